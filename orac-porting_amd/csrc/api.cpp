@@ -611,22 +611,31 @@ static int force_impl(orac_hip_ctx *ctx, const int32_t *ss_index, const double *
       p.ntypes = A.ncls;
       p.type = B.put_vec("f_atype", A.cls, st, true);
       p.alch_pair = B.put_vec("f_apair", A.pair, st, true);
+      p.lj_dense = B.put_vec("f_aljd", A.lj, st, true);
+      p.tflag = B.put_vec("f_aljflag", A.flag, st, true);
       p.alch_fac = B.put("f_afac", fac, 72, st, true);
     } else if (ma <= LJ_DENSE_MAX) {
       std::vector<double2> dense((size_t)ma * ma);
+      std::vector<unsigned char> tflag(ma, 0);
       for (int i = 0; i < ma; ++i)
         for (int j = 0; j < ma; ++j) {
           int lij = type[i + (size_t)ma * j] - 1;
           ORAC_REQUIRE(lij >= 0 && (size_t)lij < npk, E_ARG, "type table index out of range");
-          dense[(size_t)i * ma + j] = make_double2(ecc12[lij], ecc6[lij]);
+          const bool lj = ecc6[lij] > 1e-12;  // (force.f:455)
+          dense[(size_t)i * ma + j] = lj ? make_double2(ecc12[lij], ecc6[lij]) : make_double2(0.0, 0.0);
+          if (lj) tflag[i] = ATOM_LJ;
         }
+      p.tflag = B.put_vec("f_ljflag", tflag, st, true);
       p.lj_dense = B.put_vec("f_ljd", dense, st, true);
     } else {
       std::vector<int> tt((size_t)ma * ma);
+      std::vector<unsigned char> tflag(ma, 0);
       for (size_t k = 0; k < tt.size(); ++k) {
         tt[k] = type[k] - 1;
         ORAC_REQUIRE(tt[k] >= 0 && (size_t)tt[k] < npk, E_ARG, "type table index out of range");
+        if (ecc6[tt[k]] > 1e-12) tflag[k % ma] = ATOM_LJ;
       }
+      p.tflag = B.put_vec("f_ljflag", tflag, st, true);
       p.type_table = B.put_vec("f_tt", tt, st, true);
       p.ecc12 = B.put("f_e12", ecc12, npk, st, true);
       p.ecc6 = B.put("f_e6", ecc6, npk, st, true);
@@ -661,8 +670,7 @@ static int force_impl(orac_hip_ctx *ctx, const int32_t *ss_index, const double *
     p.nb_off = f_off;
     p.nb_idx = f_idx;
     for (int k = 0; k < 9; ++k) p.co[k] = co[k];
-    p.alpha = alphal;
-    p.twrtpi = 2.0 / std::sqrt(4.0 * std::atan(1.0));
+    set_ewald(p, alphal);
     p.r2inn = r2inn;
     p.r2out = r2out;
     p.rinn0 = rinn0;
@@ -673,6 +681,8 @@ static int force_impl(orac_hip_ctx *ctx, const int32_t *ss_index, const double *
     p.arsout2 = rtolout * rtolout * rtolout;
     p.arsinn1 = rinn0 - 3.0 * rinn;
     p.arsinn2 = *rtolinn * *rtolinn * *rtolinn;
+    p.inv_arsout2 = 1.0 / p.arsout2;
+    p.inv_arsinn2 = 1.0 / p.arsinn2;
     p.lskip_ewald = lskip_ewald ? 1 : 0;
     p.ewald = ewald ? 1 : 0;
     p.fx = B.get<double>("f_fx", nato);
@@ -682,8 +692,6 @@ static int force_impl(orac_hip_ctx *ctx, const int32_t *ss_index, const double *
     p.nblk = std::max(1, (ngrp + PAIR_WAVES / p.split - 1) / (PAIR_WAVES / p.split));
     p.part = B.get<double>("f_part", (size_t)p.nblk * 16);
     p.sgp = B.get<double4>("f_sgp", std::max(1, ngrp));
-    p.sgi = B.get<int4>("f_sgi", std::max(1, ngrp));
-    p.sap = B.get<double4>("f_sap", std::max(1, nato));
     p.sapc = B.get<double4>("f_sapc", std::max(1, nato));
     p.sai = B.get<int2>("f_sai", std::max(1, nato));
     p.max_group = max_group;

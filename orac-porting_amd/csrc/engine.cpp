@@ -363,15 +363,20 @@ static void system_build(orac_hip_ctx *ctx, System &S, const orac_hip_system_des
     double *d6 = ctx->B.put("ljs_e6", d.ecc6, npk, st, false);
     double2 *dense = B.get<double2>("ljd", n2);
     float2 *dense32 = d.precision == 1 ? B.get<float2>("ljd32", n2) : nullptr;
-    launch_lj_dense(ma, dtt, d12, d6, dense, dense32, st);
+    unsigned char *tflag = B.get<unsigned char>("ljflag", ((size_t)ma + 7) / 8 * 8);
+    launch_lj_dense(ma, dtt, d12, d6, dense, dense32, tflag, st);
+    p.tflag = tflag;
     p.lj_dense = dense;
     if (dense32) p.lj_dense32 = dense32;
   } else {
     std::vector<int> tt((size_t)ma * ma);
+    std::vector<unsigned char> tflag(ma, 0);
     for (size_t k = 0; k < tt.size(); ++k) {
       tt[k] = d.type_table[k] - 1;
       ORAC_REQUIRE(tt[k] >= 0 && (size_t)tt[k] < npk, E_ARG, "type table index out of range");
+      if (d.ecc6[tt[k]] > 1e-12) tflag[k % ma] = ATOM_LJ;
     }
+    p.tflag = B.put_vec("ljflag", tflag, st, false);
     p.type_table = B.put_vec("tt", tt, st, false);
     p.ecc12 = B.put("e12", d.ecc12, npk, st, false);
     p.ecc6 = B.put("e6", d.ecc6, npk, st, false);
@@ -387,8 +392,7 @@ static void system_build(orac_hip_ctx *ctx, System &S, const orac_hip_system_des
   p.any_heavy = 0;
   p.massinfty = 1.0e20;
   for (int k = 0; k < 9; ++k) p.co[k] = d.co[k];
-  p.alpha = d.alpha;
-  p.twrtpi = 2.0 / std::sqrt(4.0 * std::atan(1.0));
+  set_ewald(p, d.alpha);
   // single shell: rinn = 0, rout = rcut switched over rtol (mts_forces.f:88-93)
   const double rinn = 0.0, rout = d.rcut, rtolout = d.rtol;
   p.r2inn = 0.0;
@@ -401,6 +405,7 @@ static void system_build(orac_hip_ctx *ctx, System &S, const orac_hip_system_des
   p.arsout2 = rtolout * rtolout * rtolout;
   p.arsinn1 = 0.0;
   p.arsinn2 = 0.0;
+  p.inv_arsout2 = 1.0 / p.arsout2;
   p.lskip_ewald = 0;
   p.ewald = 1;
   p.fx = S.fx;
@@ -410,8 +415,6 @@ static void system_build(orac_hip_ctx *ctx, System &S, const orac_hip_system_des
   p.nblk = (ng + PAIR_WAVES / p.split - 1) / (PAIR_WAVES / p.split);
   p.part = B.get<double>("ppart", (size_t)p.nblk * 16);
   p.sgp = B.get<double4>("sgp", ng);
-  p.sgi = B.get<int4>("sgi", ng);
-  p.sap = B.get<double4>("sap", n);
   if (d.precision == 1) p.sapf = B.get<float4>("sapf", n);
   else p.sapc = B.get<double4>("sapc", n);
   p.sai = B.get<int2>("sai", n);
@@ -486,6 +489,7 @@ static void system_build(orac_hip_ctx *ctx, System &S, const orac_hip_system_des
     const double pairs = 0.5 * ng * (4.0 / 3.0 * M_PI * rl * rl * rl * dens);
     size_half_slots(S, (long long)(1.5 * pairs * S.max_group) + 4096);
     p.half = 1;
+    p.sgi = B.get<int4>("sgi", ng);
     p.nb_mirror = L.mirror;
     p.nb_rcount = L.rcount;
     p.nb_rbase = L.rbase;
@@ -1354,6 +1358,15 @@ extern "C" int orac_hip_system_set_alchemy(orac_hip_ctx *ctx, int32_t sys, const
     S.pair.type = B.put_vec("atype", A.cls, st, false);
     S.pair.ntypes = A.ncls;
     S.pair.alch_pair = B.put_vec("apair", A.pair, st, false);
+    S.pair.lj_dense = B.put_vec("aljd", A.lj, st, false);
+    S.pair.lj_dense32 = nullptr;
+    if (S.precision == 1) {
+      std::vector<float2> lj32(A.lj.size());
+      for (size_t k = 0; k < lj32.size(); ++k) lj32[k] = make_float2((float)A.lj[k].x, (float)A.lj[k].y);
+      S.pair.lj_dense32 = B.put_vec("aljd32", lj32, st, false);
+      ORAC_HIP(hipStreamSynchronize(st));  // (the staging vector ends here)
+    }
+    S.pair.tflag = B.put_vec("aljflag", A.flag, st, false);
     S.afac = B.get<double>("afac", 72);
     S.pair.alch_fac = S.afac;
     S.qc = B.get<double>("qc", n);
@@ -1598,6 +1611,7 @@ extern "C" int orac_hip_system_set_shells(orac_hip_ctx *ctx, int32_t sys, double
       p.r2inn0 = p.rinn0 * p.rinn0;
       p.arsinn1 = p.rinn0 - 3.0 * rcutm;
       p.arsinn2 = rtolm * rtolm * rtolm;
+      p.inv_arsinn2 = 1.0 / p.arsinn2;
       int32_t skip = 0;
       ORAC_REQUIRE(orac_hip_decide_force(rcutm, S.alpha, &skip) == 0, E_STATE, "decide_force failed");
       p.lskip_ewald = skip;
@@ -1610,6 +1624,7 @@ extern "C" int orac_hip_system_set_shells(orac_hip_ctx *ctx, int32_t sys, double
       m.r2out0 = m.rout0 * m.rout0;
       m.arsout1 = m.rout0 - 3.0 * rcutm;
       m.arsout2 = rtolm * rtolm * rtolm;
+      m.inv_arsout2 = 1.0 / m.arsout2;
       m.lskip_ewald = 0;
       if (!S.fmx) {
         S.fmx = S.B.get<double>("fmx", S.natoms);

@@ -1,12 +1,8 @@
 // force_pairs.hip -- the direct-space pair kernel (force.f:235-870) on gfx950.
 //
-// One wavefront per owner group.  Lane l serves owner atom ai = l % nI for
-// the neighbour-group slot l / nI, so a pass covers 64 / nI neighbour groups
-// (21 for a water owner) and each lane evaluates one owner atom against the
-// atoms of one neighbour group.  The neighbour list is full (both directions),
-// so every atom's force is summed by its own wavefront: no atomics, and the
-// order of every sum is fixed.  Energies are taken from the j > i direction
-// only, so each pair counts once.
+// One wavefront per owner group (k_pairs, below).  The neighbour list is full
+// (both directions), so every atom's force is summed by its own wavefront: no
+// atomics, and the order of every sum is fixed.
 //
 // Molecular virial.  force.f accumulates st += f_ab (x) (C_a - C_b - s) per pair
 // (C = molecule centre, s = the group-pair image shift) and, for switched
@@ -18,6 +14,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <string>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -35,35 +32,33 @@ namespace orac {
 // Cell-ordered copies of the step's group and atom data: sorted position t
 // holds group perm[t] (identity without a permutation) and its atoms from
 // soff[t] on.  Neighbours listed next to each other are then next to each
-// other in memory, and one group is one 32-byte and one 16-byte record.
+// other in memory, and one group is one 32-byte record.
 __global__ void __launch_bounds__(256) k_pack_sorted(const PairDesc *__restrict__ D) {
   const PairDesc &d = D[blockIdx.y];
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= d.ngrp) return;
   const int g = d.perm ? gmem(d.perm)[t] : t;
   const int f0 = gmem(d.gfirst)[g], n = gmem(d.glast)[g] - f0 + 1;
-  const int sf = d.soff ? gmem(d.soff)[t] : f0;
-  gstore(d.sgp + t, make_double4(gmem(d.xpg)[g], gmem(d.ypg)[g], gmem(d.zpg)[g], 0.0));
-  gstore(d.sgi + t, make_int4(sf, f0, n | (gmem(d.gss)[g] << 8), g));
+  const int sf = d.soff ? gmem(d.soff)[t] : f0, gss = gmem(d.gss)[g];
   const double gx = gmem(d.xpg)[g], gy = gmem(d.ypg)[g], gz = gmem(d.zpg)[g];
+  const int w[2] = {sf, n | (gss << 8)};
+  double4 gp = make_double4(gx, gy, gz, 0.0);
+  __builtin_memcpy(&gp.w, w, 8);
+  gstore(d.sgp + t, gp);
+  if (d.half) gstore(d.sgi + t, make_int4(sf, f0, n | (gss << 8), g));
   for (int k = 0; k < n; ++k) {
     const int a = f0 + k;
-    const double x = gmem(d.xp)[a], y = gmem(d.yp)[a], z = gmem(d.zp)[a], q = gmem(d.q)[a];
-    gstore(d.sap + sf + k, make_double4(x, y, z, q));
-    gstore(d.sai + sf + k, make_int2(gmem(d.type)[a], gmem(d.ex_inter)[a] ? 1 : 0));
-    if (d.sapc) {
-      // FP64 Cartesian offset from the group centre (upper triangle of co, as force.f)
-      const double dx = x - gx, dy = y - gy, dz = z - gz;
-      gstore(d.sapc + sf + k, make_double4(d.co[0] * dx + d.co[3] * dy + d.co[6] * dz, d.co[4] * dy + d.co[7] * dz,
-                                           d.co[8] * dz, q));
-    }
-    if (d.sapf) {
-      // Cartesian offset from the group centre: a pair's separation is the
-      // group separation (FP64) plus the difference of two small offsets
-      const double dx = x - gx, dy = y - gy, dz = z - gz;
-      gstore(d.sapf + sf + k, make_float4((float)(d.co[0] * dx + d.co[3] * dy + d.co[6] * dz),
-                                          (float)(d.co[4] * dy + d.co[7] * dz), (float)(d.co[8] * dz), (float)q));
-    }
+    const double q = gmem(d.q)[a];
+    // Cartesian offset from the group centre (upper triangle of co, as
+    // force.f): a pair's separation is the group separation plus the
+    // difference of two small offsets
+    const double dx = gmem(d.xp)[a] - gx, dy = gmem(d.yp)[a] - gy, dz = gmem(d.zp)[a] - gz;
+    const double cx = d.co[0] * dx + d.co[3] * dy + d.co[6] * dz, cy = d.co[4] * dy + d.co[7] * dz, cz = d.co[8] * dz;
+    const int ty = gmem(d.type)[a];
+    const int fl = (gmem(d.ex_inter)[a] ? ATOM_EX : 0) | gmem(d.tflag)[ty] | (d.rematom && gmem(d.rematom)[a] ? ATOM_REM : 0);
+    gstore(d.sai + sf + k, make_int2(ty << ATOM_FLAG_BITS | fl, a));
+    if (d.sapc) gstore(d.sapc + sf + k, make_double4(cx, cy, cz, q));
+    if (d.sapf) gstore(d.sapf + sf + k, make_float4((float)cx, (float)cy, (float)cz, (float)q));
   }
 }
 
@@ -88,8 +83,8 @@ __device__ inline bool is_excluded(P ex_off, P ex_idx, int a, int b) {
 // Newton-Raphson step each (~1e-14 relative; the reference's 1/sqrt and
 // divides are correctly rounded, and the difference stays far below the
 // force tolerance) for a fraction of the instructions of an IEEE divide and
-// square root, and exp by a two-constant ln 2 reduction and a degree-10
-// Taylor series (~3e-13 relative) in place of the libm routine.  FP32
+// square root, and the exponential by a polynomial (pair_exp2) in place of
+// the libm routine.  FP32
 // (mixed precision): the hardware reciprocal, reciprocal square root and
 // exponential, 1-2 ulp each.  Pair distances are positive and finite, so no
 // special cases arise.
@@ -111,51 +106,62 @@ __device__ inline double pair_rcp<double>(double x) {
 }
 template <>
 __device__ inline float pair_rcp<float>(float x) { return __builtin_amdgcn_rcpf(x); }
+// a * b + c with c in a scalar register pair: the three-operand form, which
+// leaves the polynomials' constants out of the vector registers (the compiler
+// copies each constant to a fresh pair and accumulates into that)
+__device__ __forceinline__ double fma_const(double a, double b, double c) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+  return d;
+}
+// 2^y for the Ewald factor exp(-(alpha r)^2) = 2^(-alpha^2 log2(e) r^2), from
+// the squared distance, beside the reciprocal square root rather than after
+// it.  y = n + f, |f| <= 1/2 (exact), and 2^f = 1 + f q(f) with q of degree 8
+// interpolating (2^f - 1) / f at the Chebyshev nodes (3.7e-14 relative).
 template <typename T>
-__device__ inline T pair_exp(T x);
-// exp(x) for the Ewald factor exp(-(alpha r)^2) (x <= 0, modest): x = n ln2 +
-// r, |r| <= ln2 / 2 (ln 2 split in two constants, the reduction by FMA), e^r
-// by its Taylor series to degree 10 (truncation below 3e-13), scaled by 2^n
+__device__ inline T pair_exp2(T y);
 template <>
-__device__ inline double pair_exp<double>(double x) {
-  const double n = __builtin_rint(x * 1.4426950408889634);
-  double r = fma(-n, 0.6931471805599453, x);
-  r = fma(-n, 2.3190468138462996e-17, r);
-  double p = 2.755731922398589e-07;
-  p = fma(p, r, 2.7557319223985893e-06);
-  p = fma(p, r, 2.48015873015873e-05);
-  p = fma(p, r, 0.0001984126984126984);
-  p = fma(p, r, 0.001388888888888889);
-  p = fma(p, r, 0.008333333333333333);
-  p = fma(p, r, 0.041666666666666664);
-  p = fma(p, r, 0.16666666666666666);
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.0);
-  p = fma(p, r, 1.0);
+__device__ inline double pair_exp2<double>(double y) {
+  const double n = __builtin_rint(y), f = y - n;
+  double p = fma_const(f, 1.0203121047189341e-07, 1.3255224879317324e-06);
+  p = fma_const(p, f, 1.525268684635191e-05);
+  p = fma_const(p, f, 0.0001540345585244999);
+  p = fma_const(p, f, 0.0013333558179042969);
+  p = fma_const(p, f, 0.009618129159402565);
+  p = fma_const(p, f, 0.055504108664760424);
+  p = fma_const(p, f, 0.2402265069581299);
+  p = fma_const(p, f, 0.6931471805599453);
+  p = fma(p, f, 1.0);
   return __builtin_amdgcn_ldexp(p, (int)n);
 }
 template <>
-__device__ inline float pair_exp<float>(float x) { return __expf(x); }
+__device__ inline float pair_exp2<float>(float y) { return __builtin_amdgcn_exp2f(y); }
 
-// The pair (a, b) is masked: excluded (the symmetric exclusion list), or
-// both atoms at or above massinfty (force.f:488-489).  For the reverse
-// direction the owner group must first hold one of b's partners.
-__device__ __noinline__ bool pair_masked(const PairDesc &d, int a, int b, int ia0, int nI, bool fwd) {
-  if (!fwd && !has_partner_in(gmem(d.ex_off), gmem(d.ex_idx), b, ia0, ia0 + nI - 1)) return false;
-  if (is_excluded(gmem(d.ex_off), gmem(d.ex_idx), a, b)) return true;
-  return d.any_heavy && !(gmem(d.mass)[b] < d.massinfty || gmem(d.mass)[a] < d.massinfty);
+// The A&S 7.1.26 polynomial of erfc at qt = 1 / (1 + p x), without its exponential
+template <typename T>
+__device__ __forceinline__ T erfc_poly(T qt) {
+  if constexpr (sizeof(T) == 8) {
+    double p = fma_const(qt, AS_A5, AS_A4);
+    p = fma_const(p, qt, AS_A3);
+    p = fma_const(p, qt, AS_A2);
+    p = fma_const(p, qt, AS_A1);
+    return p * qt;
+  } else {
+    return ((((T(AS_A5) * qt + T(AS_A4)) * qt + T(AS_A3)) * qt + T(AS_A2)) * qt + T(AS_A1)) * qt;
+  }
 }
 
-__device__ inline void lj_params(const PairDesc &d, int ti, int tj, double &c12, double &c6) {
-  if (d.lj_dense) {
-    double2 v = gload_at(d.lj_dense, ti * d.ntypes + tj);
-    c12 = v.x;
-    c6 = v.y;
-  } else {
-    int lij = gmem(d.type_table)[ti + (size_t)d.ntypes * tj];
-    c12 = gmem(d.ecc12)[lij];
-    c6 = gmem(d.ecc6)[lij];
-  }
+// force.f:486-490: two atoms at or above massinfty are skipped only where the
+// list owner's atom has an exclusion partner in the other group (the owner is
+// the lower group).  a: the owner atom (flags fa) of the group at sorted
+// position t, atoms ia0 .. ia0 + nI - 1; ib: the neighbour atom's record.
+__device__ __noinline__ bool heavy_masked(const PairDesc &d, int a, int fa, int t, int ia0, int nI, int2 ib, int tj) {
+  const int b = ib.y;
+  if (gmem(d.mass)[b] < d.massinfty || gmem(d.mass)[a] < d.massinfty) return false;
+  const int g = d.perm ? gmem(d.perm)[t] : t, j = d.perm ? gmem(d.perm)[tj] : tj;
+  if (j > g)
+    return (fa & ATOM_EX) && has_partner_in(gmem(d.ex_off), gmem(d.ex_idx), a, gmem(d.gfirst)[j], gmem(d.glast)[j]);
+  return (ib.x & ATOM_EX) && has_partner_in(gmem(d.ex_off), gmem(d.ex_idx), b, ia0, ia0 + nI - 1);
 }
 
 // Group-pair geometry (force.f:265-292): the image shift s (even integers in
@@ -168,12 +174,17 @@ __device__ __forceinline__ GroupGeom group_geom(double xpgi, double ypgi, double
 #pragma clang fp contract(off)
   GroupGeom g;
   double xgg = xpgi - gpj.x, ygg = ypgi - gpj.y, zgg = zpgi - gpj.z;
-  g.sxm = 2.0 * fnint(0.5 * xgg);
-  g.sym = 2.0 * fnint(0.5 * ygg);
-  g.szm = 2.0 * fnint(0.5 * zgg);
-  xgg = xgg - g.sxm;
-  ygg = ygg - g.sym;
-  zgg = zgg - g.szm;
+  g.sxm = g.sym = g.szm = 0.0;
+  // dnint(d / 2) is zero below |d| = 1: a wavefront without a larger
+  // difference (an owner away from the cell's faces) skips the rounding
+  if (__ballot(!(fmax(fmax(fabs(xgg), fabs(ygg)), fabs(zgg)) < 1.0))) {
+    g.sxm = 2.0 * fnint(0.5 * xgg);
+    g.sym = 2.0 * fnint(0.5 * ygg);
+    g.szm = 2.0 * fnint(0.5 * zgg);
+    xgg = xgg - g.sxm;
+    ygg = ygg - g.sym;
+    zgg = zgg - g.szm;
+  }
   g.xcc = co[0] * xgg + co[3] * ygg + co[6] * zgg;
   g.ycc = co[4] * ygg + co[7] * zgg;
   g.zcc = co[8] * zgg;
@@ -181,73 +192,30 @@ __device__ __forceinline__ GroupGeom group_geom(double xpgi, double ypgi, double
   return g;
 }
 
-// the group pair is inside the shell: normal [rinn0, rout) or switched
-// [rout, rout0) and [rinn, rinn0) (force.f:293-335)
-__device__ __forceinline__ bool in_shell(const PairDesc &d, double drj) {
-  return (drj >= d.r2inn0 && drj < d.r2out) || (drj >= d.r2out && drj < d.r2out0) ||
-         (drj >= d.r2inn && drj < d.r2inn0);
-}
+// The group pair is inside the shell: normal [rinn0, rout) or switched
+// [rout, rout0) and [rinn, rinn0) (force.f:293-335), one interval since
+// rinn <= rinn0 < rout <= rout0 (force.f:166 computes nothing otherwise).
+__device__ __forceinline__ bool in_shell(const PairDesc &d, double drj) { return drj >= d.r2inn && drj < d.r2out0; }
 
-// One atom pair of a group pair (force.f:420-560): the LJ term when the pair
-// has one (c6 > 1e-12), the A&S erfc Ewald term or plain Coulomb, as the
-// scalar force factor qf (force = qf * r), the separation and the two energies.
-struct PairTerms {
-  double qf, xc, yc, zc, conf, cou;
-  __device__ __forceinline__ void add(double &uconf, double &ucoul, double &fx, double &fy, double &fz) const {
-    uconf += conf;
-    ucoul += cou;
-    fx += qf * xc;
-    fy += qf * yc;
-    fz += qf * zc;
+// LJ {c12, c6} of the type pair (ti, tj), zero when c6 <= 1e-12 (the pair then
+// has no LJ term, force.f:455; the dense tables hold such entries as zeros)
+template <typename T, bool DENSE = false>
+__device__ __forceinline__ void pair_lj(const PairDesc &d, int ti, int tj, T &c12, T &c6) {
+  if (sizeof(T) == 4 && (DENSE || d.lj_dense32)) {
+    const float2 v = gload_at(d.lj_dense32 + (size_t)ti * d.ntypes, tj);
+    c12 = T(v.x);
+    c6 = T(v.y);
+  } else if (DENSE || d.lj_dense) {
+    const double2 v = gload_at(d.lj_dense + (size_t)ti * d.ntypes, tj);
+    c12 = T(v.x);
+    c6 = T(v.y);
+  } else {
+    const int lij = gmem(d.type_table)[ti + (size_t)d.ntypes * tj];
+    const double a = gmem(d.ecc12)[lij], b = gmem(d.ecc6)[lij];
+    const bool lj = b > 1e-12;
+    c12 = lj ? T(a) : T(0);
+    c6 = lj ? T(b) : T(0);
   }
-};
-
-// The pair at Cartesian separation (xc, yc, zc) with charge product qq.
-template <typename T>
-__device__ __forceinline__ PairTerms pair_terms_c(const PairDesc &d, T xc, T yc, T zc, T qq, double c12, double c6);
-
-template <typename T>
-__device__ __forceinline__ PairTerms pair_terms(const PairDesc &d, double pxs, double pys, double pzs, double qa,
-                                                const double *co, const double4 &pb4, double c12, double c6) {
-  const double xg = pxs - pb4.x, yg = pys - pb4.y, zg = pzs - pb4.z;
-  return pair_terms_c<T>(d, T(co[0] * xg + co[3] * yg + co[6] * zg), T(co[4] * yg + co[7] * zg), T(co[8] * zg),
-                         T(qa * pb4.w), c12, c6);
-}
-
-template <typename T>
-__device__ __forceinline__ PairTerms pair_terms_c(const PairDesc &d, T xc, T yc, T zc, T qq, double c12, double c6) {
-  const T rsq = xc * xc + yc * yc + zc * zc;
-  const T rinv = pair_rsqrt<T>(rsq);
-  const T rsqi = rinv * rinv;
-  // LJ by predication: a pair without LJ takes zero parameters
-  const bool lj = c6 > 1e-12;
-  const T c12t = lj ? T(c12) : T(0), c6t = lj ? T(c6) : T(0);
-  const T c12f = lj ? T(12.0 * c12) : T(0), c6f = lj ? T(6.0 * c6) : T(0);
-  const T r6 = rsqi * rsqi * rsqi, r12 = r6 * r6;
-  T qforce = (c12f * r12 - c6f * r6) * rsqi;
-  PairTerms r;
-  r.conf = lj ? (double)(c12t * r12 - c6t * r6) : 0.0;
-  r.cou = 0.0;
-  if (!d.lskip_ewald) {
-    const T rsp = rsq * rinv;
-    const T rspqi = rsqi * rinv;
-    const T alphar = T(d.alpha) * rsp;
-    const T qt = pair_rcp<T>(T(1) + T(AS_QP) * alphar);
-    const T expcst = pair_exp<T>(-(alphar * alphar));
-    const T erfcst = ((((T(AS_A5) * qt + T(AS_A4)) * qt + T(AS_A3)) * qt + T(AS_A2)) * qt + T(AS_A1)) * qt * expcst;
-    const T furpar = qq;
-    r.cou = (double)(furpar * erfcst * rinv);
-    qforce += furpar * (erfcst + T(d.twrtpi) * alphar * expcst) * rspqi;
-  } else if (!d.ewald) {
-    const T ssv = qq * rinv;
-    r.cou = (double)ssv;
-    qforce += ssv * rsqi;
-  }
-  r.qf = (double)qforce;
-  r.xc = (double)xc;
-  r.yc = (double)yc;
-  r.zc = (double)zc;
-  return r;
 }
 
 // One atom pair in soft-core form (force_alchemy.f:439-523): F = the pair's
@@ -256,31 +224,18 @@ __device__ __forceinline__ PairTerms pair_terms_c(const PairDesc &d, T xc, T yc,
 // Coulomb q_a q_b fq2 erfc(alpha r) / sqrt(qsoft fq1^2 + r^2) (or without
 // erfc, plain); the energies at lambda0 come from the same distances with
 // the lambda0 factors.  dw = U(lambda) - U(lambda0) of the pair.
+template <typename T>
 struct AlchTerms {
-  double qf, xc, yc, zc, conf, cou, dw;
-  __device__ __forceinline__ void add(double &uconf, double &ucoul, double &dwa, double &fx, double &fy,
-                                      double &fz) const {
-    uconf += conf;
-    ucoul += cou;
-    dwa += dw;
-    fx += qf * xc;
-    fy += qf * yc;
-    fz += qf * zc;
-  }
+  T qf, conf, cou;
+  double dw;
 };
 
 template <typename T>
-__device__ __forceinline__ AlchTerms alch_terms(const PairDesc &d, double pxs, double pys, double pzs, double qa,
-                                                const double *co, const double4 &pb4, const double4 &ap,
-                                                const double *F) {
-  const double xg = pxs - pb4.x, yg = pys - pb4.y, zg = pzs - pb4.z;
-  const T xc = T(co[0] * xg + co[3] * yg + co[6] * zg);
-  const T yc = T(co[4] * yg + co[7] * zg);
-  const T zc = T(co[8] * zg);
+__device__ __forceinline__ AlchTerms<T> alch_terms(const PairDesc &d, T xc, T yc, T zc, T qq, const double4 &ap,
+                                                   const double *F) {
   const T rsq = xc * xc + yc * yc + zc * zc;
   const T rinv = pair_rsqrt<T>(rsq);
   T qforce = T(0), conf = T(0), conf0 = T(0), cou = T(0), cou0 = T(0);
-  const T qq = T(qa * pb4.w);
   if (d.alch_shifted) {
     // force_alchemy_shifted.f:469-509: LJ at r + ljshift 2^(1/6) sigma f1, Coulomb over
     // r + qshift fq1 (erfc of the real distance)
@@ -298,7 +253,7 @@ __device__ __forceinline__ AlchTerms alch_terms(const PairDesc &d, double pxs, d
     if (!d.lskip_ewald) {
       const T alphar = T(d.alpha) * r;
       const T qt = pair_rcp<T>(T(1) + T(AS_QP) * alphar);
-      const T expcst = pair_exp<T>(-(alphar * alphar));
+      const T expcst = pair_exp2<T>(T(d.ew_exp2) * rsq);
       const T erfcst = ((((T(AS_A5) * qt + T(AS_A4)) * qt + T(AS_A3)) * qt + T(AS_A2)) * qt + T(AS_A1)) * qt * expcst;
       const T furpar = T(F[5]) * qq;
       cou = furpar * erfcst * irq;
@@ -325,7 +280,7 @@ __device__ __forceinline__ AlchTerms alch_terms(const PairDesc &d, double pxs, d
     if (!d.lskip_ewald) {
       const T alphar = T(d.alpha) * (rsq * rinv);
       const T qt = pair_rcp<T>(T(1) + T(AS_QP) * alphar);
-      const T expcst = pair_exp<T>(-(alphar * alphar));
+      const T expcst = pair_exp2<T>(T(d.ew_exp2) * rsq);
       const T erfcst = ((((T(AS_A5) * qt + T(AS_A4)) * qt + T(AS_A3)) * qt + T(AS_A2)) * qt + T(AS_A1)) * qt * expcst;
       const T furpar = T(F[5]) * qq, furpar0 = T(F[7]) * qq;
       cou = furpar * erfcst * auxaa;
@@ -337,296 +292,546 @@ __device__ __forceinline__ AlchTerms alch_terms(const PairDesc &d, double pxs, d
       qforce += cou * (auxaa * auxaa);
     }
   }
-  AlchTerms r;
-  r.qf = (double)qforce;
-  r.xc = (double)xc;
-  r.yc = (double)yc;
-  r.zc = (double)zc;
-  r.conf = (double)conf;
-  r.cou = (double)cou;
+  AlchTerms<T> r;
+  r.qf = qforce;
+  r.conf = conf;
+  r.cou = cou;
   r.dw = (double)(conf - conf0) + (double)(cou - cou0);
   return r;
 }
 
-constexpr int PAIR_NACC = 16;      // per-lane sums: uconf[3], ucoul[3], st[9], dwrk
+constexpr int PAIR_NACC = 16;      // energies and virial of a block: uconf[3], ucoul[3], st[9], dwrk
+
+// ================================================================ k_pairs
+//
+// The lanes of a wavefront take the atoms of the owner's in-shell neighbour
+// groups, one atom each, and loop over the owner group's atoms, whose records
+// are the same across the wavefront and sit in SGPRs: a pair costs three
+// additions before its distance and reads no memory but its LJ entry, and a
+// neighbour atom's record is read once for all owner atoms.  The list entries
+// are classified 64 at a time; a kept entry's Cartesian group separation,
+// image shift and switch are computed once and kept in a small LDS ring, and
+// its atoms are appended to a ring of lane slots, from which passes of 64 are
+// taken, so that every lane of a pass has an atom (the last pass aside),
+// whatever the sizes of the groups.
+//
+// Bound by VALU issue (about 60 FP64 instructions and two quarter-rate seeds
+// per pair, no matrix instruction fits a scalar function of each distance).
+// What keeps the count down:
+//  * an owner atom whose LJ row is empty (water hydrogens) skips the LJ gather
+//    and arithmetic, a wave-uniform branch;
+//  * the S'(r) V term of switched group pairs is linear in V, so each lane
+//    adds its own share -S'(r)/r v (C_i - C_j) and no lane needs the group
+//    pair's total;
+//  * the list is full, so every pair is seen from both sides: energies and
+//    image-shift virial are summed over both and halved, with no test which
+//    side counts;
+//  * exclusions of an owner atom are walked as a wave-uniform loop;
+//  * the 64-lane sums go through LDS eight values at a time (8 writes, 8 reads
+//    per lane and three exchanges for eight sums).
+// Measured on the 24,460-atom system (11.9 M pair evaluations from both sides):
+// 86 us in FP64 and 79 us in FP32, against 182 and 151 us with lanes on (owner
+// atom, neighbour group) that recomputed the group geometry per lane; 26 M
+// vector instructions against 43 M.  16 systems in one launch: 56 us each (FP32).
+
+constexpr int OWN_U = 3;        // owner atoms whose sums stay in registers during a list walk
+constexpr int ENT_RING = 128;   // entries kept: at most 63 with atoms waiting + 64 new ones
+constexpr int SLOT_RING = 256;  // lane slots: at most 63 waiting + one round's atoms
+constexpr int RED_STRIDE = 72;  // 8 rows of 64 values, rows 16 banks apart
+
+struct PairWave {
+  double gx[ENT_RING], gy[ENT_RING], gz[ENT_RING];  // centre separation, image applied (T = float: {hi, lo} floats)
+  double sw[ENT_RING], dsw[ENT_RING];               // S and S'(r) / r of the group distance (1 and 0 unswitched)
+  int sx[ENT_RING], sy[ENT_RING], sz[ENT_RING];     // image shift (even integers, reduced units)
+  int bs[ENT_RING];                                 // sorted first atom | solute neighbour << 26 | shifted << 27
+  int tj[ENT_RING];                                 // neighbour group, sorted position
+  unsigned short slot[SLOT_RING];                   // entry | atom within the group << 7
+  double4 own[OWN_U];                               // the owner atoms' records (T = float: four floats)
+};
+static_assert(sizeof(PairWave) >= 8 * RED_STRIDE * sizeof(double), "the lane sums reuse the ring");
 
 struct PairShared {
-  double red[PAIR_WAVES][PAIR_NACC];
-  double facc[PAIR_WAVES][64][3];
-  double acc[PAIR_WAVES][PAIR_NACC][64];  // per-lane energy and virial sums (lane-private slots)
-  double alch[9][8];                      // the system's soft-core factors (alchemical kernels)
+  PairWave w[PAIR_WAVES];
+  double fsum[PAIR_WAVES][64][3];          // owner-atom forces of a wave's part of the list
+  double red[PAIR_WAVES][3 + PAIR_NACC];   // S'V vector, then energies and virial
+  double alch[9][8];                       // the system's soft-core factors (alchemical kernels)
 };
 
-// One work item: block blk of system d (PAIR_WAVES owner groups).  ALCH:
-// the kernel also takes the soft-core form for systems that carry alch_pair.
-template <typename T, bool ALCH>
+// A wave-uniform value the compiler must take anew here: tests of it stay at
+// their place instead of being held in (and spilled from) scalar registers
+// across the whole list walk.
+__device__ __forceinline__ int here(int v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
+// A wave's LDS writes above are read by its other lanes below.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ int lanes_below(unsigned long long m) {
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
+__device__ __forceinline__ double uniform(double v) {
+  int w[2];
+  __builtin_memcpy(w, &v, 8);
+  w[0] = __builtin_amdgcn_readfirstlane(w[0]);
+  w[1] = __builtin_amdgcn_readfirstlane(w[1]);
+  __builtin_memcpy(&v, w, 8);
+  return v;
+}
+__device__ __forceinline__ float uniform(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Sums of eight values over the 64 lanes; lane l returns the sum of v[l >> 3].
+// Fixed order: lane l adds the eight lanes = l mod 8, then lanes 1, 2, 4 apart.
+__device__ __forceinline__ double wave_sum8(const double *v, double *buf, int lane) {
+  wave_lds_sync();
+#pragma unroll
+  for (int k = 0; k < 8; ++k) buf[k * RED_STRIDE + lane] = v[k];
+  wave_lds_sync();
+  const double *row = buf + (lane >> 3) * RED_STRIDE + (lane & 7);
+  double s = row[0];
+#pragma unroll
+  for (int k = 1; k < 8; ++k) s += row[8 * k];
+  s += __shfl_xor(s, 1, 64);
+  s += __shfl_xor(s, 2, 64);
+  s += __shfl_xor(s, 4, 64);
+  return s;
+}
+
+// An atom's Cartesian offset from its group centre and its charge, in the pair precision.
+template <typename T>
+struct AtomRec {
+  T x, y, z, q;
+};
+template <typename T>
+__device__ __forceinline__ AtomRec<T> atom_rec(const PairDesc &d, int s) {
+  if constexpr (sizeof(T) == 4) {
+    const float4 v = gload_at(d.sapf, s);
+    return {v.x, v.y, v.z, v.w};
+  } else {
+    const double4 v = gload_at(d.sapc, s);
+    return {v.x, v.y, v.z, v.w};
+  }
+}
+
+// The pair forms of a kernel: plain (every system with the Ewald term, a dense
+// LJ table and no atom at massinfty: what a simulation runs), soft core
+// (alchemical systems), REM segment scaling, and plain without those limits
+// (an outer shell that skips the Ewald term, more than LJ_DENSE_MAX types).
+enum { PAIR_PLAIN = 0, PAIR_ALCH = 1, PAIR_REM = 2, PAIR_ANY = 3 };
+
+// One work item: block blk of system d (PAIR_WAVES waves, split of them per owner group).
+template <typename T, int MODE>
 __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShared &sh) {
   if (blk >= d.nblk || d.half) return;
-  double(&red)[PAIR_WAVES][PAIR_NACC] = sh.red;
-  double(&facc)[PAIR_WAVES][64][3] = sh.facc;
-  double(&acc)[PAIR_WAVES][PAIR_NACC][64] = sh.acc;
-  const bool alch = ALCH && d.alch_pair != nullptr;
-  if (alch) {
-    if (threadIdx.x < 72) sh.alch[threadIdx.x >> 3][threadIdx.x & 7] = gmem(d.alch_fac)[threadIdx.x];
+  constexpr bool F32 = sizeof(T) == 4;
+  constexpr bool DW = MODE == PAIR_ALCH || MODE == PAIR_REM;  // a 16th sum: dwrk or the segment energy
+  const bool alch = MODE == PAIR_ALCH && d.alch_pair != nullptr;
+  if (MODE == PAIR_ALCH) {
+    if (alch && threadIdx.x < 72) sh.alch[threadIdx.x >> 3][threadIdx.x & 7] = gmem(d.alch_fac)[threadIdx.x];
     __syncthreads();
   }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  // (wave-uniform for the compiler too: the loop control then stays in scalar registers)
+  const int lane = threadIdx.x & 63, wid = uniform((int)(threadIdx.x >> 6));
   // S waves share one owner group, each taking a contiguous part of its list
   const int S = d.split, part = wid % S;
-  const int t = blk * (PAIR_WAVES / S) + wid / S;  // owner group, sorted position
-  double fxa = 0.0, fya = 0.0, fza = 0.0;
-  double *en = &acc[wid][0][0];  // en[k * 64 + lane]: uconf[typeij], ucoul[typeij]
-  double *st = &acc[wid][6][0];  // st[k * 64 + lane]
+  const int t = uniform(blk * (PAIR_WAVES / S) + wid / S);  // owner group, sorted position
+  PairWave &W = sh.w[wid];
+  double *buf = reinterpret_cast<double *>(&W);
+  double x3[3] = {0.0, 0.0, 0.0};                 // S'(r) V vectors of the switched group pairs
+  double ec[2] = {0.0, 0.0}, eq[2] = {0.0, 0.0};  // LJ and Coulomb energy by the neighbour's class
+  double st[9], dwl = 0.0;
 #pragma unroll
-  for (int k = 0; k < PAIR_NACC; ++k) acc[wid][k][lane] = 0.0;
-  int ia0 = 0, nI = 1, nslot = 64;  // ia0: owner's first atom, original numbering
+  for (int k = 0; k < 9; ++k) st[k] = 0.0;
+  bool any_st = false;                            // wave-uniform
+  int ia0 = 0, nI = 0, typei = 1;
   if (t < d.ngrp) {
-    const int4 gi = gload(d.sgi + t);
-    const int g = gi.w;
-    ia0 = gi.y;
-    nI = gi.z & 255;
-    nslot = 64 / nI;
-    const int slot = lane / nI, ai = lane - slot * nI;
-    const bool active = slot < nslot;
-    const int a = ia0 + (active ? ai : 0);        // original index
-    const int as = gi.x + (active ? ai : 0);      // sorted index
-    const double4 pa4 = gload(d.sap + as);
-    const int2 ia4 = gload(d.sai + as);
-    // mixed precision reads compact FP32 records (the soft-core form keeps the FP64 ones)
-    constexpr bool FREC = sizeof(T) == 4;
-    const float4 paf = (FREC && !alch) ? gload(d.sapf + as) : make_float4(0.f, 0.f, 0.f, 0.f);
-    const double ma = gmem(d.gmass)[a];
-    const int typei = gi.z >> 8;
     const double4 gpi = gload(d.sgp + t);
-    const double xpgi = gpi.x, ypgi = gpi.y, zpgi = gpi.z;
-    double co[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) co[k] = d.co[k];
-    const double co0 = co[0], co3 = co[3], co6 = co[6], co4 = co[4], co7 = co[7], co8 = co[8];
+    const double xpgi = uniform(gpi.x), ypgi = uniform(gpi.y), zpgi = uniform(gpi.z);
+    int gw[2];
+    __builtin_memcpy(gw, &gpi.w, 8);
+    const int as0 = uniform(gw[0]);
+    nI = uniform(gw[1] & 255);
+    typei = uniform(gw[1] >> 8);
+    ia0 = uniform(gload_at(d.sai, as0).y);
     int nb0, nb1;
     if (d.nb_slab > 0) {
       nb0 = t * d.nb_slab;
-      nb1 = nb0 + min(gmem(d.nb_cnt)[t], d.nb_slab);
+      nb1 = nb0 + min(uniform(gmem(d.nb_cnt)[t]), d.nb_slab);
     } else {
-      nb0 = gmem(d.nb_off)[t];
-      nb1 = gmem(d.nb_off)[t + 1];
+      nb0 = uniform(gmem(d.nb_off)[t]);
+      nb1 = uniform(gmem(d.nb_off)[t + 1]);
     }
     if (S > 1) {
       const int len = nb1 - nb0;
       nb1 = nb0 + (len * (part + 1)) / S;
       nb0 = nb0 + (len * part) / S;
     }
-    // The list reaches rc + rtol + rnei; only groups inside the shell do work.
-    // Entries are classified 64 at a time and the survivors compacted, in list
-    // order, into this wave's part of facc (unused until the force reduction),
-    // so every slot of the pair loop is busy.
-    int *cbuf = reinterpret_cast<int *>(&facc[wid][0][0]);
-    constexpr int CBUF = (int)(sizeof(facc[0]) / sizeof(int));
-    for (int c0 = nb0; c0 < nb1;) {
-      int nc = 0;
-      for (; c0 < nb1 && nc <= CBUF - 64; c0 += 64) {
-        const int jj = c0 + lane;
-        const bool in = jj < nb1;
-        const int tj = in ? gmem(d.nb_idx)[jj] : t;
-        const GroupGeom gg = group_geom(xpgi, ypgi, zpgi, gload_at(d.sgp, tj), co);
-        const bool keep = in && in_shell(d, gg.drj);
-        const unsigned long long m = __ballot(keep);
-        if (keep) cbuf[nc + __popcll(m & ((1ull << lane) - 1ull))] = tj;
-        nc += __popcll(m);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      for (int base = 0; base < nc; base += nslot) {
-        const int jj = base + slot;
-        const bool have = active && jj < nc;
-        const int tj = have ? cbuf[jj] : t;
-        const double4 gpj = gload_at(d.sgp, tj);
-        const int4 gij = gload_at(d.sgi, tj);
-        const int j = gij.w;
-        const GroupGeom gg = group_geom(xpgi, ypgi, zpgi, gpj, co);
-        const double sxm = gg.sxm, sym = gg.sym, szm = gg.szm, xcc = gg.xcc, ycc = gg.ycc, zcc = gg.zcc,
-                     drj = gg.drj;
-        int cls = 0;  // 0 none, 1 normal, 2 switched
-        double sw = 1.0, dsw = 0.0;
-        if (have) {
-          if (drj >= d.r2inn0 && drj < d.r2out) {
-            cls = 1;
-          } else if (drj >= d.r2out && drj < d.r2out0) {
-            cls = 2;
-            double rsp = sqrt(drj);
-            double auxa = (d.arsout1 + 2.0 * rsp) / d.arsout2;
-            double auxb = d.rout0 - rsp;
-            sw = auxa * (auxb * auxb);
-            dsw = (-(2.0 * auxa * auxb) + 2.0 * (auxb * auxb) / d.arsout2) / rsp;
-          } else if (drj >= d.r2inn && drj < d.r2inn0) {
-            cls = 2;
-            double rsp = sqrt(drj);
-            double auxa = (d.arsinn1 + 2.0 * rsp) / d.arsinn2;
-            double auxb = d.rinn0 - rsp;
-            sw = 1.0 - auxa * (auxb * auxb);
-            dsw = (2.0 * auxa * auxb - 2.0 * (auxb * auxb) / d.arsinn2) / rsp;
-          }
+    // entries per classification round: all of a round's atoms fit the slots beside 63 waiting ones
+    const int mg = d.max_group;
+    const int per_round = min(64, (SLOT_RING - 63) / mg);
+    const bool lskip = (MODE == PAIR_ALCH || MODE == PAIR_ANY) && d.lskip_ewald != 0, plainq = !d.ewald;
+    const double inv_o2 = d.inv_arsout2, inv_i2 = d.inv_arsinn2;
+    for (int u0 = 0; u0 < nI; u0 += OWN_U) {
+      const int nu = min(OWN_U, nI - u0);
+      int ot[OWN_U];  // type << ATOM_FLAG_BITS | flags
+      int xn[OWN_U], xv[OWN_U];
+      double fr[OWN_U][3];
+#pragma unroll
+      for (int u = 0; u < OWN_U; ++u) {
+        const int a = as0 + u0 + min(u, nu - 1);
+        const AtomRec<T> r = atom_rec<T>(d, a);
+        if (lane == 0) __builtin_memcpy(&W.own[u], &r, sizeof r);
+        ot[u] = uniform(gload_at(d.sai, a).x);
+        fr[u][0] = fr[u][1] = fr[u][2] = 0.0;
+        // an atom with exclusions outside its group: the first 64, one a lane
+        xn[u] = 0;
+        xv[u] = -1;
+        if (ot[u] & ATOM_EX) {
+          const int x0 = uniform(gmem(d.ex_off)[ia0 + u0 + min(u, nu - 1)]);
+          xn[u] = uniform(gmem(d.ex_off)[ia0 + u0 + min(u, nu - 1) + 1]) - x0;
+          if (lane < xn[u]) xv[u] = gmem(d.ex_idx)[x0 + lane];
         }
-        const bool fwd = j > g;
-        const bool shifted = sxm != 0.0 || sym != 0.0 || szm != 0.0;
-        double cm = 0.0;                      // this lane's part of V (switched pairs)
-        double fgx = 0.0, fgy = 0.0, fgz = 0.0;  // this lane's pair forces for the group pair
-        if (cls != 0) {
-          const int nJ = gij.z & 255;
-          const int jb0 = gij.y, jb1 = jb0 + nJ - 1, jbs = gij.x;  // original range, sorted start
-          const int typeij = typei + (gij.z >> 8) - 2;  // 0..2
-          const bool mask_a = fwd && (ia4.y & 1) && has_partner_in(gmem(d.ex_off), gmem(d.ex_idx), a, jb0, jb1);
-          // owner position minus the image shift: one association for every class
-          const double pxs = pa4.x - sxm, pys = pa4.y - sym, pzs = pa4.z - szm;
-          // unswitched sums over the neighbour's atoms; the switch (a function of
-          // the group distance only) scales them once below
-          double ucoula = 0.0, uconfa = 0.0, dwa = 0.0;
-          double sega = 0.0, cmr = 0.0;  // REM: segment energy, V with the selected pairs scaled
-          if (alch) {
-            for (int k = 0; k < nJ; ++k) {
-              const int2 ib0 = gload_at(d.sai, jbs + k);
-              const double4 pb0 = gload_at(d.sap, jbs + k);
-              const double4 ap = gload_at(d.alch_pair, ia4.x * d.ntypes + ib0.x);
-              bool skip0 = d.lskip_ewald && ap.y < 1e-12 && d.ewald;
-              if (fwd ? mask_a : (ib0.y & 1) != 0) skip0 = skip0 || pair_masked(d, a, jb0 + k, ia0, nI, fwd);
-              const AlchTerms r0 = alch_terms<T>(d, pxs, pys, pzs, pa4.w, co, pb0, ap, sh.alch[(int)ap.z]);
-              if (!skip0) r0.add(uconfa, ucoula, dwa, fgx, fgy, fgz);
-            }
-          } else if constexpr (FREC) {
-            // compact records: separation = group separation (FP64) + offset difference
-            for (int k = 0; k < nJ; ++k) {
-              const int2 ib0 = gload_at(d.sai, jbs + k);
-              const float4 pb0 = gload_at(d.sapf, jbs + k);
-              double c12a, c6a;
-              if (d.lj_dense32) {
-                const float2 lj = gload_at(d.lj_dense32, ia4.x * d.ntypes + ib0.x);
-                c12a = lj.x;
-                c6a = lj.y;
+      }
+      int c0 = nb0, ecount = 0, shead = 0, ns = 0;
+      for (;;) {
+        while (ns < 64 && c0 < nb1) {
+          // ---- classify per_round entries; the in-shell ones are kept in list order
+          const int jj = c0 + lane;
+          const bool in = lane < per_round && jj < nb1;
+          c0 += per_round;
+          const int tj = in ? gmem(d.nb_idx)[jj] : t;
+          const double4 gpj = gload_at(d.sgp, tj);
+          const GroupGeom gg = group_geom(xpgi, ypgi, zpgi, gpj, d.co);
+          const bool keep = in && in_shell(d, gg.drj);
+          int jw[2];
+          __builtin_memcpy(jw, &gpj.w, 8);
+          const int nJ = keep ? (jw[1] & 255) : 0;
+          const unsigned long long m = __ballot(keep);
+          // exclusive prefix of the kept entries' atom counts, one bit of the counts at a time
+          int apos = 0, atot = 0;
+          for (int b = 0; (mg >> b) != 0; ++b) {
+            const unsigned long long mb = __ballot((nJ >> b) & 1);
+            apos += lanes_below(mb) << b;
+            atot += __popcll(mb) << b;
+          }
+          if (keep) {
+            const int e = (ecount + lanes_below(m)) & (ENT_RING - 1);
+            double sw = 1.0, dsw = 0.0;
+            if (!(gg.drj >= d.r2inn0 && gg.drj < d.r2out)) {
+              const double rinv = pair_rsqrt<double>(gg.drj), rsp = gg.drj * rinv;
+              if (gg.drj >= d.r2out && gg.drj < d.r2out0) {
+                const double auxa = (d.arsout1 + 2.0 * rsp) * inv_o2, auxb = d.rout0 - rsp;
+                sw = auxa * (auxb * auxb);
+                dsw = (-(2.0 * auxa * auxb) + 2.0 * (auxb * auxb) * inv_o2) * rinv;
               } else {
-                lj_params(d, ia4.x, ib0.x, c12a, c6a);
+                const double auxa = (d.arsinn1 + 2.0 * rsp) * inv_i2, auxb = d.rinn0 - rsp;
+                sw = 1.0 - auxa * (auxb * auxb);
+                dsw = (2.0 * auxa * auxb - 2.0 * (auxb * auxb) * inv_i2) * rinv;
               }
-              bool skip0 = d.lskip_ewald && c6a < 1e-12 && d.ewald;
-              if (fwd ? mask_a : (ib0.y & 1) != 0) skip0 = skip0 || pair_masked(d, a, jb0 + k, ia0, nI, fwd);
-              const PairTerms r0 =
-                  pair_terms_c<T>(d, T(gg.xcc + (double)(paf.x - pb0.x)), T(gg.ycc + (double)(paf.y - pb0.y)),
-                                  T(gg.zcc + (double)(paf.z - pb0.z)), T(paf.w * pb0.w), c12a, c6a);
-              if (!skip0) r0.add(uconfa, ucoula, fgx, fgy, fgz);
             }
-          } else if (d.rematom) {
-            // force_REM.f:491-494, 649-664, 679-682 (Ewald branch): a selected
-            // pair's force is scaled by rem_f3 and its energy goes to the
-            // segment energy; its share of V for the switch derivative is
-            // scaled too (cmap2), the shell energies are not
-            const bool ra = gmem(d.rematom)[a] != 0;
-            for (int k = 0; k < nJ; ++k) {
-              const int2 ib0 = gload_at(d.sai, jbs + k);
-              const double4 pb0 = gload_at(d.sap, jbs + k);
-              double c12a, c6a;
-              lj_params(d, ia4.x, ib0.x, c12a, c6a);
-              bool skip0 = false;
-              if (fwd ? mask_a : (ib0.y & 1) != 0) skip0 = pair_masked(d, a, jb0 + k, ia0, nI, fwd);
-              const PairTerms r0 = pair_terms<T>(d, pxs, pys, pzs, pa4.w, co, pb0, c12a, c6a);
-              if (skip0) continue;
-              const bool rb = gmem(d.rematom)[jb0 + k] != 0;
-              const bool sel = d.rem_kind == 0 ? (ra || rb) : (d.rem_kind == 1 ? (ra && rb) : (ra != rb));
-              const double f = sel ? d.rem_f3 : 1.0;
-              uconfa += r0.conf;
-              ucoula += r0.cou;
-              fgx += (f * r0.qf) * r0.xc;
-              fgy += (f * r0.qf) * r0.yc;
-              fgz += (f * r0.qf) * r0.zc;
-              if (sel) sega += r0.conf + r0.cou;
-              cmr += f * r0.conf + f * r0.cou;
+            if constexpr (F32) {
+              float2 g;
+              g.x = (float)gg.xcc;
+              g.y = (float)(gg.xcc - (double)g.x);
+              __builtin_memcpy(&W.gx[e], &g, 8);
+              g.x = (float)gg.ycc;
+              g.y = (float)(gg.ycc - (double)g.x);
+              __builtin_memcpy(&W.gy[e], &g, 8);
+              g.x = (float)gg.zcc;
+              g.y = (float)(gg.zcc - (double)g.x);
+              __builtin_memcpy(&W.gz[e], &g, 8);
+            } else {
+              W.gx[e] = gg.xcc;
+              W.gy[e] = gg.ycc;
+              W.gz[e] = gg.zcc;
             }
-          } else {
-            for (int k = 0; k < nJ; ++k) {
-              const int2 ib0 = gload_at(d.sai, jbs + k);
-              const double4 pb0 = gload_at(d.sap, jbs + k);
-              double c12a, c6a;
-              lj_params(d, ia4.x, ib0.x, c12a, c6a);
-              bool skip0 = d.lskip_ewald && c6a < 1e-12 && d.ewald;
-              if (fwd ? mask_a : (ib0.y & 1) != 0) skip0 = skip0 || pair_masked(d, a, jb0 + k, ia0, nI, fwd);
-              const PairTerms r0 = pair_terms<T>(d, pxs, pys, pzs, pa4.w, co, pb0, c12a, c6a);
-              if (!skip0) r0.add(uconfa, ucoula, fgx, fgy, fgz);
+            W.sw[e] = sw;
+            W.dsw[e] = dsw;
+            const bool shifted = gg.sxm != 0.0 || gg.sym != 0.0 || gg.szm != 0.0;
+            if (shifted) {
+              W.sx[e] = (int)gg.sxm;
+              W.sy[e] = (int)gg.sym;
+              W.sz[e] = (int)gg.szm;
             }
+            W.bs[e] = jw[0] | ((jw[1] >> 8) == 1 ? 1 << 26 : 0) | (shifted ? 1 << 27 : 0);
+            if (MODE != PAIR_PLAIN) W.tj[e] = tj;
+            const int s0 = shead + ns + apos;
+            for (int k = 0; k < mg; ++k)
+              if (k < nJ) W.slot[(s0 + k) & (SLOT_RING - 1)] = (unsigned short)(e | (k << 7));
           }
-          const double s = cls == 2 ? sw : 1.0;
-          fgx *= s;
-          fgy *= s;
-          fgz *= s;
-          fxa += fgx;
-          fya += fgy;
-          fza += fgz;
-          if (fwd) {
-            en[typeij * 64 + lane] += s * uconfa;
-            en[(3 + typeij) * 64 + lane] += s * ucoula;
-            if (ALCH) acc[wid][15][lane] += s * dwa;
-            if (!ALCH && FREC == false && d.rematom) acc[wid][15][lane] += s * sega;
-          }
-          if (cls == 2) cm = (!ALCH && !FREC && d.rematom) ? cmr : uconfa + ucoula;
+          ecount += __popcll(m);
+          ns += atot;
         }
-        // total V of the group pair over the slot's lanes (every lane shuffles)
-        double cmt = 0.0;
-        for (int u = 0; u < nI; ++u) cmt += __shfl(cm, (slot * nI + u) & 63, 64);
-        if (cls == 2) {
-          // S'(r) V spread over group atoms by mass fraction (force.f:756-817)
-          const double x3 = -(dsw * cmt * xcc), y3 = -(dsw * cmt * ycc), z3 = -(dsw * cmt * zcc);
-          fxa += ma * x3;
-          fya += ma * y3;
-          fza += ma * z3;
-          if (fwd && shifted && ai == 0) {
-            fgx += x3;
-            fgy += y3;
-            fgz += z3;
-          }
+        if (ns <= 0) break;
+        wave_lds_sync();
+        // ---- one pass: up to 64 neighbour atoms
+        const int np = min(ns, 64);
+        const bool have = lane < np;
+        const int sl = W.slot[(shead + (have ? lane : 0)) & (SLOT_RING - 1)];
+        const int e = sl & 127, k = sl >> 7;
+        const int eb = W.bs[e];
+        const int js = (eb & 0x3ffffff) + k;
+        const AtomRec<T> rb = atom_rec<T>(d, js);
+        const int2 ib = gload_at(d.sai, js);
+        const double sw = have ? W.sw[e] : 0.0, dsw = have ? W.dsw[e] : 0.0;
+        // separation = (owner centre - neighbour centre - image) + owner offset - neighbour offset;
+        // FP32: the centre separation as hi + lo, so that the last addition alone rounds at its size
+        T bx, by, bz, hx = T(0), hy = T(0), hz = T(0), lx = T(0), ly = T(0), lz = T(0);
+        if constexpr (F32) {
+          float2 g;
+          __builtin_memcpy(&g, &W.gx[e], 8);
+          hx = g.x;
+          lx = g.y;
+          __builtin_memcpy(&g, &W.gy[e], 8);
+          hy = g.x;
+          ly = g.y;
+          __builtin_memcpy(&g, &W.gz[e], 8);
+          hz = g.x;
+          lz = g.y;
+          bx = lx - rb.x;
+          by = ly - rb.y;
+          bz = lz - rb.z;
+        } else {
+          bx = W.gx[e] - rb.x;
+          by = W.gy[e] - rb.y;
+          bz = W.gz[e] - rb.z;
         }
-        if (fwd && shifted) {
-          st[0 * 64 + lane] -= fgx * sxm; st[1 * 64 + lane] -= fgx * sym; st[2 * 64 + lane] -= fgx * szm;
-          st[3 * 64 + lane] -= fgy * sxm; st[4 * 64 + lane] -= fgy * sym; st[5 * 64 + lane] -= fgy * szm;
-          st[6 * 64 + lane] -= fgz * sxm; st[7 * 64 + lane] -= fgz * sym; st[8 * 64 + lane] -= fgz * szm;
+        const bool shifted = have && ((eb >> 27) & 1) != 0, solute = ((eb >> 26) & 1) != 0;
+        const bool pass_st = __ballot(shifted) != 0ull, pass_solute = __ballot(have && solute) != 0ull;
+        const bool pass_ex = __ballot((ib.x & ATOM_EX) != 0) != 0ull;
+        any_st = any_st || pass_st;
+        const int tb = ib.x >> ATOM_FLAG_BITS;
+        // a pass without alchemical atoms takes the plain form of an alchemical system's pairs
+        const bool soft_b = alch && __ballot(have && (ib.x & ATOM_ALCH)) != 0ull;
+        // the first owner atom's LJ entry (a water's only one), requested before the arithmetic that hides it
+        T c12a = T(0), c6a = T(0);
+        if (ot[0] & ATOM_LJ) pair_lj<T, MODE == PAIR_PLAIN>(d, ot[0] >> ATOM_FLAG_BITS, tb, c12a, c6a);
+        double vc = 0.0, vq = 0.0, fsx = 0.0, fsy = 0.0, fsz = 0.0, seg = 0.0, vr = 0.0;
+        auto owner_atoms = [&](auto st_tag) {
+          constexpr bool ST = decltype(st_tag)::value;
+#pragma unroll
+          for (int u = 0; u < OWN_U; ++u) {
+            if (u < nu) {
+              const int fl = here(ot[u]);
+              AtomRec<T> ra;
+              __builtin_memcpy(&ra, &W.own[u], sizeof ra);
+              T x, y, z;
+              if constexpr (F32) {
+                x = hx + (bx + ra.x);
+                y = hy + (by + ra.y);
+                z = hz + (bz + ra.z);
+              } else {
+                x = bx + ra.x;
+                y = by + ra.y;
+                z = bz + ra.z;
+              }
+              T qq = ra.q * rb.q;
+              bool masked = false;
+              const bool heavy = MODE != PAIR_PLAIN && d.any_heavy != 0;
+              if (((fl & ATOM_EX) && pass_ex) || heavy) {  // wave-uniform
+                const int a = ia0 + u0 + u;
+                if ((fl & ATOM_EX) && pass_ex) {  // the owner atom's exclusions
+                  const int nx = min(xn[u], 64);
+                  for (int q = 0; q < nx; ++q) masked |= __builtin_amdgcn_readlane(xv[u], q) == ib.y;
+                  for (int q = 64; q < xn[u]; ++q) masked |= gmem(d.ex_idx)[gmem(d.ex_off)[a] + q] == ib.y;
+                }
+                if (heavy) masked |= heavy_masked(d, a, fl, t, ia0, nI, ib, W.tj[e]);
+                // no charge, no LJ, and a distance that keeps the zeros finite
+                qq = masked ? T(0) : qq;
+                x = masked ? T(1) : x;
+              }
+              T qf, cou, conf = T(0);
+              double dw = 0.0;
+              if (MODE == PAIR_ALCH && (soft_b || (alch && (fl & ATOM_ALCH)))) {
+                const double4 ap = gload_at(d.alch_pair, (fl >> ATOM_FLAG_BITS) * d.ntypes + tb);
+                const AlchTerms<T> r = alch_terms<T>(d, x, y, z, qq, ap, sh.alch[(int)ap.z]);
+                qf = r.qf;
+                conf = r.conf;
+                cou = r.cou;
+                dw = r.dw;
+              } else {
+                const T rsq = x * x + y * y + z * z;
+                const T rinv = pair_rsqrt<T>(rsq);
+                const T rsqi = rinv * rinv;
+                if (!lskip) {
+                  const T expcst = pair_exp2<T>(T(d.ew_exp2) * rsq), r = rsq * rinv;
+                  const T erfcst = erfc_poly<T>(pair_rcp<T>(T(1) + T(d.ew_qp) * r)) * expcst;
+                  const T qr = qq * rinv;
+                  cou = qr * erfcst;
+                  qf = (erfcst + (T(d.ew_twa) * r) * expcst) * (qr * rsqi);
+                } else {
+                  cou = plainq ? qq * rinv : T(0);
+                  qf = cou * rsqi;
+                }
+                if (fl & ATOM_LJ) {  // some type has LJ with this owner atom's
+                  T c12 = c12a, c6 = c6a;
+                  if (u > 0) pair_lj<T, MODE == PAIR_PLAIN>(d, fl >> ATOM_FLAG_BITS, tb, c12, c6);
+                  c12 = masked ? T(0) : c12;
+                  c6 = masked ? T(0) : c6;
+                  const T r6 = rsqi * rsqi * rsqi;
+                  const T e6 = c6 * r6, e12 = c12 * r6 * r6;
+                  conf = e12 - e6;
+                  if (MODE != PAIR_ALCH) vc += (double)conf;
+                  qf += (T(12) * e12 - T(6) * e6) * rsqi;
+                }
+              }
+              if (MODE == PAIR_ALCH) {  // (the soft core takes its own parameters)
+                qf = masked ? T(0) : qf;
+                conf = masked ? T(0) : conf;
+                cou = masked ? T(0) : cou;
+                seg += masked ? 0.0 : dw;
+              }
+              if (MODE == PAIR_ALCH) vc += (double)conf;
+              vq += (double)cou;
+              double w = (double)qf * sw;
+              if (MODE == PAIR_REM) {
+                // force_REM.f:491-494, 649-664, 679-682 (Ewald branch): a selected pair's force is scaled by
+                // rem_f3 and its energy goes to the segment energy; its share of V for the switch derivative
+                // is scaled too (cmap2), the shell energies are not
+                const bool ra = (fl & ATOM_REM) != 0, rbs = (ib.x & ATOM_REM) != 0;
+                const bool sel = d.rem_kind == 0 ? (ra || rbs) : (d.rem_kind == 1 ? (ra && rbs) : (ra != rbs));
+                const double f = sel ? d.rem_f3 : 1.0, en = (double)conf + (double)cou;
+                w *= f;
+                if (sel) seg += en;
+                vr += f * en;
+              }
+              fr[u][0] += w * (double)x;
+              fr[u][1] += w * (double)y;
+              fr[u][2] += w * (double)z;
+              if (ST) {
+                fsx += w * (double)x;
+                fsy += w * (double)y;
+                fsz += w * (double)z;
+              }
+            }
+          }
+        };
+        // the image-shift virial needs the lane's summed force: a path of its own
+        if (pass_st)
+          owner_atoms(std::true_type{});
+        else
+          owner_atoms(std::false_type{});
+        // ---- the lane's share of the group pair's energies, S'V term and image-shift virial
+        if (pass_solute) {
+          ec[0] += solute ? sw * vc : 0.0;
+          eq[0] += solute ? sw * vq : 0.0;
+          ec[1] += solute ? 0.0 : sw * vc;
+          eq[1] += solute ? 0.0 : sw * vq;
+        } else {
+          ec[1] += sw * vc;
+          eq[1] += sw * vq;
+        }
+        if (DW) dwl += sw * seg;
+        double gx, gy, gz;
+        if constexpr (F32) {
+          gx = (double)hx + (double)lx;
+          gy = (double)hy + (double)ly;
+          gz = (double)hz + (double)lz;
+        } else {
+          gx = W.gx[e];
+          gy = W.gy[e];
+          gz = W.gz[e];
+        }
+        const double v = -dsw * (MODE == PAIR_REM ? vr : vc + vq);
+        x3[0] += v * gx;
+        x3[1] += v * gy;
+        x3[2] += v * gz;
+        if (pass_st) {
+          fsx += v * gx;
+          fsy += v * gy;
+          fsz += v * gz;
+          const double sx = shifted ? (double)W.sx[e] : 0.0, sy = shifted ? (double)W.sy[e] : 0.0,
+                       sz = shifted ? (double)W.sz[e] : 0.0;
+          st[0] -= fsx * sx; st[1] -= fsx * sy; st[2] -= fsx * sz;
+          st[3] -= fsy * sx; st[4] -= fsy * sy; st[5] -= fsy * sz;
+          st[6] -= fsz * sx; st[7] -= fsz * sy; st[8] -= fsz * sz;
+        }
+        shead = (shead + np) & (SLOT_RING - 1);
+        ns -= np;
+      }
+      // ---- this batch's owner-atom forces: value 3 u + c on lanes 8 (3 u + c) ..
+      double v[8];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (h == 0 || nu >= 3) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const int w = 8 * h + q;
+          v[q] = w < 3 * OWN_U ? fr[w / 3 < OWN_U ? w / 3 : 0][w % 3] : 0.0;
+        }
+        const double s = wave_sum8(v, buf, lane);
+        const int w = 8 * h + (lane >> 3);
+        if ((lane & 7) == 0 && w < 3 * nu) sh.fsum[wid][u0 + w / 3][w % 3] = s;
         }
       }
-      // every lane is done with this chunk before the next fill
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
   }
-  // owner-atom forces: the owner's waves in part order, in each the lanes
-  // ai, ai + nI, ... in lane order
-  facc[wid][lane][0] = fxa;
-  facc[wid][lane][1] = fya;
-  facc[wid][lane][2] = fza;
-  __syncthreads();
-  if (t < d.ngrp && part == 0 && lane < nI) {
-    double sx = 0.0, sy = 0.0, sz = 0.0;
-    for (int p = 0; p < S; ++p)
-      for (int s = 0; s < nslot; ++s) {
-        sx += facc[wid + p][s * nI + lane][0];
-        sy += facc[wid + p][s * nI + lane][1];
-        sz += facc[wid + p][s * nI + lane][2];
-      }
-    const int a = ia0 + lane;
-    gmem(d.fx)[a] = sx;
-    gmem(d.fy)[a] = sy;
-    gmem(d.fz)[a] = sz;
-    const int pa = gmem(d.atomp)[a];
-    const double cx = gmem(d.xpcm)[pa], cy = gmem(d.ypcm)[pa], cz = gmem(d.zpcm)[pa];
-    st[0 * 64 + lane] += sx * cx; st[1 * 64 + lane] += sx * cy; st[2 * 64 + lane] += sx * cz;
-    st[3 * 64 + lane] += sy * cx; st[4 * 64 + lane] += sy * cy; st[5 * 64 + lane] += sy * cz;
-    st[6 * 64 + lane] += sz * cx; st[7 * 64 + lane] += sz * cy; st[8 * 64 + lane] += sz * cz;
+  // ---- energies, S'V vector and virial of the wave
+  {
+    double v[8] = {x3[0], x3[1], x3[2], ec[1], eq[1], DW ? dwl : 0.0, ec[0], eq[0]};
+    const double s = wave_sum8(v, buf, lane);
+    double *red = sh.red[wid];
+    if (lane < PAIR_NACC) red[3 + lane] = 0.0;
+    wave_lds_sync();
+    if ((lane & 7) == 0) {
+      // uconf / ucoul by typeij = typei + typej - 2 (0 slt-slt, 1 slt-slv, 2 slv-slv); both sides counted
+      const int q = lane >> 3;
+      if (q < 3) red[q] = s;
+      else if (q == 3) red[3 + typei] = 0.5 * s;
+      else if (q == 4) red[3 + 3 + typei] = 0.5 * s;
+      else if (q == 5) red[3 + 15] = 0.5 * s;
+      else if (q == 6) red[3 + typei - 1] = 0.5 * s;
+      else red[3 + 3 + typei - 1] = 0.5 * s;
+    }
+    if (any_st) {
+      const double s0 = wave_sum8(st, buf, lane);
+      if ((lane & 7) == 0) red[3 + 6 + (lane >> 3)] = 0.5 * s0;
+      const double s8 = wave_sum(st[8]);
+      if (lane == 0) red[3 + 14] = 0.5 * s8;
+    }
   }
-  // energies and virial: wave then block, fixed order
-#pragma unroll
-  for (int k = 0; k < PAIR_NACC; ++k) {
-    double v = wave_sum(acc[wid][k][lane]);
-    if (lane == 0) red[wid][k] = v;
+  __syncthreads();
+  // ---- owner-atom forces: the owner's waves in part order, then the S'V terms by mass fraction
+  if (t < d.ngrp && part == 0) {
+    double X[3] = {0.0, 0.0, 0.0}, f[3] = {0.0, 0.0, 0.0};
+    for (int p = 0; p < S; ++p)
+      for (int c = 0; c < 3; ++c) X[c] += sh.red[wid + p][c];
+    if (lane < nI) {
+      for (int p = 0; p < S; ++p)
+        for (int c = 0; c < 3; ++c) f[c] += sh.fsum[wid + p][lane][c];
+      const int a = ia0 + lane;
+      const double gm = gmem(d.gmass)[a];
+      const int pa = gmem(d.atomp)[a];
+      const double cm[3] = {gmem(d.xpcm)[pa], gmem(d.ypcm)[pa], gmem(d.zpcm)[pa]};
+      for (int c = 0; c < 3; ++c) f[c] += gm * X[c];
+      gmem(d.fx)[a] = f[0];
+      gmem(d.fy)[a] = f[1];
+      gmem(d.fz)[a] = f[2];
+      for (int c = 0; c < 3; ++c) {
+        sh.fsum[wid][lane][c] = f[c];
+        buf[3 * lane + c] = cm[c];
+      }
+    }
+    wave_lds_sync();
+    if (lane < 9) {  // the molecular virial F_a (x) C_a, in atom order
+      double s = 0.0;
+      for (int u = 0; u < nI; ++u) s += sh.fsum[wid][u][lane / 3] * buf[3 * u + lane % 3];
+      sh.red[wid][3 + 6 + lane] += s;
+    }
   }
   __syncthreads();
   if (threadIdx.x < PAIR_NACC) {
     double s = 0.0;
-    for (int w = 0; w < PAIR_WAVES; ++w) s += red[w][threadIdx.x];
+    for (int w = 0; w < PAIR_WAVES; ++w) s += sh.red[w][3 + threadIdx.x];
     gmem(d.part)[(size_t)blk * 16 + threadIdx.x] = s;
   }
 }
@@ -639,36 +844,36 @@ __device__ __forceinline__ void pairs_item_index(int h, int nitems, int nblkmax,
 }
 
 // W = minimum waves per SIMD the register allocation must allow (occupancy target)
-template <typename T, int W, bool ALCH>
+template <typename T, int W, int MODE>
 __global__ void __launch_bounds__(256, W) k_pairs(const PairDesc *__restrict__ D, int remap) {
   __shared__ PairShared sh;
   int sys, blk;
   pairs_item_index(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y, gridDim.x, remap, sys, blk);
-  pairs_item<T, ALCH>(D[sys], blk, sh);
+  pairs_item<T, MODE>(D[sys], blk, sh);
 }
 
 // Persistent form: a fixed grid (a multiple of 8 workgroups, so each keeps to
 // one XCD) walks all items of the batch with a grid stride.
-template <typename T, int W, bool ALCH>
+template <typename T, int W, int MODE>
 __global__ void __launch_bounds__(256, W) k_pairs_persistent(const PairDesc *__restrict__ D, int remap, int nitems,
                                                              int nblkmax) {
   __shared__ PairShared sh;
   for (int h = blockIdx.x; h < nitems; h += gridDim.x) {
     int sys, blk;
     pairs_item_index(h, nitems, nblkmax, remap, sys, blk);
-    pairs_item<T, ALCH>(D[sys], blk, sh);
+    pairs_item<T, MODE>(D[sys], blk, sh);
     __syncthreads();
   }
 }
 
-template <typename T, int W, bool ALCH>
+template <typename T, int W, int MODE>
 static void launch_pair_kernel(bool persistent, dim3 grd, int g, hipStream_t st, const PairDesc *d_desc, int remap,
                                int nitems, int max_blk) {
   const dim3 blk(64 * PAIR_WAVES);
   if (persistent)
-    hipLaunchKernelGGL((k_pairs_persistent<T, W, ALCH>), dim3(g), blk, 0, st, d_desc, remap, nitems, max_blk);
+    hipLaunchKernelGGL((k_pairs_persistent<T, W, MODE>), dim3(g), blk, 0, st, d_desc, remap, nitems, max_blk);
   else
-    hipLaunchKernelGGL((k_pairs<T, W, ALCH>), grd, blk, 0, st, d_desc, remap);
+    hipLaunchKernelGGL((k_pairs<T, W, MODE>), grd, blk, 0, st, d_desc, remap);
 }
 
 // d.out[16]: uconf[3], ucoul[3] (slt, slt-slv, slv order of typeij), st[9] row-major,
@@ -708,10 +913,7 @@ __global__ void __launch_bounds__(256) k_pairs_finalize(const PairDesc *__restri
 //
 // Pair separations are the Cartesian group separation (image applied, FP64)
 // plus the difference of the two atoms' Cartesian offsets from their group
-// centres, so each pair costs three additions before its distance.  FP64
-// reciprocal, reciprocal square root and exponential are the hardware seeds
-// refined by one Newton step (~1e-14 relative) and a degree-10 Taylor
-// polynomial after a two-constant ln 2 reduction (~3e-13 relative).
+// centres, so each pair costs three additions before its distance.
 
 // (OWN_REG, the owner atoms whose force sums stay in registers: water, single atoms, is in kernels.hpp)
 
@@ -731,61 +933,8 @@ struct OwnShared {
 };
 
 template <typename T>
-__device__ __forceinline__ T own_rsqrt(T x);
-template <>
-__device__ __forceinline__ double own_rsqrt<double>(double x) { return pair_rsqrt<double>(x); }
-template <>
-__device__ __forceinline__ float own_rsqrt<float>(float x) { return __builtin_amdgcn_rsqf(x); }
-template <typename T>
-__device__ __forceinline__ T own_rcp(T x);
-template <>
-__device__ __forceinline__ double own_rcp<double>(double x) { return pair_rcp<double>(x); }
-template <>
-__device__ __forceinline__ float own_rcp<float>(float x) { return __builtin_amdgcn_rcpf(x); }
-template <typename T>
-__device__ __forceinline__ T own_exp(T x);
-template <>
-__device__ __forceinline__ double own_exp<double>(double x) { return pair_exp<double>(x); }
-template <>
-__device__ __forceinline__ float own_exp<float>(float x) { return __expf(x); }
-
-// LJ {c12, c6} of the type pair (ti, tj), zero when c6 <= 1e-12 (the pair
-// then has no LJ term, force.f:455)
-template <typename T>
-__device__ __forceinline__ void own_lj(const PairDesc &d, int ti, int tj, T &c12, T &c6) {
-  double a, b;
-  if (sizeof(T) == 4 && d.lj_dense32) {
-    const float2 v = gload_at(d.lj_dense32, ti * d.ntypes + tj);
-    a = v.x;
-    b = v.y;
-  } else {
-    lj_params(d, ti, tj, a, b);
-  }
-  const bool lj = b > 1e-12;
-  c12 = lj ? T(a) : T(0);
-  c6 = lj ? T(b) : T(0);
-}
-
-// The owner-side and neighbour-side records of one atom: Cartesian offset
-// from the group centre and the charge, in the pair precision.
-template <typename T>
-struct OwnRec {
-  T x, y, z, q;
-};
-template <typename T>
-__device__ __forceinline__ OwnRec<T> own_rec(const PairDesc &d, int s) {
-  if constexpr (sizeof(T) == 4) {
-    const float4 v = gload(d.sapf + s);
-    return {v.x, v.y, v.z, v.w};
-  } else {
-    const double4 v = gload(d.sapc + s);
-    return {v.x, v.y, v.z, v.w};
-  }
-}
-
-template <typename T, bool HALF>
 __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &sh) {
-  if (blk >= d.nblk || (d.half != 0) != HALF) return;
+  if (blk >= d.nblk || !d.half) return;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   OwnWave &W = sh.w[wid];
   // the owner group: wave-uniform, so its records come through scalar loads
@@ -801,7 +950,6 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
   int ia0 = 0, nI = 0, typei = 1, as0 = 0;
   if (t < d.ngrp) {
     const int4 gi = gload(d.sgi + t);
-    const int g = gi.w;
     as0 = gi.x;
     ia0 = gi.y;
     nI = gi.z & 255;
@@ -825,7 +973,7 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
       const int nJin = in ? (gload_at(d.sgi, tj).z & 255) : 0;
       const int nJ = keep ? nJin : 0;
       int mslot = -1;
-      if (HALF && in) {
+      if (in) {
         // every forward entry's slots are written: the pair forces, or zeros outside the shell
         mslot = gmem(d.nb_mirror)[jj];
         if (!keep && mslot >= 0)
@@ -859,7 +1007,7 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
           dsw = (2.0 * auxa * auxb - 2.0 * (auxb * auxb) / d.arsinn2) / rsp;
         }
         W.ent[pos] = tj;
-        if (HALF) W.pb[pos] = mslot;
+        W.pb[pos] = mslot;
         W.aoff[pos] = incl - nJ;
         W.nj[pos] = nJ;
         W.gx[pos] = gg.xcc;
@@ -898,15 +1046,15 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
         int typej = 1, bs = 0, bo = 0, nJl = 0;
         bool fwd = false;
         int2 ib = make_int2(0, 0);
-        OwnRec<T> rb = {T(0), T(0), T(0), T(0)};
+        AtomRec<T> rb = {T(0), T(0), T(0), T(0)};
         if (have) {
           const int4 gij = gload_at(d.sgi, W.ent[e]);
           typej = gij.z >> 8;
-          fwd = HALF || gij.w > g;
+          fwd = true;  // a half list: this group is the lower one
           bs = gij.x + k;
           bo = gij.y + k;
           nJl = gij.z & 255;
-          rb = own_rec<T>(d, bs);
+          rb = atom_rec<T>(d, bs);
           ib = gload_at(d.sai, bs);
         }
         // separation = (owner centre - neighbour centre - image) + owner offset - neighbour offset
@@ -918,27 +1066,27 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
           for (int u = 0; u < OWN_REG; ++u) {
             c12[u] = T(0);
             c6[u] = T(0);
-            if (u < nI) own_lj<T>(d, gload(d.sai + as0 + u).x, ib.x, c12[u], c6[u]);
+            if (u < nI) pair_lj<T>(d, gload(d.sai + as0 + u).x >> ATOM_FLAG_BITS, ib.x >> ATOM_FLAG_BITS, c12[u], c6[u]);
           }
 #pragma unroll
           for (int u = 0; u < OWN_REG; ++u) {
             if (u >= nI) break;
-            const OwnRec<T> ra = own_rec<T>(d, as0 + u);
+            const AtomRec<T> ra = atom_rec<T>(d, as0 + u);
             const int2 ia = gload(d.sai + as0 + u);
             bool masked = false;
-            if (ia.y & ib.y & 1) masked = is_excluded(gmem(d.ex_off), gmem(d.ex_idx), ia0 + u, bo);
+            if (ia.x & ib.x & ATOM_EX) masked = is_excluded(gmem(d.ex_off), gmem(d.ex_idx), ia0 + u, bo);
             if (d.any_heavy && !masked && !(gmem(d.mass)[bo] < d.massinfty || gmem(d.mass)[ia0 + u] < d.massinfty)) {
               // force.f:486-490: two atoms at or above massinfty are skipped only where the
               // list owner's atom has an exclusion partner in the other group (the owner
               // is the lower group: this one when fwd, the neighbour's otherwise)
               if (fwd)
-                masked = (ia.y & 1) && has_partner_in(gmem(d.ex_off), gmem(d.ex_idx), ia0 + u, bo - k, bo - k + nJl - 1);
+                masked = (ia.x & ATOM_EX) && has_partner_in(gmem(d.ex_off), gmem(d.ex_idx), ia0 + u, bo - k, bo - k + nJl - 1);
               else
-                masked = (ib.y & 1) && has_partner_in(gmem(d.ex_off), gmem(d.ex_idx), bo, ia0, ia0 + nI - 1);
+                masked = (ib.x & ATOM_EX) && has_partner_in(gmem(d.ex_off), gmem(d.ex_idx), bo, ia0, ia0 + nI - 1);
             }
             const T xc = bx + ra.x, yc = by + ra.y, zc = bz + ra.z;
             const T rsq = xc * xc + yc * yc + zc * zc;
-            const T rinv = own_rsqrt<T>(rsq);
+            const T rinv = pair_rsqrt<T>(rsq);
             const T rsqi = rinv * rinv;
             const T r6 = rsqi * rsqi * rsqi;
             const T e6 = c6[u] * r6, e12 = c12[u] * r6 * r6;
@@ -949,8 +1097,8 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
             if (!d.lskip_ewald) {
               const T rsp = rsq * rinv;
               const T alphar = T(d.alpha) * rsp;
-              const T qt = own_rcp<T>(T(1) + T(AS_QP) * alphar);
-              const T expcst = own_exp<T>(-(alphar * alphar));
+              const T qt = pair_rcp<T>(T(1) + T(AS_QP) * alphar);
+              const T expcst = pair_exp2<T>(T(d.ew_exp2) * rsq);
               const T erfcst =
                   ((((T(AS_A5) * qt + T(AS_A4)) * qt + T(AS_A3)) * qt + T(AS_A2)) * qt + T(AS_A1)) * qt * expcst;
               cou = qq * erfcst * rinv;
@@ -972,11 +1120,9 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
             fsx += fx;
             fsy += fy;
             fsz += fz;
-            if (HALF) {
-              fbx -= fx;
-              fby -= fy;
-              fbz -= fz;
-            }
+            fbx -= fx;
+            fby -= fy;
+            fbz -= fz;
             vc += (double)conf;
             vq += (double)cou;
           }
@@ -1006,7 +1152,7 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
             x3y += y3;
             x3z += z3;
           }
-          if (HALF && have && dsw != 0.0) {
+          if (have && dsw != 0.0) {
             // the neighbour group's share, -x3 by its atoms' mass fractions
             const double mb = gmem(d.gmass)[bo];
             fbx -= mb * x3;
@@ -1014,7 +1160,7 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
             fbz -= mb * z3;
           }
         }
-        if (HALF && have) {
+        if (have) {
           const int slot = W.pb[e];
           if (slot >= 0) {
             gmem(d.jpx)[slot + k] = fbx;
@@ -1067,13 +1213,7 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
       gmem(d.fx)[a] = fxa;
       gmem(d.fy)[a] = fya;
       gmem(d.fz)[a] = fza;
-      if (!HALF) {  // (the half form adds the molecular virial once the neighbour-side forces are in)
-        const int pa = gmem(d.atomp)[a];
-        const double cx = gmem(d.xpcm)[pa], cy = gmem(d.ypcm)[pa], cz = gmem(d.zpcm)[pa];
-        st[0] += fxa * cx; st[1] += fxa * cy; st[2] += fxa * cz;
-        st[3] += fya * cx; st[4] += fya * cy; st[5] += fya * cz;
-        st[6] += fza * cx; st[7] += fza * cy; st[8] += fza * cz;
-      }
+      // (k_pairs_jsum adds the molecular virial once the neighbour-side forces are in)
     }
   }
   // ---- energies and virial: wave, then block, fixed order
@@ -1100,34 +1240,34 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
   }
 }
 
-template <typename T, int W, bool HALF>
+template <typename T, int W>
 __global__ void __launch_bounds__(256, W) k_pairs_own(const PairDesc *__restrict__ D, int remap) {
   __shared__ OwnShared sh;
   int sys, blk;
   pairs_item_index(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y, gridDim.x, remap, sys, blk);
-  own_item<T, HALF>(D[sys], blk, sh);
+  own_item<T>(D[sys], blk, sh);
 }
 
-template <typename T, int W, bool HALF>
+template <typename T, int W>
 __global__ void __launch_bounds__(256, W) k_pairs_own_persistent(const PairDesc *__restrict__ D, int remap,
                                                                  int nitems, int nblkmax) {
   __shared__ OwnShared sh;
   for (int h = blockIdx.x; h < nitems; h += gridDim.x) {
     int sys, blk;
     pairs_item_index(h, nitems, nblkmax, remap, sys, blk);
-    own_item<T, HALF>(D[sys], blk, sh);
+    own_item<T>(D[sys], blk, sh);
     __syncthreads();
   }
 }
 
-template <typename T, int W, bool HALF>
+template <typename T, int W>
 static void launch_own_kernel(bool persistent, dim3 grd, int g, hipStream_t st, const PairDesc *d_desc, int remap,
                               int nitems, int max_blk) {
   const dim3 blk(64 * PAIR_WAVES);
   if (persistent)
-    hipLaunchKernelGGL((k_pairs_own_persistent<T, W, HALF>), dim3(g), blk, 0, st, d_desc, remap, nitems, max_blk);
+    hipLaunchKernelGGL((k_pairs_own_persistent<T, W>), dim3(g), blk, 0, st, d_desc, remap, nitems, max_blk);
   else
-    hipLaunchKernelGGL((k_pairs_own<T, W, HALF>), grd, blk, 0, st, d_desc, remap);
+    hipLaunchKernelGGL((k_pairs_own<T, W>), grd, blk, 0, st, d_desc, remap);
 }
 
 // Half form, after the pair kernel: each group's atoms add the neighbour-side
@@ -1206,24 +1346,23 @@ int pair_split_for(int ngrp) {
   return 1;  // measured: extra waves per owner cost more than the tail they trim
 }
 
-// Occupancy target of k_pairs: measured best on MI355X for the 24.5k-atom
-// system is 3 waves/SIMD for FP64 (4 spills) and 4 for FP32.  The tuning
-// value, then ORAC_HIP_PAIR_WAVES=2|3|4, override it.
+// Occupancy target of k_pairs (plain form): on the 24.5k-atom system 4 waves
+// per SIMD take 86 us in FP64 (3 registers spilled) and 3 take 96; FP32 fits
+// 4.  The tuning value, then ORAC_HIP_PAIR_WAVES=2|3|4, override it.
 template <typename T>
 static int pair_occupancy(int tuned) {
   if (tuned == 2 || tuned == 3 || tuned == 4) return tuned;
   static int w = [] {
     const char *e = getenv("ORAC_HIP_PAIR_WAVES");
-    int v = e ? atoi(e) : (sizeof(T) == 8 ? 3 : 4);
-    return (v == 2 || v == 3 || v == 4) ? v : 3;
+    int v = e ? atoi(e) : 4;
+    return (v == 2 || v == 3 || v == 4) ? v : 4;
   }();
   return w;
 }
 
-// The owner-atom loop form (and with it the half-list layout of resident
-// systems) is selected by ORAC_HIP_PAIR_KERNEL=own: read when a resident
-// system is created (its list layout) and at each launch of a system on the
-// full list; by default every system takes k_pairs on the full list.
+// The half-list form (k_pairs_own) is selected by ORAC_HIP_PAIR_KERNEL=own,
+// read when a resident system is created (its list layout); by default every
+// system takes k_pairs on the full list.
 // Measured on MI355X on the 24,460-atom system (one evaluation with a list
 // rebuild): the half-list form's per-pair slots and its list build (split,
 // reverse ranking, mirror search) cost more than the halved arithmetic saves
@@ -1237,24 +1376,23 @@ template <typename T>
 void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream_t st, const Tuning &tu,
                   hipEvent_t kbeg, hipEvent_t kend) {
   int max_grp = 1, max_blk = 1;
-  // half-list systems take the half form; the others the full owner-atom form
-  // when every one of them qualifies, else k_pairs
-  bool any_alch = false, own = use_owner_kernel(), any_half = false, any_full = false;
+  // half-list systems take the half form, the others k_pairs
+  bool any_alch = false, any_rem = false, any_other = false, any_half = false, any_full = false;
   for (int s = 0; s < nsys; ++s) {
     // every system's groups are packed and its blocks launched, whichever form serves it
     max_grp = std::max(max_grp, h[s].ngrp);
     max_blk = std::max(max_blk, h[s].nblk);
-    const bool fits = h[s].alch_pair == nullptr && h[s].rematom == nullptr && h[s].split == 1 &&
-                      h[s].max_group <= OWN_REG &&
-                      (sizeof(T) == 4 ? h[s].sapf != nullptr : h[s].sapc != nullptr);
+    if (sizeof(T) == 4 ? !h[s].sapf : !h[s].sapc) throw Error(E_STATE, "no atom records in this precision");
     if (h[s].half) {
-      if (!fits) throw Error(E_STATE, "half-list pair form on a system it does not serve");
+      if (h[s].alch_pair || h[s].rematom || h[s].split != 1 || h[s].max_group > OWN_REG)
+        throw Error(E_STATE, "half-list pair form on a system it does not serve");
       any_half = true;
       continue;
     }
     any_full = true;
     any_alch = any_alch || h[s].alch_pair != nullptr;
-    own = own && fits;
+    any_rem = any_rem || h[s].rematom != nullptr;
+    any_other = any_other || h[s].lskip_ewald || h[s].any_heavy || !h[s].lj_dense;
     if (h[s].max_group > 64)
       throw Error(E_UNSUPPORTED, "groups larger than 64 atoms are not supported by the pair kernel");
   }
@@ -1279,28 +1417,30 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
   const bool pers = tu.persistent != 0;
   if (any_half) {
     switch (waves) {
-      case 3: launch_own_kernel<T, 3, true>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
-      case 4: launch_own_kernel<T, 4, true>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
-      default: launch_own_kernel<T, 2, true>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
+      case 3: launch_own_kernel<T, 3>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
+      case 4: launch_own_kernel<T, 4>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
+      default: launch_own_kernel<T, 2>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
     }
     hipLaunchKernelGGL(k_pairs_jsum, grd, dim3(64 * PAIR_WAVES), 0, st, d_desc);
   }
   if (!any_full) {
     // (every system in the half-list form)
-  } else if (own) {
-    switch (waves) {
-      case 3: launch_own_kernel<T, 3, false>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
-      case 4: launch_own_kernel<T, 4, false>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
-      default: launch_own_kernel<T, 2, false>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
-    }
   } else if (any_alch) {
     // the soft-core form at the default occupancy target only
-    launch_pair_kernel<T, sizeof(T) == 8 ? 3 : 4, true>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
+    if (any_rem) throw Error(E_STATE, "alchemical and REM systems in one launch");
+    launch_pair_kernel<T, 3, PAIR_ALCH>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
+  } else if (any_rem) {
+    if constexpr (sizeof(T) == 8)
+      launch_pair_kernel<T, 3, PAIR_REM>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
+    else
+      throw Error(E_STATE, "REM pairs are evaluated in double precision");
+  } else if (any_other) {
+    launch_pair_kernel<T, 3, PAIR_ANY>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
   } else {
     switch (waves) {
-      case 3: launch_pair_kernel<T, 3, false>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
-      case 4: launch_pair_kernel<T, 4, false>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
-      default: launch_pair_kernel<T, 2, false>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
+      case 3: launch_pair_kernel<T, 3, PAIR_PLAIN>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
+      case 4: launch_pair_kernel<T, 4, PAIR_PLAIN>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
+      default: launch_pair_kernel<T, 2, PAIR_PLAIN>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
     }
   }
   if (kend) ORAC_HIP(hipEventRecord(kend, st));

@@ -359,6 +359,9 @@ AlchTables alch_tables(int n, const int32_t *ss_alchemy, const double *rmin, con
   T.ncls = (int)cr.size();
   ORAC_REQUIRE(T.ncls <= LJ_DENSE_MAX, E_UNSUPPORTED, "more than 2048 alchemical classes");
   T.pair.resize((size_t)T.ncls * T.ncls);
+  T.lj.resize(T.pair.size());
+  T.flag.resize(T.ncls);
+  for (int i = 0; i < T.ncls; ++i) T.flag[i] = cs[i] == 1 ? 0 : ATOM_ALCH;
   for (int i = 0; i < T.ncls; ++i)
     for (int j = 0; j < T.ncls; ++j) {
       // force_alchemy.f:432-437
@@ -366,6 +369,9 @@ AlchTables alch_tables(int n, const int32_t *ss_alchemy, const double *rmin, con
       const double epsmin = 4.0 * std::sqrt(ce[i] * ce[j]);
       const double s6 = std::pow(sigma, 6.0);
       T.pair[(size_t)i * T.ncls + j] = make_double4(s6 > 0.0 ? 1.0 / s6 : 0.0, epsmin, cs[i] + cs[j] + 4, sigma);
+      const bool lj = epsmin > 1e-12;
+      T.lj[(size_t)i * T.ncls + j] = lj ? make_double2(epsmin * s6 * s6, epsmin * s6) : make_double2(0.0, 0.0);
+      if (lj) T.flag[i] |= ATOM_LJ;
     }
   return T;
 }

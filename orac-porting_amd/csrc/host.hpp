@@ -164,6 +164,8 @@ struct AlchTables {
   std::vector<int> cls;  // class of each atom
   int ncls = 0;
   std::vector<double4> pair;
+  std::vector<double2> lj;           // {eps sigma^12, eps sigma^6}: the plain LJ form of two normal atoms' pair
+  std::vector<unsigned char> flag;   // per class: ATOM_LJ, ATOM_ALCH
 };
 AlchTables alch_tables(int n, const int32_t *ss_alchemy, const double *rmin, const double *epsm, int opls);
 // alch_fact(1:2, -4:4) as fact[2 * (typeaij + 4) + k]

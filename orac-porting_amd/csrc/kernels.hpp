@@ -6,6 +6,8 @@
 // range by that system's own sizes, so systems of different sizes share a
 // launch and each system's result does not depend on what it is batched with.
 #pragma once
+#include <cmath>
+
 #include "common.hpp"
 
 namespace orac {
@@ -61,7 +63,8 @@ struct PairDesc {
   int ntypes;
   const int *type_table;            // ma x ma, 0-based packed index
   const double *ecc12, *ecc6;
-  const double2 *lj_dense;          // ma x ma {ecc12, ecc6}, or null
+  const double2 *lj_dense;          // ma x ma {ecc12, ecc6} (zeros where ecc6 <= 1e-12), or null
+  const unsigned char *tflag;       // per type: ATOM_LJ when some pair of the type has LJ, ATOM_ALCH
   const int *ex_off, *ex_idx;       // symmetric exclusion CSR (sorted partners)
   const unsigned char *ex_inter;    // atom has an excluded partner outside its own group
   int any_heavy;
@@ -71,7 +74,9 @@ struct PairDesc {
   int nb_slab;                      //   nb_cnt[t] of them (at most nb_slab are stored)
   double co[9];
   double alpha, twrtpi;
+  double ew_exp2, ew_qp, ew_twa;    // -alpha^2 log2(e), 0.3275911 alpha, 2 alpha / sqrt(pi) (set_ewald)
   double r2inn, r2out, rinn0, r2inn0, rout0, r2out0, arsout1, arsout2, arsinn1, arsinn2;
+  double inv_arsout2, inv_arsinn2;  // 1 / arsout2, 1 / arsinn2 (read for switched group pairs only)
   int lskip_ewald, ewald;
   double *fx, *fy, *fz;             // direct forces (written)
   double *part;                     // per-block partials [nblk][16]: uconf[3] ucoul[3] st[9]
@@ -82,11 +87,10 @@ struct PairDesc {
   // atoms start at sorted atom soff[t] (gfirst[t] without).
   const int *perm;
   const int *soff;
-  double4 *sgp;                     // [ngrp] {xpg, ypg, zpg, 0}
-  int4 *sgi;                        // [ngrp] {sorted first atom, first atom, natoms | gss << 8, group}
-  double4 *sap;                     // [natoms] {xp, yp, zp, q}
+  double4 *sgp;                     // [ngrp] {xpg, ypg, zpg, two ints: sorted first atom, natoms | gss << 8}
+  int4 *sgi;                        // half form: [ngrp] {sorted first atom, first atom, natoms | gss << 8, group}
   float4 *sapf;                     // [natoms] {Cartesian offset from the group centre, q}: mixed-precision pairs
-  double4 *sapc;                    // [natoms] the same in FP64 (FP64 pairs of the owner-atom loop form)
+  double4 *sapc;                    // [natoms] the same in FP64 (FP64 pairs)
   // Half-list form (half = 1, split list layout): the list holds each group
   // pair once (forward entries, upper group l > owner); the forces on the
   // neighbour's atoms go to per-pair slots, mirror[t * nb_slab + e] the first
@@ -106,7 +110,7 @@ struct PairDesc {
   int rem_kind;
   double rem_f3;
   const float2 *lj_dense32;         // the dense LJ table in FP32 (mixed-precision pairs), or null
-  int2 *sai;                        // [natoms] {type, flags}; flags bit 0 = ex_inter
+  int2 *sai;                        // [natoms] {type << ATOM_FLAG_BITS | ATOM_* flags, atom}
   double *out;                      // [16]: uconf[3], ucoul[3] by typeij, st[9] row-major, dwrk
   int max_group;                    // largest group (atoms)
   // Alchemy (force_alchemy.f): with alch_pair set, `type` is each atom's
@@ -119,6 +123,20 @@ struct PairDesc {
   int alch_shifted;                 // 1: shifted potential (force_alchemy_shifted.f)
 };
 
+// per-atom flags of PairDesc::sai (and of tflag)
+constexpr int ATOM_EX = 1;          // has an excluded partner outside its own group
+constexpr int ATOM_LJ = 2;          // its LJ type has a partner type with LJ
+constexpr int ATOM_ALCH = 4;        // an alchemical (added or removed) atom
+constexpr int ATOM_REM = 8;         // in the REM segment
+constexpr int ATOM_FLAG_BITS = 4;
+// alpha and the factors of r and r^2 that the pair kernel takes from it
+inline void set_ewald(PairDesc &p, double alpha) {
+  p.alpha = alpha;
+  p.twrtpi = 2.0 / std::sqrt(4.0 * std::atan(1.0));
+  p.ew_exp2 = -alpha * alpha * 1.4426950408889634;
+  p.ew_qp = 0.3275911 * alpha;
+  p.ew_twa = p.twrtpi * alpha;
+}
 constexpr int PAIR_WAVES = 4;       // owner groups per 256-thread block
 constexpr int OWN_REG = 3;          // largest owner group of the owner-atom loop form (k_pairs_own)
 // whether the owner-atom loop form (and with it the half-list layout) is in use
@@ -191,10 +209,10 @@ enum ListPhase { LIST_COUNT = 1, LIST_WRITE = 2 };
 void launch_list_build(const ListDesc *d_desc, const ListDesc *h, int nsys, int phases, hipStream_t st);
 // the inner lists of a batch's systems after a slab-layout build (systems with r2m > 0)
 void launch_list_inner(const ListDesc *d_desc, const ListDesc *h, int nsys, hipStream_t st);
-// dense {ecc12, ecc6} table (and its FP32 copy if dense32) from the packed
-// type_table (ma x ma, 1-based, column-major) and ecc12/ecc6
+// dense {ecc12, ecc6} table (and its FP32 copy if dense32) and the types' flags from the packed
+// type_table (ma x ma, 1-based, column-major) and ecc12/ecc6 (tflag: ma rounded up to 8 bytes)
 void launch_lj_dense(int ma, const int *tt, const double *e12, const double *e6, double2 *dense, float2 *dense32,
-                     hipStream_t st);
+                     unsigned char *tflag, hipStream_t st);
 void launch_exclusive_scan(const int *in, int *out, int n, int *total, hipStream_t st);
 
 // half list (CSR) -> full list (CSR) with deterministic order

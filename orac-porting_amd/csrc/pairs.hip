@@ -747,21 +747,26 @@ void launch_list_inner(const ListDesc *d_desc, const ListDesc *h, int nsys, hipS
 // when asked (the mixed-precision pair kernel's).  The host has checked the
 // indices.
 __global__ void __launch_bounds__(256) k_lj_dense(int ma, const int *__restrict__ tt, const double *__restrict__ e12,
-                                                  const double *__restrict__ e6, double2 *dense, float2 *dense32) {
+                                                  const double *__restrict__ e6, double2 *dense, float2 *dense32,
+                                                  unsigned char *tflag) {
   const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= (size_t)ma * ma) return;
   const int i = (int)(k / ma), j = (int)(k - (size_t)i * ma);
   const int lij = tt[i + (size_t)ma * j] - 1;
-  const double2 v = make_double2(e12[lij], e6[lij]);
+  // a pair has LJ where ecc6 > 1e-12 (force.f:455); entries without are zero
+  const bool lj = e6[lij] > 1e-12;
+  const double2 v = make_double2(lj ? e12[lij] : 0.0, lj ? e6[lij] : 0.0);
+  if (lj) tflag[i] = ATOM_LJ;  // (every thread of a row stores the same value)
   dense[k] = v;
   if (dense32) dense32[k] = make_float2((float)v.x, (float)v.y);
 }
 
 void launch_lj_dense(int ma, const int *tt, const double *e12, const double *e6, double2 *dense, float2 *dense32,
-                     hipStream_t st) {
+                     unsigned char *tflag, hipStream_t st) {
   const size_t n = (size_t)ma * ma;
+  launch_zero_u64(reinterpret_cast<unsigned long long *>(tflag), ((size_t)ma + 7) / 8, st);
   if (n > 0) hipLaunchKernelGGL(k_lj_dense, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, ma, tt, e12, e6,
-                                dense, dense32);
+                                dense, dense32, tflag);
 }
 
 // ---------------------------------------------------------------- half -> full

@@ -1,0 +1,116 @@
+"""k_pairs at the sizes where its mapping has edges: owner groups of one to 64
+atoms (batches of owner atoms, classification rounds of fewer entries), passes
+whose lane slots straddle groups, atoms with more exclusions than lanes, and
+lists short enough to end in the first pass; against the oracle's force at the
+tolerances of the other FP64 parity tests (the sums run in another order:
+sqrt(pairs) x 1e-16 and the polynomial exponential's 4e-14)."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import rel, relrms
+from test_gpu_parity import E_TOL, F_TOL, _force_gpu, _oracle_list, _stress_close
+
+pytestmark = pytest.mark.gpu
+
+
+def grouped(sizes, side=12, spacing=2.2, seed=3, many_excluded=False, solute=0.4):
+    """side^3 atoms on a jittered lattice, consecutive atoms in groups of the
+    given sizes (repeated), one group in three a solute group."""
+    from orac_hip import synth
+    rng = np.random.default_rng(seed)
+    n = side ** 3
+    L = side * spacing
+    g = (np.arange(side) + 0.5) * spacing - L / 2
+    x = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3) + rng.uniform(-0.2, 0.2, (n, 3))
+    first = []
+    a = k = 0
+    while a < n:
+        first.append(a)
+        a += sizes[k % len(sizes)]
+        k += 1
+    first = np.array(first)
+    last = np.append(first[1:], n) - 1
+    ng = len(first)
+    atomg = np.repeat(np.arange(1, ng + 1), last - first + 1).astype(np.int32)
+    mass = rng.uniform(1.0, 16.0, n)
+    pmass = mass / np.bincount(atomg - 1, weights=mass)[atomg - 1]
+    sol = rng.random(ng) < solute
+    nt = 5
+    tt, e12, e6 = synth._lj_tables(rng.uniform(1.6, 2.4, nt), np.array([0.15, 0.0, 0.1, 0.2, 0.0]))
+    cons = np.zeros((2, 0), np.int32)
+    if many_excluded:  # atom 1 excludes 100 atoms of other groups, 30 more chain pairs
+        far = rng.choice(np.arange(70, n), 100, replace=False)
+        cons = np.concatenate([np.stack([np.zeros(100, int), far]),
+                               np.stack([np.arange(200, 230), np.arange(201, 231)])], axis=1) + 1
+    half = L / 2
+    q = rng.normal(0, 0.3, n)
+    return synth.System(
+        L=L, xp0=x[:, 0] / half, yp0=x[:, 1] / half, zp0=x[:, 2] / half, charge=synth.charge_internal(q - q.mean()),
+        mass=mass, nbtype=rng.integers(1, nt + 1, n).astype(np.int32), ntypes=nt, type_table=tt, ecc12=e12, ecc6=e6,
+        grppt=np.asfortranarray(np.stack([first + 1, last + 1]).astype(np.int32)), atomg=atomg,
+        atomp=atomg.copy(), ss_index=np.where(sol, 1, 2)[atomg - 1].astype(np.int32), pmass=pmass,
+        co=np.asfortranarray(np.diag([half] * 3)), oc=np.asfortranarray(np.diag([1 / half] * 3)),
+        volume=L ** 3, alpha=0.35, nfft=(24, 24, 24), order=4, rcut=6.0, constraints=cons.astype(np.int32))
+
+
+CASES = {
+    "singles": dict(sizes=[1]),
+    "waters": dict(sizes=[3]),
+    "four": dict(sizes=[4]),
+    "mixed": dict(sizes=[1, 3, 2, 5, 1, 4]),
+    "seven_one": dict(sizes=[7, 1, 1]),
+    "largest": dict(sizes=[64, 1, 3, 17]),
+    "exclusions": dict(sizes=[1, 3], many_excluded=True),
+    "few": dict(sizes=[3, 1], side=5, spacing=4.0),
+}
+
+
+@pytest.mark.parametrize("shell", ["single", "outer", "plain"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_force_forms(gpu_ctx, name, shell):
+    s = grouped(**CASES[name])
+    nnlpp, fa, _ = _oracle_list(s)
+    kw = dict(rinn=0.0, rout=s.rcut, rtolinn=0.0, rtolout=s.rtol, rneigh=0.0)
+    if shell == "outer":
+        kw.update(rinn=3.5, rtolinn=0.4, lskip_ewald=True)
+    elif shell == "plain":
+        kw.update(lskip_ewald=True, ewald=False)
+    g = _force_gpu(gpu_ctx, s, nnlpp, fa, **kw)
+    o = O.force(s, nnlpp, fa=fa, **kw)
+    assert relrms(g["f"], o["f"]) < F_TOL
+    for k in ("uconf_slt", "uconf_slv", "uconf_ss", "ucoul_slt", "ucoul_slv", "ucoul_ss"):
+        scale = max(abs(o[k]), 1e-3 * abs(o["uconf_ss"]) + 1e-3 * abs(o["ucoul_ss"]))  # sums of both signs cancel
+        assert abs(g[k] - o[k]) <= E_TOL * max(scale, 1e-300), k
+    assert _stress_close(g["stress"], o["stress"])
+
+
+@pytest.mark.parametrize("name", ["mixed", "largest", "exclusions"])
+def test_mixed_precision_forms(gpu_ctx, name):
+    """The FP32 pair form on the same groups: forces within the mixed-precision bar of FP64."""
+    from orac_hip.api import ResidentSystem
+    s = grouped(**CASES[name])
+    f = []
+    for precision in (0, 1):
+        rs = ResidentSystem(gpu_ctx, s, precision=precision)
+        rs.eval()
+        f.append(rs.results())
+        rs.close()
+    assert relrms(f[1]["f"], f[0]["f"]) < 5e-6
+    assert rel(f[1]["uconf_ss"], f[0]["uconf_ss"]) < 1e-5
+
+
+def test_owner_atoms_order(gpu_ctx):
+    """Groups in another order than their atoms: owners and neighbours are found by their records."""
+    s = grouped(sizes=[3, 1, 2])
+    p = np.random.default_rng(1).permutation(s.ngrp)
+    inv = np.argsort(p)
+    s2 = dataclasses.replace(s, grppt=np.asfortranarray(s.grppt[:, p]), atomg=(inv[s.atomg - 1] + 1).astype(np.int32))
+    nnlpp, fa, _ = _oracle_list(s2)
+    kw = dict(rinn=0.0, rout=s.rcut, rtolinn=0.0, rtolout=s.rtol, rneigh=0.0)
+    g = _force_gpu(gpu_ctx, s2, nnlpp, fa, **kw)
+    o = O.force(s2, nnlpp, fa=fa, **kw)
+    assert relrms(g["f"], o["f"]) < F_TOL
+    assert _stress_close(g["stress"], o["stress"])
