@@ -519,25 +519,25 @@ static int force_impl(orac_hip_ctx *ctx, const int32_t *ss_index, const double *
       max_group = std::max(max_group, glast[g] - gfirst[g] + 1);
       for (int a = gfirst[g]; a <= glast[g]; ++a) agroup[a] = g;
     }
-    // half list (serial nnlpp layout) -> CSR
-    std::vector<int> h_off(ngrp + 1, 0), h_idx;
+    // half list: the prefix of its counts; its entries go to the device as they are
+    std::vector<int> h_off(ngrp + 1, 0);
+    size_t nn = 0;
     if (iz == 1) {
-      size_t n = 0;
       for (int g = 0; g < ngrp; ++g) {
-        int m = nnlpp[n];
+        const int m = nnlpp[nn];
         ORAC_REQUIRE(m >= 0, E_ARG, "negative count in nnlpp");
+        int lo = 1, hi = 1;
         for (int t = 1; t <= m; ++t) {
-          int j = nnlpp[n + t] - 1;
-          ORAC_REQUIRE(j >= 0 && j < ngrp, E_ARG, "nnlpp holds a group index out of range");
-          h_idx.push_back(j);
+          lo = std::min(lo, (int)nnlpp[nn + t]);
+          hi = std::max(hi, (int)nnlpp[nn + t]);
         }
-        h_off[g + 1] = (int)h_idx.size();
-        n += (size_t)m + 1;
+        ORAC_REQUIRE(lo >= 1 && hi <= ngrp, E_ARG, "nnlpp holds a group index out of range");
+        h_off[g + 1] = h_off[g] + m;
+        nn += (size_t)m + 1;
       }
     }
-    if (h_idx.empty()) h_idx.push_back(0);
     int *d_hoff = B.put_vec("f_hoff", h_off, st, false);
-    int *d_hidx = B.put_vec("f_hidx", h_idx, st, false);
+    int *d_nnlpp = B.put("f_nnlpp", nnlpp, nn, st, false);
     double *d_xpg = B.put("f_xpg", xpg, ngrp, st, false), *d_ypg = B.put("f_ypg", ypg, ngrp, st, false),
            *d_zpg = B.put("f_zpg", zpg, ngrp, st, false);
 
@@ -547,7 +547,7 @@ static int force_impl(orac_hip_ctx *ctx, const int32_t *ss_index, const double *
           *itot = B.get<int>("f_itot", 2);
       int tot = 0;
       if (r2inn > 1.0e-5) {
-        launch_inner_list(ngrp, iz, d_hoff, d_hidx, d_xpg, d_ypg, d_zpg, co, r2neigh, cnt, nullptr, nullptr, 0, st);
+        launch_inner_list(ngrp, iz, d_hoff, d_nnlpp, d_xpg, d_ypg, d_zpg, co, r2neigh, cnt, nullptr, nullptr, 0, st);
         launch_exclusive_scan(cnt, ioff, ngrp, itot, st);
         ORAC_HIP(hipMemcpyAsync(&tot, itot, sizeof(int), hipMemcpyDeviceToHost, st));
         ORAC_HIP(hipStreamSynchronize(st));
@@ -557,7 +557,7 @@ static int force_impl(orac_hip_ctx *ctx, const int32_t *ss_index, const double *
                    "force: dimensions of NNLPP1 are insufficient (" + std::to_string(need) + " needed)");
       int *out = B.get<int>("f_iout", (size_t)need + 2);
       if (r2inn > 1.0e-5) {
-        launch_inner_list(ngrp, iz, d_hoff, d_hidx, d_xpg, d_ypg, d_zpg, co, r2neigh, nullptr, ioff, out, 1, st);
+        launch_inner_list(ngrp, iz, d_hoff, d_nnlpp, d_xpg, d_ypg, d_zpg, co, r2neigh, nullptr, ioff, out, 1, st);
       } else {
         // every group gets an empty record [0]
         launch_zero_u64(reinterpret_cast<unsigned long long *>(out), (size_t)(need + 1) / 2, st);
@@ -663,10 +663,10 @@ static int force_impl(orac_hip_ctx *ctx, const int32_t *ss_index, const double *
     p.any_heavy = heavy;
     p.massinfty = massinfty;
     // full list from the half list
-    int *incount = B.get<int>("f_incount", ngrp + 1), *cursor = B.get<int>("f_cursor", ngrp + 1),
+    int *counts = B.get<int>("f_counts", 2 * (size_t)ngrp + 1), *rev = B.get<int>("f_rev", (size_t)h_off[ngrp] + 1),
         *f_off = B.get<int>("f_foff", ngrp + 1), *ftot = B.get<int>("f_ftot", 2);
     int *f_idx = B.get<int>("f_fidx", 2 * (size_t)h_off[ngrp] + 1);
-    launch_half_to_full(ngrp, d_hoff, d_hidx, incount, f_off, f_idx, cursor, ftot, st);
+    launch_half_to_full(ngrp, d_hoff, d_nnlpp, counts, f_off, f_idx, rev, ftot, st);
     p.nb_off = f_off;
     p.nb_idx = f_idx;
     for (int k = 0; k < 9; ++k) p.co[k] = co[k];

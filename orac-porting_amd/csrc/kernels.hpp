@@ -215,12 +215,13 @@ void launch_lj_dense(int ma, const int *tt, const double *e12, const double *e6,
                      unsigned char *tflag, hipStream_t st);
 void launch_exclusive_scan(const int *in, int *out, int n, int *total, hipStream_t st);
 
-// half list (CSR) -> full list (CSR) with deterministic order
-void launch_half_to_full(int ngrp, const int *h_off, const int *h_idx, int *incount, int *f_off, int *f_idx,
-                         int *cursor, int *total, hipStream_t st);
+// half list (nnlpp layout, h_off the prefix of its counts) -> full list (CSR)
+// with deterministic order; counts: 2 ngrp + 1 ints, rev: one per half entry
+void launch_half_to_full(int ngrp, const int *h_off, const int *nnlpp, int *counts, int *f_off, int *f_idx, int *rev,
+                         int *total, hipStream_t st);
 
 // next-inner-shell list written by force.f:259-286
-void launch_inner_list(int ngrp, int iz, const int *h_off, const int *h_idx, const double *xpg, const double *ypg,
+void launch_inner_list(int ngrp, int iz, const int *h_off, const int *nnlpp, const double *xpg, const double *ypg,
                        const double *zpg, const double *co, double r2neigh, int *count, const int *off, int *out,
                        int pass, hipStream_t st);
 

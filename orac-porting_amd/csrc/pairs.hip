@@ -771,57 +771,76 @@ void launch_lj_dense(int ma, const int *tt, const double *e12, const double *e6,
 
 // ---------------------------------------------------------------- half -> full
 
-__global__ void k_h2f_count(int ngrp, const int *h_off, const int *h_idx, int *incount) {
-  int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= ngrp) return;
-  for (int t = h_off[g]; t < h_off[g + 1]; ++t) atomicAdd(&incount[h_idx[t]], 1);
+// The caller's half list stays in its own layout (per group [nv, l1..lnv],
+// 1-based): entry t of group g is at nnlpp[h_off[g] + g + 1 + t], h_off the
+// prefix of the counts.  Each kernel gives a group to a wavefront, its lanes
+// taking the entries: the transpose is bound by the scattered 4-byte counts and
+// entries, and by a sort of ~100 numbers per group, so what matters is lanes in
+// flight (16k atoms, 0.66 M entries: the five kernels take 60 us; with a thread
+// per group and an insertion sort in memory they took 2.3 ms).
+__device__ __forceinline__ int half_entry(const int *nnlpp, const int *h_off, int g, int t) {
+  return nnlpp[(size_t)h_off[g] + g + 1 + t] - 1;
 }
 
-__global__ void k_h2f_total(int ngrp, const int *h_off, int *incount) {
-  int g = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256) k_h2f_count(int ngrp, const int *__restrict__ h_off,
+                                                   const int *__restrict__ nnlpp, int *incount) {
+  const int g = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (g >= ngrp) return;
-  incount[g] += h_off[g + 1] - h_off[g];
+  const int nh = h_off[g + 1] - h_off[g];
+  for (int t = lane; t < nh; t += 64) atomicAdd(&incount[half_entry(nnlpp, h_off, g, t)], 1);
+  if (lane == 0) atomicAdd(&incount[g], nh);
 }
 
-__global__ void k_h2f_fill(int ngrp, const int *h_off, const int *h_idx, const int *f_off, int *f_idx, int *cursor) {
-  int g = blockIdx.x * blockDim.x + threadIdx.x;
+// forward entries to their place in the full list; the reverse ones, in
+// arrival order, to rev (group j's from f_off[j] - h_off[j] on)
+__global__ void __launch_bounds__(256) k_h2f_fill(int ngrp, const int *__restrict__ h_off,
+                                                  const int *__restrict__ nnlpp, const int *__restrict__ f_off,
+                                                  int *__restrict__ f_idx, int *__restrict__ rev, int *cursor) {
+  const int g = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (g >= ngrp) return;
-  int nh = h_off[g + 1] - h_off[g];
-  for (int t = 0; t < nh; ++t) f_idx[f_off[g] + t] = h_idx[h_off[g] + t];
-  for (int t = h_off[g]; t < h_off[g + 1]; ++t) {
-    int j = h_idx[t];
-    int nhj = h_off[j + 1] - h_off[j];
-    int pos = atomicAdd(&cursor[j], 1);
-    f_idx[f_off[j] + nhj + pos] = g;
+  const int nh = h_off[g + 1] - h_off[g], f0 = f_off[g];
+  for (int t = lane; t < nh; t += 64) {
+    const int j = half_entry(nnlpp, h_off, g, t);
+    f_idx[f0 + t] = j;
+    rev[f_off[j] - h_off[j] + atomicAdd(&cursor[j], 1)] = g;
   }
 }
 
-__global__ void k_h2f_sort(int ngrp, const int *h_off, const int *f_off, int *f_idx) {
-  int g = blockIdx.x * blockDim.x + threadIdx.x;
+// the reverse entries in ascending order: an entry's place is the number of
+// entries below it (of equal ones, those before it: a pair listed twice)
+__global__ void __launch_bounds__(256) k_h2f_sort(int ngrp, const int *__restrict__ h_off,
+                                                  const int *__restrict__ f_off, const int *__restrict__ rev,
+                                                  int *__restrict__ f_idx) {
+  const int g = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (g >= ngrp) return;
-  int s = f_off[g] + (h_off[g + 1] - h_off[g]), n = f_off[g + 1] - s;
-  for (int i = 1; i < n; ++i) {
-    int v = f_idx[s + i];
-    int j = i - 1;
-    while (j >= 0 && f_idx[s + j] > v) {
-      f_idx[s + j + 1] = f_idx[s + j];
-      --j;
+  const int nh = h_off[g + 1] - h_off[g], n = f_off[g + 1] - f_off[g] - nh;
+  const int *src = rev + (f_off[g] - h_off[g]);
+  int *dst = f_idx + f_off[g] + nh;
+  for (int i0 = 0; i0 < n; i0 += 64) {
+    const int i = i0 + lane;
+    const int v = i < n ? src[i] : 0;
+    int rank = 0;
+    for (int j0 = 0; j0 < n; j0 += 64) {
+      const int w = j0 + lane < n ? src[j0 + lane] : 0, m = min(64, n - j0);
+      for (int q = 0; q < m; ++q) {
+        const int o = __builtin_amdgcn_readlane(w, q);
+        rank += (o < v || (o == v && j0 + q < i)) ? 1 : 0;
+      }
     }
-    f_idx[s + j + 1] = v;
+    if (i < n) dst[rank] = v;
   }
 }
 
-void launch_half_to_full(int ngrp, const int *h_off, const int *h_idx, int *incount, int *f_off, int *f_idx,
-                         int *cursor, int *total, hipStream_t st) {
-  dim3 b(256), g((ngrp + 255) / 256);
+void launch_half_to_full(int ngrp, const int *h_off, const int *nnlpp, int *counts, int *f_off, int *f_idx, int *rev,
+                         int *total, hipStream_t st) {
   if (ngrp <= 0) return;
-  hipLaunchKernelGGL(k_zero_i32, g, b, 0, st, incount, ngrp + 1);
-  hipLaunchKernelGGL(k_zero_i32, g, b, 0, st, cursor, ngrp);
-  hipLaunchKernelGGL(k_h2f_count, g, b, 0, st, ngrp, h_off, h_idx, incount);
-  hipLaunchKernelGGL(k_h2f_total, g, b, 0, st, ngrp, h_off, incount);
+  const dim3 b(256), g((ngrp + 3) / 4);
+  int *incount = counts, *cursor = counts + ngrp + 1;
+  hipLaunchKernelGGL(k_zero_i32, dim3((2 * ngrp + 1 + 255) / 256), b, 0, st, counts, 2 * ngrp + 1);
+  hipLaunchKernelGGL(k_h2f_count, g, b, 0, st, ngrp, h_off, nnlpp, incount);
   launch_exclusive_scan(incount, f_off, ngrp + 1, total, st);
-  hipLaunchKernelGGL(k_h2f_fill, g, b, 0, st, ngrp, h_off, h_idx, f_off, f_idx, cursor);
-  hipLaunchKernelGGL(k_h2f_sort, g, b, 0, st, ngrp, h_off, f_off, f_idx);
+  hipLaunchKernelGGL(k_h2f_fill, g, b, 0, st, ngrp, h_off, nnlpp, f_off, f_idx, rev, cursor);
+  hipLaunchKernelGGL(k_h2f_sort, g, b, 0, st, ngrp, h_off, f_off, rev, f_idx);
 }
 
 // ---------------------------------------------------------------- inner-shell list
@@ -845,17 +864,17 @@ struct Co9 {
   double m[9];
 };
 
-__global__ void k_inner_list(int ngrp, int iz, const int *h_off, const int *h_idx, const double *xpg,
+__global__ void k_inner_list(int ngrp, int iz, const int *h_off, const int *nnlpp, const double *xpg,
                              const double *ypg, const double *zpg, Co9 co, double r2neigh, int *count, const int *off,
                              int *out, int pass) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= ngrp) return;
   int nv = 0;
-  int b = iz == 1 ? h_off[i] : 0, e = iz == 1 ? h_off[i + 1] : 0;
+  int b = 0, e = iz == 1 ? h_off[i + 1] - h_off[i] : 0;
   int jlo = iz == 1 ? 0 : i + 1, jhi = iz == 1 ? 0 : ngrp;
   int o = pass ? off[i] + i + 1 : 0;
   for (int t = b; t < e; ++t) {
-    int j = h_idx[t];
+    int j = half_entry(nnlpp, h_off, i, t);
     if (centre_d2(xpg, ypg, zpg, co.m, i, j) < r2neigh) {
       if (pass) out[o + nv] = j + 1;
       ++nv;
@@ -871,13 +890,13 @@ __global__ void k_inner_list(int ngrp, int iz, const int *h_off, const int *h_id
   else count[i] = nv;
 }
 
-void launch_inner_list(int ngrp, int iz, const int *h_off, const int *h_idx, const double *xpg, const double *ypg,
+void launch_inner_list(int ngrp, int iz, const int *h_off, const int *nnlpp, const double *xpg, const double *ypg,
                        const double *zpg, const double *co, double r2neigh, int *count, const int *off, int *out,
                        int pass, hipStream_t st) {
   if (ngrp <= 0) return;
   Co9 c;
   for (int k = 0; k < 9; ++k) c.m[k] = co[k];
-  hipLaunchKernelGGL(k_inner_list, dim3((ngrp + 127) / 128), dim3(128), 0, st, ngrp, iz, h_off, h_idx, xpg, ypg, zpg,
+  hipLaunchKernelGGL(k_inner_list, dim3((ngrp + 127) / 128), dim3(128), 0, st, ngrp, iz, h_off, nnlpp, xpg, ypg, zpg,
                      c, r2neigh, count, off, out, pass);
 }
 

@@ -114,3 +114,19 @@ def test_owner_atoms_order(gpu_ctx):
     o = O.force(s2, nnlpp, fa=fa, **kw)
     assert relrms(g["f"], o["f"]) < F_TOL
     assert _stress_close(g["stress"], o["stress"])
+
+
+@pytest.mark.parametrize("ngrp", [1, 2, 64, 65, 130, 216])
+def test_half_list_transpose(gpu_ctx, water216, ngrp):
+    """Every pair of the first ngrp groups listed (group i lists all j > i, in
+    descending order): reverse lists of 0 to ngrp - 1 entries, around the 64
+    lanes of the transpose's sort; forces against the oracle on the same list."""
+    s = water216
+    nnlpp = np.concatenate([np.concatenate([[max(0, ngrp - i)], np.arange(ngrp, i, -1)]) if i <= ngrp else [0]
+                            for i in range(1, s.ngrp + 1)]).astype(np.int32)
+    fa = O.ForceArgs(s)
+    kw = dict(rinn=0.0, rout=s.rcut, rtolinn=0.0, rtolout=s.rtol, rneigh=0.0)
+    g = _force_gpu(gpu_ctx, s, nnlpp, fa, **kw)
+    o = O.force(s, nnlpp, fa=fa, **kw)
+    assert np.abs(g["f"] - o["f"]).max() <= F_TOL * max(np.abs(o["f"]).max(), 1e-300)
+    assert _stress_close(g["stress"], o["stress"])
