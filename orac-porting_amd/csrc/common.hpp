@@ -77,11 +77,11 @@ struct PmeDesc {
   int gather_nblk;
   // LDS-tiled spread: grid tiles of st1 x st2 x st3 points (st = 0: global-atomic spread)
   int st1, st2, st3, nb1, nb2, nb3;
-  int *bin_cnt, *bin_start;     // [nb1*nb2*nb3] atoms per tile bin, exclusive prefix
-  int2 *atom_bin;               // [natoms] {bin, position in bin}
-  double4 *afr;                 // [natoms] {fr1, fr2, fr3, q}
-  double4 *sfr;                 // [natoms] the same, sorted by bin
-  double *swt;                  // [natoms][3][order] B-spline weights of the sorted atoms (exact T values)
+  int *bin_cnt;                 // [nb1*nb2*nb3 + 1] atoms per tile bin; the last: atoms that found their bin full.
+                                //   Zero before an evaluation (the forward FFT leaves them so)
+  double4 *bin_fr;              // [nb1*nb2*nb3][bin_cap] {fr1, fr2, fr3, q} of each bin's atoms
+  double4 *over_fr;             // [natoms] the same of the atoms beyond their bin's capacity
+  int bin_cap;
   int tiled;                    // 1: LDS-tiled spread, 0: global-atomic spread
   double *out;                  // [20]: eer, vir (3x3 col-major), stc1..stc9
   int energy_only;              // 1: spread, forward FFT and energy only (a lambda0 charge grid)
@@ -148,16 +148,26 @@ __host__ __device__ inline T recip_km1(int k) {
   }
 }
 
+// (one rounding per written operation, no contraction: every caller, unrolled
+// or not, gets the same weights bit for bit, and the host the reference's)
+template <typename T>
+__host__ __device__ inline T bspline_term(T div, T w, int k, int j, T lo, T hi) {
+#pragma clang fp contract(off)
+  return div * ((w + T(j)) * lo + (T(k - j) - w) * hi);
+}
+
 template <typename T>
 __host__ __device__ inline void bspline_pass(T *c, T w, int k) {
+#pragma clang fp contract(off)
   T div = recip_km1<T>(k);
   c[k - 1] = div * w * c[k - 2];
-  for (int j = 1; j <= k - 2; ++j) c[k - j - 1] = div * ((w + T(j)) * c[k - j - 2] + (T(k - j) - w) * c[k - j - 1]);
+  for (int j = 1; j <= k - 2; ++j) c[k - j - 1] = bspline_term(div, w, k, j, c[k - j - 2], c[k - j - 1]);
   c[0] = div * (T(1) - w) * c[0];
 }
 
 template <typename T>
 __host__ __device__ inline void fill_bspline(T w, int order, T *c, T *d) {
+#pragma clang fp contract(off)
   c[order - 1] = T(0);
   c[1] = w;
   c[0] = T(1) - w;
@@ -165,6 +175,30 @@ __host__ __device__ inline void fill_bspline(T w, int order, T *c, T *d) {
   d[0] = -c[0];
   for (int j = 2; j <= order; ++j) d[j - 1] = c[j - 2] - c[j - 1];
   bspline_pass(c, w, order);
+}
+
+// the same for an order known at compile time (the loops unroll, and the
+// weights stay in registers)
+template <typename T, int ORDER>
+__device__ __forceinline__ void fill_bspline_n(T w, T *c, T *d) {
+#pragma clang fp contract(off)
+  c[ORDER - 1] = T(0);
+  c[1] = w;
+  c[0] = T(1) - w;
+#pragma unroll
+  for (int k = 3; k <= ORDER; ++k) {
+    if (k == ORDER) {
+      d[0] = -c[0];
+#pragma unroll
+      for (int j = 2; j <= ORDER; ++j) d[j - 1] = c[j - 2] - c[j - 1];
+    }
+    const T div = recip_km1<T>(k);
+    c[k - 1] = div * w * c[k - 2];
+#pragma unroll
+    for (int j = 1; j <= ORDER - 2; ++j)
+      if (j <= k - 2) c[k - j - 1] = bspline_term(div, w, k, j, c[k - j - 2], c[k - j - 1]);
+    c[0] = div * (T(1) - w) * c[0];
+  }
 }
 
 // 64-bit fixed point: round-to-nearest of v*scale, two's complement.

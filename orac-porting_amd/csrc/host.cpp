@@ -256,6 +256,23 @@ CellGrid make_cellgrid(BufSet &B, const std::string &pfx, int ncx, int ncy, int 
   return cg;
 }
 
+// Spread tiles of the largest or smallest edges the grid admits, and the room
+// of their bins: 1.5 x the mean, or 0.2 atoms per cubic A of the tile (above
+// any liquid's or solid's density, so that vacuum elsewhere does not fill a
+// bin), at most about twice the atoms in all.  Atoms beyond it go through the
+// overflow list, which every tile reads.
+static void pme_tiling(PmeDesc &d, bool smallest) {
+  d.st1 = spread_tile_edge(d.K1, d.order, smallest);
+  d.st2 = spread_tile_edge(d.K2, d.order, smallest);
+  d.st3 = spread_tile_edge(d.K3, d.order, smallest);
+  d.nb1 = d.K1 / d.st1;
+  d.nb2 = d.K2 / d.st2;
+  d.nb3 = d.K3 / d.st3;
+  const double nbin = (double)d.nb1 * d.nb2 * d.nb3, mean = d.natoms / nbin;
+  const double want = std::max(1.5 * mean, 0.2 * d.volume / nbin) + 16.0;
+  d.bin_cap = (int)std::min({want, 2.0 * mean + 48.0, (double)std::max(1, d.natoms)});
+}
+
 // Device PME descriptor of one system: grids, B-spline moduli, partial-sum
 // buffers sized for any tuning, spread bins when the grid admits tiles.
 PmeDesc pme_desc_base(BufSet &B, const std::string &pfx, const PmePlan &P, int natoms, const double *oc,
@@ -293,12 +310,15 @@ PmeDesc pme_desc_base(BufSet &B, const std::string &pfx, const PmePlan &P, int n
             e3 = spread_tile_edge(P.K3, P.order, true);
   if (e1 && e2 && e3) {
     const size_t nbin = (size_t)(P.K1 / e1) * (P.K2 / e2) * (P.K3 / e3);
-    d.bin_cnt = B.get<int>(pfx + "bin_cnt", nbin);
-    d.bin_start = B.get<int>(pfx + "bin_start", nbin);
-    d.atom_bin = B.get<int2>(pfx + "atom_bin", std::max(1, natoms));
-    d.afr = B.get<double4>(pfx + "afr", std::max(1, natoms));
-    d.sfr = B.get<double4>(pfx + "sfr", std::max(1, natoms));
-    d.swt = B.get<double>(pfx + "swt", (size_t)std::max(1, natoms) * 3 * P.order);
+    size_t slots = 0;
+    for (const bool smallest : {false, true}) {
+      pme_tiling(d, smallest);
+      slots = std::max(slots, (size_t)d.nb1 * d.nb2 * d.nb3 * d.bin_cap);
+    }
+    d.bin_cnt = B.get<int>(pfx + "bin_cnt", (nbin + 2) / 2 * 2);
+    launch_zero_u64(reinterpret_cast<unsigned long long *>(d.bin_cnt), (nbin + 2) / 2, st);
+    d.bin_fr = B.get<double4>(pfx + "bin_fr", std::max<size_t>(1, slots));
+    d.over_fr = B.get<double4>(pfx + "over_fr", std::max(1, natoms));
   }
   pme_apply_tuning(d, tu);
   return d;
@@ -311,19 +331,7 @@ void pme_apply_tuning(PmeDesc &d, const Tuning &tu) {
   pme_set_tiles(d, tu.lds_elems);
   d.tiled = 0;
   if (!d.bin_cnt || !tu.spread_tiled || std::getenv("ORAC_HIP_SPREAD_ATOMIC")) return;
-  const int K[3] = {d.K1, d.K2, d.K3};
-  int big[3], small[3];
-  for (int a = 0; a < 3; ++a) {
-    big[a] = spread_tile_edge(K[a], d.order, false);
-    small[a] = spread_tile_edge(K[a], d.order, true);
-  }
-  const int *e = tu.spread_tiled == 2 ? small : big;
-  d.st1 = e[0];
-  d.st2 = e[1];
-  d.st3 = e[2];
-  d.nb1 = K[0] / e[0];
-  d.nb2 = K[1] / e[1];
-  d.nb3 = K[2] / e[2];
+  pme_tiling(d, tu.spread_tiled == 2);
   d.tiled = 1;
 }
 

@@ -36,20 +36,35 @@ __device__ inline cx<T> cscale(cx<T> a, T s) { return {a.x * s, a.y * s}; }
 template <typename T, int S>
 __device__ inline cx<T> cmuli(cx<T> a) { return S > 0 ? cx<T>{-a.y, a.x} : cx<T>{a.y, -a.x}; }
 
+// Quotient of a small index (below 2^20) by a runtime divisor (below 2^11): the
+// float quotient of the half-shifted index is off by less than 2^-2 / d, so its
+// floor is exact, in three instructions rather than an integer division.
+struct FastDiv {
+  int d;
+  float inv;
+  __device__ __forceinline__ explicit FastDiv(int n) : d(n), inv(1.0f / (float)n) {}
+  __device__ __forceinline__ int div(int x) const { return (int)(((float)x + 0.5f) * inv); }
+  __device__ __forceinline__ int div(int x, int &rem) const {
+    const int q = div(x);
+    rem = x - q * d;
+    return q;
+  }
+};
+
+// the axis's twiddle table into LDS (one load per entry and workgroup)
 template <typename T>
-__device__ inline cx<T> twiddle(const FftAxis &ax, int m);
-template <>
-__device__ inline cx<double> twiddle<double>(const FftAxis &ax, int m) {
-  double2 w = ax.tw64[m];
-  return {w.x, w.y};
-}
-template <>
-__device__ inline cx<float> twiddle<float>(const FftAxis &ax, int m) {
-  float2 w = ax.tw32[m];
-  return {w.x, w.y};
+__device__ __forceinline__ void load_twiddles(cx<T> *tw, const FftAxis &ax) {
+  for (int i = threadIdx.x; i < ax.n; i += blockDim.x) {
+    if constexpr (sizeof(T) == 8) {
+      const double2 w = gload(ax.tw64 + i);
+      tw[i] = {w.x, w.y};
+    } else {
+      const float2 w = gload(ax.tw32 + i);
+      tw[i] = {w.x, w.y};
+    }
+  }
 }
 
-// R-point DFT in registers, S = -1 forward (e^{-i}), +1 backward.
 template <typename T, int R, int S>
 __device__ inline void dft(cx<T> *v) {
   if constexpr (R == 2) {
@@ -88,44 +103,44 @@ __device__ inline void dft(cx<T> *v) {
 }
 
 template <typename T, int R, int S>
-__device__ inline void stockham_pass(const cx<T> *a, cx<T> *b, int N, int TP, int Ns, const FftAxis &ax) {
-  const int NR = N / R;
-  const int twstep = N / (Ns * R);
+__device__ inline void stockham_pass(const cx<T> *a, cx<T> *b, int N, int TP, int Ns, const cx<T> *tw) {
+  const FastDiv dNs(Ns), dNR(N / R);
+  const int NR = dNR.d, twstep = FastDiv(Ns * R).div(N);
   for (int bi = threadIdx.x; bi < TP * NR; bi += blockDim.x) {
-    int t = bi / NR, j = bi - t * NR;
+    int j, k;
+    const int t = dNR.div(bi, j), jq = dNs.div(j, k);
     const cx<T> *src = a + t * N;
     cx<T> *dst = b + t * N;
-    int k = j % Ns;
     cx<T> v[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) v[r] = src[j + r * NR];
     if (Ns > 1) {
 #pragma unroll
       for (int r = 1; r < R; ++r) {
-        cx<T> w = twiddle<T>(ax, r * k * twstep);
+        cx<T> w = tw[r * k * twstep];
         if (S > 0) w.y = -w.y;
         v[r] = cmul(v[r], w);
       }
     }
     dft<T, R, S>(v);
-    int idxD = (j / Ns) * Ns * R + k;
+    const int idxD = jq * Ns * R + k;
 #pragma unroll
     for (int r = 0; r < R; ++r) dst[idxD + r * Ns] = v[r];
   }
 }
 
-// TP pencils of length N held in LDS buffer a (b is scratch); returns the
-// buffer that holds the result.
+// TP pencils of length N held in LDS buffer a (b is scratch, tw the axis's
+// twiddles in LDS); returns the buffer that holds the result.
 template <typename T, int S>
-__device__ cx<T> *lds_fft(cx<T> *a, cx<T> *b, int N, int TP, const FftAxis &ax) {
+__device__ cx<T> *lds_fft(cx<T> *a, cx<T> *b, int N, int TP, const FftAxis &ax, const cx<T> *tw) {
   int Ns = 1;
   for (int p = 0; p < ax.nr; ++p) {
     int R = ax.radix[p];
     switch (R) {
-      case 2: stockham_pass<T, 2, S>(a, b, N, TP, Ns, ax); break;
-      case 3: stockham_pass<T, 3, S>(a, b, N, TP, Ns, ax); break;
-      case 4: stockham_pass<T, 4, S>(a, b, N, TP, Ns, ax); break;
-      default: stockham_pass<T, 5, S>(a, b, N, TP, Ns, ax); break;
+      case 2: stockham_pass<T, 2, S>(a, b, N, TP, Ns, tw); break;
+      case 3: stockham_pass<T, 3, S>(a, b, N, TP, Ns, tw); break;
+      case 4: stockham_pass<T, 4, S>(a, b, N, TP, Ns, tw); break;
+      default: stockham_pass<T, 5, S>(a, b, N, TP, Ns, tw); break;
     }
     __syncthreads();
     cx<T> *t = a;
@@ -204,84 +219,56 @@ __global__ void __launch_bounds__(256) k_spread(const PmeDesc *__restrict__ D) {
 // atoms with b in [t0, t0 + st + order - 2] per axis, i.e. from bins T and
 // T + 1 (mod nb) when st >= order - 1 and st divides K.  One workgroup per
 // tile accumulates those contributions in LDS with int64 atomics and stores
-// its points: every grid point has one owner, no global atomics, no clearing.
-
-__global__ void __launch_bounds__(256) k_bin_zero(const PmeDesc *__restrict__ D) {
-  const PmeDesc &d = D[blockIdx.y];
-  if (!d.tiled) return;
-  int nb = d.nb1 * d.nb2 * d.nb3;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += gridDim.x * blockDim.x) d.bin_cnt[i] = 0;
-}
-
-// Neighbouring atoms fall in the same tile, so a wavefront's atoms share a
-// handful of bins: lanes of one bin are counted with one atomic by their
-// lowest lane, and each lane takes base + its rank among them.
-__global__ void __launch_bounds__(256) k_bin_count(const PmeDesc *__restrict__ D) {
+// its points: every grid point has one owner, no global atomics, no clearing,
+// and sums of integers do not depend on their order.
+//
+// k_bin puts each atom straight into its bin's slots (fixed capacity, an
+// overflow list beyond it), so no scan and no second pass over the atoms is
+// needed: 20 + 5 + 6 us of counting, scanning and filling for 24,460 atoms
+// became one kernel of 5.5 us.
+__global__ void __launch_bounds__(256) k_bin(const PmeDesc *__restrict__ D) {
   const PmeDesc &d = D[blockIdx.y];
   if (!d.tiled) return;
   const int a = blockIdx.x * blockDim.x + threadIdx.x;
   const int lane = threadIdx.x & 63;
   int bin = -1;
+  double4 f = make_double4(0.0, 0.0, 0.0, 0.0);
   if (a < d.natoms) {
     double x, y, z;
-    cartesian(d.co, d.xp[a], d.yp[a], d.zp[a], x, y, z);
+    cartesian(d.co, gmem(d.xp)[a], gmem(d.yp)[a], gmem(d.zp)[a], x, y, z);
     double fr1 = frac_coord(x, y, z, d.recip, 0, d.K1);
     double fr2 = frac_coord(x, y, z, d.recip, 1, d.K2);
     double fr3 = frac_coord(x, y, z, d.recip, 2, d.K3);
-    if (!(fr1 >= 0.0 && fr1 <= d.K1 && fr2 >= 0.0 && fr2 <= d.K2 && fr3 >= 0.0 && fr3 <= d.K3)) {
-      d.atom_bin[a] = make_int2(-1, 0);  // non-finite coordinates are not spread
-    } else {
+    // (non-finite coordinates are not spread)
+    if (fr1 >= 0.0 && fr1 <= d.K1 && fr2 >= 0.0 && fr2 <= d.K2 && fr3 >= 0.0 && fr3 <= d.K3) {
       // fr = K (w - anint(w) = 0.5 exactly) is the grid origin: same spline weights
       if (fr1 >= d.K1) fr1 -= d.K1;
       if (fr2 >= d.K2) fr2 -= d.K2;
       if (fr3 >= d.K3) fr3 -= d.K3;
-      d.afr[a] = make_double4(fr1, fr2, fr3, d.q[a]);
-      int b1 = (int)fr1, b2 = (int)fr2, b3 = (int)fr3;
-      bin = b1 / d.st1 + d.nb1 * (b2 / d.st2 + d.nb2 * (b3 / d.st3));
+      f = make_double4(fr1, fr2, fr3, gmem(d.q)[a]);
+      bin = (int)fr1 / d.st1 + d.nb1 * ((int)fr2 / d.st2 + d.nb2 * ((int)fr3 / d.st3));
     }
   }
-  unsigned long long todo = __ballot(bin >= 0);
-  int pos = 0;
+  // Neighbouring atoms fall in the same tile: the lanes of one bin are counted
+  // by one atomic of their lowest lane, all bins' atomics in flight together.
+  unsigned long long todo = __ballot(bin >= 0), mine = 0ull;
   while (todo) {  // the same on every lane of the wavefront
-    const int leader = __ffsll((long long)todo) - 1;
-    const int lb = __shfl(bin, leader, 64);
+    const int lb = __builtin_amdgcn_readlane(bin, __ffsll((long long)todo) - 1);
     const unsigned long long same = __ballot(bin == lb);
-    int base = 0;
-    if (lane == leader) base = atomicAdd(&d.bin_cnt[lb], __popcll(same));
-    base = __shfl(base, leader, 64);
-    if (bin == lb) pos = base + __popcll(same & ((1ull << lane) - 1ull));
+    if (bin == lb) mine = same;
     todo &= ~same;
   }
-  if (bin >= 0) d.atom_bin[a] = make_int2(bin, pos);
-}
-
-// one block per system: exclusive prefix of the bin counts, fixed order
-__global__ void __launch_bounds__(1024) k_bin_scan(const PmeDesc *__restrict__ D) {
-  const PmeDesc &d = D[blockIdx.x];
-  if (!d.tiled) return;
-  block_exclusive_scan(d.bin_cnt, d.bin_start, d.nb1 * d.nb2 * d.nb3);
-}
-
-// atoms into bin order, with their B-spline weights along the three axes
-// (computed once here instead of once per tile and stencil plane)
-template <typename T>
-__global__ void __launch_bounds__(256) k_bin_fill(const PmeDesc *__restrict__ D) {
-  const PmeDesc &d = D[blockIdx.y];
-  int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (!d.tiled || a >= d.natoms) return;
-  int2 bp = d.atom_bin[a];
-  if (bp.x < 0) return;
-  const int s = d.bin_start[bp.x] + bp.y, order = d.order;
-  const double4 f = d.afr[a];
-  d.sfr[s] = f;
-  double *w = d.swt + (size_t)s * 3 * order;
-  T th[MAX_ORDER], dd[MAX_ORDER];
-  fill_bspline<T>(T(f.x - (int)f.x), order, th, dd);
-  for (int i = 0; i < order; ++i) w[i] = (double)th[i];
-  fill_bspline<T>(T(f.y - (int)f.y), order, th, dd);
-  for (int i = 0; i < order; ++i) w[order + i] = (double)th[i];
-  fill_bspline<T>(T(f.z - (int)f.z), order, th, dd);
-  for (int i = 0; i < order; ++i) w[2 * order + i] = (double)th[i];
+  if (bin < 0) mine = 1ull << lane;
+  const int leader = __ffsll((long long)mine) - 1;
+  int base = 0;
+  if (bin >= 0 && lane == leader) base = atomicAdd(&d.bin_cnt[bin], __popcll(mine));
+  base = __shfl(base, leader, 64);
+  if (bin < 0) return;
+  const int pos = base + __popcll(mine & ((1ull << lane) - 1ull));
+  if (pos < d.bin_cap)
+    gstore(d.bin_fr + (size_t)bin * d.bin_cap + pos, f);
+  else
+    gstore(d.over_fr + atomicAdd(&d.bin_cnt[d.nb1 * d.nb2 * d.nb3], 1), f);
 }
 
 constexpr int SPREAD_TILE_MAX = 8;
@@ -310,65 +297,158 @@ __device__ inline AxisRange axis_range(int b, int order, int t0, int st, int K, 
   return r;
 }
 
-// The tile is held in LDS with padded strides (st1 + 1, st2 + 1): z-planes and
-// y-rows of one column then fall on different banks, which the int64 atomics
-// of neighbouring stencil points would otherwise serialise on.  Threads take
-// (atom, z-plane) pairs, 8 planes per atom (order <= 8), 64 atoms per sweep;
-// a pair whose plane lies outside the tile stops at once, the others add
-// their in-tile rows.  Local indices need no modulo: the bin offset tells
-// which atoms come across the periodic boundary.
-constexpr int SPREAD_THREADS = 512;  // 64 atoms x 8 z-planes per sweep
+// k_spread_tile, in two alternating phases.  (1) One thread per candidate of
+// the eight bins, taken as one flat sequence (a lookup in nine prefix sums),
+// so the loads of all bins are in flight together; a candidate that reaches
+// the tile writes its spline weights and tile-local ranges to LDS.  (2) The
+// threads take (listed atom, z-plane, y-row) tasks and add a row's points.
+// Bound by the latency of phase 1 and the LDS atomics of phase 2; 24,460 atoms on
+// 64^3: 16 us, against 33 us when the bins were walked one after the other by
+// (atom, plane) threads that re-read their weights from memory; 16 such systems
+// in one launch 129 us against 344.  256 candidates a round keep the list within
+// 64 KB of LDS at any order; 512 threads share its tasks (22 us with 256).  The tile is padded (st1 + 1,
+// st2 + 1), which keeps z-planes and y-rows of one column on different banks.
+constexpr int SPREAD_THREADS = 512, SPREAD_CAND = 256;  // threads; candidates per round
+constexpr int SPREAD_TILE_WORDS = (SPREAD_TILE_MAX + 1) * (SPREAD_TILE_MAX + 1) * SPREAD_TILE_MAX;
 
+// one listed atom: ranges (l0, ia | ib << 8 per axis), then 3 * order weights, the third times q
 template <typename T>
+__host__ __device__ constexpr int spread_rec_bytes(int order) {
+  return 24 + ((3 * order * (int)sizeof(T) + 7) / 8) * 8;
+}
+template <typename T>
+static size_t spread_lds_bytes(int order) {
+  return (size_t)SPREAD_CAND * spread_rec_bytes<T>(order);
+}
+
+template <typename T, int ORDER>
 __global__ void __launch_bounds__(SPREAD_THREADS) k_spread_tile(const PmeDesc *__restrict__ D) {
-  __shared__ unsigned long long tile[(SPREAD_TILE_MAX + 1) * (SPREAD_TILE_MAX + 1) * SPREAD_TILE_MAX];
+  extern __shared__ __align__(16) unsigned char list[];
+  __shared__ unsigned long long tile[SPREAD_TILE_WORDS];
+  __shared__ int pre[10], bins[8], listed;
   const PmeDesc &d = D[blockIdx.y];
   if (!d.tiled || (int)blockIdx.x >= d.nb1 * d.nb2 * d.nb3) return;
-  const int order = d.order;
-  const int T1 = blockIdx.x % d.nb1, T2 = (blockIdx.x / d.nb1) % d.nb2, T3 = blockIdx.x / (d.nb1 * d.nb2);
+  const int order = ORDER > 0 ? ORDER : d.order;
+  const int nb1 = d.nb1, nb2 = d.nb2, nb3 = d.nb3, cap = d.bin_cap;
+  const int T1 = blockIdx.x % nb1, T2 = (blockIdx.x / nb1) % nb2, T3 = blockIdx.x / (nb1 * nb2);
   const int st1 = d.st1, st2 = d.st2, st3 = d.st3, P1 = st1 + 1, P2 = st2 + 1;
   const int t01 = T1 * st1, t02 = T2 * st2, t03 = T3 * st3;
   const int npts = st1 * st2 * st3;
-  for (int i = threadIdx.x; i < P1 * P2 * st3; i += blockDim.x) tile[i] = 0ull;
+  if (threadIdx.x < 8) {
+    const int sb = threadIdx.x, o1 = sb & 1, o2 = (sb >> 1) & 1, o3 = sb >> 2;
+    // with a single bin along an axis, the +1 neighbour is the same bin: visited once
+    const bool skip = (o1 && nb1 == 1) || (o2 && nb2 == 1) || (o3 && nb3 == 1);
+    const int B1 = T1 + o1 - (T1 + o1 >= nb1 ? nb1 : 0), B2 = T2 + o2 - (T2 + o2 >= nb2 ? nb2 : 0),
+              B3 = T3 + o3 - (T3 + o3 >= nb3 ? nb3 : 0);
+    const int bin = B1 + nb1 * (B2 + nb2 * B3);
+    const int n = skip ? 0 : min(gmem(d.bin_cnt)[bin], cap);
+    bins[sb] = bin;
+    int x = n;
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) {
+      const int y = __shfl_up(x, off, 8);
+      if (sb >= off) x += y;
+    }
+    pre[sb + 1] = x;
+    if (sb == 0) pre[0] = 0;
+    if (sb == 7) pre[9] = x + gmem(d.bin_cnt)[nb1 * nb2 * nb3];  // then the overflow list
+  }
+  if (threadIdx.x == 0) listed = 0;
+  for (int i = threadIdx.x; i < P1 * P2 * st3; i += SPREAD_THREADS) tile[i] = 0ull;
   __syncthreads();
   const double scale = d.fixscale;
-  const int slot = threadIdx.x >> 3, i3 = threadIdx.x & 7;
-  for (int sb = 0; sb < 8; ++sb) {
-    const int o1 = sb & 1, o2 = (sb >> 1) & 1, o3 = sb >> 2;
-    // with a single bin along an axis, the +1 neighbour is the same bin: visit it once
-    if ((o1 && d.nb1 == 1) || (o2 && d.nb2 == 1) || (o3 && d.nb3 == 1)) continue;
-    const int w1 = T1 + o1 >= d.nb1, w2 = T2 + o2 >= d.nb2, w3 = T3 + o3 >= d.nb3;
-    const int B1 = T1 + o1 - (w1 ? d.nb1 : 0), B2 = T2 + o2 - (w2 ? d.nb2 : 0), B3 = T3 + o3 - (w3 ? d.nb3 : 0);
-    const int bin = B1 + d.nb1 * (B2 + d.nb2 * B3);
-    const int s = d.bin_start[bin], n = d.bin_cnt[bin];
-    for (int at = slot; at < n; at += SPREAD_THREADS / 8) {
-      if (i3 >= order) continue;
-      const double4 f = d.sfr[s + at];
-      const AxisRange z = axis_range((int)f.z, order, t03, st3, d.K3, w3);
-      int lz = z.l0 + i3;
-      if (lz < 0) lz += z.wrap;
-      if (lz < 0 || lz >= st3) continue;
-      const AxisRange x = axis_range((int)f.x, order, t01, st1, d.K1, w1);
-      const AxisRange y = axis_range((int)f.y, order, t02, st2, d.K2, w2);
-      const double *wt = d.swt + (size_t)(s + at) * 3 * order;
-      const T q3 = T(wt[2 * order + i3]) * T(f.w);
-      for (int i2 = y.ia; i2 < y.ib; ++i2) {
-        int ly = y.l0 + i2;
-        if (ly < 0) ly += y.wrap;
-        const T prod = T(wt[order + i2]) * q3;
-        unsigned long long *row = tile + P1 * (ly + P2 * lz);
-        for (int i1 = x.ia; i1 < x.ib; ++i1) {
-          int lx = x.l0 + i1;
-          if (lx < 0) lx += x.wrap;
-          atomicAdd(&row[lx], to_fix((double)(T(wt[i1]) * prod), scale));
+  const int in_bins = pre[8], total = pre[9], rec = spread_rec_bytes<T>(order);
+  const FastDiv dO2(order * order), dO(order);
+  for (int q0 = 0; q0 < total; q0 += SPREAD_CAND) {
+    // ---- (1) candidates
+    const int qi = q0 + threadIdx.x;
+    if (qi < total && (int)threadIdx.x < SPREAD_CAND) {
+      double4 f;
+      if (qi < in_bins) {
+        int sb = 0;
+#pragma unroll
+        for (int k = 1; k < 8; ++k) sb += pre[k] <= qi ? 1 : 0;
+        f = gload(d.bin_fr + (size_t)bins[sb] * cap + (qi - pre[sb]));
+      } else {
+        f = gload(d.over_fr + (qi - in_bins));
+      }
+      const int b1 = (int)f.x, b2 = (int)f.y, b3 = (int)f.z;
+      // the atom comes across the periodic boundary when its base point lies below the tile's origin
+      const AxisRange x = axis_range(b1, order, t01, st1, d.K1, b1 < t01), y = axis_range(b2, order, t02, st2, d.K2, b2 < t02),
+                      z = axis_range(b3, order, t03, st3, d.K3, b3 < t03);
+      if (x.ia < x.ib && y.ia < y.ib && z.ia < z.ib) {
+        unsigned char *rp = list + (size_t)atomicAdd(&listed, 1) * rec;
+        int *ri = reinterpret_cast<int *>(rp);
+        T *w = reinterpret_cast<T *>(rp + 24);
+        ri[0] = x.l0;
+        ri[1] = x.ia | x.ib << 8;
+        ri[2] = y.l0;
+        ri[3] = y.ia | y.ib << 8;
+        ri[4] = z.l0;
+        ri[5] = z.ia | z.ib << 8;
+        constexpr int NO = ORDER > 0 ? ORDER : MAX_ORDER;
+        T th[NO], dd[NO];
+        const T qt = T(f.w);
+        if constexpr (ORDER > 0) {
+          fill_bspline_n<T, ORDER>(T(f.x - b1), th, dd);
+#pragma unroll
+          for (int i = 0; i < NO; ++i) w[i] = th[i];
+          fill_bspline_n<T, ORDER>(T(f.y - b2), th, dd);
+#pragma unroll
+          for (int i = 0; i < NO; ++i) w[NO + i] = th[i];
+          fill_bspline_n<T, ORDER>(T(f.z - b3), th, dd);
+#pragma unroll
+          for (int i = 0; i < NO; ++i) w[2 * NO + i] = th[i] * qt;
+        } else {
+          fill_bspline<T>(T(f.x - b1), order, th, dd);
+          for (int i = 0; i < order; ++i) w[i] = th[i];
+          fill_bspline<T>(T(f.y - b2), order, th, dd);
+          for (int i = 0; i < order; ++i) w[order + i] = th[i];
+          fill_bspline<T>(T(f.z - b3), order, th, dd);
+          for (int i = 0; i < order; ++i) w[2 * order + i] = th[i] * qt;
         }
       }
     }
+    __syncthreads();
+    // ---- (2) rows
+    const int ntask = listed * order * order;
+    for (int task = threadIdx.x; task < ntask; task += SPREAD_THREADS) {
+      int row, i2;
+      const int at = dO2.div(task, row), i3 = dO.div(row, i2);
+      const unsigned char *rp = list + (size_t)at * rec;
+      const int *ri = reinterpret_cast<const int *>(rp);
+      if (i3 < (ri[5] & 255) || i3 >= ri[5] >> 8 || i2 < (ri[3] & 255) || i2 >= ri[3] >> 8) continue;
+      int lz = ri[4] + i3, ly = ri[2] + i2;
+      if (lz < 0) lz += d.K3;  // (one tile along the axis: the only case with negative in-range points)
+      if (ly < 0) ly += d.K2;
+      const T *w = reinterpret_cast<const T *>(rp + 24);
+      const T prod = w[order + i2] * w[2 * order + i3];
+      unsigned long long *trow = tile + P1 * (ly + P2 * lz);
+      const int l0 = ri[0], ia = ri[1] & 255, ib = ri[1] >> 8;
+      if constexpr (ORDER > 0) {
+#pragma unroll
+        for (int i1 = 0; i1 < ORDER; ++i1) {
+          int lx = l0 + i1;
+          if (lx < 0) lx += d.K1;
+          if (i1 >= ia && i1 < ib) atomicAdd(&trow[lx], to_fix((double)(w[i1] * prod), scale));
+        }
+      } else {
+        for (int i1 = ia; i1 < ib; ++i1) {
+          int lx = l0 + i1;
+          if (lx < 0) lx += d.K1;
+          atomicAdd(&trow[lx], to_fix((double)(w[i1] * prod), scale));
+        }
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) listed = 0;
+    __syncthreads();
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < npts; i += blockDim.x) {
-    const int lx = i % st1, ly = (i / st1) % st2, lz = i / (st1 * st2);
-    d.Qfix[(size_t)(t01 + lx) + (size_t)d.K1 * ((t02 + ly) + (size_t)d.K2 * (t03 + lz))] =
+  const FastDiv d1(st1), d2(st2);
+  for (int i = threadIdx.x; i < npts; i += SPREAD_THREADS) {
+    int lx, ly;
+    const int yz = d1.div(i, lx), lz = d2.div(yz, ly);
+    gmem(d.Qfix)[(size_t)(t01 + lx) + (size_t)d.K1 * ((t02 + ly) + (size_t)d.K2 * (t03 + lz))] =
         tile[lx + P1 * (ly + P2 * lz)];
   }
 }
@@ -398,21 +478,28 @@ __global__ void __launch_bounds__(256) k_fft_x_r2c(const PmeDesc *__restrict__ D
   if ((int)blockIdx.x >= d.gx) return;
   cx<T> *a = reinterpret_cast<cx<T> *>(smem);
   cx<T> *b = a + TP * N;
+  cx<T> *tw = b + TP * N;
   const int row0 = blockIdx.x * TP;
   const double inv = d.fixinv;
+  const FastDiv dN(N), dH(H);
+  load_twiddles(tw, d.ax1);
   for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
-    int t = i / N, e = i - t * N;
-    int row = row0 + t;
+    int e;
+    const int row = row0 + dN.div(i, e);
     T v = T(0);
-    if (row < rows) v = T((double)(long long)d.Qfix[(size_t)row * N + e] * inv);
+    if (row < rows) v = T((double)(long long)gmem(d.Qfix)[(size_t)row * N + e] * inv);
     a[i] = {v, T(0)};
   }
+  // the spread is done with its bins: empty for the next evaluation
+  if (d.tiled)
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i <= d.nb1 * d.nb2 * d.nb3; i += d.gx * blockDim.x)
+      gmem(d.bin_cnt)[i] = 0;
   __syncthreads();
-  cx<T> *r = lds_fft<T, -1>(a, b, N, TP, d.ax1);
+  cx<T> *r = lds_fft<T, -1>(a, b, N, TP, d.ax1, tw);
   cx<T> *FQ = reinterpret_cast<cx<T> *>(d.FQ);
   for (int i = threadIdx.x; i < TP * H; i += blockDim.x) {
-    int t = i / H, e = i - t * H;
-    int row = row0 + t;
+    int e;
+    const int t = dH.div(i, e), row = row0 + t;
     if (row < rows) FQ[(size_t)row * H + e] = r[t * N + e];
   }
 }
@@ -435,19 +522,22 @@ __global__ void __launch_bounds__(256) k_fft_pencil(const PmeDesc *__restrict__ 
   cx<T> *a = reinterpret_cast<cx<T> *>(smem);
   cx<T> *b = a + TP * N;
   cx<T> *FQ = reinterpret_cast<cx<T> *>(d.FQ);
+  cx<T> *tw = b + TP * N;
+  const FastDiv dTP(TP), dH(H);
+  load_twiddles(tw, ax);
   for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
-    int e = i / TP, t = i - e * TP;
-    int p = p0 + t;
+    int t, pr;
+    const int e = dTP.div(i, t), p = p0 + t, pq = dH.div(p, pr);
     cx<T> v = {T(0), T(0)};
-    if (p < npen) v = FQ[(size_t)(p % H) + (size_t)(p / H) * S1 + (size_t)e * Se];
+    if (p < npen) v = FQ[(size_t)pr + (size_t)pq * S1 + (size_t)e * Se];
     a[t * N + e] = v;
   }
   __syncthreads();
-  cx<T> *r = lds_fft<T, S>(a, b, N, TP, ax);
+  cx<T> *r = lds_fft<T, S>(a, b, N, TP, ax, tw);
   for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
-    int e = i / TP, t = i - e * TP;
-    int p = p0 + t;
-    if (p < npen) FQ[(size_t)(p % H) + (size_t)(p / H) * S1 + (size_t)e * Se] = r[t * N + e];
+    int t, pr;
+    const int e = dTP.div(i, t), p = p0 + t, pq = dH.div(p, pr);
+    if (p < npen) FQ[(size_t)pr + (size_t)pq * S1 + (size_t)e * Se] = r[t * N + e];
   }
 }
 
@@ -467,17 +557,19 @@ __global__ void __launch_bounds__(256) k_fft_z_conv(const PmeDesc *__restrict__ 
   double acc[7] = {0, 0, 0, 0, 0, 0, 0};
   cx<T> *FQ = reinterpret_cast<cx<T> *>(d.FQ);
   cx<T> *a = reinterpret_cast<cx<T> *>(smem);
-  cx<T> *b = a + TP * N;
+  cx<T> *b = a + TP * N, *tw = b + TP * N;
+  const FastDiv dTP(TP), dH(H);
   if (p0 < npen) {
+    load_twiddles(tw, d.ax3);
     for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
-      int e = i / TP, t = i - e * TP;
-      int p = p0 + t;
+      int t;
+      const int e = dTP.div(i, t), p = p0 + t;
       cx<T> v = {T(0), T(0)};
       if (p < npen) v = FQ[(size_t)p + (size_t)e * Se];
       a[t * N + e] = v;
     }
     __syncthreads();
-    cx<T> *r = lds_fft<T, -1>(a, b, N, TP, d.ax3);
+    cx<T> *r = lds_fft<T, -1>(a, b, N, TP, d.ax3, tw);
     cx<T> *s = (r == a) ? b : a;
     const int nfft1 = d.K1, nfft2 = d.K2, nfft3 = d.K3, ndim1 = H;
     int nf1 = nfft1 / 2; if (2 * nf1 < nfft1) nf1 += 1;
@@ -485,10 +577,11 @@ __global__ void __launch_bounds__(256) k_fft_z_conv(const PmeDesc *__restrict__ 
     int nf3 = nfft3 / 2; if (2 * nf3 < nfft3) nf3 += 1;
     const double pi = d.pi_f32, fac = d.fac;
     for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
-      int e = i / TP, t = i - e * TP;
-      int p = p0 + t;
+      int t, pr;
+      const int e = dTP.div(i, t), p = p0 + t;
       if (p >= npen) continue;
-      int k1 = p % H + 1, k2 = p / H + 1, k3 = e + 1;  // 1-based as in scalar_sum
+      const int pq = dH.div(p, pr);
+      int k1 = pr + 1, k2 = pq + 1, k3 = e + 1;  // 1-based as in scalar_sum
       cx<T> qv = r[t * N + e];
       if (k1 == 1 && k2 == 1 && k3 == 1) continue;     // ind = 0 is never scaled
       int m1 = k1 - 1; if (k1 > nf1) m1 = k1 - 1 - nfft1;
@@ -530,10 +623,10 @@ __global__ void __launch_bounds__(256) k_fft_z_conv(const PmeDesc *__restrict__ 
     }
     __syncthreads();
     if (!d.energy_only) {
-      cx<T> *o = lds_fft<T, +1>(r, s, N, TP, d.ax3);
+      cx<T> *o = lds_fft<T, +1>(r, s, N, TP, d.ax3, tw);
       for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
-        int e = i / TP, t = i - e * TP;
-        int p = p0 + t;
+        int t;
+        const int e = dTP.div(i, t), p = p0 + t;
         if (p < npen) FQ[(size_t)p + (size_t)e * Se] = o[t * N + e];
       }
     }
@@ -562,11 +655,14 @@ __global__ void __launch_bounds__(256) k_fft_x_c2r(const PmeDesc *__restrict__ D
   if ((int)blockIdx.x >= d.gx || d.energy_only) return;
   cx<T> *a = reinterpret_cast<cx<T> *>(smem);
   cx<T> *b = a + TP * N;
+  cx<T> *tw = b + TP * N;
   const int row0 = blockIdx.x * TP;
   const cx<T> *FQ = reinterpret_cast<const cx<T> *>(d.FQ);
+  const FastDiv dN(N), dH(H);
+  load_twiddles(tw, d.ax1);
   for (int i = threadIdx.x; i < TP * H; i += blockDim.x) {
-    int t = i / H, e = i - t * H;
-    int row = row0 + t;
+    int e;
+    const int t = dH.div(i, e), row = row0 + t;
     cx<T> v = {T(0), T(0)};
     if (row < rows) v = FQ[(size_t)row * H + e];
     if (e == 0 || 2 * e == N) v.y = T(0);
@@ -574,11 +670,11 @@ __global__ void __launch_bounds__(256) k_fft_x_c2r(const PmeDesc *__restrict__ D
     if (e > 0 && N - e >= H) a[t * N + (N - e)] = {v.x, -v.y};
   }
   __syncthreads();
-  cx<T> *r = lds_fft<T, +1>(a, b, N, TP, d.ax1);
+  cx<T> *r = lds_fft<T, +1>(a, b, N, TP, d.ax1, tw);
   T *Qr = reinterpret_cast<T *>(d.Qr);
   for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
-    int t = i / N, e = i - t * N;
-    int row = row0 + t;
+    int e;
+    const int t = dN.div(i, e), row = row0 + t;
     if (row < rows) Qr[(size_t)row * N + e] = r[t * N + e].x;
   }
 }
@@ -587,13 +683,17 @@ __global__ void __launch_bounds__(256) k_fft_x_c2r(const PmeDesc *__restrict__ D
 
 // `order` lanes per atom, 64 / order atoms per wavefront: lane i3 sums the
 // z-plane i3 of the atom's order^3 stencil, and the partial f1, f2, f3 are
-// summed over the atom's lanes in plane order (fixed order).
-template <typename T>
+// summed over the atom's lanes in plane order (fixed order).  Bound by the
+// latency of order^2 scattered grid loads a lane: with the order known at
+// compile time (ORDER > 0) they are all in flight at once (24,460 atoms, order
+// 5: 20 -> 14 us in FP64).  Orders 4 to 6, what simulations use, are written
+// out; a launch of other or mixed orders takes the order at run time.
+template <typename T, int ORDER>
 __global__ void __launch_bounds__(256) k_gather(const PmeDesc *__restrict__ D) {
   __shared__ double red[8][9];
   const PmeDesc &d = D[blockIdx.y];
   if ((int)blockIdx.x >= d.gather_nblk || d.energy_only) return;
-  const int order = d.order;
+  const int order = ORDER > 0 ? ORDER : d.order;
   const int apw = 64 / order;
   const int lane = threadIdx.x & 63;
   const int slot = lane / order, sub = lane - slot * order;
@@ -619,26 +719,60 @@ __global__ void __launch_bounds__(256) k_gather(const PmeDesc *__restrict__ D) {
     b1 = (int)fr1;
     b2 = (int)fr2;
     b3 = (int)fr3;
-    T th1[MAX_ORDER], th2[MAX_ORDER], th3[MAX_ORDER], dt1[MAX_ORDER], dt2[MAX_ORDER], dt3[MAX_ORDER];
-    fill_bspline<T>(T(fr1 - b1), order, th1, dt1);
-    fill_bspline<T>(T(fr2 - b2), order, th2, dt2);
-    fill_bspline<T>(T(fr3 - b3), order, th3, dt3);
-    const T *Qr = reinterpret_cast<const T *>(d.Qr);
+    constexpr int NO = ORDER > 0 ? ORDER : MAX_ORDER;
+    T th1[NO], th2[NO], th3[NO], dt1[NO], dt2[NO], dt3[NO];
+    const auto Qr = gmem(reinterpret_cast<const T *>(d.Qr));
     const int i3 = sub;
-    int kk = wrapK(b3 - order + i3 + 1, d.K3);
-    for (int i2 = 0; i2 < order; ++i2) {
-      int jj = wrapK(b2 - order + i2 + 1, d.K2);
-      const T *row = Qr + (size_t)d.K1 * (jj + (size_t)d.K2 * kk);
-      T s1 = T(0), s23 = T(0);
-      for (int i1 = 0; i1 < order; ++i1) {
-        int ii = wrapK(b1 - order + i1 + 1, d.K1);
-        T g = row[ii];
-        s1 += dt1[i1] * g;
-        s23 += th1[i1] * g;
+    const int kk = wrapK(b3 - order + i3 + 1, d.K3);
+    const unsigned plane = (unsigned)d.K1 * d.K2 * kk;
+    if constexpr (ORDER > 0) {
+      unsigned ii[NO];
+#pragma unroll
+      for (int i1 = 0; i1 < NO; ++i1) ii[i1] = plane + wrapK(b1 - NO + i1 + 1, d.K1);
+      T g[NO][NO];
+#pragma unroll
+      for (int i2 = 0; i2 < NO; ++i2) {
+        const unsigned row = (unsigned)d.K1 * wrapK(b2 - NO + i2 + 1, d.K2);
+#pragma unroll
+        for (int i1 = 0; i1 < NO; ++i1) g[i2][i1] = Qr[row + ii[i1]];
       }
-      f1 -= (double)(s1 * th2[i2] * th3[i3]);
-      f2 -= (double)(s23 * dt2[i2] * th3[i3]);
-      f3 -= (double)(s23 * th2[i2] * dt3[i3]);
+      fill_bspline_n<T, ORDER>(T(fr1 - b1), th1, dt1);
+      fill_bspline_n<T, ORDER>(T(fr2 - b2), th2, dt2);
+      fill_bspline_n<T, ORDER>(T(fr3 - b3), th3, dt3);
+      T t3 = th3[0], d3 = dt3[0];  // this lane's plane
+#pragma unroll
+      for (int k = 1; k < NO; ++k) {
+        t3 = i3 == k ? th3[k] : t3;
+        d3 = i3 == k ? dt3[k] : d3;
+      }
+#pragma unroll
+      for (int i2 = 0; i2 < NO; ++i2) {
+        T s1 = T(0), s23 = T(0);
+#pragma unroll
+        for (int i1 = 0; i1 < NO; ++i1) {
+          s1 += dt1[i1] * g[i2][i1];
+          s23 += th1[i1] * g[i2][i1];
+        }
+        f1 -= (double)(s1 * th2[i2] * t3);
+        f2 -= (double)(s23 * dt2[i2] * t3);
+        f3 -= (double)(s23 * th2[i2] * d3);
+      }
+    } else {
+      fill_bspline<T>(T(fr1 - b1), order, th1, dt1);
+      fill_bspline<T>(T(fr2 - b2), order, th2, dt2);
+      fill_bspline<T>(T(fr3 - b3), order, th3, dt3);
+      for (int i2 = 0; i2 < order; ++i2) {
+        const unsigned row = plane + (unsigned)d.K1 * wrapK(b2 - order + i2 + 1, d.K2);
+        T s1 = T(0), s23 = T(0);
+        for (int i1 = 0; i1 < order; ++i1) {
+          T g = Qr[row + wrapK(b1 - order + i1 + 1, d.K1)];
+          s1 += dt1[i1] * g;
+          s23 += th1[i1] * g;
+        }
+        f1 -= (double)(s1 * th2[i2] * th3[i3]);
+        f2 -= (double)(s23 * dt2[i2] * th3[i3]);
+        f3 -= (double)(s23 * th2[i2] * dt3[i3]);
+      }
     }
   }
   {
@@ -736,7 +870,7 @@ __global__ void __launch_bounds__(256) k_pme_finalize(const PmeDesc *__restrict_
 // ---------------------------------------------------------------- launchers
 
 static int tile_pencils(int n, int npen, int elems) {
-  int tp = elems / n;
+  int tp = std::min(elems / n, (4096 / n - 1) / 2);  // two buffers and the twiddles within 64 KB in FP64
   if (tp < 1) tp = 1;
   if (tp > npen) tp = npen;
   return tp;
@@ -761,6 +895,7 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
   (void)tu;
   if (nsys <= 0) return;
   int max_atoms = 1, max_bins = 1, any_tiled = 0, any_atomic = 0, max_gx = 1, max_gy = 1, max_gz = 1, max_gg = 1;
+  int order = 0, max_order = 0;
   size_t max_grid = 1, shx = 0, shy = 0, shz = 0, max_work = 1;
   for (int s = 0; s < nsys; ++s) {
     const PmeDesc &d = h[s];
@@ -769,9 +904,12 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
     max_gy = std::max(max_gy, d.gy);
     max_gz = std::max(max_gz, d.conv_nblk);
     max_gg = std::max(max_gg, d.gather_nblk);
-    shx = std::max(shx, 2 * (size_t)d.tpx * d.K1 * sizeof(cx<T>));
-    shy = std::max(shy, 2 * (size_t)d.tpy * d.K2 * sizeof(cx<T>));
-    shz = std::max(shz, 2 * (size_t)d.tpz * d.K3 * sizeof(cx<T>));
+    shx = std::max(shx, (2 * (size_t)d.tpx + 1) * d.K1 * sizeof(cx<T>));
+    shy = std::max(shy, (2 * (size_t)d.tpy + 1) * d.K2 * sizeof(cx<T>));
+    shz = std::max(shz, (2 * (size_t)d.tpz + 1) * d.K3 * sizeof(cx<T>));
+    // one spline order in the whole launch: the kernels written out for it
+    order = s == 0 || order == d.order ? d.order : 0;
+    max_order = std::max(max_order, d.order);
     if (d.tiled) {
       any_tiled = 1;
       max_bins = std::max(max_bins, d.nb1 * d.nb2 * d.nb3);
@@ -784,12 +922,15 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
   dim3 blk(256);
   if (ev) ORAC_HIP(hipEventRecord(ev[0], st));
   if (any_tiled) {
-    dim3 ga((max_atoms + 255) / 256, nsys);
-    hipLaunchKernelGGL(k_bin_zero, dim3((max_bins + 255) / 256, nsys), blk, 0, st, d_desc);
-    hipLaunchKernelGGL(k_bin_count, ga, blk, 0, st, d_desc);
-    hipLaunchKernelGGL(k_bin_scan, dim3(nsys), dim3(1024), 0, st, d_desc);
-    hipLaunchKernelGGL(k_bin_fill<T>, ga, blk, 0, st, d_desc);
-    hipLaunchKernelGGL(k_spread_tile<T>, dim3(max_bins, nsys), dim3(SPREAD_THREADS), 0, st, d_desc);
+    hipLaunchKernelGGL(k_bin, dim3((max_atoms + 255) / 256, nsys), blk, 0, st, d_desc);
+    const dim3 gt(max_bins, nsys), bt(SPREAD_THREADS);
+    const size_t sh = spread_lds_bytes<T>(max_order);
+    switch (order) {
+      case 4: hipLaunchKernelGGL((k_spread_tile<T, 4>), gt, bt, sh, st, d_desc); break;
+      case 5: hipLaunchKernelGGL((k_spread_tile<T, 5>), gt, bt, sh, st, d_desc); break;
+      case 6: hipLaunchKernelGGL((k_spread_tile<T, 6>), gt, bt, sh, st, d_desc); break;
+      default: hipLaunchKernelGGL((k_spread_tile<T, 0>), gt, bt, sh, st, d_desc); break;
+    }
   }
   if (any_atomic) {
     unsigned gzero = (unsigned)std::min<size_t>((max_grid + 255) / 256, 4096);
@@ -803,7 +944,12 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
   hipLaunchKernelGGL((k_fft_pencil<T, +1>), dim3(max_gy, nsys), blk, shy, st, d_desc, 2);
   hipLaunchKernelGGL(k_fft_x_c2r<T>, dim3(max_gx, nsys), blk, shx, st, d_desc);
   if (ev) ORAC_HIP(hipEventRecord(ev[2], st));
-  hipLaunchKernelGGL(k_gather<T>, dim3(max_gg, nsys), blk, 0, st, d_desc);
+  switch (order) {
+    case 4: hipLaunchKernelGGL((k_gather<T, 4>), dim3(max_gg, nsys), blk, 0, st, d_desc); break;
+    case 5: hipLaunchKernelGGL((k_gather<T, 5>), dim3(max_gg, nsys), blk, 0, st, d_desc); break;
+    case 6: hipLaunchKernelGGL((k_gather<T, 6>), dim3(max_gg, nsys), blk, 0, st, d_desc); break;
+    default: hipLaunchKernelGGL((k_gather<T, 0>), dim3(max_gg, nsys), blk, 0, st, d_desc); break;
+  }
   if (ev) ORAC_HIP(hipEventRecord(ev[3], st));
   hipLaunchKernelGGL(k_pme_finalize, dim3(16, nsys), dim3(256), 0, st, d_desc);
 }
