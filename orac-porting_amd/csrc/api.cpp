@@ -402,7 +402,7 @@ extern "C" int orac_hip_lc_list(orac_hip_ctx *ctx, int32_t ncx, int32_t ncy, int
     L.cell_of = B.get<int>("l_cellof", natp);
     L.cell_cnt = B.get<int>("l_cnt", ncell + 1);
     L.cell_start = B.get<int>("l_start", ncell + 1);
-    L.cell_cursor = B.get<int>("l_cur", ncell + 1);
+    L.cell_pos = B.get<int>("l_pos", natp);
     L.cell_items = B.get<int>("l_items", natp);
     L.cell_fill = B.get<int>("l_fill", natp);
     L.count = B.get<int>("l_count", natp + 1);
@@ -412,7 +412,7 @@ extern "C" int orac_hip_lc_list(orac_hip_ctx *ctx, int32_t ncx, int32_t ncy, int
     L.mode = 1;
     // pass 1: counts and the capacity check against the caller's array
     ListDesc *dd = B.put("l_desc", &L, 1, st, false);
-    launch_list_build(dd, &L, 1, LIST_COUNT, st);
+    launch_list_build(dd, &L, 1, LIST_ZERO | LIST_COUNT, st);
     int tot[2] = {0, 0};
     ORAC_HIP(hipMemcpyAsync(tot, L.total, sizeof tot, hipMemcpyDeviceToHost, st));
     ORAC_HIP(hipStreamSynchronize(st));

@@ -85,7 +85,7 @@ struct PmeDesc {
   int tiled;                    // 1: LDS-tiled spread, 0: global-atomic spread
   double *out;                  // [20]: eer, vir (3x3 col-major), stc1..stc9
   int energy_only;              // 1: spread, forward FFT and energy only (a lambda0 charge grid)
-  double *fx_dst, *fy_dst, *fz_dst;  // when set, launch_pme_combine adds fx/fy/fz into these
+  double *fx_dst, *fy_dst, *fz_dst;  // when set, launch_tail adds fx/fy/fz into these
   const double *cfx, *cfy, *cfz;     // and then these (the system's correction forces), when set
 };
 
@@ -213,43 +213,135 @@ __device__ inline T wave_sum(T v) {
   return v;
 }
 
-// Exclusive prefix sum of in[0..n) into out by one 1024-thread workgroup, in
-// fixed order; returns the total to every thread.
+// A wave's LDS writes above are read by its other lanes below.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ int lanes_below(unsigned long long m) {
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
+__device__ __forceinline__ double uniform(double v) {
+  int w[2];
+  __builtin_memcpy(w, &v, 8);
+  w[0] = __builtin_amdgcn_readfirstlane(w[0]);
+  w[1] = __builtin_amdgcn_readfirstlane(w[1]);
+  __builtin_memcpy(&v, w, 8);
+  return v;
+}
+__device__ __forceinline__ float uniform(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Quotient of a small index (below 2^20) by a runtime divisor (below 2^11): the
+// float quotient of the half-shifted index is off by less than 2^-2 / d, so its
+// floor is exact, in three instructions rather than an integer division.
+struct FastDiv {
+  int d;
+  float inv;
+  __device__ __forceinline__ explicit FastDiv(int n) : d(n), inv(1.0f / (float)n) {}
+  __device__ __forceinline__ int div(int x) const { return (int)(((float)x + 0.5f) * inv); }
+  __device__ __forceinline__ int div(int x, int &rem) const {
+    const int q = div(x);
+    rem = x - q * d;
+    return q;
+  }
+};
+
+// Sum over a 1024-thread workgroup in fixed order, to every thread.
+__device__ inline double block_sum_1024(double v) {
+  __shared__ double red[16];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) s += red[w];
+  return s;
+}
+
+// Exclusive prefix sum of in[0..n) into out (may be in) by one 1024-thread
+// workgroup; returns the total to every thread.  Each thread takes a contiguous
+// part, so the whole scan has two barriers whatever n.
 __device__ inline int block_exclusive_scan(const int *in, int *out, int n) {
   __shared__ int wsum[16];
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  for (int base = 0; base < n; base += 1024) {
-    const int i = base + threadIdx.x;
-    const int v = i < n ? in[i] : 0;
-    int x = v;
+  const int per = (n + 1023) >> 10, i0 = min(n, (int)threadIdx.x * per), i1 = min(n, i0 + per);
+  int s = 0;
+  for (int i = i0; i < i1; ++i) s += gmem(in)[i];
+  int x = s;
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      int y = __shfl_up(x, off, 64);
-      if (lane >= off) x += y;
-    }
-    if (lane == 63) wsum[wid] = x;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int s = 0;
-      for (int w = 0; w < 16; ++w) {
-        int t = wsum[w];
-        wsum[w] = s;
-        s += t;
-      }
-    }
-    __syncthreads();
-    const int excl = carry + wsum[wid] + x - v;
-    if (i < n) out[i] = excl;
-    __syncthreads();
-    if (threadIdx.x == 1023) carry = excl + v;
-    __syncthreads();
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(x, off, 64);
+    if (lane >= off) x += y;
   }
-  const int total = carry;
-  __syncthreads();  // every thread has read carry before a later call resets it
+  if (lane == 63) wsum[wid] = x;
+  __syncthreads();
+  int base = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    const int v = wsum[w];
+    base += w < wid ? v : 0;
+    total += v;
+  }
+  int run = base + x - s;
+  for (int i = i0; i < i1; ++i) {
+    const int v = gmem(in)[i];
+    gmem(out)[i] = run;
+    run += v;
+  }
+  __syncthreads();  // every thread has read wsum before a later call writes it
   return total;
+}
+
+// d.out[20]: eer, vir(3x3 col-major), stc(3x3 row-major as stc1..stc9).  A
+// 1024-thread workgroup reduces one component in fixed order: k < 7 the
+// convolution partials (scalar_sum.f:125-133 halving and symmetrisation),
+// k >= 7 the molecular-virial partials.
+__device__ inline void pme_finalize(const PmeDesc &d, int k) {
+  if (k >= 7 && d.energy_only) {  // no gather: no molecular-virial terms
+    if (threadIdx.x == 0) d.out[10 + (k - 7)] = 0.0;
+    return;
+  }
+  const double *src = k < 7 ? d.conv_part + k : d.gather_part + (k - 7);
+  const int nrow = k < 7 ? d.conv_nblk : d.gather_nblk, stride = k < 7 ? 8 : 9;
+  double s = 0.0;
+#pragma unroll 4
+  for (int r = threadIdx.x; r < nrow; r += 1024) s += gmem(src)[(size_t)r * stride];
+  s = block_sum_1024(s);
+  if (threadIdx.x != 0) return;
+  double *o = d.out;
+  switch (k) {
+    case 0: o[0] = 0.5 * s; break;
+    case 1: o[1] = 0.5 * s; break;
+    case 2: o[5] = 0.5 * s; break;
+    case 3: o[9] = 0.5 * s; break;
+    case 4: o[4] = o[2] = 0.5 * s; break;  // vir(1,2) = vir(2,1)
+    case 5: o[7] = o[3] = 0.5 * s; break;  // vir(1,3) = vir(3,1)
+    case 6: o[8] = o[6] = 0.5 * s; break;  // vir(2,3) = vir(3,2)
+    default: o[10 + (k - 7)] = s; break;
+  }
+}
+
+// The reciprocal forces of a system evaluated beside its direct sum are
+// written to their own arrays; atom a's are added to its direct force once
+// both are done, and then the corrections.
+__device__ inline void pme_combine(const PmeDesc &d, int a) {
+  if (!d.fx_dst || a >= d.natoms) return;
+  double x = gmem(d.fx_dst)[a] + gmem(d.fx)[a], y = gmem(d.fy_dst)[a] + gmem(d.fy)[a],
+         z = gmem(d.fz_dst)[a] + gmem(d.fz)[a];
+  if (d.cfx) {
+    x += gmem(d.cfx)[a];
+    y += gmem(d.cfy)[a];
+    z += gmem(d.cfz)[a];
+  }
+  gmem(d.fx_dst)[a] = x;
+  gmem(d.fy_dst)[a] = y;
+  gmem(d.fz_dst)[a] = z;
 }
 
 // Workgroups are dealt to the 8 XCDs round robin (hardware id h runs on XCD

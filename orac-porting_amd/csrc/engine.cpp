@@ -109,7 +109,7 @@ struct Batch {
   ListDesc *dl = nullptr;
   CorrDesc *dc = nullptr;
   bool any_corr = false;
-  hipEvent_t fork = nullptr, join = nullptr;  // reciprocal sum on the side stream
+  hipEvent_t fork = nullptr, join = nullptr;  // reciprocal sum and corrections on the side stream
   hipGraph_t graph[2] = {nullptr, nullptr};  // [rebuild]
   hipGraphExec_t exec[2] = {nullptr, nullptr};
   bool profile = false;
@@ -139,8 +139,8 @@ struct Batch {
     }
     for (auto &e : ev)
       if (e) (void)hipEventDestroy(e);
-    if (fork) (void)hipEventDestroy(fork);
-    if (join) (void)hipEventDestroy(join);
+    for (hipEvent_t e : {fork, join})
+      if (e) (void)hipEventDestroy(e);
   }
 };
 
@@ -452,7 +452,7 @@ static void system_build(orac_hip_ctx *ctx, System &S, const orac_hip_system_des
     L.cell_of = B.get<int>("cellof", ng);
     L.cell_cnt = B.get<int>("ccnt", ncell + 1);
     L.cell_start = B.get<int>("cstart", ncell + 1);
-    L.cell_cursor = B.get<int>("ccur", ncell + 1);
+    L.cell_pos = B.get<int>("cpos_in", ng);
     L.cell_items = B.get<int>("citems", ng);
     L.cell_fill = B.get<int>("cfill", ng);
     L.count = B.get<int>("lcount", ng + 1);
@@ -653,8 +653,8 @@ static int batch_create(orac_hip_ctx *ctx, const int32_t *ids, int n) {
     b->sys.push_back(&S);
   }
   for (auto &e : b->ev) ORAC_HIP(hipEventCreate(&e));
-  ORAC_HIP(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
-  ORAC_HIP(hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
+  for (hipEvent_t *e : {&b->fork, &b->join})
+    ORAC_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
   batch_upload(ctx, *b);
   const int id = E.next_batch++;
   E.batches[id] = std::move(b);
@@ -672,38 +672,42 @@ static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events
   auto pme = [&](hipStream_t s) {
     const hipEvent_t *pev = events ? &b.ev[ST_P0] : nullptr;
     if (b.precision == 0)
-      launch_pme<double>(b.dp, b.hp.data(), npme, s, b.tu, pev);
+      launch_pme<double>(b.dp, b.hp.data(), npme, s, b.tu, pev, false);
     else
-      launch_pme<float>(b.dp, b.hp.data(), npme, s, b.tu, pev);
+      launch_pme<float>(b.dp, b.hp.data(), npme, s, b.tu, pev, false);
   };
   mark(ST_BEGIN);
-  launch_centres(b.dq, b.hq.data(), n, st);
+  // in group order (no cell permutation) the pair kernel's records are written with the centres
+  const bool pack = !b.tu.cell_order, lists = md_lists || rebuild;
+  const ListDesc *dl = md_lists ? b.dl_md : b.dl;
+  const std::vector<ListDesc> &hl = md_lists ? b.hl_md : b.hl;  // (md: every system on its own update schedule)
+  launch_centres(b.dq, b.hq.data(), n, st, pack, dl, lists ? hl.data() : nullptr);
   mark(ST_CENTRES);
-  // The reciprocal sum needs the coordinates and the molecule centres only:
-  // unless the stages are being timed it runs on the side stream beside the
-  // list build and the pair kernel (both latency bound), and joins before
-  // its forces are added.
+  // The reciprocal sum needs the coordinates and the molecule centres only,
+  // the corrections the coordinates: unless the stages are being timed they
+  // run on the side stream beside the list build and the pair kernel, and join
+  // before the tail.  One fork and one join: every further edge between the
+  // streams cost more than it overlapped (a fork before the centres with a
+  // wait at the gather, and a third stream for the corrections: 279 against
+  // 231 us for the 24,460-atom system; everything on one stream 269).
   const bool side = !events && ctx->side;
   if (side) {
     ORAC_HIP(hipEventRecord(b.fork, st));
     ORAC_HIP(hipStreamWaitEvent(ctx->side, b.fork, 0));
     pme(ctx->side);
-    if (b.any_corr) launch_corr(b.dc, b.hc.data(), n, ctx->side);
+    if (b.any_corr) launch_corr(b.dc, b.hc.data(), n, ctx->side, false);
     ORAC_HIP(hipEventRecord(b.join, ctx->side));
   }
-  if (md_lists) {  // every system on its own update schedule (device step counters)
-    launch_list_build(b.dl_md, b.hl_md.data(), n, LIST_COUNT | LIST_WRITE, st);
-    if (b.shells) launch_list_inner(b.dl_md, b.hl_md.data(), n, st);
-  } else if (rebuild) {
-    launch_list_build(b.dl, b.hl.data(), n, LIST_COUNT | LIST_WRITE, st);
-    if (b.shells) launch_list_inner(b.dl, b.hl.data(), n, st);
+  if (lists) {
+    launch_list_build(dl, hl.data(), n, LIST_COUNT | LIST_WRITE, st);
+    if (b.shells) launch_list_inner(dl, hl.data(), n, st);
   }
   mark(ST_LIST);
   hipEvent_t kb = events ? b.ev[ST_KBEG] : nullptr, ke = events ? b.ev[ST_KEND] : nullptr;
   if (b.precision == 0)
-    launch_pairs<double>(b.dq, b.hq.data(), n, st, b.tu, kb, ke);
+    launch_pairs<double>(b.dq, b.hq.data(), n, st, b.tu, pack, false, kb, ke);
   else
-    launch_pairs<float>(b.dq, b.hq.data(), n, st, b.tu, kb, ke);
+    launch_pairs<float>(b.dq, b.hq.data(), n, st, b.tu, pack, false, kb, ke);
   mark(ST_PAIRS);
   if (side) {
     ORAC_HIP(hipStreamWaitEvent(st, b.join, 0));
@@ -711,9 +715,9 @@ static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events
   } else {
     pme(st);
     mark(ST_PME);
-    if (b.any_corr) launch_corr(b.dc, b.hc.data(), n, st);
+    if (b.any_corr) launch_corr(b.dc, b.hc.data(), n, st, false);
   }
-  launch_pme_combine(b.dp, b.hp.data(), npme, st);
+  launch_tail(b.dp, b.hp.data(), npme, b.dq, b.any_corr ? b.dc : nullptr, lists ? dl : nullptr, n, st);
   mark(ST_END);
 }
 
@@ -722,11 +726,13 @@ static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events
 static void batch_enqueue_mid(orac_hip_ctx *ctx, Batch &b) {
   hipStream_t st = ctx->stream;
   const int n = (int)b.sys.size();
-  launch_centres(b.dq, b.hq.data(), n, st);
+  // (the inner shell's descriptors share the records of the outer ones)
+  const bool pack = !b.tu.cell_order;
+  launch_centres(b.dq, b.hq.data(), n, st, pack);
   if (b.precision == 0)
-    launch_pairs<double>(b.dqm, b.hqm.data(), n, st, b.tu, nullptr, nullptr);
+    launch_pairs<double>(b.dqm, b.hqm.data(), n, st, b.tu, pack);
   else
-    launch_pairs<float>(b.dqm, b.hqm.data(), n, st, b.tu, nullptr, nullptr);
+    launch_pairs<float>(b.dqm, b.hqm.data(), n, st, b.tu, pack);
 }
 
 static void batch_eval(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool use_graph) {
@@ -777,7 +783,7 @@ static void size_list(orac_hip_ctx *ctx, int32_t id) {
   Batch &b = get_batch(ctx, solo_batch(ctx, id));
   ensure_fresh(ctx, b);
   hipStream_t st = ctx->stream;
-  launch_centres(b.dq, b.hq.data(), 1, st);
+  launch_centres(b.dq, b.hq.data(), 1, st, false, b.dl, b.hl.data());
   launch_list_build(b.dl, b.hl.data(), 1, LIST_COUNT, st);
   int tot[4] = {0, 0, 0, 0};
   ORAC_HIP(hipMemcpyAsync(tot, S.list.total, sizeof tot, hipMemcpyDeviceToHost, st));

@@ -29,37 +29,15 @@ namespace orac {
 #define AS_A5 1.0614054
 #define AS_QP 0.3275911
 
-// Cell-ordered copies of the step's group and atom data: sorted position t
-// holds group perm[t] (identity without a permutation) and its atoms from
-// soff[t] on.  Neighbours listed next to each other are then next to each
-// other in memory, and one group is one 32-byte record.
+// The pair kernel's records in cell order (or, for coordinates that come with
+// their centres, in group order): sorted position t holds group perm[t].
 __global__ void __launch_bounds__(256) k_pack_sorted(const PairDesc *__restrict__ D) {
   const PairDesc &d = D[blockIdx.y];
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= d.ngrp) return;
   const int g = d.perm ? gmem(d.perm)[t] : t;
   const int f0 = gmem(d.gfirst)[g], n = gmem(d.glast)[g] - f0 + 1;
-  const int sf = d.soff ? gmem(d.soff)[t] : f0, gss = gmem(d.gss)[g];
-  const double gx = gmem(d.xpg)[g], gy = gmem(d.ypg)[g], gz = gmem(d.zpg)[g];
-  const int w[2] = {sf, n | (gss << 8)};
-  double4 gp = make_double4(gx, gy, gz, 0.0);
-  __builtin_memcpy(&gp.w, w, 8);
-  gstore(d.sgp + t, gp);
-  if (d.half) gstore(d.sgi + t, make_int4(sf, f0, n | (gss << 8), g));
-  for (int k = 0; k < n; ++k) {
-    const int a = f0 + k;
-    const double q = gmem(d.q)[a];
-    // Cartesian offset from the group centre (upper triangle of co, as
-    // force.f): a pair's separation is the group separation plus the
-    // difference of two small offsets
-    const double dx = gmem(d.xp)[a] - gx, dy = gmem(d.yp)[a] - gy, dz = gmem(d.zp)[a] - gz;
-    const double cx = d.co[0] * dx + d.co[3] * dy + d.co[6] * dz, cy = d.co[4] * dy + d.co[7] * dz, cz = d.co[8] * dz;
-    const int ty = gmem(d.type)[a];
-    const int fl = (gmem(d.ex_inter)[a] ? ATOM_EX : 0) | gmem(d.tflag)[ty] | (d.rematom && gmem(d.rematom)[a] ? ATOM_REM : 0);
-    gstore(d.sai + sf + k, make_int2(ty << ATOM_FLAG_BITS | fl, a));
-    if (d.sapc) gstore(d.sapc + sf + k, make_double4(cx, cy, cz, q));
-    if (d.sapf) gstore(d.sapf + sf + k, make_float4((float)cx, (float)cy, (float)cz, (float)q));
-  }
+  pack_group(d, t, g, d.soff ? gmem(d.soff)[t] : f0, f0, n, gmem(d.xpg)[g], gmem(d.ypg)[g], gmem(d.zpg)[g]);
 }
 
 template <typename P>
@@ -364,30 +342,6 @@ __device__ __forceinline__ int here(int v) {
   asm volatile("" : "+s"(v));
   return v;
 }
-
-// A wave's LDS writes above are read by its other lanes below.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ int lanes_below(unsigned long long m) {
-  return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-}
-
-__device__ __forceinline__ double uniform(double v) {
-  int w[2];
-  __builtin_memcpy(w, &v, 8);
-  w[0] = __builtin_amdgcn_readfirstlane(w[0]);
-  w[1] = __builtin_amdgcn_readfirstlane(w[1]);
-  __builtin_memcpy(&v, w, 8);
-  return v;
-}
-__device__ __forceinline__ float uniform(float v) {
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // Sums of eight values over the 64 lanes; lane l returns the sum of v[l >> 3].
 // Fixed order: lane l adds the eight lanes = l mod 8, then lanes 1, 2, 4 apart.
@@ -876,24 +830,8 @@ static void launch_pair_kernel(bool persistent, dim3 grd, int g, hipStream_t st,
     hipLaunchKernelGGL((k_pairs<T, W, MODE>), grd, blk, 0, st, d_desc, remap);
 }
 
-// d.out[16]: uconf[3], ucoul[3] (slt, slt-slv, slv order of typeij), st[9] row-major,
-// dwrk; block k reduces component k over the per-block partials in fixed order
-__global__ void __launch_bounds__(256) k_pairs_finalize(const PairDesc *__restrict__ D) {
-  __shared__ double red[4];
-  const PairDesc &d = D[blockIdx.y];
-  const int k = blockIdx.x;
-  double s = 0.0;
-  for (int b = threadIdx.x; b < d.nblk; b += blockDim.x) s += gmem(d.part)[(size_t)b * 16 + k];
-  if (d.half && k >= 6 && k < 15)  // the half form's molecular virial of the total forces
-    for (int b = threadIdx.x; b < d.nblk; b += blockDim.x) s += gmem(d.part2)[(size_t)b * 9 + (k - 6)];
-  s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += red[w];
-    d.out[k] = t;
-  }
+__global__ void __launch_bounds__(1024) k_pairs_finalize(const PairDesc *__restrict__ D) {
+  pairs_finalize(D[blockIdx.y], blockIdx.x);
 }
 
 // ================================================================ owner-atom loop form
@@ -1374,7 +1312,7 @@ bool use_owner_kernel() {
 
 template <typename T>
 void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream_t st, const Tuning &tu,
-                  hipEvent_t kbeg, hipEvent_t kend) {
+                  bool packed, bool finalize, hipEvent_t kbeg, hipEvent_t kend) {
   int max_grp = 1, max_blk = 1;
   // half-list systems take the half form, the others k_pairs
   bool any_alch = false, any_rem = false, any_other = false, any_half = false, any_full = false;
@@ -1396,7 +1334,7 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
     if (h[s].max_group > 64)
       throw Error(E_UNSUPPORTED, "groups larger than 64 atoms are not supported by the pair kernel");
   }
-  hipLaunchKernelGGL(k_pack_sorted, dim3((max_grp + 255) / 256, nsys), dim3(256), 0, st, d_desc);
+  if (!packed) hipLaunchKernelGGL(k_pack_sorted, dim3((max_grp + 255) / 256, nsys), dim3(256), 0, st, d_desc);
   dim3 grd(max_blk, nsys);
   const int remap = tu.xcd_remap ? 1 : 0;
   const int waves = pair_occupancy<T>(tu.pair_waves);
@@ -1444,12 +1382,12 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
     }
   }
   if (kend) ORAC_HIP(hipEventRecord(kend, st));
-  hipLaunchKernelGGL(k_pairs_finalize, dim3(PAIR_NACC, nsys), dim3(256), 0, st, d_desc);
+  if (finalize) hipLaunchKernelGGL(k_pairs_finalize, dim3(PAIR_NACC, nsys), dim3(1024), 0, st, d_desc);
 }
 
-template void launch_pairs<double>(const PairDesc *, const PairDesc *, int, hipStream_t, const Tuning &, hipEvent_t,
-                                   hipEvent_t);
-template void launch_pairs<float>(const PairDesc *, const PairDesc *, int, hipStream_t, const Tuning &, hipEvent_t,
-                                  hipEvent_t);
+template void launch_pairs<double>(const PairDesc *, const PairDesc *, int, hipStream_t, const Tuning &, bool, bool,
+                                   hipEvent_t, hipEvent_t);
+template void launch_pairs<float>(const PairDesc *, const PairDesc *, int, hipStream_t, const Tuning &, bool, bool,
+                                  hipEvent_t, hipEvent_t);
 
 }  // namespace orac

@@ -250,6 +250,26 @@ CellGrid make_cellgrid(BufSet &B, const std::string &pfx, int ncx, int ncy, int 
     sten[3 * m + 2] = indxk[1 + 2 * m];
   }
   cg.sten = B.put_vec(pfx + "sten", sten, st, true);
+  // the stencil's runs along z, where every (x, y) offset has one
+  cg.ncol = 0;
+  cg.col = nullptr;
+  if (!half) {
+    std::map<std::pair<int, int>, std::vector<int>> runs;
+    for (int m = 0; m < cg.nsten; ++m) runs[{sten[3 * m], sten[3 * m + 1]}].push_back(sten[3 * m + 2]);
+    std::vector<int4> col;
+    for (auto &r : runs) {
+      std::vector<int> &z = r.second;
+      std::sort(z.begin(), z.end());
+      if (z.back() - z.front() + 1 != (int)z.size() || (int)z.size() > ncz || std::abs(r.first.first) >= ncx ||
+          std::abs(r.first.second) >= ncy || z.front() <= -ncz || z.back() >= ncz) {
+        col.clear();
+        break;
+      }
+      col.push_back(make_int4(r.first.first, r.first.second, z.front(), z.back()));
+    }
+    cg.ncol = (int)col.size();
+    if (cg.ncol > 0) cg.col = B.put_vec(pfx + "col", col, st, true);
+  }
   for (int k = 0; k < 9; ++k) cg.co[k] = co[k];
   cg.sqcut = rcut * rcut;
   cg.half = half;

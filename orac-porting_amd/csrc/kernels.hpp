@@ -29,11 +29,10 @@ struct Tuning {
 void pme_set_tiles(PmeDesc &d, int lds_elems);
 template <typename T>
 // ev (optional, 4 events): recorded before the spread, before the forward FFT,
-// before the gather and after it (the stage timings of a profiled evaluation)
+// before the gather and after it (the stage timings of a profiled evaluation).
+// finalize: reduce the partial sums (else launch_tail does).
 void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st, const Tuning &tu,
-                const hipEvent_t *ev = nullptr);
-// fx_dst += fx (and y, z) for every descriptor that has a destination
-void launch_pme_combine(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st);
+                const hipEvent_t *ev = nullptr, bool finalize = true);
 // tile edge of the LDS-tiled spread along an axis of K points (0: use the atomic spread)
 int spread_tile_edge(int K, int order, bool smallest);
 // Waves per owner group of the pair kernel for a system of ngrp groups (1
@@ -147,13 +146,59 @@ constexpr int MOL_SMALL = 16;       // molecules up to this size get one thread 
 // type_table of the reference (two dependent gathers per pair)
 constexpr int LJ_DENSE_MAX = 2048;
 
+// Group record t (group g, atoms f0 .. f0 + n - 1, centre gx, gy, gz) and its
+// atoms' records from sf on.  Neighbours listed next to each other are next to
+// each other in memory, and one group is one 32-byte record.
+__device__ inline void pack_group(const PairDesc &d, int t, int g, int sf, int f0, int n, double gx, double gy,
+                                  double gz) {
+  const int gss = gmem(d.gss)[g], w[2] = {sf, n | (gss << 8)};
+  double4 gp = make_double4(gx, gy, gz, 0.0);
+  __builtin_memcpy(&gp.w, w, 8);
+  gstore(d.sgp + t, gp);
+  if (d.half) gstore(d.sgi + t, make_int4(sf, f0, n | (gss << 8), g));
+  for (int k = 0; k < n; ++k) {
+    const int a = f0 + k;
+    const double q = gmem(d.q)[a];
+    // Cartesian offset from the group centre (upper triangle of co, as
+    // force.f): a pair's separation is the group separation plus the
+    // difference of two small offsets
+    const double dx = gmem(d.xp)[a] - gx, dy = gmem(d.yp)[a] - gy, dz = gmem(d.zp)[a] - gz;
+    const double cx = d.co[0] * dx + d.co[3] * dy + d.co[6] * dz, cy = d.co[4] * dy + d.co[7] * dz, cz = d.co[8] * dz;
+    const int ty = gmem(d.type)[a];
+    const int fl = (gmem(d.ex_inter)[a] ? ATOM_EX : 0) | gmem(d.tflag)[ty] |
+                   (d.rematom && gmem(d.rematom)[a] ? ATOM_REM : 0);
+    gstore(d.sai + sf + k, make_int2(ty << ATOM_FLAG_BITS | fl, a));
+    if (d.sapc) gstore(d.sapc + sf + k, make_double4(cx, cy, cz, q));
+    if (d.sapf) gstore(d.sapf + sf + k, make_float4((float)cx, (float)cy, (float)cz, (float)q));
+  }
+}
+
+// packed: the systems' records are in place (launch_centres with pack).
+// finalize: reduce the partial sums (else launch_tail does).
 // kbeg/kend (optional) are recorded right before and after the pair kernel itself
 template <typename T>
 void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream_t st, const Tuning &tu,
-                  hipEvent_t kbeg = nullptr, hipEvent_t kend = nullptr);
+                  bool packed = false, bool finalize = true, hipEvent_t kbeg = nullptr, hipEvent_t kend = nullptr);
 
-// group centres (appbou.f) and molecule centres of mass of every system
-void launch_centres(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream_t st);
+// d.out[16]: uconf[3], ucoul[3] (slt, slt-slv, slv order of typeij), st[9]
+// row-major, dwrk; a 1024-thread workgroup reduces component k over the
+// per-block partials in fixed order
+__device__ inline void pairs_finalize(const PairDesc &d, int k) {
+  double s = 0.0;
+#pragma unroll 4
+  for (int b = threadIdx.x; b < d.nblk; b += 1024) s += gmem(d.part)[(size_t)b * 16 + k];
+  if (d.half && k >= 6 && k < 15)  // the half form's molecular virial of the total forces
+    for (int b = threadIdx.x; b < d.nblk; b += 1024) s += gmem(d.part2)[(size_t)b * 9 + (k - 6)];
+  s = block_sum_1024(s);
+  if (threadIdx.x == 0) gmem(d.out)[k] = s;
+}
+
+// group centres (appbou.f) and molecule centres of mass of every system; with
+// pack the pair kernel's records in group order, with a list descriptor per
+// system the counters of the build that follows (LIST_ZERO left out)
+struct ListDesc;
+void launch_centres(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream_t st, bool pack = false,
+                    const ListDesc *d_list = nullptr, const ListDesc *h_list = nullptr);
 
 // linked cells (lc_list.f)
 struct CellGrid {
@@ -164,6 +209,8 @@ struct CellGrid {
   double sqcut;
   int half;                  // 1: l > n only (reference lc_list); 0: every l != n
   double4 *cpos;             // [ngrp] {xpg, ypg, zpg, group} in cell order (filled by the cell build)
+  int ncol;                  // the stencil as runs of cells along z: {dx, dy, first dz, last dz} (0: not as runs)
+  const int4 *col;
 };
 
 // One system's list build: cells of the group centres, then the stencil walk.
@@ -171,7 +218,7 @@ struct ListDesc {
   int ngrp;
   const double *xpg, *ypg, *zpg;
   CellGrid cg;
-  int *cell_of, *cell_cnt, *cell_start, *cell_cursor, *cell_items;
+  int *cell_of, *cell_cnt, *cell_start, *cell_pos, *cell_items;
   int *cell_fill;            // [ngrp] cell members in arrival order, before the sort
   int *count;                // [ngrp] entries per group
   int *off;                  // [ngrp+1] CSR offsets (mode 0) / prefix of count (mode 1)
@@ -203,8 +250,8 @@ struct ListDesc {
   double r2m;
   long long pcap;
 };
-enum ListPhase { LIST_COUNT = 1, LIST_WRITE = 2 };
-// LIST_COUNT: cells, per-group counts, offsets and the capacity check;
+enum ListPhase { LIST_COUNT = 1, LIST_WRITE = 2, LIST_ZERO = 4 };
+// LIST_ZERO: the counters; LIST_COUNT: cells, per-group counts, offsets and the capacity check;
 // LIST_WRITE: the entries.  On overflow total[1] = 1 and nothing is written.
 void launch_list_build(const ListDesc *d_desc, const ListDesc *h, int nsys, int phases, hipStream_t st);
 // the inner lists of a batch's systems after a slab-layout build (systems with r2m > 0)
@@ -271,7 +318,14 @@ struct CorrDesc {
   const int *remf;
   double remf2;
 };
-void launch_corr(const CorrDesc *d_desc, const CorrDesc *h, int nsys, hipStream_t st);
+// energies: reduce the energy columns (else launch_tail does)
+void launch_corr(const CorrDesc *d_desc, const CorrDesc *h, int nsys, hipStream_t st, bool energies = true);
+
+// The end of a resident evaluation: forces combined, every partial sum
+// reduced.  d_corr: null without corrections; d_list: the list build's
+// descriptors, null without one.
+void launch_tail(const PmeDesc *d_pme, const PmeDesc *h_pme, int npme, const PairDesc *d_pair, const CorrDesc *d_corr,
+                 const ListDesc *d_list, int nsys, hipStream_t st);
 
 // Proper torsions (fptors.f): one thread per torsion writes its four atoms'
 // forces and its energy; a per-atom gather sums them in a fixed order.

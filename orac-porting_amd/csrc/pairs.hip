@@ -34,36 +34,45 @@ __device__ inline int fmodp(int a, int n) { return ((a % n) + n) % n; }
 
 // ---------------------------------------------------------------- centres
 
-// group centres (appbou.f): mass-fraction weighted sum, no contraction
-__global__ void __launch_bounds__(256) k_group_centres(const PairDesc *__restrict__ D) {
-#pragma clang fp contract(off)
-  const PairDesc &d = D[blockIdx.y];
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= d.ngrp) return;
-  double sx = 0.0, sy = 0.0, sz = 0.0;
-  for (int m = d.gfirst[g]; m <= d.glast[g]; ++m) {
-    sx = sx + d.gmass[m] * d.xp[m];
-    sy = sy + d.gmass[m] * d.yp[m];
-    sz = sz + d.gmass[m] * d.zp[m];
-  }
-  d.xpg[g] = sx;
-  d.ypg[g] = sy;
-  d.zpg[g] = sz;
+// the build of a system with a step counter runs only on its update steps
+__device__ inline bool list_due(const ListDesc &d) { return !d.step || (*d.step % d.every) == 0; }
+
+// workgroup blk of nblk clears a build's counters
+__device__ inline void list_zero(const ListDesc &d, int blk, int nblk) {
+  if (!list_due(d)) return;
+  const int ncell = d.cg.ncx * d.cg.ncy * d.cg.ncz + 1;  // + the parking cell
+  for (int i = blk * blockDim.x + threadIdx.x; i < ncell; i += nblk * blockDim.x) gmem(d.cell_cnt)[i] = 0;
+  if (blk == 0 && threadIdx.x < 3) d.total[threadIdx.x] = 0;
 }
 
-// Molecule centres of mass.  Blocks [0, nbb) give each large molecule (more
-// than MOL_SMALL atoms) a wavefront: lanes stride over its atoms, fixed-order
-// butterfly sum.  The blocks after them give every small molecule (a water) a
-// thread that sums its atoms in order.  Each molecule has one fixed path.
-__global__ void __launch_bounds__(256) k_mol_com(const PairDesc *__restrict__ D, int nbb) {
+__global__ void __launch_bounds__(256) k_list_zero(const ListDesc *__restrict__ D) {
+  list_zero(D[blockIdx.y], blockIdx.x, gridDim.x);
+}
+
+
+// One launch prepares an evaluation; its workgroups take, in this order,
+//   the molecules of more than MOL_SMALL atoms (one workgroup each: threads
+//     stride over the atoms, fixed-order sums; a 20,000-atom solute takes 9 us
+//     where one wavefront took 95),
+//   the other molecules (a thread each),
+//   the groups (a thread each): centres (appbou.f), and with pack the records
+//     the pair kernel reads in group order,
+//   the counters of the list build L, when one follows.
+constexpr int PREP_THREADS = 1024;
+
+__global__ void __launch_bounds__(PREP_THREADS) k_prepare(const PairDesc *__restrict__ D,
+                                                          const ListDesc *__restrict__ L, int nbig, int nsmall,
+                                                          int ngrpb, int pack) {
   const PairDesc &d = D[blockIdx.y];
-  if ((int)blockIdx.x < nbb) {
-    const int lane = threadIdx.x & 63;
-    const int k = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (k >= d.nbig) return;
-    const int m = gmem(d.mbig)[k];
+  int blk = blockIdx.x;
+  if (blk < nbig) {
+    __shared__ double red[PREP_THREADS / 64][4];
+    if (blk >= d.nbig) return;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int m = gmem(d.mbig)[blk], a0 = gmem(d.mfirst)[m], a1 = gmem(d.mlast)[m];
     double sx = 0.0, sy = 0.0, sz = 0.0, sm = 0.0;
-    for (int a = gmem(d.mfirst)[m] + lane; a <= gmem(d.mlast)[m]; a += 64) {
+#pragma unroll 4
+    for (int a = a0 + (int)threadIdx.x; a <= a1; a += PREP_THREADS) {
       const double w = gmem(d.mass)[a];
       sx += w * gmem(d.xp)[a];
       sy += w * gmem(d.yp)[a];
@@ -75,41 +84,84 @@ __global__ void __launch_bounds__(256) k_mol_com(const PairDesc *__restrict__ D,
     sz = wave_sum(sz);
     sm = wave_sum(sm);
     if (lane == 0) {
-      gmem(d.xpcm)[m] = sx / sm;
-      gmem(d.ypcm)[m] = sy / sm;
-      gmem(d.zpcm)[m] = sz / sm;
+      red[wid][0] = sx;
+      red[wid][1] = sy;
+      red[wid][2] = sz;
+      red[wid][3] = sm;
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+      double s = 0.0, w = 0.0;
+      for (int k = 0; k < PREP_THREADS / 64; ++k) {
+        s += red[k][threadIdx.x];
+        w += red[k][3];
+      }
+      if (threadIdx.x == 0) gmem(d.xpcm)[m] = s / w;
+      if (threadIdx.x == 1) gmem(d.ypcm)[m] = s / w;
+      if (threadIdx.x == 2) gmem(d.zpcm)[m] = s / w;
     }
     return;
   }
-  const int m = (blockIdx.x - nbb) * blockDim.x + threadIdx.x;
-  if (m >= d.nmol) return;
-  const int a0 = gmem(d.mfirst)[m], a1 = gmem(d.mlast)[m];
-  if (a1 - a0 + 1 > MOL_SMALL) return;
-  double sx = 0.0, sy = 0.0, sz = 0.0, sm = 0.0;
-  for (int a = a0; a <= a1; ++a) {
-    const double w = gmem(d.mass)[a];
-    sx += w * gmem(d.xp)[a];
-    sy += w * gmem(d.yp)[a];
-    sz += w * gmem(d.zp)[a];
-    sm += w;
+  blk -= nbig;
+  if (blk < nsmall) {
+    const int m = blk * PREP_THREADS + threadIdx.x;
+    if (!d.mfirst || m >= d.nmol) return;
+    const int a0 = gmem(d.mfirst)[m], a1 = gmem(d.mlast)[m];
+    if (a1 - a0 + 1 > MOL_SMALL) return;
+    double sx = 0.0, sy = 0.0, sz = 0.0, sm = 0.0;
+    for (int a = a0; a <= a1; ++a) {
+      const double w = gmem(d.mass)[a];
+      sx += w * gmem(d.xp)[a];
+      sy += w * gmem(d.yp)[a];
+      sz += w * gmem(d.zp)[a];
+      sm += w;
+    }
+    gmem(d.xpcm)[m] = sx / sm;
+    gmem(d.ypcm)[m] = sy / sm;
+    gmem(d.zpcm)[m] = sz / sm;
+    return;
   }
-  gmem(d.xpcm)[m] = sx / sm;
-  gmem(d.ypcm)[m] = sy / sm;
-  gmem(d.zpcm)[m] = sz / sm;
+  blk -= nsmall;
+  if (blk < ngrpb) {
+    const int g = blk * PREP_THREADS + threadIdx.x;
+    if (g >= d.ngrp) return;
+    const int f0 = gmem(d.gfirst)[g], f1 = gmem(d.glast)[g];
+    double sx = 0.0, sy = 0.0, sz = 0.0;
+    {
+#pragma clang fp contract(off)
+      // mass-fraction weighted sum in atom order, no contraction (appbou.f)
+      for (int m = f0; m <= f1; ++m) {
+        const double w = gmem(d.gmass)[m];
+        sx = sx + w * gmem(d.xp)[m];
+        sy = sy + w * gmem(d.yp)[m];
+        sz = sz + w * gmem(d.zp)[m];
+      }
+    }
+    gmem(d.xpg)[g] = sx;
+    gmem(d.ypg)[g] = sy;
+    gmem(d.zpg)[g] = sz;
+    if (pack) pack_group(d, g, g, f0, f0, f1 - f0 + 1, sx, sy, sz);
+    return;
+  }
+  blk -= ngrpb;
+  if (L) list_zero(L[blockIdx.y], blk, (int)gridDim.x - nbig - nsmall - ngrpb);
 }
 
-void launch_centres(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream_t st) {
-  int max_mol = 0, max_grp = 0, max_big = 0;
+void launch_centres(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream_t st, bool pack,
+                    const ListDesc *d_list, const ListDesc *h_list) {
+  int max_mol = 0, max_grp = 0, max_big = 0, max_cell = 0;
   for (int s = 0; s < nsys; ++s) {
     max_mol = std::max(max_mol, h[s].mfirst ? h[s].nmol : 0);
     max_big = std::max(max_big, h[s].mfirst ? h[s].nbig : 0);
     max_grp = std::max(max_grp, h[s].ngrp);
+    if (h_list) max_cell = std::max(max_cell, h_list[s].cg.ncx * h_list[s].cg.ncy * h_list[s].cg.ncz + 1);
   }
-  if (max_mol > 0) {
-    const int nbb = (max_big + 3) / 4;
-    hipLaunchKernelGGL(k_mol_com, dim3(nbb + (max_mol + 255) / 256, nsys), dim3(256), 0, st, d_desc, nbb);
-  }
-  if (max_grp > 0) hipLaunchKernelGGL(k_group_centres, dim3((max_grp + 255) / 256, nsys), dim3(256), 0, st, d_desc);
+  const int nsmall = (max_mol + PREP_THREADS - 1) / PREP_THREADS, ngrpb = (max_grp + PREP_THREADS - 1) / PREP_THREADS,
+            nzero = h_list ? std::min(16, (max_cell + PREP_THREADS - 1) / PREP_THREADS) : 0;
+  const int n = max_big + nsmall + ngrpb + nzero;
+  if (n > 0)
+    hipLaunchKernelGGL(k_prepare, dim3(n, nsys), dim3(PREP_THREADS), 0, st, d_desc, h_list ? d_list : nullptr, max_big,
+                       nsmall, ngrpb, pack ? 1 : 0);
 }
 
 // ---------------------------------------------------------------- cells
@@ -125,20 +177,6 @@ __device__ inline int cell_axis(double xr, double dcell, int nc) {
   double sg = (x1 - (double)ix) >= 0.0 ? 1.0 : -1.0;
   int n = (int)((double)ix + (sg - 1.0) / 2.0);
   return fmodp(n, nc);
-}
-
-// the build of a system with a step counter runs only on its update steps
-__device__ inline bool list_due(const ListDesc &d) { return !d.step || (*d.step % d.every) == 0; }
-
-__global__ void __launch_bounds__(256) k_list_zero(const ListDesc *__restrict__ D) {
-  const ListDesc &d = D[blockIdx.y];
-  if (!list_due(d)) return;
-  const int ncell = d.cg.ncx * d.cg.ncy * d.cg.ncz + 1;  // + the parking cell
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ncell; i += gridDim.x * blockDim.x) {
-    d.cell_cnt[i] = 0;
-    d.cell_cursor[i] = 0;
-  }
-  if (blockIdx.x == 0 && threadIdx.x < 2) d.total[threadIdx.x] = 0;
 }
 
 __global__ void __launch_bounds__(256) k_cell_assign(const ListDesc *__restrict__ D) {
@@ -158,8 +196,8 @@ __global__ void __launch_bounds__(256) k_cell_assign(const ListDesc *__restrict_
     // stencil visits; the group gets no neighbours and is nobody's neighbour
     c = cg.ncx * cg.ncy * cg.ncz;
   }
-  d.cell_of[g] = c;
-  atomicAdd(&d.cell_cnt[c], 1);
+  gmem(d.cell_of)[g] = c;
+  gmem(d.cell_pos)[g] = atomicAdd(&d.cell_cnt[c], 1);  // arrival order within the cell
 }
 
 __global__ void __launch_bounds__(1024) k_cell_scan(const ListDesc *__restrict__ D) {
@@ -172,41 +210,41 @@ __global__ void __launch_bounds__(256) k_cell_fill(const ListDesc *__restrict__ 
   const ListDesc &d = D[blockIdx.y];
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= d.ngrp || !list_due(d)) return;
-  const int c = d.cell_of[g];
-  const int pos = atomicAdd(&d.cell_cursor[c], 1);
-  d.cell_fill[d.cell_start[c] + pos] = g;
+  gmem(d.cell_fill)[gmem(d.cell_start)[gmem(d.cell_of)[g]] + gmem(d.cell_pos)[g]] = g;
 }
 
 // each cell's members in descending group order: the order of the
-// reference's head-inserted chains (lc_list.f:104-108).  One wavefront per
-// cell ranks its members (group indices are distinct): a member's place is
-// the number of members above it, so the cost per cell is n^2 / 64 compares
-// and one cell holding every group (the single-cell fallback of a small box)
-// is as cheap as many small ones.
+// reference's head-inserted chains (lc_list.f:104-108), and their centres in
+// that order for the stencil walk.  A wavefront ranks a cell's members (group
+// indices are distinct): a member's place is the number of members above it,
+// compared lane by lane from registers.  Where cells are few and crowded (the
+// single cell of a small box) CELL_SHARE wavefronts share one (216 members: 62
+// us when one wavefront read every member from memory for each 64, now 5).
+constexpr int CELL_FEW = 64, CELL_SHARE = 16;
+
 __global__ void __launch_bounds__(256) k_cell_sort(const ListDesc *__restrict__ D) {
   const ListDesc &d = D[blockIdx.y];
-  const int c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (c > d.cg.ncx * d.cg.ncy * d.cg.ncz || !list_due(d)) return;
-  const int s = gmem(d.cell_start)[c], n = gmem(d.cell_cnt)[c];
+  const int ncell = d.cg.ncx * d.cg.ncy * d.cg.ncz + 1, share = ncell <= CELL_FEW ? CELL_SHARE : 1;
+  const int unit = blockIdx.x * 4 + uniform((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int c = unit / share, part = unit - c * share;
+  if (c >= ncell || !list_due(d)) return;
+  const int s = uniform(gmem(d.cell_start)[c]), n = uniform(gmem(d.cell_cnt)[c]);
   const auto in = gmem(d.cell_fill + s);
-  for (int i0 = 0; i0 < n; i0 += 64) {
+  for (int i0 = 64 * part; i0 < n; i0 += 64 * share) {
     const int i = i0 + lane;
     const int v = i < n ? in[i] : -1;
     int rank = 0;
-    for (int j = 0; j < n; ++j) rank += in[j] > v ? 1 : 0;
-    if (i < n) d.cell_items[s + rank] = v;
+    for (int j0 = 0; j0 < n; j0 += 64) {
+      const int w = j0 == i0 ? v : (j0 + lane < n ? in[j0 + lane] : -1), m = min(64, n - j0);
+      for (int q = 0; q < m; ++q) rank += __builtin_amdgcn_readlane(w, q) > v ? 1 : 0;
+    }
+    if (i < n) {
+      const int t = s + rank;
+      gmem(d.cell_items)[t] = v;
+      gstore(d.cg.cpos + t, make_double4(gmem(d.xpg)[v], gmem(d.ypg)[v], gmem(d.zpg)[v], (double)v));
+      if (d.soff && d.cellorder) gmem(d.soff)[t] = gmem(d.gsize)[v];  // sizes in cell order; scanned in place below
+    }
   }
-}
-
-// centres copied into cell order, with the group index, so a stencil walk
-// reads each cell's candidates from contiguous memory
-__global__ void __launch_bounds__(256) k_cell_pack(const ListDesc *__restrict__ D) {
-  const ListDesc &d = D[blockIdx.y];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= d.ngrp || !list_due(d)) return;
-  const int g = d.cell_items[t];
-  d.cg.cpos[t] = make_double4(gmem(d.xpg)[g], gmem(d.ypg)[g], gmem(d.zpg)[g], (double)g);
-  if (d.soff && d.cellorder) d.soff[t] = gmem(d.gsize)[g];  // group sizes in cell order; scanned in place below
 }
 
 // first atom of each group in cell order (exclusive prefix of the sizes), one block per system
@@ -233,12 +271,16 @@ void launch_exclusive_scan(const int *in, int *out, int n, int *total, hipStream
 
 // Pair test of lc_list.f:159-170 (full co, minimum image), no contraction.
 // p = {xpg, ypg, zpg, group} of the candidate, from the cell-ordered copy.
+// dnint(d / 2) is zero below |d| = 1: a wavefront none of whose candidates is
+// further away skips the rounding.
 __device__ inline bool list_hit(double x1, double y1, double z1, double4 p, const double *co, double sqcut) {
 #pragma clang fp contract(off)
   double x2 = x1 - p.x, y2 = y1 - p.y, z2 = z1 - p.z;
-  x2 = x2 - 2.0 * fnint(0.5 * x2);
-  y2 = y2 - 2.0 * fnint(0.5 * y2);
-  z2 = z2 - 2.0 * fnint(0.5 * z2);
+  if (__ballot(!(fmax(fmax(fabs(x2), fabs(y2)), fabs(z2)) < 1.0))) {
+    x2 = x2 - 2.0 * fnint(0.5 * x2);
+    y2 = y2 - 2.0 * fnint(0.5 * y2);
+    z2 = z2 - 2.0 * fnint(0.5 * z2);
+  }
   double xx = co[0] * x2 + co[3] * y2 + co[6] * z2;
   double yy = co[1] * x2 + co[4] * y2 + co[7] * z2;
   double zz = co[2] * x2 + co[5] * y2 + co[8] * z2;
@@ -259,6 +301,72 @@ __device__ inline int wave_excl_scan_int(int v, int lane) {
     if (lane >= off) x += y;
   }
   return x - v;
+}
+
+// Column walk for group n by one wavefront (the resident lists, whose entries
+// may come in any fixed order): the stencil's cells over one (x, y) offset are
+// a run of cells along z, contiguous in the cell order, so a run's members are
+// one range of memory (two where it wraps).  Lane m reads the bounds of run m,
+// and the runs' members are tested 64 at a time as one flat sequence; a
+// candidate finds its run by a binary search over the runs' offsets, read
+// across lanes.  24,460 atoms: 37 runs for 200 cells, k_list_write 44 -> 26 us.
+template <bool WRITE>
+__device__ __forceinline__ int list_walk_runs(int n, const ListDesc &d, int *out, int entry, int cap) {
+  const CellGrid &cg = d.cg;
+  const int lane = threadIdx.x & 63, ncy = cg.ncy, ncz = cg.ncz;
+  const int c = uniform(gmem(d.cell_of)[n]);
+  if (c >= cg.ncx * ncy * ncz) return 0;  // parked (non-finite centre)
+  const double x1 = uniform(gmem(d.xpg)[n]), y1 = uniform(gmem(d.ypg)[n]), z1 = uniform(gmem(d.zpg)[n]);
+  const int cj = c / ncz, k = c - cj * ncz, i = cj / ncy, j = cj - i * ncy;
+  int base = 0;
+  for (int m0 = 0; m0 < cg.ncol; m0 += 64) {
+    const int m = m0 + lane;
+    int s[2] = {0, 0}, cnt[2] = {0, 0};
+    if (m < cg.ncol) {
+      const int4 col = gload(cg.col + m);
+      int nx = i + col.x, ny = j + col.y;  // |offsets| are below the cell counts
+      nx += nx < 0 ? cg.ncx : 0;
+      nx -= nx >= cg.ncx ? cg.ncx : 0;
+      ny += ny < 0 ? ncy : 0;
+      ny -= ny >= ncy ? ncy : 0;
+      const auto start = gmem(d.cell_start + ncz * (ny + ncy * nx));
+      const int za = k + col.z, zb = k + col.w;
+      s[0] = start[max(za, 0)];
+      cnt[0] = start[min(zb, ncz - 1) + 1] - s[0];
+      if (za < 0) {
+        s[1] = start[za + ncz];
+        cnt[1] = start[ncz] - s[1];
+      } else if (zb >= ncz) {
+        s[1] = start[0];
+        cnt[1] = start[zb - ncz + 1] - s[1];
+      }
+    }
+    for (int w = 0; w < 2; ++w) {
+      if (w == 1 && !__ballot(cnt[1] > 0)) break;
+      const int sw = s[w], ofs = wave_excl_scan_int(cnt[w], lane);
+      const int total = __builtin_amdgcn_readlane(ofs + cnt[w], 63);
+      for (int q0 = 0; q0 < total; q0 += 64) {
+        const int q = q0 + lane;
+        int r = 0;  // the last run whose offset is <= q (r + step <= 63 at every step)
+#pragma unroll
+        for (int step = 32; step > 0; step >>= 1)
+          if (__shfl(ofs, r + step, 64) <= q) r += step;
+        const int t = __shfl(sw - ofs, r, 64) + q;
+        const bool in = q < total;
+        double4 p = make_double4(x1, y1, z1, (double)n);
+        if (in) p = gload(cg.cpos + t);
+        const int l = (int)p.w;
+        const bool hit = list_hit(x1, y1, z1, p, cg.co, cg.sqcut) && in && l != n;
+        const unsigned long long mask = __ballot(hit);
+        if (WRITE && hit) {
+          const int pos = base + lanes_below(mask);
+          if (pos < cap) gmem(out)[pos] = entry == 1 ? t : l;
+        }
+        base += __popcll(mask);
+      }
+    }
+  }
+  return base;
 }
 
 // Stencil walk for group n (lc_list.f:133-201) by one wavefront: the lanes
@@ -355,7 +463,7 @@ __global__ void __launch_bounds__(256) k_list_count(const ListDesc *__restrict__
   const int o = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (o >= d.ngrp || !list_due(d)) return;
   const int n = (d.mode == 0 && d.cellorder) ? d.cell_items[o] : o;
-  const int c = list_walk_wave<false>(n, d, nullptr, 0);
+  const int c = d.cg.ncol > 0 ? list_walk_runs<false>(uniform(n), d, nullptr, 0, 0) : list_walk_wave<false>(n, d, nullptr, 0);
   if ((threadIdx.x & 63) == 0) d.count[o] = c;
 }
 
@@ -386,17 +494,24 @@ enum { LW_REF = 0, LW_SLAB = 1, LW_CSR = 2 };
 template <int LAYOUT>
 __global__ void __launch_bounds__(256) k_list_write(const ListDesc *__restrict__ D) {
   const ListDesc &d = D[blockIdx.y];
-  const int o = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (o >= d.ngrp || d.total[1] || !list_due(d)) return;
+  const int wid = uniform((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int o = blockIdx.x * 4 + wid;
+  if (!list_due(d)) return;
+  if (LAYOUT == LW_SLAB) {
+    if (d.split) return;  // k_list_write_split
+    if (o >= d.ngrp) return;
+    const int n = d.cellorder ? uniform(gmem(d.cell_items)[o]) : o;
+    int *out = d.out + (size_t)o * d.slab;
+    const int entry = d.cellorder ? 1 : 2;
+    const int c = d.cg.ncol > 0 ? list_walk_runs<true>(n, d, out, entry, d.slab) : list_walk_wave<true>(n, d, out, entry, d.slab);
+    if (lane == 0) gmem(d.count)[o] = c;
+    return;
+  }
+  if (o >= d.ngrp || d.total[1]) return;
   if (LAYOUT == LW_REF) {
     const int w = d.off[o] + o;  // one count slot per preceding group
     const int nv = list_walk_wave<true>(o, d, d.out + w + 1, 0);
-    if ((threadIdx.x & 63) == 0) d.out[w] = nv;
-  } else if (LAYOUT == LW_SLAB) {
-    if (d.split) return;  // k_list_write_split
-    const int n = d.cellorder ? d.cell_items[o] : o;
-    const int c = list_walk_wave<true>(n, d, d.out + (size_t)o * d.slab, d.cellorder ? 1 : 2, d.slab);
-    if ((threadIdx.x & 63) == 0) d.count[o] = c;
+    if (lane == 0) d.out[w] = nv;
   } else {
     const int n = d.cellorder ? d.cell_items[o] : o;
     list_walk_wave<true>(n, d, d.out + d.off[o], d.cellorder ? 1 : 2);
@@ -597,26 +712,19 @@ __global__ void __launch_bounds__(256) k_list_mirror(const ListDesc *__restrict_
   }
 }
 
-// slab layout, one block per system: total and largest count (fixed order),
+// slab layout, one 1024-thread workgroup per system: total and largest count,
 // overflow when a count exceeds the slab
-__global__ void __launch_bounds__(1024) k_list_total(const ListDesc *__restrict__ D, int split_written) {
-  __shared__ int wmax[16];
-  const ListDesc &d = D[blockIdx.x];
+__device__ inline void list_total(const ListDesc &d, bool split_written) {
+  __shared__ int wmax[16], wsum[16];
   if (!list_due(d)) return;
-  __shared__ int wsum[16];
   const int n = d.ngrp;
-  // the slab layout reads counts only: sum and largest count, no offsets
-  int tot = 0, mx = 0, s = 0;
-  if (d.slab > 0) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      // after a split write: forward and reverse entries (both directions), the larger part against the slab
-      const int c = d.count[i], r = (split_written && d.split) ? d.rcount[i] : 0;
-      s += c + r;
-      mx = max(mx, max(c, r));
-    }
-  } else {
-    tot = block_exclusive_scan(d.count, d.off, n);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) mx = max(mx, d.count[i]);
+  int mx = 0, s = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    // after a split write: forward and reverse entries (both directions), the larger part against the slab
+    const int c = gmem(d.count)[i], r = (split_written && d.split) ? gmem(d.rcount)[i] : 0;
+    s += c + r;
+    mx = max(mx, max(c, r));
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -629,17 +737,20 @@ __global__ void __launch_bounds__(1024) k_list_total(const ListDesc *__restrict_
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 0; w < 16; ++w) mx = max(mx, wmax[w]);
-    if (d.slab > 0) {
-      tot = 0;
-      for (int w = 0; w < 16; ++w) tot += wsum[w];
+    int tot = 0;
+    for (int w = 0; w < 16; ++w) {
+      mx = max(mx, wmax[w]);
+      tot += wsum[w];
     }
-    d.off[n] = tot;
     d.total[0] = tot;
     d.total[1] = mx > d.slab ? 1 : 0;
     d.total[2] = mx;
     if (mx > d.slab) d.total[3] = 1;  // sticky: cleared only by the host
   }
+}
+
+__global__ void __launch_bounds__(1024) k_list_total(const ListDesc *__restrict__ D, int split_written) {
+  list_total(D[blockIdx.x], split_written != 0);
 }
 
 void launch_list_build(const ListDesc *d_desc, const ListDesc *h, int nsys, int phases, hipStream_t st) {
@@ -665,13 +776,20 @@ void launch_list_build(const ListDesc *d_desc, const ListDesc *h, int nsys, int 
   }
   const int layout = h[0].mode == 1 ? LW_REF : (slab ? LW_SLAB : LW_CSR);
   if (phases & LIST_COUNT) {
-    hipLaunchKernelGGL(k_list_zero, dim3(std::min(64, (max_cell + 255) / 256), nsys), b, 0, st, d_desc);
+    int max_unit = 1;
+    bool any_cellorder = false;
+    for (int s = 0; s < nsys; ++s) {
+      const int ncell = h[s].cg.ncx * h[s].cg.ncy * h[s].cg.ncz + 1;
+      max_unit = std::max(max_unit, ncell <= CELL_FEW ? ncell * CELL_SHARE : ncell);
+      any_cellorder = any_cellorder || h[s].cellorder;
+    }
+    if (phases & LIST_ZERO)
+      hipLaunchKernelGGL(k_list_zero, dim3(std::min(64, (max_cell + 255) / 256), nsys), b, 0, st, d_desc);
     hipLaunchKernelGGL(k_cell_assign, gg, b, 0, st, d_desc);
     hipLaunchKernelGGL(k_cell_scan, dim3(nsys), dim3(1024), 0, st, d_desc);
     hipLaunchKernelGGL(k_cell_fill, gg, b, 0, st, d_desc);
-    hipLaunchKernelGGL(k_cell_sort, dim3((max_cell + 3) / 4, nsys), b, 0, st, d_desc);
-    hipLaunchKernelGGL(k_cell_pack, gg, b, 0, st, d_desc);
-    hipLaunchKernelGGL(k_soff_scan, dim3(nsys), dim3(1024), 0, st, d_desc);
+    hipLaunchKernelGGL(k_cell_sort, dim3((max_unit + 3) / 4, nsys), b, 0, st, d_desc);
+    if (any_cellorder) hipLaunchKernelGGL(k_soff_scan, dim3(nsys), dim3(1024), 0, st, d_desc);
     if (!slab || !(phases & LIST_WRITE)) {
       // counts only (or the compact layout's first pass)
       hipLaunchKernelGGL(k_list_count, gw, b, 0, st, d_desc);
@@ -694,8 +812,8 @@ void launch_list_build(const ListDesc *d_desc, const ListDesc *h, int nsys, int 
     } else {
       hipLaunchKernelGGL(k_list_write<LW_CSR>, gw, b, 0, st, d_desc);
     }
-    if (slab) hipLaunchKernelGGL(k_list_total, dim3(nsys), dim3(1024), 0, st, d_desc, any_split ? 1 : 0);
     if (any_split) {
+      hipLaunchKernelGGL(k_list_total, dim3(nsys), dim3(1024), 0, st, d_desc, 1);
       hipLaunchKernelGGL(k_list_rbase, dim3(nsys), dim3(1024), 0, st, d_desc);
       hipLaunchKernelGGL(k_list_mirror, gw, b, 0, st, d_desc);
     }
@@ -1162,26 +1280,22 @@ __global__ void __launch_bounds__(256) k_corr_gather(const CorrDesc *__restrict_
 }
 
 // d.out[ncol]: coul(slt), coul(slv), lj(slt), lj(slv) (and the alchemical
-// columns of kinds 3 and 4); block k reduces column k in fixed order
-__global__ void __launch_bounds__(256) k_corr_energy(const CorrDesc *__restrict__ D) {
-  __shared__ double red[4];
-  const CorrDesc &d = D[blockIdx.y];
-  const int k = blockIdx.x;
+// columns of kinds 3 and 4); a 1024-thread workgroup reduces column k in fixed order
+__device__ inline void corr_energy(const CorrDesc &d, int k) {
   const int ncol = d.ncol ? d.ncol : 4;
   if (k >= ncol) return;
   double s = 0.0;
-  for (int p = threadIdx.x; p < d.npairs; p += blockDim.x) s += d.pe[ncol * (size_t)p + k];
-  s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += red[w];
-    d.out[k] = t;
-  }
+#pragma unroll 4
+  for (int p = threadIdx.x; p < d.npairs; p += 1024) s += gmem(d.pe)[ncol * (size_t)p + k];
+  s = block_sum_1024(s);
+  if (threadIdx.x == 0) gmem(d.out)[k] = s;
 }
 
-void launch_corr(const CorrDesc *d_desc, const CorrDesc *h, int nsys, hipStream_t st) {
+__global__ void __launch_bounds__(1024) k_corr_energy(const CorrDesc *__restrict__ D) {
+  corr_energy(D[blockIdx.y], blockIdx.x);
+}
+
+void launch_corr(const CorrDesc *d_desc, const CorrDesc *h, int nsys, hipStream_t st, bool energies) {
   int max_pairs = 0, max_atoms = 0, max_col = 4;
   for (int s = 0; s < nsys; ++s) {
     max_pairs = std::max(max_pairs, h[s].npairs);
@@ -1192,7 +1306,54 @@ void launch_corr(const CorrDesc *d_desc, const CorrDesc *h, int nsys, hipStream_
     hipLaunchKernelGGL(k_corr_pairs, dim3((max_pairs + 255) / 256, nsys), dim3(256), 0, st, d_desc);
   if (max_atoms > 0)
     hipLaunchKernelGGL(k_corr_gather, dim3((max_atoms + 255) / 256, nsys), dim3(256), 0, st, d_desc);
-  hipLaunchKernelGGL(k_corr_energy, dim3(max_col, nsys), dim3(256), 0, st, d_desc);
+  if (energies) hipLaunchKernelGGL(k_corr_energy, dim3(max_col, nsys), dim3(1024), 0, st, d_desc);
+}
+
+// ---------------------------------------------------------------- the end of an evaluation
+
+// One launch, after the direct sum, the reciprocal sum and the corrections are
+// done; its workgroups take, in this order,
+//   the atoms: reciprocal and correction forces added to the direct ones, in
+//     that order, as accumulating in sequence would,
+//   the direct sum's 16 energy and virial columns (d.out[16]: uconf[3],
+//     ucoul[3], st[9] row-major, dwrk),
+//   the reciprocal sum's 16 columns,
+//   the corrections' energy columns,
+//   the list's totals, when a list was built (L).
+// Five launches of 3 to 6 us each, three of them in series, became one.
+constexpr int TAIL_THREADS = 1024, TAIL_COLS = 16 + 16 + 8 + 1;
+
+__global__ void __launch_bounds__(TAIL_THREADS) k_tail(const PmeDesc *__restrict__ P, const PairDesc *__restrict__ Q,
+                                                       const CorrDesc *__restrict__ Cc,
+                                                       const ListDesc *__restrict__ L, int nsys, int natomb) {
+  const int sys = blockIdx.y;
+  int blk = blockIdx.x;
+  if (blk < natomb) {
+    pme_combine(P[sys], blk * TAIL_THREADS + threadIdx.x);
+    return;
+  }
+  blk -= natomb;
+  if (blk >= 16 && blk < 32) {  // (the energy-only grids of alchemical systems follow the systems' own)
+    pme_finalize(P[sys], blk - 16);
+    return;
+  }
+  if (sys >= nsys) return;
+  if (blk < 16) pairs_finalize(Q[sys], blk);
+  else if (blk < 40) {
+    if (Cc) corr_energy(Cc[sys], blk - 32);
+  } else if (L) {
+    if (!L[sys].split) list_total(L[sys], false);
+  }
+}
+
+void launch_tail(const PmeDesc *d_pme, const PmeDesc *h_pme, int npme, const PairDesc *d_pair, const CorrDesc *d_corr,
+                 const ListDesc *d_list, int nsys, hipStream_t st) {
+  int max_atoms = 1;
+  for (int s = 0; s < npme; ++s)
+    if (h_pme[s].fx_dst) max_atoms = std::max(max_atoms, h_pme[s].natoms);
+  const int natomb = (max_atoms + TAIL_THREADS - 1) / TAIL_THREADS;
+  hipLaunchKernelGGL(k_tail, dim3(natomb + TAIL_COLS, npme), dim3(TAIL_THREADS), 0, st, d_pme, d_pair, d_corr, d_list,
+                     nsys, natomb);
 }
 
 // ---------------------------------------------------------------- cself

@@ -36,21 +36,6 @@ __device__ inline cx<T> cscale(cx<T> a, T s) { return {a.x * s, a.y * s}; }
 template <typename T, int S>
 __device__ inline cx<T> cmuli(cx<T> a) { return S > 0 ? cx<T>{-a.y, a.x} : cx<T>{a.y, -a.x}; }
 
-// Quotient of a small index (below 2^20) by a runtime divisor (below 2^11): the
-// float quotient of the half-shifted index is off by less than 2^-2 / d, so its
-// floor is exact, in three instructions rather than an integer division.
-struct FastDiv {
-  int d;
-  float inv;
-  __device__ __forceinline__ explicit FastDiv(int n) : d(n), inv(1.0f / (float)n) {}
-  __device__ __forceinline__ int div(int x) const { return (int)(((float)x + 0.5f) * inv); }
-  __device__ __forceinline__ int div(int x, int &rem) const {
-    const int q = div(x);
-    rem = x - q * d;
-    return q;
-  }
-};
-
 // the axis's twiddle table into LDS (one load per entry and workgroup)
 template <typename T>
 __device__ __forceinline__ void load_twiddles(cx<T> *tw, const FftAxis &ax) {
@@ -832,39 +817,8 @@ __global__ void __launch_bounds__(256) k_gather(const PmeDesc *__restrict__ D) {
   }
 }
 
-// d.out[20]: eer, vir(3x3 col-major), stc(3x3 row-major as stc1..stc9).
-// Block k reduces one component in fixed order: k < 7 the convolution
-// partials (scalar_sum.f:125-133 halving and symmetrisation), k >= 7 the
-// molecular-virial partials.
-__global__ void __launch_bounds__(256) k_pme_finalize(const PmeDesc *__restrict__ D) {
-  __shared__ double red[4];
-  const PmeDesc &d = D[blockIdx.y];
-  const int k = blockIdx.x;
-  if (k >= 7 && d.energy_only) {  // no gather: no molecular-virial terms
-    if (threadIdx.x == 0) d.out[10 + (k - 7)] = 0.0;
-    return;
-  }
-  const double *src = k < 7 ? d.conv_part + k : d.gather_part + (k - 7);
-  const int nrow = k < 7 ? d.conv_nblk : d.gather_nblk, stride = k < 7 ? 8 : 9;
-  double s = 0.0;
-  for (int r = threadIdx.x; r < nrow; r += blockDim.x) s += src[(size_t)r * stride];
-  s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  s = 0.0;
-  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) s += red[w];
-  double *o = d.out;
-  switch (k) {
-    case 0: o[0] = 0.5 * s; break;
-    case 1: o[1] = 0.5 * s; break;
-    case 2: o[5] = 0.5 * s; break;
-    case 3: o[9] = 0.5 * s; break;
-    case 4: o[4] = o[2] = 0.5 * s; break;  // vir(1,2) = vir(2,1)
-    case 5: o[7] = o[3] = 0.5 * s; break;  // vir(1,3) = vir(3,1)
-    case 6: o[8] = o[6] = 0.5 * s; break;  // vir(2,3) = vir(3,2)
-    default: o[10 + (k - 7)] = s; break;
-  }
+__global__ void __launch_bounds__(1024) k_pme_finalize(const PmeDesc *__restrict__ D) {
+  pme_finalize(D[blockIdx.y], blockIdx.x);
 }
 
 // ---------------------------------------------------------------- launchers
@@ -891,7 +845,7 @@ void pme_set_tiles(PmeDesc &d, int lds_elems) {
 
 template <typename T>
 void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st, const Tuning &tu,
-                const hipEvent_t *ev) {
+                const hipEvent_t *ev, bool finalize) {
   (void)tu;
   if (nsys <= 0) return;
   int max_atoms = 1, max_bins = 1, any_tiled = 0, any_atomic = 0, max_gx = 1, max_gy = 1, max_gz = 1, max_gg = 1;
@@ -951,37 +905,12 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
     default: hipLaunchKernelGGL((k_gather<T, 0>), dim3(max_gg, nsys), blk, 0, st, d_desc); break;
   }
   if (ev) ORAC_HIP(hipEventRecord(ev[3], st));
-  hipLaunchKernelGGL(k_pme_finalize, dim3(16, nsys), dim3(256), 0, st, d_desc);
-}
-
-// The reciprocal forces of a system evaluated beside its direct sum are
-// written to their own arrays; this adds them to the direct forces once both
-// are done, so the sum is the same as accumulating in sequence.
-__global__ void __launch_bounds__(256) k_pme_combine(const PmeDesc *__restrict__ D) {
-  const PmeDesc &d = D[blockIdx.y];
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (!d.fx_dst || a >= d.natoms) return;
-  double x = d.fx_dst[a] + d.fx[a], y = d.fy_dst[a] + d.fy[a], z = d.fz_dst[a] + d.fz[a];
-  if (d.cfx) {  // the corrections, in the order of a sequential evaluation
-    x += d.cfx[a];
-    y += d.cfy[a];
-    z += d.cfz[a];
-  }
-  d.fx_dst[a] = x;
-  d.fy_dst[a] = y;
-  d.fz_dst[a] = z;
-}
-
-void launch_pme_combine(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st) {
-  int max_atoms = 1;
-  for (int s = 0; s < nsys; ++s)
-    if (h[s].fx_dst) max_atoms = std::max(max_atoms, h[s].natoms);
-  hipLaunchKernelGGL(k_pme_combine, dim3((max_atoms + 255) / 256, nsys), dim3(256), 0, st, d_desc);
+  if (finalize) hipLaunchKernelGGL(k_pme_finalize, dim3(16, nsys), dim3(1024), 0, st, d_desc);
 }
 
 template void launch_pme<double>(const PmeDesc *, const PmeDesc *, int, hipStream_t, const Tuning &,
-                                 const hipEvent_t *);
+                                 const hipEvent_t *, bool);
 template void launch_pme<float>(const PmeDesc *, const PmeDesc *, int, hipStream_t, const Tuning &,
-                                const hipEvent_t *);
+                                const hipEvent_t *, bool);
 
 }  // namespace orac
