@@ -717,18 +717,19 @@ static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events
     mark(ST_PME);
     if (b.any_corr) launch_corr(b.dc, b.hc.data(), n, st, false);
   }
-  launch_tail(b.dp, b.hp.data(), npme, b.dq, b.any_corr ? b.dc : nullptr, lists ? dl : nullptr, n, st);
+  launch_tail(b.dp, b.hp.data(), npme, b.dq, b.any_corr ? b.dc : nullptr, lists ? dl : nullptr, n, md_lists, st);
   mark(ST_END);
 }
 
-// The inner shell of every system (systems with two shells): centres, then the
-// pair kernel on the inner-shell descriptors, on the list of the last build.
-static void batch_enqueue_mid(orac_hip_ctx *ctx, Batch &b) {
+// The inner shell of every system (systems with two shells): centres (unless
+// those of an outer evaluation at the same positions stand), then the pair
+// kernel on the inner-shell descriptors, on the list of the last build.
+static void batch_enqueue_mid(orac_hip_ctx *ctx, Batch &b, bool centres = true) {
   hipStream_t st = ctx->stream;
   const int n = (int)b.sys.size();
   // (the inner shell's descriptors share the records of the outer ones)
   const bool pack = !b.tu.cell_order;
-  launch_centres(b.dq, b.hq.data(), n, st, pack);
+  if (centres) launch_centres(b.dq, b.hq.data(), n, st, pack);
   if (b.precision == 0)
     launch_pairs<double>(b.dqm, b.hqm.data(), n, st, b.tu, pack);
   else
@@ -857,6 +858,109 @@ static double batch_time(orac_hip_ctx *ctx, Batch &b, int reps, bool rebuild) {
 
 // ---------------------------------------------------------------- molecular dynamics
 
+// The units as launch_md_advance takes them: without terms; connected by terms
+// within MD_WG_SLOTS atoms, none of a rigid unit (small sets share a
+// workgroup); the rest.
+static void md_partition(BufSet &B, MdDesc &d, const std::vector<int> &ufirst,
+                         const std::vector<unsigned char> &urigid, const std::vector<double> &ud2,
+                         const std::vector<int> &goff, const std::vector<int> &gt, const std::vector<int> &bi,
+                         const std::vector<int> &bj, const std::vector<double> &bk, const std::vector<double> &br0,
+                         hipStream_t st) {
+  const int n = d.natoms, nu = (int)ufirst.size();
+  std::vector<int> root(n), size(n, 1), unit_of(n);
+  for (int a = 0; a < n; ++a) root[a] = a;
+  auto find = [&](int a) {
+    while (root[a] != a) a = root[a] = root[root[a]];
+    return a;
+  };
+  auto join = [&](int a, int b) {
+    a = find(a);
+    b = find(b);
+    if (a == b) return;
+    if (size[a] < size[b]) std::swap(a, b);
+    root[b] = a;
+    size[a] += size[b];
+  };
+  for (int t = 0; t < d.nbond; ++t) join(bi[t], bj[t]);
+  std::vector<char> rigid_set(n, 0);  // (by root) terms reach a rigid unit
+  for (int u = 0; u < nu; ++u)
+    for (int k = 0; k < (urigid[u] ? 3 : 1); ++k) {
+      unit_of[ufirst[u] + k] = u;
+      if (urigid[u] && goff[ufirst[u] + k + 1] > goff[ufirst[u] + k]) rigid_set[find(ufirst[u] + k)] = 1;
+    }
+  std::vector<int> free_atom, rest;
+  std::vector<double> free_d2;
+  std::vector<std::vector<int>> sets;
+  std::vector<int> set_of(n, -1);
+  for (int pass = 1; pass >= 0; --pass)  // rigid ones first
+    for (int u = 0; u < nu; ++u) {
+      if (urigid[u] != pass) continue;
+      const int a = ufirst[u];
+      if (goff[a + (pass ? 3 : 1)] == goff[a]) {
+        free_atom.push_back(a);
+        for (int k = 0; pass && k < 3; ++k) free_d2.push_back(ud2[3 * (size_t)u + k]);
+      } else if (pass || rigid_set[find(a)] || size[find(a)] > MD_WG_SLOTS) {
+        rest.push_back(u);
+      } else {
+        int &s = set_of[find(a)];
+        if (s < 0) {
+          s = (int)sets.size();
+          sets.emplace_back();
+        }
+        sets[s].push_back(a);
+      }
+    }
+  d.nfree = (int)free_atom.size();
+  d.nfree_rigid = (int)free_d2.size() / 3;
+  // workgroups: sets in order, filled up to MD_WG slots (a larger set has one of its own)
+  std::vector<int> wg_slot(1, 0), slot_atom, slot_of(n, -1);
+  d.wg_most = 0;
+  auto close = [&] {
+    d.wg_most = std::max(d.wg_most, (int)slot_atom.size() - wg_slot.back());
+    slot_atom.resize((slot_atom.size() + 63) / 64 * 64, -1);
+    wg_slot.push_back((int)slot_atom.size());
+  };
+  for (const std::vector<int> &s : sets) {
+    const int used = (int)slot_atom.size() - wg_slot.back();
+    if (used > 0 && used + (int)s.size() > MD_WG) close();
+    for (int a : s) {
+      slot_of[a] = (int)slot_atom.size() - wg_slot.back();
+      slot_atom.push_back(a);
+    }
+  }
+  if ((int)slot_atom.size() > wg_slot.back()) close();
+  d.nwg = (int)wg_slot.size() - 1;
+  std::vector<int> slot_deg(slot_atom.size(), 0), slice_off(slot_atom.size() / 64, 0), ent_slot;
+  std::vector<double2> ent_kr;
+  for (size_t s0 = 0; s0 < slot_atom.size(); s0 += 64) {
+    int most = 0;
+    for (int k = 0; k < 64; ++k)
+      if (const int a = slot_atom[s0 + k]; a >= 0) most = std::max(most, slot_deg[s0 + k] = goff[a + 1] - goff[a]);
+    const size_t off = ent_slot.size();
+    slice_off[s0 / 64] = (int)off;
+    ORAC_REQUIRE(off + 64 * (size_t)most <= (size_t)INT32_MAX, E_ARG, "too many harmonic terms");
+    ent_slot.resize(off + 64 * (size_t)most, 0);
+    ent_kr.resize(off + 64 * (size_t)most, make_double2(0.0, 0.0));
+    for (int k = 0; k < 64; ++k)
+      for (int e = 0; e < slot_deg[s0 + k]; ++e) {
+        const int a = slot_atom[s0 + k], t = std::abs(gt[goff[a] + e]) - 1;
+        ent_slot[off + 64 * (size_t)e + k] = slot_of[bi[t] == a ? bj[t] : bi[t]];
+        ent_kr[off + 64 * (size_t)e + k] = make_double2(bk[t], br0[t]);
+      }
+  }
+  d.nrest = (int)rest.size();
+  d.free_atom = B.put_vec("md_free", free_atom, st, false);
+  d.free_d2 = B.put_vec("md_freed2", free_d2, st, false);
+  d.wg_slot = B.put_vec("md_wgslot", wg_slot, st, false);
+  d.slot_atom = B.put_vec("md_slot", slot_atom, st, false);
+  d.slot_deg = B.put_vec("md_slotdeg", slot_deg, st, false);
+  d.slice_off = B.put_vec("md_slice", slice_off, st, false);
+  d.ent_slot = B.put_vec("md_ent", ent_slot, st, false);
+  d.ent_kr = B.put_vec("md_entkr", ent_kr, st, false);
+  d.rest_unit = B.put_vec("md_rest", rest, st, false);
+  ORAC_HIP(hipStreamSynchronize(st));  // (the uploads read vectors of this scope)
+}
+
 static void md_setup(orac_hip_ctx *ctx, System &S, int nrigid, const int32_t *rigid_first, const double *rigid_len,
                      int nterm, const int32_t *terms, const double *tk, const double *tr0) {
   hipStream_t st = ctx->stream;
@@ -952,6 +1056,7 @@ static void md_setup(orac_hip_ctx *ctx, System &S, int nrigid, const int32_t *ri
   d.bpe = B.get<double>("md_bpe", (size_t)std::max(1, nterm));
   d.bg_off = B.put_vec("md_bgoff", goff, st, false);
   d.bg_term = B.put_vec("md_bgterm", gt, st, false);
+  md_partition(B, d, ufirst, urigid, ud2, goff, gt, bi, bj, bk, br0, st);
   for (int k = 0; k < 9; ++k) d.oc[k] = S.oc[k];
   d.out = B.get<double>("md_out", 8);
   d.fail = B.get<int>("md_fail", 2);
@@ -1033,44 +1138,39 @@ static void md_prime(orac_hip_ctx *ctx, Batch &b) {
   E.batches.erase(pid);
 }
 
-// one outer r-RESPA step of every system in the batch (see md.hip)
+// The force part of one outer r-RESPA step of every system in the batch and
+// the launches that lead to the next force (see md.hip).  The step's start is
+// the launch before: md_start for a run's first step, the last launch here for
+// the others, which past the run's last step only ends it.
+static void md_start(orac_hip_ctx *ctx, Batch &b, double dt, int nmid, int ninner, int nsteps) {
+  hipStream_t st = ctx->stream;
+  const int n = (int)b.sys.size();
+  const double hm = nmid > 0 ? dt / nmid : 0.0, h = (nmid > 0 ? hm : dt) / ninner;
+  launch_md_begin(b.dm, n, nsteps, st);
+  launch_md_advance(b.dm, b.hm.data(), n, dt, hm, h, MD_KICK_SLOW | (nmid > 0 ? MD_KICK_MID : 0), ninner, st);
+}
+
 static void md_enqueue_step(orac_hip_ctx *ctx, Batch &b, double dt, int nmid, int ninner) {
   hipStream_t st = ctx->stream;
   const int n = (int)b.sys.size();
   if (nmid <= 0) {
-    const double h = dt / ninner;
-    // slow half kick, then the first fast substep's drift
-    launch_md_units(b.dm, b.hm.data(), n, dt, 0.0, h, MD_KICK_SLOW | MD_VERLET, st);
-    launch_md_fast_forces(b.dm, b.hm.data(), n, st);
-    // end of one fast substep (half kick), start of the next (drift)
-    for (int k = 1; k < ninner; ++k) {
-      launch_md_units(b.dm, b.hm.data(), n, dt, 0.0, h, MD_KICK_FAST | MD_VERLET, st);
-      launch_md_fast_forces(b.dm, b.hm.data(), n, st);
-    }
     batch_enqueue(ctx, b, true, false, true);
-    // end of the last fast substep, then the slow half kick
-    launch_md_units(b.dm, b.hm.data(), n, dt, 0.0, h, MD_KICK_FAST | MD_KICK_SLOW, st);
-  } else {
-    // two nonbonded shells, three levels in mtsmd.f's order: the outer shell
-    // with PME and corrections over dt, nmid steps of the inner shell over
-    // hm = dt/nmid, each with ninner fast substeps over h = hm/ninner
-    const double hm = dt / nmid, h = hm / ninner;
-    launch_md_units(b.dm, b.hm.data(), n, dt, hm, h, MD_KICK_SLOW, st);
-    for (int im = 0; im < nmid; ++im) {
-      launch_md_units(b.dm, b.hm.data(), n, dt, hm, h, MD_KICK_MID | MD_VERLET, st);
-      launch_md_fast_forces(b.dm, b.hm.data(), n, st);
-      for (int k = 1; k < ninner; ++k) {
-        launch_md_units(b.dm, b.hm.data(), n, dt, hm, h, MD_KICK_FAST | MD_VERLET, st);
-        launch_md_fast_forces(b.dm, b.hm.data(), n, st);
-      }
-      launch_md_units(b.dm, b.hm.data(), n, dt, hm, h, MD_KICK_FAST, st);
-      if (im == nmid - 1) batch_enqueue(ctx, b, true, false, true);  // the outer shell at the step's end
-      batch_enqueue_mid(ctx, b);
-      launch_md_units(b.dm, b.hm.data(), n, dt, hm, h, MD_KICK_MID, st);
-    }
-    launch_md_units(b.dm, b.hm.data(), n, dt, hm, h, MD_KICK_SLOW, st);
+    launch_md_advance(b.dm, b.hm.data(), n, dt, 0.0, dt / ninner, MD_END_SLOW | MD_KICK_SLOW | MD_BETWEEN, ninner, st);
+    return;
   }
-  launch_md_tick(b.dm, n, st);
+  // two nonbonded shells, three levels in mtsmd.f's order: the outer shell
+  // with PME and corrections over dt, nmid steps of the inner shell over
+  // hm = dt/nmid, each with ninner fast substeps over h = hm/ninner
+  const double hm = dt / nmid, h = hm / ninner;
+  for (int im = 0; im < nmid; ++im) {
+    const bool last = im == nmid - 1;  // the outer shell at the step's end
+    if (last) batch_enqueue(ctx, b, true, false, true);
+    batch_enqueue_mid(ctx, b, !last);
+    launch_md_advance(b.dm, b.hm.data(), n, dt, hm, h,
+                      last ? MD_END_MID | MD_END_SLOW | MD_KICK_SLOW | MD_KICK_MID | MD_BETWEEN
+                           : MD_END_MID | MD_KICK_MID,
+                      ninner, st);
+  }
 }
 
 static void md_run(orac_hip_ctx *ctx, Batch &b, int nsteps, double dt, int nmid, int ninner, int list_every,
@@ -1096,6 +1196,7 @@ static void md_run(orac_hip_ctx *ctx, Batch &b, int nsteps, double dt, int nmid,
     b.md_nmid = nmid;
   }
   hipStream_t st = ctx->stream;
+  if (nsteps > 0) md_start(ctx, b, dt, nmid, ninner, nsteps);
   for (int s = 0; s < nsteps; ++s) {
     if (use_graph) {
       if (!b.mexec) {

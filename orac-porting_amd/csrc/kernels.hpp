@@ -226,7 +226,7 @@ struct ListDesc {
   long long cap;             // capacity of out (ints, count slots included in mode 1)
   int *total;                // [0] entries (count slots excluded), [1] overflow flag, [2] largest count
   int mode;                  // 0: CSR, 0-based; 1: reference layout per group [nv, l1..lnv], 1-based
-  const int *step;           // optional step counter of the system: the build runs only
+  int *step;                 // optional step counter of the system: the build runs only
   int every;                 //   when *step % every == 0 (device-side update schedule)
   // mode 0 only.  cellorder = 1: owners are taken in cell order (cell_items)
   // and entries are cell-order positions, soff[t] = first atom of the t-th
@@ -323,9 +323,9 @@ void launch_corr(const CorrDesc *d_desc, const CorrDesc *h, int nsys, hipStream_
 
 // The end of a resident evaluation: forces combined, every partial sum
 // reduced.  d_corr: null without corrections; d_list: the list build's
-// descriptors, null without one.
+// descriptors, null without one.  step: a step of dynamics, counted in *d_list->step.
 void launch_tail(const PmeDesc *d_pme, const PmeDesc *h_pme, int npme, const PairDesc *d_pair, const CorrDesc *d_corr,
-                 const ListDesc *d_list, int nsys, hipStream_t st);
+                 const ListDesc *d_list, int nsys, bool step, hipStream_t st);
 
 // Proper torsions (fptors.f): one thread per torsion writes its four atoms'
 // forces and its energy; a per-atom gather sums them in a fixed order.
@@ -377,18 +377,42 @@ struct MdDesc {
   double oc[9];
   double *out;                       // [5]: kinetic, bond energy, momentum x, y, z
   int *fail;                         // constraint iterations that did not converge
-  int *step;                         // outer steps taken (device counter, drives the list schedule)
+  int *step;                         // [2]: outer steps taken (drives the list schedule), steps at the run's end
+  // what launch_md_advance takes: units without terms (rigid ones first), and
+  // workgroups of up to MD_WG_SLOTS atoms connected by terms among themselves
+  // only, in slots of 64 (entries of a slice of 64 slots: entry e of slot s at
+  // slice_off + 64 e + s mod 64)
+  int nfree, nfree_rigid, nwg, wg_most;
+  const int *free_atom;              // first atom
+  const double *free_d2;             // ud2 of the rigid ones
+  const int *wg_slot;                // [nwg + 1] first slot
+  const int *slot_atom, *slot_deg;   // -1: empty slot
+  const int *slice_off, *ent_slot;   // the term's other atom, as a slot of the workgroup
+  const double2 *ent_kr;             // k, r0
+  int nrest;                         // the other units: a launch per kick and substep
+  const int *rest_unit;
 };
-// stages of launch_md_units, applied in this order when combined: half kick
-// by the fast forces over h + RATTLE; half kick by the inner-shell forces
-// over hm + RATTLE; half kick by the slow forces over dt + RATTLE; drift over
-// h (ORAC's verlet with the fast forces) + SHAKE; RATTLE
-constexpr int MD_KICK_FAST = 1, MD_KICK_SLOW = 2, MD_VERLET = 4, MD_RATTLE = 8, MD_KICK_MID = 16;
+// Connected atoms per workgroup.  Larger sets, and sets with rigid units, go by
+// launches, a kick or substep each.  A step with four substeps of a chain of
+// 2,048 atoms takes 109 us in one workgroup and 137 by launches; each further
+// 1,024 atoms add 20 to the one and 4 to the other, and the positions of 3,072
+// exceed 64 KB of LDS.
+constexpr int MD_WG = 1024, MD_WG_SLOTS = 2 * MD_WG, MD_FREE = 256;
+// stages, applied in this order when combined: half kick by the fast forces
+// over h + RATTLE; the half kicks that end a step, by the inner-shell forces
+// over hm + RATTLE and by the slow forces over dt + RATTLE; those that start
+// one, slow and inner; drift over h (ORAC's verlet with the fast forces) +
+// SHAKE; RATTLE.  MD_BETWEEN: past the run's last step only the ends are done.
+constexpr int MD_KICK_FAST = 1, MD_KICK_SLOW = 2, MD_VERLET = 4, MD_RATTLE = 8, MD_KICK_MID = 16, MD_END_MID = 32,
+              MD_END_SLOW = 64, MD_BETWEEN = 128;
 void launch_md_units(const MdDesc *d, const MdDesc *h, int nsys, double dt, double hm, double hin, int flags,
                      hipStream_t st);
 void launch_md_fast_forces(const MdDesc *d, const MdDesc *h, int nsys, hipStream_t st);
 void launch_md_energy(const MdDesc *d, int nsys, hipStream_t st);
-void launch_md_tick(const MdDesc *d, int nsys, hipStream_t st);
+void launch_md_begin(const MdDesc *d, int nsys, int nsteps, hipStream_t st);
+// kicks (flags), then nsub fast substeps: drift + SHAKE, fast forces, half kick + RATTLE
+void launch_md_advance(const MdDesc *d, const MdDesc *h, int nsys, double dt, double hm, double hin, int flags,
+                       int nsub, hipStream_t st);
 void launch_md_relax(const MdDesc *d, const MdDesc *h, int nsys, double hstep, double dmax, hipStream_t st);
 void launch_md_scale_v(const MdDesc *d, const MdDesc *h, int nsys, const double *scale, hipStream_t st);
 

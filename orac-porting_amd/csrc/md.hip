@@ -15,6 +15,12 @@
 //   Fs(x)          (the force evaluation of the engine)
 //   v += Fs*0.5*dt/m; RATTLE                                 (:3121-3146)
 //
+// A unit without harmonic terms moves alone between two slow forces, and an
+// atom with terms moves with the atoms its terms reach, so the whole fast level
+// of a step is one launch (k_md_advance): the units' kicks and substeps stay in
+// registers, the atoms that terms connect share a workgroup.  It also closes
+// the step before it.
+//
 // Positions are Cartesian FP64 with the reduced copy xp = oc x refreshed after
 // every drift; the force path reads the reduced copy.  A unit is one atom or
 // one rigid 3-atom molecule; one thread advances a unit, so constraint
@@ -40,10 +46,23 @@ __device__ inline void to_reduced(const double *oc, double x, double y, double z
 // (0,1), (0,2), (1,2); im = 1/m; dss the squared lengths.  mim_dir gives the
 // direction in which atom `at` moves for constraint (ca, cb) with bond vector
 // d (rattle_verlet.f:286-303): -d for its first atom, +d for its second.
-__device__ inline double3 mim_dir(int at, int ca, int cb, double3 d) {
-  if (at == ca) return make_double3(-d.x, -d.y, -d.z);
-  if (at == cb) return d;
-  return make_double3(0.0, 0.0, 0.0);
+// That is mim_sgn times d; its zeros are left out of the sums below (a third of
+// their terms), which changes no value.
+constexpr int MIM_CA[3] = {0, 0, 1}, MIM_CB[3] = {1, 2, 2};
+__device__ constexpr int mim_sgn(int at, int k) {
+  return at == (k == 2 ? 1 : 0) ? -1 : (at == (k == 0 ? 1 : 2) ? 1 : 0);
+}
+__device__ inline double3 mim_fma(double c, double3 d, double3 s) {
+  return make_double3(s.x + d.x * c, s.y + d.y * c, s.z + d.z * c);
+}
+__device__ inline double mim_dot(double3 a, double3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+__device__ inline double3 mim_diff(double3 a, double3 b) { return make_double3(a.x - b.x, a.y - b.y, a.z - b.z); }
+
+// one element of the constraint matrix: (direction of ka's atoms for kb) . x, by inverse masses
+__device__ inline double mim_elem(int ka, int kb, double dot, const double (&im)[3]) {
+  const int sa = mim_sgn(MIM_CA[ka], kb), sb = mim_sgn(MIM_CB[ka], kb);
+  if (sa && sb) return dot * im[MIM_CA[ka]] + dot * im[MIM_CB[ka]];
+  return sa ? -sa * dot * im[MIM_CA[ka]] : sb * dot * im[MIM_CB[ka]];
 }
 
 // 3x3 solve by cofactors (rattle_verlet.f:381-397); later solves reuse them
@@ -89,56 +108,38 @@ constexpr int MIM_MAXIT = 120;      // rattle_verlet.f:461
 // molecule over; here the unit is counted as failed and keeps what it has).
 __device__ inline bool shake_mim3(double3 (&q)[3], const double3 (&p)[3], const double (&im)[3], const double *dss,
                                   double dti, double3 (&v)[3]) {
-  constexpr int ca[3] = {0, 0, 1}, cb[3] = {1, 2, 2};
-  double3 x0[3], xc[3], da[3][3], db[3][3];
+  double3 x0[3], xc[3];
   double dd[3], mat[3][3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    x0[k] = make_double3(p[ca[k]].x - p[cb[k]].x, p[ca[k]].y - p[cb[k]].y, p[ca[k]].z - p[cb[k]].z);
-    xc[k] = make_double3(q[ca[k]].x - q[cb[k]].x, q[ca[k]].y - q[cb[k]].y, q[ca[k]].z - q[cb[k]].z);
+    x0[k] = mim_diff(p[MIM_CA[k]], p[MIM_CB[k]]);
+    xc[k] = mim_diff(q[MIM_CA[k]], q[MIM_CB[k]]);
   }
 #pragma unroll
   for (int ka = 0; ka < 3; ++ka) {
-    const int la = ca[ka], lb = cb[ka];
-    dd[ka] = dss[ka] - (xc[ka].x * xc[ka].x + xc[ka].y * xc[ka].y + xc[ka].z * xc[ka].z);
+    dd[ka] = dss[ka] - mim_dot(xc[ka], xc[ka]);
 #pragma unroll
-    for (int kb = 0; kb < 3; ++kb) {
-      const double3 a = mim_dir(la, ca[kb], cb[kb], x0[kb]);
-      const double3 b = mim_dir(lb, ca[kb], cb[kb], x0[kb]);
-      da[ka][kb] = a;
-      db[ka][kb] = b;
-      double aux3 = (-a.x * xc[ka].x + -a.y * xc[ka].y + -a.z * xc[ka].z) * im[la];
-      aux3 = aux3 + (b.x * xc[ka].x + b.y * xc[ka].y + b.z * xc[ka].z) * im[lb];
-      mat[ka][kb] = -(aux3 * 4.0);
-    }
+    for (int kb = 0; kb < 3; ++kb) mat[ka][kb] = -(mim_elem(ka, kb, mim_dot(x0[kb], xc[ka]), im) * 4.0);
   }
   const MimInv inv = mim_inverse(mat);
-  const double gg1 = im[ca[2]] * 2.0, gg2 = im[cb[2]] * 2.0;  // the last constraint's atoms
+  const double gg1 = im[MIM_CA[2]] * 2.0, gg2 = im[MIM_CB[2]] * 2.0;  // the last constraint's atoms
   double gam[3] = {0.0, 0.0, 0.0};
   bool ok = true;
   for (int iter = 0;;) {
     const double gamo[3] = {gam[0], gam[1], gam[2]};
     double g[3];
-    if (iter == 0) {
 #pragma unroll
-      for (int ka = 0; ka < 3; ++ka) g[ka] = dd[ka];
-    } else {
-#pragma unroll
-      for (int ka = 0; ka < 3; ++ka) {
-        double xd = 0.0, yd = 0.0, zd = 0.0;
+    for (int ka = 0; ka < 3; ++ka) {
+      double3 s = make_double3(0.0, 0.0, 0.0);
+      if (iter > 0) {
 #pragma unroll
         for (int kb = 0; kb < 3; ++kb) {
-          double aux = gam[kb] * gg1;
-          xd = xd + da[ka][kb].x * aux;
-          yd = yd + da[ka][kb].y * aux;
-          zd = zd + da[ka][kb].z * aux;
-          aux = gam[kb] * gg2;
-          xd = xd + -db[ka][kb].x * aux;
-          yd = yd + -db[ka][kb].y * aux;
-          zd = zd + -db[ka][kb].z * aux;
+          const int sa = mim_sgn(MIM_CA[ka], kb), sb = mim_sgn(MIM_CB[ka], kb);
+          if (sa) s = mim_fma(sa * (gam[kb] * gg1), x0[kb], s);
+          if (sb) s = mim_fma(-sb * (gam[kb] * gg2), x0[kb], s);
         }
-        g[ka] = dd[ka] - (xd * xd + yd * yd + zd * zd);
       }
+      g[ka] = dd[ka] - mim_dot(s, s);
     }
     mim_solve(inv, g);
 #pragma unroll
@@ -151,41 +152,22 @@ __device__ inline bool shake_mim3(double3 (&q)[3], const double3 (&p)[3], const 
     bool more = false;
 #pragma unroll
     for (int ka = 0; ka < 3; ++ka)
-      if (gam[ka] != 0.0 && fabs((gam[ka] - gamo[ka]) / gam[ka]) > MIM_TOL) more = true;
+      if (gam[ka] != 0.0 && fabs(gam[ka] - gamo[ka]) > MIM_TOL * fabs(gam[ka])) more = true;
     if (!more) break;
   }
   // corrections, each atom once: by the first constraint that holds it
   // (rattle_verlet.f:514-541)
-  bool mask[3] = {true, true, true};
 #pragma unroll
-  for (int ka = 0; ka < 3; ++ka) {
-    const int la = ca[ka], lb = cb[ka];
-    const double xd = im[la] * 2.0, yd = im[lb] * 2.0;
+  for (int at = 0; at < 3; ++at) {
+    const double w = im[at] * 2.0;
 #pragma unroll
     for (int kb = 0; kb < 3; ++kb) {
-      if (mask[la]) {
-        double aux = gam[kb] * xd;
-        q[la].x = q[la].x + da[ka][kb].x * aux;
-        q[la].y = q[la].y + da[ka][kb].y * aux;
-        q[la].z = q[la].z + da[ka][kb].z * aux;
-        aux = aux * dti;
-        v[la].x = v[la].x + da[ka][kb].x * aux;
-        v[la].y = v[la].y + da[ka][kb].y * aux;
-        v[la].z = v[la].z + da[ka][kb].z * aux;
-      }
-      if (mask[lb]) {
-        double aux = gam[kb] * yd;
-        q[lb].x = q[lb].x + db[ka][kb].x * aux;
-        q[lb].y = q[lb].y + db[ka][kb].y * aux;
-        q[lb].z = q[lb].z + db[ka][kb].z * aux;
-        aux = aux * dti;
-        v[lb].x = v[lb].x + db[ka][kb].x * aux;
-        v[lb].y = v[lb].y + db[ka][kb].y * aux;
-        v[lb].z = v[lb].z + db[ka][kb].z * aux;
-      }
+      const int s = mim_sgn(at, kb);
+      if (!s) continue;
+      const double aux = s * (gam[kb] * w);
+      q[at] = mim_fma(aux, x0[kb], q[at]);
+      v[at] = mim_fma(aux * dti, x0[kb], v[at]);
     }
-    mask[la] = false;
-    mask[lb] = false;
   }
   return ok;
 }
@@ -193,68 +175,59 @@ __device__ inline bool shake_mim3(double3 (&q)[3], const double3 (&p)[3], const 
 // RATTLE: velocities made orthogonal to the bonds at positions r by one
 // linear solve (rattle_correc.f:176-385).
 __device__ inline void rattle_mim3(const double3 (&r)[3], double3 (&v)[3], const double (&im)[3]) {
-  constexpr int ca[3] = {0, 0, 1}, cb[3] = {1, 2, 2};
-  double3 bv[3], da[3][3], db[3][3];
+  double3 bv[3];
   double mat[3][3], gam[3];
 #pragma unroll
-  for (int k = 0; k < 3; ++k)
-    bv[k] = make_double3(r[ca[k]].x - r[cb[k]].x, r[ca[k]].y - r[cb[k]].y, r[ca[k]].z - r[cb[k]].z);
+  for (int k = 0; k < 3; ++k) bv[k] = mim_diff(r[MIM_CA[k]], r[MIM_CB[k]]);
 #pragma unroll
   for (int ka = 0; ka < 3; ++ka) {
-    const int la = ca[ka], lb = cb[ka];
-    const double3 xc = make_double3(v[la].x - v[lb].x, v[la].y - v[lb].y, v[la].z - v[lb].z);
-    gam[ka] = -(xc.x * bv[ka].x + xc.y * bv[ka].y + xc.z * bv[ka].z);
+    gam[ka] = -mim_dot(mim_diff(v[MIM_CA[ka]], v[MIM_CB[ka]]), bv[ka]);
 #pragma unroll
-    for (int kb = 0; kb < 3; ++kb) {
-      const double3 a = mim_dir(la, ca[kb], cb[kb], bv[kb]);
-      const double3 b = mim_dir(lb, ca[kb], cb[kb], bv[kb]);
-      da[ka][kb] = a;
-      db[ka][kb] = b;
-      double aux3 = (bv[ka].x * -a.x + bv[ka].y * -a.y + bv[ka].z * -a.z) * im[la];
-      aux3 = aux3 + (bv[ka].x * b.x + bv[ka].y * b.y + bv[ka].z * b.z) * im[lb];
-      mat[ka][kb] = -(aux3 * 2.0);
-    }
+    for (int kb = 0; kb < 3; ++kb) mat[ka][kb] = -(mim_elem(ka, kb, mim_dot(bv[ka], bv[kb]), im) * 2.0);
   }
   mim_solve(mim_inverse(mat), gam);
-  bool mask[3] = {true, true, true};
 #pragma unroll
-  for (int ka = 0; ka < 3; ++ka) {
-    const int la = ca[ka], lb = cb[ka];
-    const double xd = im[la] * 2.0, yd = im[lb] * 2.0;
+  for (int at = 0; at < 3; ++at) {
+    const double w = im[at] * 2.0;
 #pragma unroll
     for (int kb = 0; kb < 3; ++kb) {
-      if (mask[la]) {
-        v[la].x = v[la].x + (da[ka][kb].x * gam[kb]) * xd;
-        v[la].y = v[la].y + (da[ka][kb].y * gam[kb]) * xd;
-        v[la].z = v[la].z + (da[ka][kb].z * gam[kb]) * xd;
-      }
-      if (mask[lb]) {
-        v[lb].x = v[lb].x + (db[ka][kb].x * gam[kb]) * yd;
-        v[lb].y = v[lb].y + (db[ka][kb].y * gam[kb]) * yd;
-        v[lb].z = v[lb].z + (db[ka][kb].z * gam[kb]) * yd;
-      }
+      const int s = mim_sgn(at, kb);
+      if (!s) continue;
+      v[at].x = v[at].x + (bv[kb].x * (s * gam[kb])) * w;
+      v[at].y = v[at].y + (bv[kb].y * (s * gam[kb])) * w;
+      v[at].z = v[at].z + (bv[kb].z * (s * gam[kb])) * w;
     }
-    mask[la] = false;
-    mask[lb] = false;
   }
 }
 
-// One unit's share of an integration stage, in ORAC's order (mtsmd.f):
-//   MD_KICK_FAST  v += Ff*0.5*h/m, RATTLE        correc + rattle_correc (:2876-2884)
-//   MD_KICK_MID   v += Fm*0.5*hm/m, RATTLE       the inner nonbonded shell (two shells)
-//   MD_KICK_SLOW  v += Fs*0.5*dt/m, RATTLE       correc + rattle_correc (:2598-2604, :3121-3146)
-//   MD_VERLET     x += h*v + Ff*0.5*h^2/m, v += Ff*0.5*h/m, then SHAKE against the
-//                 positions before the drift      verlet + rattle_verlet (:2663-2683)
-//   MD_RATTLE     RATTLE alone
-// applied in that order when several are set (a stage that ends one level's
-// step and starts the next).  Ff are the fast forces, Fs the slow ones; the
-// expressions keep verlet.f's and correc.f's association.  One thread per
-// unit; NA atoms per unit as a template parameter so the unit stays in
-// registers.
+// v += f*0.5*dt/m, then RATTLE of a rigid unit (correc + rattle_correc): verlet.f's and correc.f's association
 template <int NA>
-__device__ __forceinline__ void md_unit(const MdDesc &d, int u, int a0, double dt, double hm, double h, int flags) {
-  double3 x[NA], v[NA], ff[NA];
-  double m[NA], im[NA];
+__device__ __forceinline__ void md_kick(const double *fx, const double *fy, const double *fz, int a0, double dt,
+                                        const double3 (&x)[NA], double3 (&v)[NA], const double (&m)[NA],
+                                        const double (&im)[NA]) {
+#pragma unroll
+  for (int k = 0; k < NA; ++k) {
+    v[k].x = v[k].x + gmem(fx)[a0 + k] * 0.5 * dt / m[k];
+    v[k].y = v[k].y + gmem(fy)[a0 + k] * 0.5 * dt / m[k];
+    v[k].z = v[k].z + gmem(fz)[a0 + k] * 0.5 * dt / m[k];
+  }
+  if constexpr (NA == 3) rattle_mim3(x, v, im);
+}
+
+// the kicks that end a step and those that start the next, in mtsmd.f's order
+template <int NA>
+__device__ __forceinline__ void md_kicks(const MdDesc &d, int a0, double dt, double hm, int flags,
+                                         const double3 (&x)[NA], double3 (&v)[NA], const double (&m)[NA],
+                                         const double (&im)[NA]) {
+  if (flags & MD_END_MID) md_kick<NA>(d.fmx, d.fmy, d.fmz, a0, hm, x, v, m, im);
+  if (flags & MD_END_SLOW) md_kick<NA>(d.fx, d.fy, d.fz, a0, dt, x, v, m, im);
+  if (flags & MD_KICK_SLOW) md_kick<NA>(d.fx, d.fy, d.fz, a0, dt, x, v, m, im);
+  if (flags & MD_KICK_MID) md_kick<NA>(d.fmx, d.fmy, d.fmz, a0, hm, x, v, m, im);
+}
+
+template <int NA>
+__device__ __forceinline__ void md_load(const MdDesc &d, int a0, double3 (&x)[NA], double3 (&v)[NA], double (&m)[NA],
+                                        double (&im)[NA]) {
 #pragma unroll
   for (int k = 0; k < NA; ++k) {
     const int a = a0 + k;
@@ -262,49 +235,63 @@ __device__ __forceinline__ void md_unit(const MdDesc &d, int u, int a0, double d
     im[k] = 1.0 / m[k];
     x[k] = make_double3(gmem(d.x)[a], gmem(d.y)[a], gmem(d.z)[a]);
     v[k] = make_double3(gmem(d.vx)[a], gmem(d.vy)[a], gmem(d.vz)[a]);
-    ff[k] = make_double3(gmem(d.bfx)[a], gmem(d.bfy)[a], gmem(d.bfz)[a]);
   }
-  if (flags & MD_KICK_FAST) {
-#pragma unroll
-    for (int k = 0; k < NA; ++k) {
-      v[k].x = v[k].x + ff[k].x * 0.5 * h / m[k];
-      v[k].y = v[k].y + ff[k].y * 0.5 * h / m[k];
-      v[k].z = v[k].z + ff[k].z * 0.5 * h / m[k];
-    }
-    if constexpr (NA == 3) rattle_mim3(x, v, im);
-  }
-  if (flags & MD_KICK_MID) {
-#pragma unroll
-    for (int k = 0; k < NA; ++k) {
-      const int a = a0 + k;
-      v[k].x = v[k].x + gmem(d.fmx)[a] * 0.5 * hm / m[k];
-      v[k].y = v[k].y + gmem(d.fmy)[a] * 0.5 * hm / m[k];
-      v[k].z = v[k].z + gmem(d.fmz)[a] * 0.5 * hm / m[k];
-    }
-    if constexpr (NA == 3) rattle_mim3(x, v, im);
-  }
-  if (flags & MD_KICK_SLOW) {
-#pragma unroll
-    for (int k = 0; k < NA; ++k) {
-      const int a = a0 + k;
-      v[k].x = v[k].x + gmem(d.fx)[a] * 0.5 * dt / m[k];
-      v[k].y = v[k].y + gmem(d.fy)[a] * 0.5 * dt / m[k];
-      v[k].z = v[k].z + gmem(d.fz)[a] * 0.5 * dt / m[k];
-    }
-    if constexpr (NA == 3) rattle_mim3(x, v, im);
-  }
+}
+
+__device__ __forceinline__ void md_store_v(const MdDesc &d, int a, double3 v) {
+  gmem(d.vx)[a] = v.x;
+  gmem(d.vy)[a] = v.y;
+  gmem(d.vz)[a] = v.z;
+}
+
+__device__ __forceinline__ void md_store_x(const MdDesc &d, int a, double3 x) {
+  gmem(d.x)[a] = x.x;
+  gmem(d.y)[a] = x.y;
+  gmem(d.z)[a] = x.z;
+  double xp, yp, zp;
+  to_reduced(d.oc, x.x, x.y, x.z, xp, yp, zp);
+  gmem(d.xp)[a] = xp;
+  gmem(d.yp)[a] = yp;
+  gmem(d.zp)[a] = zp;
+}
+
+// a stage between two steps of one run: past the run's last step only what ends that step is left
+__device__ inline int md_stage(const MdDesc &d, int flags) {
+  if ((flags & MD_BETWEEN) && gmem(d.step)[0] == gmem(d.step)[1]) flags &= MD_END_MID | MD_END_SLOW;
+  return flags;
+}
+
+// One unit's share of an integration stage, in ORAC's order (mtsmd.f):
+//   MD_KICK_FAST  v += Ff*0.5*h/m, RATTLE        correc + rattle_correc (:2876-2884)
+//   MD_END_MID    v += Fm*0.5*hm/m, RATTLE       the inner nonbonded shell (two shells)
+//   MD_END_SLOW   v += Fs*0.5*dt/m, RATTLE       correc + rattle_correc (:3121-3146)
+//   MD_KICK_SLOW, MD_KICK_MID                    the same kicks, starting the next step (:2598-2604)
+//   MD_VERLET     x += h*v + Ff*0.5*h^2/m, v += Ff*0.5*h/m, then SHAKE against the
+//                 positions before the drift      verlet + rattle_verlet (:2663-2683)
+//   MD_RATTLE     RATTLE alone
+// applied in that order when several are set.  Ff are the fast forces, Fs the
+// slow ones.  One thread per unit; NA atoms per unit as a template parameter
+// so the unit stays in registers.
+template <int NA>
+__device__ __forceinline__ void md_unit(const MdDesc &d, int u, int a0, double dt, double hm, double h, int flags) {
+  double3 x[NA], v[NA];
+  double m[NA], im[NA];
+  md_load<NA>(d, a0, x, v, m, im);
+  if (flags & MD_KICK_FAST) md_kick<NA>(d.bfx, d.bfy, d.bfz, a0, h, x, v, m, im);
+  md_kicks<NA>(d, a0, dt, hm, flags, x, v, m, im);
   if (flags & MD_VERLET) {
     double3 p[NA];
     const double ts2 = h * h;
 #pragma unroll
     for (int k = 0; k < NA; ++k) {
+      const double3 f = make_double3(gmem(d.bfx)[a0 + k], gmem(d.bfy)[a0 + k], gmem(d.bfz)[a0 + k]);
       p[k] = x[k];
-      x[k].x = x[k].x + h * v[k].x + ff[k].x * 0.5 * ts2 / m[k];
-      x[k].y = x[k].y + h * v[k].y + ff[k].y * 0.5 * ts2 / m[k];
-      x[k].z = x[k].z + h * v[k].z + ff[k].z * 0.5 * ts2 / m[k];
-      v[k].x = v[k].x + ff[k].x * 0.5 * h / m[k];
-      v[k].y = v[k].y + ff[k].y * 0.5 * h / m[k];
-      v[k].z = v[k].z + ff[k].z * 0.5 * h / m[k];
+      x[k].x = x[k].x + h * v[k].x + f.x * 0.5 * ts2 / m[k];
+      x[k].y = x[k].y + h * v[k].y + f.y * 0.5 * ts2 / m[k];
+      x[k].z = x[k].z + h * v[k].z + f.z * 0.5 * ts2 / m[k];
+      v[k].x = v[k].x + f.x * 0.5 * h / m[k];
+      v[k].y = v[k].y + f.y * 0.5 * h / m[k];
+      v[k].z = v[k].z + f.z * 0.5 * h / m[k];
     }
     if constexpr (NA == 3)
       if (!shake_mim3(x, p, im, d.ud2 + 3 * (size_t)u, h != 0.0 ? 1.0 / h : 0.0, v)) atomicAdd(d.fail, 1);
@@ -313,28 +300,20 @@ __device__ __forceinline__ void md_unit(const MdDesc &d, int u, int a0, double d
     if (flags & MD_RATTLE) rattle_mim3(x, v, im);
 #pragma unroll
   for (int k = 0; k < NA; ++k) {
-    const int a = a0 + k;
-    gmem(d.vx)[a] = v[k].x;
-    gmem(d.vy)[a] = v[k].y;
-    gmem(d.vz)[a] = v[k].z;
-    if (flags & MD_VERLET) {
-      gmem(d.x)[a] = x[k].x;
-      gmem(d.y)[a] = x[k].y;
-      gmem(d.z)[a] = x[k].z;
-      double xp, yp, zp;
-      to_reduced(d.oc, x[k].x, x[k].y, x[k].z, xp, yp, zp);
-      gmem(d.xp)[a] = xp;
-      gmem(d.yp)[a] = yp;
-      gmem(d.zp)[a] = zp;
-    }
+    md_store_v(d, a0 + k, v[k]);
+    if (flags & MD_VERLET) md_store_x(d, a0 + k, x[k]);
   }
 }
 
+// rest: only the units that k_md_advance does not take
 __global__ void __launch_bounds__(256) k_md_units(const MdDesc *__restrict__ D, double dt, double hm, double h,
-                                                  int flags) {
+                                                  int flags, int rest) {
   const MdDesc &d = D[blockIdx.y];
-  const int u = blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= d.nunits) return;
+  int u = blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= (rest ? d.nrest : d.nunits)) return;
+  if (rest) u = gmem(d.rest_unit)[u];
+  flags = md_stage(d, flags);
+  if (!(flags & ~MD_BETWEEN)) return;
   const int a0 = gmem(d.ufirst)[u];
   if (gmem(d.urigid)[u])
     md_unit<3>(d, u, a0, dt, hm, h, flags);
@@ -342,10 +321,152 @@ __global__ void __launch_bounds__(256) k_md_units(const MdDesc *__restrict__ D, 
     md_unit<1>(d, u, a0, dt, hm, h, flags);
 }
 
-__global__ void __launch_bounds__(256) k_md_bonds(const MdDesc *__restrict__ D) {
+// ---------------------------------------------------------------- a step's fast level in one launch
+
+// A unit without terms: kicks, then nsub times drift, SHAKE, RATTLE (its fast forces are zero).
+template <int NA>
+__device__ __forceinline__ void md_free(const MdDesc &d, int a0, const double *dss, double dt, double hm, double h,
+                                        int flags, int nsub) {
+  double3 x[NA], v[NA];
+  double m[NA], im[NA];
+  md_load<NA>(d, a0, x, v, m, im);
+  md_kicks<NA>(d, a0, dt, hm, flags, x, v, m, im);
+  const double dti = h != 0.0 ? 1.0 / h : 0.0;
+  for (int s = 0; s < nsub; ++s) {
+    double3 p[NA];
+#pragma unroll
+    for (int k = 0; k < NA; ++k) {
+      p[k] = x[k];
+      x[k] = mim_fma(h, v[k], x[k]);
+    }
+    if constexpr (NA == 3) {
+      if (!shake_mim3(x, p, im, dss, dti, v)) atomicAdd(d.fail, 1);
+      rattle_mim3(x, v, im);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NA; ++k) {
+    md_store_v(d, a0 + k, v[k]);
+    if (nsub) md_store_x(d, a0 + k, x[k]);
+  }
+}
+
+// The atoms of one workgroup's slots (K a thread), connected by terms among
+// themselves only: positions in LDS, everything else in registers.  An atom
+// sums its own terms, in the order of the terms, from both ends' positions:
+// twice the arithmetic of one thread per term, but no second pass.
+template <int K>
+__device__ __forceinline__ void md_connected(const MdDesc &d, int s0, int n, double (*pos)[3], double dt, double hm,
+                                             double h, int flags, int nsub) {
+  const double ts2 = h * h;
+  double3 x[K][1], v[K][1], f[K];
+  double m[K][1], im[K][1];
+  int at[K], deg[K], off[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int s = k * MD_WG + threadIdx.x;
+    at[k] = s < n ? gmem(d.slot_atom)[s0 + s] : -1;
+    deg[k] = off[k] = 0;
+    if (at[k] < 0) continue;
+    deg[k] = gmem(d.slot_deg)[s0 + s];
+    off[k] = gmem(d.slice_off)[(s0 + s) >> 6] + (threadIdx.x & 63);
+    md_load<1>(d, at[k], x[k], v[k], m[k], im[k]);
+    f[k] = make_double3(gmem(d.bfx)[at[k]], gmem(d.bfy)[at[k]], gmem(d.bfz)[at[k]]);
+    md_kicks<1>(d, at[k], dt, hm, flags, x[k], v[k], m[k], im[k]);
+  }
+  for (int s = 0; s < nsub; ++s) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (at[k] < 0) continue;
+      double3 &xx = x[k][0], &vv = v[k][0];
+      const double w = m[k][0];
+      xx.x = xx.x + h * vv.x + f[k].x * 0.5 * ts2 / w;
+      xx.y = xx.y + h * vv.y + f[k].y * 0.5 * ts2 / w;
+      xx.z = xx.z + h * vv.z + f[k].z * 0.5 * ts2 / w;
+      vv.x = vv.x + f[k].x * 0.5 * h / w;
+      vv.y = vv.y + f[k].y * 0.5 * h / w;
+      vv.z = vv.z + f[k].z * 0.5 * h / w;
+      double *p = pos[k * MD_WG + threadIdx.x];
+      p[0] = xx.x;
+      p[1] = xx.y;
+      p[2] = xx.z;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (at[k] < 0) continue;
+      double3 &xx = x[k][0], &vv = v[k][0];
+      double3 sum = make_double3(0.0, 0.0, 0.0);
+#pragma unroll 2
+      for (int e = 0; e < deg[k]; ++e) {
+        const double *p = pos[gmem(d.ent_slot)[off[k] + 64 * e]];
+        const double2 kr = gload(d.ent_kr + off[k] + 64 * e);
+        const double dx = xx.x - p[0], dy = xx.y - p[1], dz = xx.z - p[2];
+        const double r = sqrt(dx * dx + dy * dy + dz * dz);
+        const double g = -2.0 * kr.x * (r - kr.y) / r;  // force along (x_i - x_j)
+        {
+#pragma clang fp contract(off)
+          // each term's vector rounded before it is added, as k_md_bonds stores it
+          sum.x = sum.x + g * dx;
+          sum.y = sum.y + g * dy;
+          sum.z = sum.z + g * dz;
+        }
+      }
+      f[k] = sum;
+      const double w = m[k][0];
+      vv.x = vv.x + sum.x * 0.5 * h / w;
+      vv.y = vv.y + sum.y * 0.5 * h / w;
+      vv.z = vv.z + sum.z * 0.5 * h / w;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    if (at[k] < 0) continue;
+    md_store_v(d, at[k], v[k][0]);
+    if (!nsub) continue;
+    md_store_x(d, at[k], x[k][0]);
+    gmem(d.bfx)[at[k]] = f[k].x;
+    gmem(d.bfy)[at[k]] = f[k].y;
+    gmem(d.bfz)[at[k]] = f[k].z;
+  }
+}
+
+// The kicks that end a step and start the next, then the next step's nsub fast
+// substeps, in one launch; its workgroups take the connected atoms first, then
+// MD_FREE units without terms each (a wavefront a SIMD: a unit's constraints
+// are one serial chain of FP64 instructions, so spreading the units over the
+// chip is what counts).  Four substeps of 216 waters: 11 us, where five
+// launches over the units and four over the atoms took 42 and the gaps between
+// them; of 4,900 waters and a 1,660-atom solute 19 us instead of 66.
+__global__ void __launch_bounds__(MD_WG) k_md_advance(const MdDesc *__restrict__ D, int nconn, double dt, double hm,
+                                                      double h, int flags, int nsub) {
+  extern __shared__ __align__(16) double md_pos[];
+  const MdDesc &d = D[blockIdx.y];
+  const int blk = blockIdx.x;
+  if (md_stage(d, flags) != flags) {
+    flags = md_stage(d, flags);
+    nsub = 0;
+  }
+  if (blk < nconn) {
+    if (blk >= d.nwg) return;
+    const int s0 = gmem(d.wg_slot)[blk], n = gmem(d.wg_slot)[blk + 1] - s0;
+    double(*pos)[3] = reinterpret_cast<double(*)[3]>(md_pos);
+    if (n <= MD_WG) md_connected<1>(d, s0, n, pos, dt, hm, h, flags, nsub);
+    else md_connected<2>(d, s0, n, pos, dt, hm, h, flags, nsub);
+    return;
+  }
+  const int u = (blk - nconn) * MD_FREE + threadIdx.x;
+  if (threadIdx.x >= MD_FREE || u >= d.nfree) return;
+  const int a0 = gmem(d.free_atom)[u];
+  if (u < d.nfree_rigid) md_free<3>(d, a0, d.free_d2 + 3 * (size_t)u, dt, hm, h, flags, nsub);
+  else md_free<1>(d, a0, nullptr, dt, hm, h, flags, nsub);
+}
+
+__global__ void __launch_bounds__(256) k_md_bonds(const MdDesc *__restrict__ D, int rest) {
   const MdDesc &d = D[blockIdx.y];
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= d.nbond) return;
+  if (t >= d.nbond || (rest && !d.nrest)) return;
   const int i = d.bi[t], j = d.bj[t];
   const double dx = d.x[i] - d.x[j], dy = d.y[i] - d.y[j], dz = d.z[i] - d.z[j];
   const double r = sqrt(dx * dx + dy * dy + dz * dz);
@@ -358,10 +479,10 @@ __global__ void __launch_bounds__(256) k_md_bonds(const MdDesc *__restrict__ D) 
 }
 
 // fast forces per atom from its terms, in fixed order
-__global__ void __launch_bounds__(256) k_md_bond_gather(const MdDesc *__restrict__ D) {
+__global__ void __launch_bounds__(256) k_md_bond_gather(const MdDesc *__restrict__ D, int rest) {
   const MdDesc &d = D[blockIdx.y];
   const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= d.natoms) return;
+  if (a >= d.natoms || (rest && !d.nrest)) return;
   double sx = 0.0, sy = 0.0, sz = 0.0;
   for (int t = d.bg_off[a]; t < d.bg_off[a + 1]; ++t) {
     const int sp = d.bg_term[t];
@@ -476,9 +597,9 @@ __global__ void __launch_bounds__(256) k_md_scale_v(const MdDesc *__restrict__ D
   d.vz[a] *= s;
 }
 
-// one outer step done: advance every system's step counter
-__global__ void k_md_tick(const MdDesc *__restrict__ D) {
-  if (threadIdx.x == 0) *D[blockIdx.y].step += 1;
+// the step count at which the run of nsteps that starts here ends
+__global__ void k_md_begin(const MdDesc *__restrict__ D, int nsteps) {
+  if (threadIdx.x == 0) D[blockIdx.y].step[1] = D[blockIdx.y].step[0] + nsteps;
 }
 
 static void md_dims(const MdDesc *h, int nsys, int &max_units, int &max_atoms, int &max_bonds) {
@@ -494,18 +615,47 @@ void launch_md_units(const MdDesc *d, const MdDesc *h, int nsys, double dt, doub
                      hipStream_t st) {
   int mu, ma, mb;
   md_dims(h, nsys, mu, ma, mb);
-  if (mu > 0) hipLaunchKernelGGL(k_md_units, dim3((mu + 255) / 256, nsys), dim3(256), 0, st, d, dt, hm, hin, flags);
+  if (mu > 0) hipLaunchKernelGGL(k_md_units, dim3((mu + 255) / 256, nsys), dim3(256), 0, st, d, dt, hm, hin, flags, 0);
+}
+
+static void fast_forces(const MdDesc *d, const MdDesc *h, int nsys, bool rest, hipStream_t st) {
+  int mu, ma, mb;
+  md_dims(h, nsys, mu, ma, mb);
+  if (mb > 0) hipLaunchKernelGGL(k_md_bonds, dim3((mb + 255) / 256, nsys), dim3(256), 0, st, d, rest ? 1 : 0);
+  if (ma > 0) hipLaunchKernelGGL(k_md_bond_gather, dim3((ma + 255) / 256, nsys), dim3(256), 0, st, d, rest ? 1 : 0);
 }
 
 void launch_md_fast_forces(const MdDesc *d, const MdDesc *h, int nsys, hipStream_t st) {
-  int mu, ma, mb;
-  md_dims(h, nsys, mu, ma, mb);
-  if (mb > 0) hipLaunchKernelGGL(k_md_bonds, dim3((mb + 255) / 256, nsys), dim3(256), 0, st, d);
-  if (ma > 0) hipLaunchKernelGGL(k_md_bond_gather, dim3((ma + 255) / 256, nsys), dim3(256), 0, st, d);
+  fast_forces(d, h, nsys, false, st);
 }
 
-void launch_md_tick(const MdDesc *d, int nsys, hipStream_t st) {
-  hipLaunchKernelGGL(k_md_tick, dim3(1, nsys), dim3(64), 0, st, d);
+void launch_md_begin(const MdDesc *d, int nsys, int nsteps, hipStream_t st) {
+  hipLaunchKernelGGL(k_md_begin, dim3(1, nsys), dim3(64), 0, st, d, nsteps);
+}
+
+void launch_md_advance(const MdDesc *d, const MdDesc *h, int nsys, double dt, double hm, double hin, int flags,
+                       int nsub, hipStream_t st) {
+  int mw = 0, ms = 0, mf = 0, mr = 0;
+  for (int s = 0; s < nsys; ++s) {
+    mw = std::max(mw, h[s].nwg);
+    ms = std::max(ms, h[s].wg_most);
+    mf = std::max(mf, h[s].nfree);
+    mr = std::max(mr, h[s].nrest);
+  }
+  const int nb = mw + (mf + MD_FREE - 1) / MD_FREE;
+  if (nb > 0)
+    hipLaunchKernelGGL(k_md_advance, dim3(nb, nsys), dim3(MD_WG), ms * 3 * sizeof(double), st, d, mw, dt, hm, hin,
+                       flags, nsub);
+  if (mr == 0) return;
+  // units the launch above does not take: one launch per kick and substep
+  const dim3 g((mr + 255) / 256, nsys), b(256);
+  const int between = flags & MD_BETWEEN;
+  hipLaunchKernelGGL(k_md_units, g, b, 0, st, d, dt, hm, hin, flags | (nsub > 0 ? MD_VERLET : 0), 1);
+  for (int k = 0; k < nsub; ++k) {
+    fast_forces(d, h, nsys, true, st);
+    hipLaunchKernelGGL(k_md_units, g, b, 0, st, d, dt, hm, hin,
+                       between | MD_KICK_FAST | (k + 1 < nsub ? MD_VERLET : 0), 1);
+  }
 }
 
 void launch_md_energy(const MdDesc *d, int nsys, hipStream_t st) {

@@ -1325,7 +1325,8 @@ constexpr int TAIL_THREADS = 1024, TAIL_COLS = 16 + 16 + 8 + 1;
 
 __global__ void __launch_bounds__(TAIL_THREADS) k_tail(const PmeDesc *__restrict__ P, const PairDesc *__restrict__ Q,
                                                        const CorrDesc *__restrict__ Cc,
-                                                       const ListDesc *__restrict__ L, int nsys, int natomb) {
+                                                       const ListDesc *__restrict__ L, int nsys, int natomb,
+                                                       int step) {
   const int sys = blockIdx.y;
   int blk = blockIdx.x;
   if (blk < natomb) {
@@ -1343,17 +1344,19 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_tail(const PmeDesc *__restrict
     if (Cc) corr_energy(Cc[sys], blk - 32);
   } else if (L) {
     if (!L[sys].split) list_total(L[sys], false);
+    __syncthreads();  // list_total, the last to read the step, is done in every wavefront
+    if (step && threadIdx.x == 0) *L[sys].step += 1;
   }
 }
 
 void launch_tail(const PmeDesc *d_pme, const PmeDesc *h_pme, int npme, const PairDesc *d_pair, const CorrDesc *d_corr,
-                 const ListDesc *d_list, int nsys, hipStream_t st) {
+                 const ListDesc *d_list, int nsys, bool step, hipStream_t st) {
   int max_atoms = 1;
   for (int s = 0; s < npme; ++s)
     if (h_pme[s].fx_dst) max_atoms = std::max(max_atoms, h_pme[s].natoms);
   const int natomb = (max_atoms + TAIL_THREADS - 1) / TAIL_THREADS;
   hipLaunchKernelGGL(k_tail, dim3(natomb + TAIL_COLS, npme), dim3(TAIL_THREADS), 0, st, d_pme, d_pair, d_corr, d_list,
-                     nsys, natomb);
+                     nsys, natomb, step ? 1 : 0);
 }
 
 // ---------------------------------------------------------------- cself
