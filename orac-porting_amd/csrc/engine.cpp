@@ -22,8 +22,42 @@ enum Stage { ST_BEGIN, ST_CENTRES, ST_LIST, ST_PAIRS, ST_PME, ST_END, ST_KBEG, S
              NSTAGE };
 constexpr int NSTAGE_MS = 5;  // centres, list, pairs, pme, corrections; then the pair kernel alone
 
+// What the host reads after every evaluation -- a system's energies, virial and
+// list size -- lies in host memory that the kernels write: reading it is one
+// wait for the stream, where a copy of 600 bytes and one of 8 took 36 us a
+// system (16 alchemical windows spent 895 of 1,444 us in them).  Records come
+// from blocks that the engine keeps and gives back.
+struct Records {
+  static constexpr size_t SIZE = 1024, PER = 32;
+  std::vector<char *> blocks, unused;
+  ~Records() {
+    for (char *b : blocks) (void)hipHostFree(b);
+  }
+  char *take() {
+    if (unused.empty()) {
+      void *b = nullptr;
+      ORAC_HIP(hipHostMalloc(&b, SIZE * PER, hipHostMallocCoherent));
+      blocks.push_back(static_cast<char *>(b));
+      unused.reserve(blocks.size() * PER);  // (a record given back never allocates)
+      for (size_t k = PER; k-- > 0;) unused.push_back(blocks.back() + k * SIZE);
+    }
+    char *r = unused.back();
+    unused.pop_back();
+    std::memset(r, 0, SIZE);
+    return r;
+  }
+};
+
 struct System {
   BufSet B;
+  std::shared_ptr<Records> records;  // (outlives the system's record)
+  char *record = nullptr;
+  System() = default;
+  System(const System &) = delete;
+  System &operator=(const System &) = delete;
+  ~System() {
+    if (record) records->unused.push_back(record);
+  }
   int natoms = 0, ngrp = 0, nmol = 0, ntypes = 0, max_group = 1;
   int precision = 0;
   double co[9], oc[9], volume = 0, alpha = 0;
@@ -37,7 +71,10 @@ struct System {
   int slab = 0;           // neighbour-list entries per owner (slab layout)
   double *xp = nullptr, *yp = nullptr, *zp = nullptr;
   double *fx = nullptr, *fy = nullptr, *fz = nullptr;
-  double *out = nullptr;  // device: pme[20], pairs[16] at 20, corrections[4] at 36, lambda0 pme[20] at 48
+  // in the record: pme[20], pairs[16] at 20, corrections[8] at 36, lambda0 pme[20] at 48; the inner shell's
+  // pairs[16] at 72; the list's {entries, overflow, sticky overflow}
+  double *out = nullptr;
+  int *report = nullptr;
   double self_e[2] = {0, 0};
   std::vector<double> q_host;      // charges as created
   std::vector<int32_t> ss_host;    // ss_index
@@ -148,6 +185,12 @@ struct Engine {
   std::map<int, std::unique_ptr<System>> systems;
   std::map<int, std::unique_ptr<Batch>> batches;
   int next_sys = 1, next_batch = 1;
+  std::shared_ptr<Records> records = std::make_shared<Records>();
+  double *stage = nullptr;  // pinned, for read_back
+  ~Engine() {
+    systems.clear();
+    if (stage) (void)hipHostFree(stage);
+  }
   long md_gen = 0;  // bumped by every md setup or state change
 };
 
@@ -157,6 +200,47 @@ static Engine &engine(orac_hip_ctx *ctx) {
   ORAC_REQUIRE(ctx, E_ARG, "null context");
   if (!ctx->engine) ctx->engine = new Engine();
   return *ctx->engine;
+}
+
+// Arrays of n doubles to the caller's memory (null: not wanted); waits for the
+// stream.  Up to STAGE doubles go through pinned memory, joined
+// ones in one copy: six arrays of 5,000 to 50,000 bytes take
+// one transfer instead of six, each of which staged and waited by itself (91
+// to 117 us).  Larger ones are copied directly, where the bandwidth counts.
+constexpr size_t STAGE = 512 * 1024;
+// joined: the six lie one after the other in one allocation.
+static void read_back(orac_hip_ctx *ctx, double *const (&dst)[6], const double *const (&src)[6], int n, bool joined) {
+  Engine &E = engine(ctx);
+  hipStream_t st = ctx->stream;
+  const size_t nb = (size_t)n * sizeof(double);
+  size_t want = 0;
+  for (double *d : dst) want += d ? (size_t)n : 0;
+  const bool staged = want <= STAGE;
+  if (staged && want && !E.stage) ORAC_HIP(hipHostMalloc(reinterpret_cast<void **>(&E.stage), STAGE * sizeof(double)));
+  size_t at = 0;
+  for (int k = 0; k < 6;) {
+    if (!dst[k]) {
+      ++k;
+      continue;
+    }
+    if (!staged) {
+      ORAC_HIP(hipMemcpyAsync(dst[k], src[k], nb, hipMemcpyDeviceToHost, st));
+      ++k;
+      continue;
+    }
+    int m = 1;
+    while (joined && k + m < 6 && dst[k + m]) ++m;
+    ORAC_HIP(hipMemcpyAsync(E.stage + at, src[k], m * nb, hipMemcpyDeviceToHost, st));
+    at += (size_t)m * n;
+    k += m;
+  }
+  ORAC_HIP(hipStreamSynchronize(st));
+  at = 0;
+  for (int k = 0; staged && k < 6; ++k)
+    if (dst[k]) {
+      std::memcpy(dst[k], E.stage + at, nb);
+      at += n;
+    }
 }
 
 static System &get_sys(orac_hip_ctx *ctx, int32_t id) {
@@ -307,8 +391,10 @@ static void system_build(orac_hip_ctx *ctx, System &S, const orac_hip_system_des
   double *xpcm = B.get<double>("xpcm", d.nmol), *ypcm = B.get<double>("ypcm", d.nmol),
          *zpcm = B.get<double>("zpcm", d.nmol);
   double *xpg = B.get<double>("xpg", ng), *ypg = B.get<double>("ypg", ng), *zpg = B.get<double>("zpg", ng);
-  S.out = B.get<double>("out", 72);
-  launch_zero_f64(S.out, 72, st);
+  S.records = engine(ctx).records;
+  S.record = S.records->take();
+  S.out = reinterpret_cast<double *>(S.record);
+  S.report = reinterpret_cast<int *>(S.out + 88);
   S.q_host.assign(d.charge, d.charge + n);
   S.ss_host.assign(d.ss_index, d.ss_index + n);
 
@@ -460,6 +546,7 @@ static void system_build(orac_hip_ctx *ctx, System &S, const orac_hip_system_des
     L.out = B.get<int>("nbidx", S.list_cap);
     L.cap = (long long)S.list_cap;
     L.total = B.get<int>("ltotal", 4);
+    L.report = S.report;
     L.mode = 0;
     L.slab = S.slab;
     std::vector<int> gsize(ng);
@@ -793,6 +880,7 @@ static void size_list(orac_hip_ctx *ctx, int32_t id) {
   const int need = std::min(ng, ((int)(1.5 * tot[2]) + 64 + 31) / 32 * 32);
   S.have_list = false;  // the count pass rewrote the counts
   launch_zero_u64(reinterpret_cast<unsigned long long *>(S.list.total + 2), 1, st);
+  S.report[2] = 0;  // (the stream is idle but for the clearing above)
   if (need > S.slab) {
     ORAC_REQUIRE((size_t)ng * (size_t)need < (size_t)INT32_MAX, E_CAPACITY,
                  "neighbour list larger than 2^31 entries");
@@ -822,13 +910,10 @@ static void size_list(orac_hip_ctx *ctx, int32_t id) {
 // Systems of b whose neighbour list overflowed its slab at some build since
 // their list was last sized (the sticky flag total[3]); synchronises.
 static std::vector<int> list_overflows(orac_hip_ctx *ctx, Batch &b) {
-  const size_t n = b.sys.size();
-  std::vector<int> flag(n, 0), bad;
-  for (size_t k = 0; k < n; ++k)
-    ORAC_HIP(hipMemcpyAsync(&flag[k], b.sys[k]->list.total + 3, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  std::vector<int> bad;
   ORAC_HIP(hipStreamSynchronize(ctx->stream));
-  for (size_t k = 0; k < n; ++k)
-    if (flag[k]) bad.push_back(b.ids[k]);
+  for (size_t k = 0; k < b.sys.size(); ++k)
+    if (b.sys[k]->report[2]) bad.push_back(b.ids[k]);
   return bad;
 }
 
@@ -1026,12 +1111,13 @@ static void md_setup(orac_hip_ctx *ctx, System &S, int nrigid, const int32_t *ri
   d.natoms = n;
   d.nunits = (int)ufirst.size();
   d.nbond = nterm;
-  d.x = B.get<double>("md_x", n);
-  d.y = B.get<double>("md_y", n);
-  d.z = B.get<double>("md_z", n);
-  d.vx = B.get<double>("md_vx", n);
-  d.vy = B.get<double>("md_vy", n);
-  d.vz = B.get<double>("md_vz", n);
+  double *state = B.get<double>("md_state", 6 * (size_t)n);  // one copy reads it back
+  d.x = state;
+  d.y = state + n;
+  d.z = state + 2 * (size_t)n;
+  d.vx = state + 3 * (size_t)n;
+  d.vy = state + 4 * (size_t)n;
+  d.vz = state + 5 * (size_t)n;
   d.xp = S.xp;
   d.yp = S.yp;
   d.zp = S.zp;
@@ -1340,26 +1426,21 @@ extern "C" int orac_hip_system_results(orac_hip_ctx *ctx, int32_t sys, double *f
     set_device(ctx);
     System &S = get_sys(ctx, sys);
     hipStream_t st = ctx->stream;
-    double out[48], outm[16];
-    int tot[2];
-    ORAC_HIP(hipMemcpyAsync(out, S.out, sizeof out, hipMemcpyDeviceToHost, st));
-    ORAC_HIP(hipMemcpyAsync(tot, S.list.total, sizeof tot, hipMemcpyDeviceToHost, st));
-    size_t nb = (size_t)S.natoms * sizeof(double);
-    if (fx) ORAC_HIP(hipMemcpyAsync(fx, S.fx, nb, hipMemcpyDeviceToHost, st));
-    if (fy) ORAC_HIP(hipMemcpyAsync(fy, S.fy, nb, hipMemcpyDeviceToHost, st));
-    if (fz) ORAC_HIP(hipMemcpyAsync(fz, S.fz, nb, hipMemcpyDeviceToHost, st));
-    std::vector<double> mx, my, mz;
     const bool two = S.rcutm > 0.0;
-    if (two) {  // the inner shell's forces and energies join the outer ones
-      ORAC_HIP(hipMemcpyAsync(outm, S.out_m, sizeof outm, hipMemcpyDeviceToHost, st));
+    std::vector<double> mx, my, mz;
+    if (two && (fx || fy || fz)) {  // the inner shell's forces and energies join the outer ones
       mx.resize(S.natoms);
       my.resize(S.natoms);
       mz.resize(S.natoms);
-      ORAC_HIP(hipMemcpyAsync(mx.data(), S.fmx, nb, hipMemcpyDeviceToHost, st));
-      ORAC_HIP(hipMemcpyAsync(my.data(), S.fmy, nb, hipMemcpyDeviceToHost, st));
-      ORAC_HIP(hipMemcpyAsync(mz.data(), S.fmz, nb, hipMemcpyDeviceToHost, st));
     }
-    ORAC_HIP(hipStreamSynchronize(st));
+    const bool m = !mx.empty();
+    double *dst[6] = {fx, fy, fz, m ? mx.data() : nullptr, m ? my.data() : nullptr, m ? mz.data() : nullptr};
+    const double *src[6] = {S.fx, S.fy, S.fz, S.fmx, S.fmy, S.fmz};
+    read_back(ctx, dst, src, S.natoms, false);
+    double out[48];
+    std::memcpy(out, S.out, sizeof out);
+    const double *outm = S.out + 72;
+    const int tot[2] = {S.report[0], S.report[1]};
     if (two) {
       for (int a = 0; a < S.natoms; ++a) {
         if (fx) fx[a] += mx[a];
@@ -1539,9 +1620,8 @@ extern "C" int orac_hip_system_alchemy_results(orac_hip_ctx *ctx, int32_t sys, d
     System &S = get_sys(ctx, sys);
     ORAC_REQUIRE(S.alch, E_STATE, "the system is not alchemical");
     ORAC_REQUIRE(out, E_ARG, "null output");
-    double o[72];
-    ORAC_HIP(hipMemcpyAsync(o, S.out, sizeof o, hipMemcpyDeviceToHost, ctx->stream));
     ORAC_HIP(hipStreamSynchronize(ctx->stream));
+    const double *o = S.out;
     double corr = o[36] + o[37] - o[38];
     if (S.nqq > 0) corr += o[40] + o[41] - o[42];  // ferrf_alchemy_add.f:203: dwrk_al
     const double direct = o[35], recip = o[0] - o[48];
@@ -1737,7 +1817,7 @@ extern "C" int orac_hip_system_set_shells(orac_hip_ctx *ctx, int32_t sys, double
         S.fmx = S.B.get<double>("fmx", S.natoms);
         S.fmy = S.B.get<double>("fmy", S.natoms);
         S.fmz = S.B.get<double>("fmz", S.natoms);
-        S.out_m = S.B.get<double>("out_m", 16);
+        S.out_m = S.out + 72;
         for (double *q : {S.fmx, S.fmy, S.fmz}) launch_zero_f64(q, S.natoms, st);
         launch_zero_f64(S.out_m, 16, st);
       }
@@ -1827,13 +1907,9 @@ extern "C" int orac_hip_md_get_state(orac_hip_ctx *ctx, int32_t sys, double *x, 
     set_device(ctx);
     System &S = get_sys(ctx, sys);
     ORAC_REQUIRE(S.md_on, E_STATE, "dynamics is not set up for this system");
-    hipStream_t st = ctx->stream;
-    const size_t nb = (size_t)S.natoms * sizeof(double);
     double *dst[6] = {x, y, z, vx, vy, vz};
     const double *src[6] = {S.md.x, S.md.y, S.md.z, S.md.vx, S.md.vy, S.md.vz};
-    for (int k = 0; k < 6; ++k)
-      if (dst[k]) ORAC_HIP(hipMemcpyAsync(dst[k], src[k], nb, hipMemcpyDeviceToHost, st));
-    ORAC_HIP(hipStreamSynchronize(st));
+    read_back(ctx, dst, src, S.natoms, true);
   });
 }
 

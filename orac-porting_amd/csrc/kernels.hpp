@@ -225,6 +225,7 @@ struct ListDesc {
   int *out;                  // list entries
   long long cap;             // capacity of out (ints, count slots included in mode 1)
   int *total;                // [0] entries (count slots excluded), [1] overflow flag, [2] largest count
+  int *report;               // optional, host memory: total[0], total[1] and the sticky overflow flag total[3]
   int mode;                  // 0: CSR, 0-based; 1: reference layout per group [nv, l1..lnv], 1-based
   int *step;                 // optional step counter of the system: the build runs only
   int every;                 //   when *step % every == 0 (device-side update schedule)

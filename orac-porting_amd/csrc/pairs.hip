@@ -670,6 +670,14 @@ __device__ inline int entry_size(const ListDesc &d, int v) {
   return gmem(d.gsize)[d.cellorder ? gmem(d.cell_items)[v] : v];
 }
 
+// what the host reads of a build, in its own memory
+__device__ inline void list_report(const ListDesc &d, int tot, bool over) {
+  if (!d.report) return;
+  d.report[0] = tot;
+  d.report[1] = over ? 1 : 0;
+  if (over) d.report[2] = 1;
+}
+
 // one block per system: first partial slot of each owner's reverse entries
 // (owner-major, atom-minor, in reverse-list order); capacity check
 __global__ void __launch_bounds__(1024) k_list_rbase(const ListDesc *__restrict__ D) {
@@ -683,6 +691,7 @@ __global__ void __launch_bounds__(1024) k_list_rbase(const ListDesc *__restrict_
   if (threadIdx.x == 0 && (long long)tot > d.pcap) {
     d.total[1] = 1;
     d.total[3] = 1;  // sticky: cleared only by the host
+    list_report(d, d.total[0], true);
   }
 }
 
@@ -746,6 +755,7 @@ __device__ inline void list_total(const ListDesc &d, bool split_written) {
     d.total[1] = mx > d.slab ? 1 : 0;
     d.total[2] = mx;
     if (mx > d.slab) d.total[3] = 1;  // sticky: cleared only by the host
+    list_report(d, tot, mx > d.slab);
   }
 }
 

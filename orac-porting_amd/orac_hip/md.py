@@ -86,9 +86,9 @@ class Dynamics:
 
     def state(self):
         n = self.s.natoms
-        arr = [np.zeros(n) for _ in range(6)]
-        _check(lib().orac_hip_md_get_state(self.rs.ctx._h, self.rs.id, *[_p(a) for a in arr]))
-        return np.stack(arr[:3]), np.stack(arr[3:])
+        x, v = np.empty((3, n)), np.empty((3, n))
+        _check(lib().orac_hip_md_get_state(self.rs.ctx._h, self.rs.id, *[_p(a) for a in (*x, *v)]))
+        return x, v
 
     def energies(self):
         """Kinetic, harmonic-term, nonbonded (eer + direct + corrections + self)

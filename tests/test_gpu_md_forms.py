@@ -125,3 +125,26 @@ def test_fast_level_batch(gpu_ctx):
         xb, vb = _state(m[0])
         assert np.array_equal(xa, xb) and np.array_equal(va, vb)
         m[0].close()
+
+
+@pytest.mark.parametrize("n", [1, 87381, 87382])
+def test_state_read_back(gpu_ctx, n):
+    """Positions and velocities come back as set, through the staging memory
+    up to its size (6 x 87,381 doubles) and past it; records of closed systems
+    start clean for the next ones."""
+    from orac_hip.api import ResidentSystem, _check, _f, _i, _p, lib
+    s = _random(n=n, nfft=(40, 40, 40), order=4, L=110.0)
+    for k in range(2):
+        rs = ResidentSystem(gpu_ctx, s, precision=0)
+        r = rs.results()
+        assert r["list_entries"] == 0 and r["eer"] == 0.0
+        z = (_i(np.zeros(2)), _f(np.zeros(2)))
+        _check(lib().orac_hip_md_setup(gpu_ctx._h, rs.id, C.c_int32(0), _p(z[0]), _p(z[1]), C.c_int32(0), _p(z[0]),
+                                       _p(z[1]), _p(z[1])))
+        rng = np.random.default_rng(k)
+        x, v = rng.uniform(-50, 50, (3, n)), rng.normal(size=(3, n))
+        xs, vs = _start(rs, x, v)
+        assert np.array_equal(x, xs) and np.array_equal(v, vs)
+        rs.eval(rebuild_list=True)
+        assert n == 1 or rs.results()["f"].any()
+        rs.close()
