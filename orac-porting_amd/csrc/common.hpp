@@ -298,6 +298,72 @@ __device__ inline int block_exclusive_scan(const int *in, int *out, int n) {
   return total;
 }
 
+// Fractional grid coordinate along one reciprocal axis (pme_fftw3.f90:151-160).
+__device__ inline double frac_coord(double x, double y, double z, const double *recip, int col, int K) {
+  double w = x * recip[3 * col] + y * recip[3 * col + 1] + z * recip[3 * col + 2];
+  return K * (w - fnint(w) + 0.5);
+}
+
+__device__ inline void cartesian(const double *co, double xp, double yp, double zp, double &x, double &y, double &z) {
+  x = co[0] * xp + co[3] * yp + co[6] * zp;
+  y = co[1] * xp + co[4] * yp + co[7] * zp;
+  z = co[2] * xp + co[5] * yp + co[8] * zp;
+}
+
+// atom a (whole wavefronts; a at or past natoms: none) into its spread tile's bin
+__device__ inline void bin_atom(const PmeDesc &d, int a) {
+  const int lane = threadIdx.x & 63;
+  int bin = -1;
+  double4 f = make_double4(0.0, 0.0, 0.0, 0.0);
+  if (a < d.natoms) {
+    double x, y, z;
+    cartesian(d.co, gmem(d.xp)[a], gmem(d.yp)[a], gmem(d.zp)[a], x, y, z);
+    double fr1 = frac_coord(x, y, z, d.recip, 0, d.K1);
+    double fr2 = frac_coord(x, y, z, d.recip, 1, d.K2);
+    double fr3 = frac_coord(x, y, z, d.recip, 2, d.K3);
+    // (non-finite coordinates are not spread)
+    if (fr1 >= 0.0 && fr1 <= d.K1 && fr2 >= 0.0 && fr2 <= d.K2 && fr3 >= 0.0 && fr3 <= d.K3) {
+      // fr = K (w - anint(w) = 0.5 exactly) is the grid origin: same spline weights
+      if (fr1 >= d.K1) fr1 -= d.K1;
+      if (fr2 >= d.K2) fr2 -= d.K2;
+      if (fr3 >= d.K3) fr3 -= d.K3;
+      f = make_double4(fr1, fr2, fr3, gmem(d.q)[a]);
+      bin = (int)fr1 / d.st1 + d.nb1 * ((int)fr2 / d.st2 + d.nb2 * ((int)fr3 / d.st3));
+    }
+  }
+  // Neighbouring atoms fall in the same tile: the lanes of one bin are counted
+  // by one atomic of their lowest lane, all bins' atomics in flight together.
+  unsigned long long todo = __ballot(bin >= 0), mine = 0ull;
+  while (todo) {  // the same on every lane of the wavefront
+    const int lb = __builtin_amdgcn_readlane(bin, __ffsll((long long)todo) - 1);
+    const unsigned long long same = __ballot(bin == lb);
+    if (bin == lb) mine = same;
+    todo &= ~same;
+  }
+  if (bin < 0) mine = 1ull << lane;
+  const int leader = __ffsll((long long)mine) - 1;
+  int base = 0;
+  if (bin >= 0 && lane == leader) base = atomicAdd(&d.bin_cnt[bin], __popcll(mine));
+  base = __shfl(base, leader, 64);
+  if (bin < 0) return;
+  const int pos = base + __popcll(mine & ((1ull << lane) - 1ull));
+  if (pos < d.bin_cap)
+    gstore(d.bin_fr + (size_t)bin * d.bin_cap + pos, f);
+  else
+    gstore(d.over_fr + atomicAdd(&d.bin_cnt[d.nb1 * d.nb2 * d.nb3], 1), f);
+}
+
+// lane J of each group of four lanes, to all four
+template <int J>
+__device__ __forceinline__ double quad_bcast(double v) {
+  int w[2];
+  __builtin_memcpy(w, &v, 8);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) w[k] = __builtin_amdgcn_update_dpp(0, w[k], J * 0x55, 0xf, 0xf, true);
+  __builtin_memcpy(&v, w, 8);
+  return v;
+}
+
 // d.out[20]: eer, vir(3x3 col-major), stc(3x3 row-major as stc1..stc9).  A
 // 1024-thread workgroup reduces one component in fixed order: k < 7 the
 // convolution partials (scalar_sum.f:125-133 halving and symmetrisation),

@@ -759,16 +759,16 @@ static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events
   auto pme = [&](hipStream_t s) {
     const hipEvent_t *pev = events ? &b.ev[ST_P0] : nullptr;
     if (b.precision == 0)
-      launch_pme<double>(b.dp, b.hp.data(), npme, s, b.tu, pev, false);
+      launch_pme<double>(b.dp, b.hp.data(), npme, s, b.tu, pev, false, true);
     else
-      launch_pme<float>(b.dp, b.hp.data(), npme, s, b.tu, pev, false);
+      launch_pme<float>(b.dp, b.hp.data(), npme, s, b.tu, pev, false, true);
   };
   mark(ST_BEGIN);
   // in group order (no cell permutation) the pair kernel's records are written with the centres
   const bool pack = !b.tu.cell_order, lists = md_lists || rebuild;
   const ListDesc *dl = md_lists ? b.dl_md : b.dl;
   const std::vector<ListDesc> &hl = md_lists ? b.hl_md : b.hl;  // (md: every system on its own update schedule)
-  launch_centres(b.dq, b.hq.data(), n, st, pack, dl, lists ? hl.data() : nullptr);
+  launch_centres(b.dq, b.hq.data(), n, st, pack, dl, lists ? hl.data() : nullptr, b.dp, b.hp.data(), npme);
   mark(ST_CENTRES);
   // The reciprocal sum needs the coordinates and the molecule centres only,
   // the corrections the coordinates: unless the stages are being timed they

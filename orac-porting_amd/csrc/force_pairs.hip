@@ -37,7 +37,10 @@ __global__ void __launch_bounds__(256) k_pack_sorted(const PairDesc *__restrict_
   if (t >= d.ngrp) return;
   const int g = d.perm ? gmem(d.perm)[t] : t;
   const int f0 = gmem(d.gfirst)[g], n = gmem(d.glast)[g] - f0 + 1;
-  pack_group(d, t, g, d.soff ? gmem(d.soff)[t] : f0, f0, n, gmem(d.xpg)[g], gmem(d.ypg)[g], gmem(d.zpg)[g]);
+  const int sf = d.soff ? gmem(d.soff)[t] : f0;
+  const double gx = gmem(d.xpg)[g], gy = gmem(d.ypg)[g], gz = gmem(d.zpg)[g];
+  pack_head(d, t, g, sf, f0, n, gx, gy, gz);
+  for (int k = 0; k < n; ++k) pack_atom(d, sf + k, f0 + k, gx, gy, gz);
 }
 
 template <typename P>

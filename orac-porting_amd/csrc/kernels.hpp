@@ -31,8 +31,9 @@ template <typename T>
 // ev (optional, 4 events): recorded before the spread, before the forward FFT,
 // before the gather and after it (the stage timings of a profiled evaluation).
 // finalize: reduce the partial sums (else launch_tail does).
+// binned: the atoms are in their tiles' bins (launch_centres).
 void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st, const Tuning &tu,
-                const hipEvent_t *ev = nullptr, bool finalize = true);
+                const hipEvent_t *ev = nullptr, bool finalize = true, bool binned = false);
 // tile edge of the LDS-tiled spread along an axis of K points (0: use the atomic spread)
 int spread_tile_edge(int K, int order, bool smallest);
 // Waves per owner group of the pair kernel for a system of ngrp groups (1
@@ -54,7 +55,7 @@ struct PairDesc {
   double *xpcm, *ypcm, *zpcm;       // molecule centres (reduced), written by the centre kernels
   int nmol;
   const int *mfirst, *mlast;        // atom range of each molecule
-  const int *mbig;                  // molecules of more than MOL_SMALL atoms (one wavefront each)
+  const int *mbig;                  // molecules of more than MOL_SMALL atoms (a workgroup each)
   int nbig;
   const int *gfirst, *glast;        // atom range of each group
   const int *gss;                   // ss_index of the group's first atom (1 solute, 2 solvent)
@@ -140,37 +141,37 @@ constexpr int PAIR_WAVES = 4;       // owner groups per 256-thread block
 constexpr int OWN_REG = 3;          // largest owner group of the owner-atom loop form (k_pairs_own)
 // whether the owner-atom loop form (and with it the half-list layout) is in use
 bool use_owner_kernel();
-constexpr int MOL_SMALL = 16;       // molecules up to this size get one thread in k_mol_com
+constexpr int MOL_SMALL = 16;       // molecules up to this size get four lanes in k_prepare
 // LJ parameters as a dense ntypes x ntypes table of {c12, c6} (one gather per
 // pair) up to this many types (64 MB); beyond it the packed table and
 // type_table of the reference (two dependent gathers per pair)
 constexpr int LJ_DENSE_MAX = 2048;
 
-// Group record t (group g, atoms f0 .. f0 + n - 1, centre gx, gy, gz) and its
-// atoms' records from sf on.  Neighbours listed next to each other are next to
+// Group record t (group g, atoms f0 .. f0 + n - 1, centre gx, gy, gz); its
+// atoms' records lie from sf on.  Neighbours listed next to each other are next to
 // each other in memory, and one group is one 32-byte record.
-__device__ inline void pack_group(const PairDesc &d, int t, int g, int sf, int f0, int n, double gx, double gy,
-                                  double gz) {
+__device__ inline void pack_head(const PairDesc &d, int t, int g, int sf, int f0, int n, double gx, double gy,
+                                 double gz) {
   const int gss = gmem(d.gss)[g], w[2] = {sf, n | (gss << 8)};
   double4 gp = make_double4(gx, gy, gz, 0.0);
   __builtin_memcpy(&gp.w, w, 8);
   gstore(d.sgp + t, gp);
   if (d.half) gstore(d.sgi + t, make_int4(sf, f0, n | (gss << 8), g));
-  for (int k = 0; k < n; ++k) {
-    const int a = f0 + k;
-    const double q = gmem(d.q)[a];
-    // Cartesian offset from the group centre (upper triangle of co, as
-    // force.f): a pair's separation is the group separation plus the
-    // difference of two small offsets
-    const double dx = gmem(d.xp)[a] - gx, dy = gmem(d.yp)[a] - gy, dz = gmem(d.zp)[a] - gz;
-    const double cx = d.co[0] * dx + d.co[3] * dy + d.co[6] * dz, cy = d.co[4] * dy + d.co[7] * dz, cz = d.co[8] * dz;
-    const int ty = gmem(d.type)[a];
-    const int fl = (gmem(d.ex_inter)[a] ? ATOM_EX : 0) | gmem(d.tflag)[ty] |
-                   (d.rematom && gmem(d.rematom)[a] ? ATOM_REM : 0);
-    gstore(d.sai + sf + k, make_int2(ty << ATOM_FLAG_BITS | fl, a));
-    if (d.sapc) gstore(d.sapc + sf + k, make_double4(cx, cy, cz, q));
-    if (d.sapf) gstore(d.sapf + sf + k, make_float4((float)cx, (float)cy, (float)cz, (float)q));
-  }
+}
+// atom record s: atom a of the group with centre gx, gy, gz
+__device__ inline void pack_atom(const PairDesc &d, int s, int a, double gx, double gy, double gz) {
+  const double q = gmem(d.q)[a];
+  // Cartesian offset from the group centre (upper triangle of co, as
+  // force.f): a pair's separation is the group separation plus the
+  // difference of two small offsets
+  const double dx = gmem(d.xp)[a] - gx, dy = gmem(d.yp)[a] - gy, dz = gmem(d.zp)[a] - gz;
+  const double cx = d.co[0] * dx + d.co[3] * dy + d.co[6] * dz, cy = d.co[4] * dy + d.co[7] * dz, cz = d.co[8] * dz;
+  const int ty = gmem(d.type)[a];
+  const int fl = (gmem(d.ex_inter)[a] ? ATOM_EX : 0) | gmem(d.tflag)[ty] |
+                 (d.rematom && gmem(d.rematom)[a] ? ATOM_REM : 0);
+  gstore(d.sai + s, make_int2(ty << ATOM_FLAG_BITS | fl, a));
+  if (d.sapc) gstore(d.sapc + s, make_double4(cx, cy, cz, q));
+  if (d.sapf) gstore(d.sapf + s, make_float4((float)cx, (float)cy, (float)cz, (float)q));
 }
 
 // packed: the systems' records are in place (launch_centres with pack).
@@ -198,7 +199,8 @@ __device__ inline void pairs_finalize(const PairDesc &d, int k) {
 // system the counters of the build that follows (LIST_ZERO left out)
 struct ListDesc;
 void launch_centres(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream_t st, bool pack = false,
-                    const ListDesc *d_list = nullptr, const ListDesc *h_list = nullptr);
+                    const ListDesc *d_list = nullptr, const ListDesc *h_list = nullptr, const PmeDesc *d_pme = nullptr,
+                    const PmeDesc *h_pme = nullptr, int npme = 0);
 
 // linked cells (lc_list.f)
 struct CellGrid {

@@ -138,19 +138,7 @@ __device__ cx<T> *lds_fft(cx<T> *a, cx<T> *b, int N, int TP, const FftAxis &ax, 
 
 // ---------------------------------------------------------------- spread
 
-// Fractional grid coordinate along one reciprocal axis (pme_fftw3.f90:151-160).
-__device__ inline double frac_coord(double x, double y, double z, const double *recip, int col, int K) {
-  double w = x * recip[3 * col] + y * recip[3 * col + 1] + z * recip[3 * col + 2];
-  return K * (w - fnint(w) + 0.5);
-}
-
 __device__ inline int wrapK(int k0, int K) { return k0 < 0 ? k0 + K : (k0 >= K ? k0 - K : k0); }
-
-__device__ inline void cartesian(const double *co, double xp, double yp, double zp, double &x, double &y, double &z) {
-  x = co[0] * xp + co[3] * yp + co[6] * zp;
-  y = co[1] * xp + co[4] * yp + co[7] * zp;
-  z = co[2] * xp + co[5] * yp + co[8] * zp;
-}
 
 // one thread per (atom, z-offset): order^2 fixed-point atomic adds
 __global__ void __launch_bounds__(256) k_grid_zero(const PmeDesc *__restrict__ D) {
@@ -211,49 +199,10 @@ __global__ void __launch_bounds__(256) k_spread(const PmeDesc *__restrict__ D) {
 // overflow list beyond it), so no scan and no second pass over the atoms is
 // needed: 20 + 5 + 6 us of counting, scanning and filling for 24,460 atoms
 // became one kernel of 5.5 us.
+// A resident evaluation bins in its preparing launch (k_prepare).
 __global__ void __launch_bounds__(256) k_bin(const PmeDesc *__restrict__ D) {
   const PmeDesc &d = D[blockIdx.y];
-  if (!d.tiled) return;
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & 63;
-  int bin = -1;
-  double4 f = make_double4(0.0, 0.0, 0.0, 0.0);
-  if (a < d.natoms) {
-    double x, y, z;
-    cartesian(d.co, gmem(d.xp)[a], gmem(d.yp)[a], gmem(d.zp)[a], x, y, z);
-    double fr1 = frac_coord(x, y, z, d.recip, 0, d.K1);
-    double fr2 = frac_coord(x, y, z, d.recip, 1, d.K2);
-    double fr3 = frac_coord(x, y, z, d.recip, 2, d.K3);
-    // (non-finite coordinates are not spread)
-    if (fr1 >= 0.0 && fr1 <= d.K1 && fr2 >= 0.0 && fr2 <= d.K2 && fr3 >= 0.0 && fr3 <= d.K3) {
-      // fr = K (w - anint(w) = 0.5 exactly) is the grid origin: same spline weights
-      if (fr1 >= d.K1) fr1 -= d.K1;
-      if (fr2 >= d.K2) fr2 -= d.K2;
-      if (fr3 >= d.K3) fr3 -= d.K3;
-      f = make_double4(fr1, fr2, fr3, gmem(d.q)[a]);
-      bin = (int)fr1 / d.st1 + d.nb1 * ((int)fr2 / d.st2 + d.nb2 * ((int)fr3 / d.st3));
-    }
-  }
-  // Neighbouring atoms fall in the same tile: the lanes of one bin are counted
-  // by one atomic of their lowest lane, all bins' atomics in flight together.
-  unsigned long long todo = __ballot(bin >= 0), mine = 0ull;
-  while (todo) {  // the same on every lane of the wavefront
-    const int lb = __builtin_amdgcn_readlane(bin, __ffsll((long long)todo) - 1);
-    const unsigned long long same = __ballot(bin == lb);
-    if (bin == lb) mine = same;
-    todo &= ~same;
-  }
-  if (bin < 0) mine = 1ull << lane;
-  const int leader = __ffsll((long long)mine) - 1;
-  int base = 0;
-  if (bin >= 0 && lane == leader) base = atomicAdd(&d.bin_cnt[bin], __popcll(mine));
-  base = __shfl(base, leader, 64);
-  if (bin < 0) return;
-  const int pos = base + __popcll(mine & ((1ull << lane) - 1ull));
-  if (pos < d.bin_cap)
-    gstore(d.bin_fr + (size_t)bin * d.bin_cap + pos, f);
-  else
-    gstore(d.over_fr + atomicAdd(&d.bin_cnt[d.nb1 * d.nb2 * d.nb3], 1), f);
+  if (d.tiled) bin_atom(d, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 constexpr int SPREAD_TILE_MAX = 8;
@@ -845,7 +794,7 @@ void pme_set_tiles(PmeDesc &d, int lds_elems) {
 
 template <typename T>
 void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st, const Tuning &tu,
-                const hipEvent_t *ev, bool finalize) {
+                const hipEvent_t *ev, bool finalize, bool binned) {
   (void)tu;
   if (nsys <= 0) return;
   int max_atoms = 1, max_bins = 1, any_tiled = 0, any_atomic = 0, max_gx = 1, max_gy = 1, max_gz = 1, max_gg = 1;
@@ -876,7 +825,7 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
   dim3 blk(256);
   if (ev) ORAC_HIP(hipEventRecord(ev[0], st));
   if (any_tiled) {
-    hipLaunchKernelGGL(k_bin, dim3((max_atoms + 255) / 256, nsys), blk, 0, st, d_desc);
+    if (!binned) hipLaunchKernelGGL(k_bin, dim3((max_atoms + 255) / 256, nsys), blk, 0, st, d_desc);
     const dim3 gt(max_bins, nsys), bt(SPREAD_THREADS);
     const size_t sh = spread_lds_bytes<T>(max_order);
     switch (order) {
@@ -909,8 +858,8 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
 }
 
 template void launch_pme<double>(const PmeDesc *, const PmeDesc *, int, hipStream_t, const Tuning &,
-                                 const hipEvent_t *, bool);
+                                 const hipEvent_t *, bool, bool);
 template void launch_pme<float>(const PmeDesc *, const PmeDesc *, int, hipStream_t, const Tuning &,
-                                const hipEvent_t *, bool);
+                                const hipEvent_t *, bool, bool);
 
 }  // namespace orac

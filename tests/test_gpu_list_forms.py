@@ -65,3 +65,23 @@ def test_list_build(gpu_ctx, name, cell_order):
     o = O.force(s, nnlpp, fa=fa, rinn=0.0, rout=s.rcut, rtolinn=0.0, rtolout=s.rtol, rneigh=0.0)
     f = o["f"] + O.fft_pme(s, variant="fftw")["f"]
     assert relrms(g["f"], f) < F_TOL
+
+
+@pytest.mark.parametrize("sizes", [[1], [2, 4], [3, 5, 8], [16, 1, 17], [64, 7, 4]])
+def test_prepare_group_and_molecule_sizes(gpu_ctx, sizes):
+    """Centres, records and bins of groups (molecules, too) around the four
+    lanes that share one and around MOL_SMALL atoms: forces and the virial,
+    whose molecular correction reads the molecules' centres, against the oracle."""
+    from orac_hip.api import ResidentSystem
+    from test_gpu_pair_forms import grouped
+    from test_gpu_parity import _stress_close
+    from test_gpu_resident import oracle_total
+    s = grouped(sizes)
+    none = np.zeros((2, 0), np.int32)
+    rs = ResidentSystem(gpu_ctx, s, precision=0)
+    rs.eval(rebuild_list=True)
+    g = rs.results()
+    rs.close()
+    o = oracle_total(s, none, np.zeros(0))
+    assert relrms(g["f"], o["f"]) < F_TOL
+    assert _stress_close(g["stress"], o["stress"])
