@@ -1,5 +1,6 @@
 // host.cpp -- host-side tables and plans of the nonbonded path: FFT plans and
 // twiddles, B-spline moduli, linked-cell stencils, exclusion maps, PME descriptors.
+#include <climits>
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -27,17 +28,32 @@ static void make_twiddles(int n, std::vector<double2> &t64, std::vector<float2> 
 }
 
 static bool factor_radices(int n, FftAxis &ax) {
+  // The fewest passes over the radices the kernels have, then the smallest sum
+  // (the least work); larger radices first.  A pass is one round trip through
+  // LDS and one barrier, which is what a short transform waits for: 64 = 8 x 8
+  // where 4 x 4 x 4 takes three.
   ax.n = n;
   ax.nr = 0;
-  int m = n;
-  const int order[4] = {4, 2, 3, 5};
-  for (int r : order)
-    while (m % r == 0) {
-      if (ax.nr >= MAX_RADICES) return false;
-      ax.radix[ax.nr++] = r;
-      m /= r;
+  if (n > MAX_FFT_LEN || n < 2) return false;
+  const int radices[6] = {8, 6, 5, 4, 3, 2};
+  std::vector<int> passes(n + 1, INT_MAX), sum(n + 1, 0), last(n + 1, 0);
+  passes[1] = 0;
+  for (int m = 1; m < n; ++m) {  // m: product of the radices so far
+    if (passes[m] == INT_MAX) continue;
+    for (int r : radices) {
+      if ((long long)m * r > n || n % (m * r) != 0) continue;
+      const int p = passes[m] + 1, s = sum[m] + r, q = m * r;
+      if (p < passes[q] || (p == passes[q] && s < sum[q])) {
+        passes[q] = p;
+        sum[q] = s;
+        last[q] = r;
+      }
     }
-  return m == 1 && n <= MAX_FFT_LEN && n >= 2;
+  }
+  if (passes[n] > MAX_RADICES) return false;
+  for (int m = n; m > 1; m /= last[m]) ax.radix[ax.nr++] = last[m];
+  std::sort(ax.radix, ax.radix + ax.nr, [](int x, int y) { return x > y; });
+  return true;
 }
 
 // load_bsp_moduli + DFTMOD (pme_fftw3.f90:165-230), with DFTMOD's 2*pi

@@ -3,15 +3,17 @@
 // Stages (each one kernel, all systems of a batch in one launch via blockIdx.y):
 //   k_spread      fractionals + order-p B-splines + charge spreading with
 //                 64-bit fixed-point atomics (pme_fftw3.f90:132-163,234-298,487-576)
-//   k_fft_x_r2c   real rows along K1 -> half spectrum (FFTW r2c, pme_fftw3.f90:114)
-//   k_fft_pencil  complex pencils along K2 (forward / inverse)
+//   k_fft_plane_r2c  K3 planes: real rows along K1 -> half spectrum (FFTW r2c,
+//                 pme_fftw3.f90:114), then K2; per axis for large planes:
+//   k_fft_x_r2c, k_fft_pencil
 //   k_fft_z_conv  pencils along K3: forward FFT, influence function with
 //                 energy and virial (scalar_sum.f:1-135), inverse FFT, in LDS
-//   k_fft_x_c2r   half spectrum -> real rows (FFTW c2r, pme_fftw3.f90:116)
+//   k_fft_plane_c2r (k_fft_pencil, k_fft_x_c2r)  back: K2, then half spectrum
+//                 -> real rows (FFTW c2r, pme_fftw3.f90:116)
 //   k_gather      forces from the convolved grid (pme_fftw3.f90:311-372) and
 //                 the molecular-virial correction terms (fft_pme.f:65-106)
 //   k_pme_finalize fixed-order reduction of the per-block partials
-// FFTs are LDS-staged mixed radix-2/3/4/5 Stockham passes over tiles of
+// FFTs are LDS-staged mixed radix (2 to 6, 8) Stockham passes over tiles of
 // pencils; loads and stores walk the contiguous K1 direction across threads.
 #include "common.hpp"
 #include "kernels.hpp"
@@ -50,6 +52,22 @@ __device__ __forceinline__ void load_twiddles(cx<T> *tw, const FftAxis &ax) {
   }
 }
 
+// complex grid elements through the global view
+__device__ __forceinline__ cx<double> cload(const cx<double> *p) {
+  const double2 v = gload(reinterpret_cast<const double2 *>(p));
+  return {v.x, v.y};
+}
+__device__ __forceinline__ cx<float> cload(const cx<float> *p) {
+  const float2 v = gload(reinterpret_cast<const float2 *>(p));
+  return {v.x, v.y};
+}
+__device__ __forceinline__ void cstore(cx<double> *p, cx<double> v) {
+  gstore(reinterpret_cast<double2 *>(p), make_double2(v.x, v.y));
+}
+__device__ __forceinline__ void cstore(cx<float> *p, cx<float> v) {
+  gstore(reinterpret_cast<float2 *>(p), make_float2(v.x, v.y));
+}
+
 template <typename T, int R, int S>
 __device__ inline void dft(cx<T> *v) {
   if constexpr (R == 2) {
@@ -71,7 +89,7 @@ __device__ inline void dft(cx<T> *v) {
     v[2] = csub(t0, t2);
     v[1] = cadd(t1, t3);
     v[3] = csub(t1, t3);
-  } else {  // R == 5
+  } else if constexpr (R == 5) {
     const T c1 = T(0.3090169943749474241022934171828191), c2 = T(-0.8090169943749474241022934171828191);
     const T s1 = T(0.9510565162951535721164393333793821), s2 = T(0.5877852522924731291687059546390728);
     cx<T> t1 = cadd(v[1], v[4]), t2 = cadd(v[2], v[3]), t3 = csub(v[1], v[4]), t4 = csub(v[2], v[3]);
@@ -84,18 +102,37 @@ __device__ inline void dft(cx<T> *v) {
     v[4] = csub(a1, b1);
     v[2] = cadd(a2, b2);
     v[3] = csub(a2, b2);
+  } else {  // 6 and 8: even and odd inputs, then one radix-2 step
+    constexpr int Q = R / 2;
+    constexpr double c1 = R == 6 ? 0.5 : 0.7071067811865475244, s1 = R == 6 ? 0.8660254037844386468 : c1;
+    constexpr double C[4][2] = {{1.0, 0.0}, {c1, s1}, {-0.5, s1}, {-c1, s1}};  // ([2] of 8 is i)
+    cx<T> e[Q], o[Q];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+      e[k] = v[2 * k];
+      o[k] = v[2 * k + 1];
+    }
+    dft<T, Q, S>(e);
+    dft<T, Q, S>(o);
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+      if (R == 8 && k == 2) o[k] = cmuli<T, S>(o[k]);
+      else if (k > 0) o[k] = cmul(o[k], cx<T>{T(C[k][0]), T(S * C[k][1])});
+      v[k] = cadd(e[k], o[k]);
+      v[k + Q] = csub(e[k], o[k]);
+    }
   }
 }
 
 template <typename T, int R, int S>
-__device__ inline void stockham_pass(const cx<T> *a, cx<T> *b, int N, int TP, int Ns, const cx<T> *tw) {
+__device__ __forceinline__ void stockham_pass(const cx<T> *a, cx<T> *b, int N, int LD, int TP, int Ns, const cx<T> *tw) {
   const FastDiv dNs(Ns), dNR(N / R);
   const int NR = dNR.d, twstep = FastDiv(Ns * R).div(N);
   for (int bi = threadIdx.x; bi < TP * NR; bi += blockDim.x) {
     int j, k;
     const int t = dNR.div(bi, j), jq = dNs.div(j, k);
-    const cx<T> *src = a + t * N;
-    cx<T> *dst = b + t * N;
+    const cx<T> *src = a + t * LD;
+    cx<T> *dst = b + t * LD;
     cx<T> v[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) v[r] = src[j + r * NR];
@@ -114,18 +151,21 @@ __device__ inline void stockham_pass(const cx<T> *a, cx<T> *b, int N, int TP, in
   }
 }
 
-// TP pencils of length N held in LDS buffer a (b is scratch, tw the axis's
-// twiddles in LDS); returns the buffer that holds the result.
+// TP pencils of length N, LD apart, held in LDS buffer a (b is scratch, tw the
+// axis's twiddles in LDS); returns the buffer that holds the result.  Where
+// lanes step from pencil to pencil, LD = N + 1 puts them in different banks.
 template <typename T, int S>
-__device__ cx<T> *lds_fft(cx<T> *a, cx<T> *b, int N, int TP, const FftAxis &ax, const cx<T> *tw) {
+__device__ __forceinline__ cx<T> *lds_fft(cx<T> *a, cx<T> *b, int N, int LD, int TP, const FftAxis &ax, const cx<T> *tw) {
   int Ns = 1;
   for (int p = 0; p < ax.nr; ++p) {
     int R = ax.radix[p];
     switch (R) {
-      case 2: stockham_pass<T, 2, S>(a, b, N, TP, Ns, tw); break;
-      case 3: stockham_pass<T, 3, S>(a, b, N, TP, Ns, tw); break;
-      case 4: stockham_pass<T, 4, S>(a, b, N, TP, Ns, tw); break;
-      default: stockham_pass<T, 5, S>(a, b, N, TP, Ns, tw); break;
+      case 2: stockham_pass<T, 2, S>(a, b, N, LD, TP, Ns, tw); break;
+      case 3: stockham_pass<T, 3, S>(a, b, N, LD, TP, Ns, tw); break;
+      case 4: stockham_pass<T, 4, S>(a, b, N, LD, TP, Ns, tw); break;
+      case 5: stockham_pass<T, 5, S>(a, b, N, LD, TP, Ns, tw); break;
+      case 6: stockham_pass<T, 6, S>(a, b, N, LD, TP, Ns, tw); break;
+      default: stockham_pass<T, 8, S>(a, b, N, LD, TP, Ns, tw); break;
     }
     __syncthreads();
     cx<T> *t = a;
@@ -404,12 +444,122 @@ int spread_tile_edge(int K, int order, bool smallest) {
 // ---------------------------------------------------------------- FFT passes
 
 // Rows along K1: fixed-point grid -> half spectrum.  TP rows per block.
+// ---------------------------------------------------------------- transforms
+
+// The transforms along K1 and K2 of one K3 plane in one workgroup, where two
+// copies of the half spectrum and the twiddles fit its 160 KB of LDS.  Two real
+// rows go through one complex transform; neither direction writes the plane
+// between its axes.  Larger planes (100 x 100 in FP64, 144 x 144 in FP32) take
+// a kernel per axis.  The three FFT launches with planes against the five
+// without: 216 waters (FP64) 27 against 33 us, 24,460 atoms 45 against 49,
+// 103k atoms (FP32, 108^3) 68 against 90, 16 systems of 24,460 114 against 190.
+constexpr size_t PLANE_LDS = 160 * 1024;
+__host__ __device__ inline int plane_buf(int K1, int K2) {
+  const int rows = (K2 + 1) / 2 * (K1 + 1), cols = (K1 / 2 + 1) * (K2 + 1);
+  return rows > cols ? rows : cols;
+}
+template <typename T>
+__host__ __device__ inline size_t plane_lds(const PmeDesc &d) {
+  return (2 * (size_t)plane_buf(d.K1, d.K2) + d.K1 + d.K2) * sizeof(cx<T>);
+}
+template <typename T>
+__host__ __device__ inline bool use_planes(const PmeDesc &d) {
+  return plane_lds<T>(d) <= PLANE_LDS;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(1024) k_fft_plane_r2c(const PmeDesc *__restrict__ D) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const PmeDesc &d = D[blockIdx.y];
+  const int K1 = d.K1, K2 = d.K2, H = K1 / 2 + 1, P = (K2 + 1) / 2, LD1 = K1 + 1, LD2 = K2 + 1, z = blockIdx.x;
+  if (z >= d.K3 || !use_planes<T>(d)) return;
+  cx<T> *a = reinterpret_cast<cx<T> *>(smem), *b = a + plane_buf(K1, K2), *tw1 = b + plane_buf(K1, K2),
+        *tw2 = tw1 + K1;
+  const double inv = d.fixinv;
+  const FastDiv dK1(K1), dH(H);
+  const auto in = gmem(d.Qfix + (size_t)z * K1 * K2);
+  load_twiddles(tw1, d.ax1);
+  load_twiddles(tw2, d.ax2);
+#pragma unroll 4
+  for (int i = threadIdx.x; i < P * K1; i += blockDim.x) {
+    int e;
+    const int j = dK1.div(i, e);
+    const long long q0 = (long long)in[(2 * j) * K1 + e], q1 = 2 * j + 1 < K2 ? (long long)in[(2 * j + 1) * K1 + e] : 0;
+    a[j * LD1 + e] = {T((double)q0 * inv), T((double)q1 * inv)};
+  }
+  // the spread is done with its bins: empty for the next evaluation
+  if (d.tiled)
+    for (int i = z * blockDim.x + threadIdx.x; i <= d.nb1 * d.nb2 * d.nb3; i += d.K3 * blockDim.x)
+      gmem(d.bin_cnt)[i] = 0;
+  __syncthreads();
+  cx<T> *r = lds_fft<T, -1>(a, b, K1, LD1, P, d.ax1, tw1), *s = r == a ? b : a;
+  // rows 2j and 2j + 1 from their sum Z: (Z[k] + conj Z[-k]) / 2, (Z[k] - conj Z[-k]) / 2i
+  for (int i = threadIdx.x; i < P * H; i += blockDim.x) {
+    int k;
+    const int j = dH.div(i, k);
+    const cx<T> u = r[j * LD1 + k], w = r[j * LD1 + (k ? K1 - k : 0)];
+    s[k * LD2 + 2 * j] = {T(0.5) * (u.x + w.x), T(0.5) * (u.y - w.y)};
+    if (2 * j + 1 < K2) s[k * LD2 + 2 * j + 1] = {T(0.5) * (u.y + w.y), T(0.5) * (w.x - u.x)};
+  }
+  __syncthreads();
+  r = lds_fft<T, -1>(s, r, K2, LD2, H, d.ax2, tw2);
+  cx<T> *FQ = reinterpret_cast<cx<T> *>(d.FQ) + (size_t)z * K2 * H;
+  for (int i = threadIdx.x; i < K2 * H; i += blockDim.x) {
+    int k;
+    const int y = dH.div(i, k);
+    cstore(FQ + i, r[k * LD2 + y]);
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(1024) k_fft_plane_c2r(const PmeDesc *__restrict__ D) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const PmeDesc &d = D[blockIdx.y];
+  const int K1 = d.K1, K2 = d.K2, H = K1 / 2 + 1, P = (K2 + 1) / 2, LD1 = K1 + 1, LD2 = K2 + 1, z = blockIdx.x;
+  if (z >= d.K3 || d.energy_only || !use_planes<T>(d)) return;
+  cx<T> *a = reinterpret_cast<cx<T> *>(smem), *b = a + plane_buf(K1, K2), *tw1 = b + plane_buf(K1, K2),
+        *tw2 = tw1 + K1;
+  const FastDiv dK1(K1), dH(H);
+  const cx<T> *FQ = reinterpret_cast<const cx<T> *>(d.FQ) + (size_t)z * K2 * H;
+  load_twiddles(tw1, d.ax1);
+  load_twiddles(tw2, d.ax2);
+#pragma unroll 4
+  for (int i = threadIdx.x; i < K2 * H; i += blockDim.x) {
+    int k;
+    const int y = dH.div(i, k);
+    a[k * LD2 + y] = cload(FQ + i);
+  }
+  __syncthreads();
+  cx<T> *r = lds_fft<T, +1>(a, b, K2, LD2, H, d.ax2, tw2), *s = r == a ? b : a;
+  // Z = X(row 2j) + i X(row 2j + 1), both Hermitian (the imaginary parts at 0 and K1 / 2 are not read)
+  for (int i = threadIdx.x; i < P * H; i += blockDim.x) {
+    int k;
+    const int j = dH.div(i, k);
+    cx<T> u = r[k * LD2 + 2 * j], w = {T(0), T(0)};
+    if (2 * j + 1 < K2) w = r[k * LD2 + 2 * j + 1];
+    if (k == 0 || 2 * k == K1) u.y = w.y = T(0);
+    s[j * LD1 + k] = {u.x - w.y, u.y + w.x};
+    if (k > 0 && K1 - k >= H) s[j * LD1 + K1 - k] = {u.x + w.y, w.x - u.y};
+  }
+  __syncthreads();
+  r = lds_fft<T, +1>(s, r, K1, LD1, P, d.ax1, tw1);
+  T *Qr = reinterpret_cast<T *>(d.Qr) + (size_t)z * K2 * K1;
+  for (int i = threadIdx.x; i < K2 * K1; i += blockDim.x) {
+    int e;
+    const int y = dK1.div(i, e);
+    const cx<T> v = r[(y >> 1) * LD1 + e];
+    gmem(Qr)[i] = y & 1 ? v.y : v.x;
+  }
+}
+
+constexpr int CONV_PTS = 8;  // grid points per thread of k_fft_z_conv at most
+
 template <typename T>
 __global__ void __launch_bounds__(256) k_fft_x_r2c(const PmeDesc *__restrict__ D) {
   extern __shared__ __align__(16) unsigned char smem[];
   const PmeDesc &d = D[blockIdx.y];
   const int N = d.K1, H = N / 2 + 1, rows = d.K2 * d.K3, TP = d.tpx;
-  if ((int)blockIdx.x >= d.gx) return;
+  if ((int)blockIdx.x >= d.gx || use_planes<T>(d)) return;
   cx<T> *a = reinterpret_cast<cx<T> *>(smem);
   cx<T> *b = a + TP * N;
   cx<T> *tw = b + TP * N;
@@ -429,12 +579,12 @@ __global__ void __launch_bounds__(256) k_fft_x_r2c(const PmeDesc *__restrict__ D
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i <= d.nb1 * d.nb2 * d.nb3; i += d.gx * blockDim.x)
       gmem(d.bin_cnt)[i] = 0;
   __syncthreads();
-  cx<T> *r = lds_fft<T, -1>(a, b, N, TP, d.ax1, tw);
+  cx<T> *r = lds_fft<T, -1>(a, b, N, N, TP, d.ax1, tw);
   cx<T> *FQ = reinterpret_cast<cx<T> *>(d.FQ);
   for (int i = threadIdx.x; i < TP * H; i += blockDim.x) {
     int e;
     const int t = dH.div(i, e), row = row0 + t;
-    if (row < rows) FQ[(size_t)row * H + e] = r[t * N + e];
+    if (row < rows) cstore(FQ + (size_t)row * H + e, r[t * N + e]);
   }
 }
 
@@ -445,7 +595,7 @@ __global__ void __launch_bounds__(256) k_fft_pencil(const PmeDesc *__restrict__ 
   extern __shared__ __align__(16) unsigned char smem[];
   const PmeDesc &d = D[blockIdx.y];
   const int H = d.K1 / 2 + 1, TP = d.tpy;
-  if ((int)blockIdx.x >= d.gy || (S > 0 && d.energy_only)) return;
+  if ((int)blockIdx.x >= d.gy || (S > 0 && d.energy_only) || use_planes<T>(d)) return;
   const FftAxis &ax = axis == 2 ? d.ax2 : d.ax3;
   const int N = ax.n;
   const int npen = axis == 2 ? H * d.K3 : H * d.K2;
@@ -463,15 +613,15 @@ __global__ void __launch_bounds__(256) k_fft_pencil(const PmeDesc *__restrict__ 
     int t, pr;
     const int e = dTP.div(i, t), p = p0 + t, pq = dH.div(p, pr);
     cx<T> v = {T(0), T(0)};
-    if (p < npen) v = FQ[(size_t)pr + (size_t)pq * S1 + (size_t)e * Se];
+    if (p < npen) v = cload(FQ + (size_t)pr + (size_t)pq * S1 + (size_t)e * Se);
     a[t * N + e] = v;
   }
   __syncthreads();
-  cx<T> *r = lds_fft<T, S>(a, b, N, TP, ax, tw);
+  cx<T> *r = lds_fft<T, S>(a, b, N, N, TP, ax, tw);
   for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
     int t, pr;
     const int e = dTP.div(i, t), p = p0 + t, pq = dH.div(p, pr);
-    if (p < npen) FQ[(size_t)pr + (size_t)pq * S1 + (size_t)e * Se] = r[t * N + e];
+    if (p < npen) cstore(FQ + (size_t)pr + (size_t)pq * S1 + (size_t)e * Se, r[t * N + e]);
   }
 }
 
@@ -489,79 +639,107 @@ __global__ void __launch_bounds__(256) k_fft_z_conv(const PmeDesc *__restrict__ 
   const size_t Se = (size_t)H * d.K2;
   const int p0 = blockIdx.x * TP;
   double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+  const int LD = N + 1;
   cx<T> *FQ = reinterpret_cast<cx<T> *>(d.FQ);
   cx<T> *a = reinterpret_cast<cx<T> *>(smem);
-  cx<T> *b = a + TP * N, *tw = b + TP * N;
+  cx<T> *b = a + TP * LD, *tw = b + TP * LD;
   const FastDiv dTP(TP), dH(H);
   if (p0 < npen) {
-    load_twiddles(tw, d.ax3);
-    for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
-      int t;
-      const int e = dTP.div(i, t), p = p0 + t;
-      cx<T> v = {T(0), T(0)};
-      if (p < npen) v = FQ[(size_t)p + (size_t)e * Se];
-      a[t * N + e] = v;
-    }
-    __syncthreads();
-    cx<T> *r = lds_fft<T, -1>(a, b, N, TP, d.ax3, tw);
-    cx<T> *s = (r == a) ? b : a;
-    const int nfft1 = d.K1, nfft2 = d.K2, nfft3 = d.K3, ndim1 = H;
+    const int nfft1 = d.K1, nfft2 = d.K2, nfft3 = d.K3, ndim1 = H, npt = TP * N;
     int nf1 = nfft1 / 2; if (2 * nf1 < nfft1) nf1 += 1;
     int nf2 = nfft2 / 2; if (2 * nf2 < nfft2) nf2 += 1;
     int nf3 = nfft3 / 2; if (2 * nf3 < nfft3) nf3 += 1;
     const double pi = d.pi_f32, fac = d.fac;
-    for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
+    // 1-based indices as in scalar_sum; false outside the grid and at ind = 0, which is never scaled
+    auto point = [&](int i, int &k1, int &k2, int &k3, double (&mh)[3]) -> bool {
       int t, pr;
-      const int e = dTP.div(i, t), p = p0 + t;
-      if (p >= npen) continue;
-      const int pq = dH.div(p, pr);
-      int k1 = pr + 1, k2 = pq + 1, k3 = e + 1;  // 1-based as in scalar_sum
-      cx<T> qv = r[t * N + e];
-      if (k1 == 1 && k2 == 1 && k3 == 1) continue;     // ind = 0 is never scaled
+      const int e = dTP.div(i, t), p = p0 + t, pq = dH.div(p, pr);
+      k1 = pr + 1, k2 = pq + 1, k3 = e + 1;
       int m1 = k1 - 1; if (k1 > nf1) m1 = k1 - 1 - nfft1;
       int m2 = k2 - 1; if (k2 > nf2) m2 = k2 - 1 - nfft2;
       int m3 = k3 - 1; if (k3 > nf3) m3 = k3 - 1 - nfft3;
       const double *rc = d.recip;
-      double mhat1 = rc[0] * m1 + rc[3] * m2 + rc[6] * m3;
-      double mhat2 = rc[1] * m1 + rc[4] * m2 + rc[7] * m3;
-      double mhat3 = rc[2] * m1 + rc[5] * m2 + rc[8] * m3;
-      double msq = mhat1 * mhat1 + mhat2 * mhat2 + mhat3 * mhat3;
-      double eterm = 0.0;
-      if (!(msq > d.rkcut2)) {
-        double denom = pi * d.volume * d.bsp1[k1 - 1] * d.bsp2[k2 - 1] * d.bsp3[k3 - 1] * msq;
-        eterm = exp(-fac * msq) / denom;
-        double vterm = 2.0 * (fac * msq + 1.0) / msq;
-        double qr = (double)qv.x, qi = (double)qv.y;
+      mh[0] = rc[0] * m1 + rc[3] * m2 + rc[6] * m3;
+      mh[1] = rc[1] * m1 + rc[4] * m2 + rc[7] * m3;
+      mh[2] = rc[2] * m1 + rc[5] * m2 + rc[8] * m3;
+      return i < npt && p < npen && !(k1 == 1 && k2 == 1 && k3 == 1);
+    };
+    load_twiddles(tw, d.ax3);
+    cx<T> v[CONV_PTS];
+#pragma unroll
+    for (int c = 0; c < CONV_PTS; ++c) {
+      if (c * 256 >= npt) continue;
+      int t;
+      const int i = c * 256 + threadIdx.x, e = dTP.div(i, t), p = p0 + t;
+      v[c] = {T(0), T(0)};
+      if (i < npt && p < npen) v[c] = cload(FQ + (size_t)p + (size_t)e * Se);
+    }
+    // the influence function needs no data: evaluated while the loads are in flight
+    double eterm[CONV_PTS], vterm[CONV_PTS];
+#pragma unroll
+    for (int c = 0; c < CONV_PTS; ++c) {
+      if (c * 256 >= npt) continue;
+      int k1, k2, k3;
+      double mh[3];
+      eterm[c] = vterm[c] = 0.0;
+      if (!point(c * 256 + threadIdx.x, k1, k2, k3, mh)) continue;
+      const double msq = mh[0] * mh[0] + mh[1] * mh[1] + mh[2] * mh[2];
+      if (msq > d.rkcut2) continue;
+      const double denom = pi * d.volume * gmem(d.bsp1)[k1 - 1] * gmem(d.bsp2)[k2 - 1] * gmem(d.bsp3)[k3 - 1] * msq;
+      eterm[c] = exp(-fac * msq) / denom;
+      vterm[c] = 2.0 * (fac * msq + 1.0) / msq;
+    }
+#pragma unroll
+    for (int c = 0; c < CONV_PTS; ++c) {
+      if (c * 256 >= npt) continue;
+      int t;
+      const int i = c * 256 + threadIdx.x, e = dTP.div(i, t);
+      if (i < npt) a[t * LD + e] = v[c];
+    }
+    __syncthreads();
+    cx<T> *r = lds_fft<T, -1>(a, b, N, LD, TP, d.ax3, tw);
+    cx<T> *s = (r == a) ? b : a;
+#pragma unroll
+    for (int c = 0; c < CONV_PTS; ++c) {
+      if (c * 256 >= npt) continue;
+      int k1, k2, k3;
+      double mh[3];
+      if (!point(c * 256 + threadIdx.x, k1, k2, k3, mh)) continue;
+      int t;
+      const int e = dTP.div(c * 256 + threadIdx.x, t);
+      cx<T> &q = r[t * LD + e];
+      const double qr = (double)q.x, qi = (double)q.y;
+      if (vterm[c] != 0.0) {  // (within the cut-off; vterm is positive there)
         double struc2, f12 = 1.0, f13 = 1.0, f23 = 1.0;
         if (k1 == 1 || (k1 == ndim1 && (nfft1 & 1) == 0)) {
-          struc2 = eterm * qr * qr + eterm * qi * qi;
+          struc2 = eterm[c] * qr * qr + eterm[c] * qi * qi;
         } else {
-          double e2 = 2.0 * eterm;
+          double e2 = 2.0 * eterm[c];
           struc2 = e2 * qr * qr + e2 * qi * qi;
-          f12 = (mhat1 * mhat2 < 0.0 && k2 <= ndim1) ? 0.0 : 1.0;
-          f13 = (mhat1 * mhat3 < 0.0 && k3 <= ndim1) ? 0.0 : 1.0;
-          bool neg = mhat2 * mhat3 < 0.0;
+          f12 = (mh[0] * mh[1] < 0.0 && k2 <= ndim1) ? 0.0 : 1.0;
+          f13 = (mh[0] * mh[2] < 0.0 && k3 <= ndim1) ? 0.0 : 1.0;
+          bool neg = mh[1] * mh[2] < 0.0;
           bool lo2 = k2 <= ndim1, lo3 = k3 <= ndim1;
           f23 = (lo2 == lo3) ? (neg ? 0.0 : 1.0) : (neg ? 1.0 : 0.0);
         }
-        double vvir = struc2 * vterm;
+        double vvir = struc2 * vterm[c];
         acc[0] += struc2;
-        acc[1] += struc2 * (vterm * mhat1 * mhat1 - 1.0);
-        acc[2] += struc2 * (vterm * mhat2 * mhat2 - 1.0);
-        acc[3] += struc2 * (vterm * mhat3 * mhat3 - 1.0);
-        acc[4] += vvir * mhat1 * mhat2 * f12;
-        acc[5] += vvir * mhat1 * mhat3 * f13;
-        acc[6] += vvir * mhat2 * mhat3 * f23;
+        acc[1] += struc2 * (vterm[c] * mh[0] * mh[0] - 1.0);
+        acc[2] += struc2 * (vterm[c] * mh[1] * mh[1] - 1.0);
+        acc[3] += struc2 * (vterm[c] * mh[2] * mh[2] - 1.0);
+        acc[4] += vvir * mh[0] * mh[1] * f12;
+        acc[5] += vvir * mh[0] * mh[2] * f13;
+        acc[6] += vvir * mh[1] * mh[2] * f23;
       }
-      r[t * N + e] = {T((double)qv.x * eterm), T((double)qv.y * eterm)};
+      q = {T(qr * eterm[c]), T(qi * eterm[c])};
     }
     __syncthreads();
     if (!d.energy_only) {
-      cx<T> *o = lds_fft<T, +1>(r, s, N, TP, d.ax3, tw);
+      cx<T> *o = lds_fft<T, +1>(r, s, N, LD, TP, d.ax3, tw);
       for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
         int t;
         const int e = dTP.div(i, t), p = p0 + t;
-        if (p < npen) FQ[(size_t)p + (size_t)e * Se] = o[t * N + e];
+        if (p < npen) cstore(FQ + (size_t)p + (size_t)e * Se, o[t * LD + e]);
       }
     }
   }
@@ -586,7 +764,7 @@ __global__ void __launch_bounds__(256) k_fft_x_c2r(const PmeDesc *__restrict__ D
   extern __shared__ __align__(16) unsigned char smem[];
   const PmeDesc &d = D[blockIdx.y];
   const int N = d.K1, H = N / 2 + 1, rows = d.K2 * d.K3, TP = d.tpx;
-  if ((int)blockIdx.x >= d.gx || d.energy_only) return;
+  if ((int)blockIdx.x >= d.gx || d.energy_only || use_planes<T>(d)) return;
   cx<T> *a = reinterpret_cast<cx<T> *>(smem);
   cx<T> *b = a + TP * N;
   cx<T> *tw = b + TP * N;
@@ -598,18 +776,18 @@ __global__ void __launch_bounds__(256) k_fft_x_c2r(const PmeDesc *__restrict__ D
     int e;
     const int t = dH.div(i, e), row = row0 + t;
     cx<T> v = {T(0), T(0)};
-    if (row < rows) v = FQ[(size_t)row * H + e];
+    if (row < rows) v = cload(FQ + (size_t)row * H + e);
     if (e == 0 || 2 * e == N) v.y = T(0);
     a[t * N + e] = v;
     if (e > 0 && N - e >= H) a[t * N + (N - e)] = {v.x, -v.y};
   }
   __syncthreads();
-  cx<T> *r = lds_fft<T, +1>(a, b, N, TP, d.ax1, tw);
+  cx<T> *r = lds_fft<T, +1>(a, b, N, N, TP, d.ax1, tw);
   T *Qr = reinterpret_cast<T *>(d.Qr);
   for (int i = threadIdx.x; i < TP * N; i += blockDim.x) {
     int e;
     const int t = dN.div(i, e), row = row0 + t;
-    if (row < rows) Qr[(size_t)row * N + e] = r[t * N + e].x;
+    if (row < rows) gmem(Qr)[(size_t)row * N + e] = r[t * N + e].x;
   }
 }
 
@@ -773,7 +951,8 @@ __global__ void __launch_bounds__(1024) k_pme_finalize(const PmeDesc *__restrict
 // ---------------------------------------------------------------- launchers
 
 static int tile_pencils(int n, int npen, int elems) {
-  int tp = std::min(elems / n, (4096 / n - 1) / 2);  // two buffers and the twiddles within 64 KB in FP64
+  // two buffers (pencils n + 1 apart) and the twiddles within 64 KB in FP64
+  int tp = std::min(elems / n, (4096 - n) / (2 * (n + 1)));
   if (tp < 1) tp = 1;
   if (tp > npen) tp = npen;
   return tp;
@@ -797,19 +976,26 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
                 const hipEvent_t *ev, bool finalize, bool binned) {
   (void)tu;
   if (nsys <= 0) return;
-  int max_atoms = 1, max_bins = 1, any_tiled = 0, any_atomic = 0, max_gx = 1, max_gy = 1, max_gz = 1, max_gg = 1;
+  int max_atoms = 1, max_bins = 1, any_tiled = 0, any_atomic = 0, max_gx = 0, max_gy = 0, max_gz = 1, max_gg = 1;
+  int max_planes = 0, max_plane = 0;
   int order = 0, max_order = 0;
-  size_t max_grid = 1, shx = 0, shy = 0, shz = 0, max_work = 1;
+  size_t max_grid = 1, shx = 0, shy = 0, shz = 0, shp = 0, max_work = 1;
   for (int s = 0; s < nsys; ++s) {
     const PmeDesc &d = h[s];
     max_atoms = std::max(max_atoms, d.natoms);
-    max_gx = std::max(max_gx, d.gx);
-    max_gy = std::max(max_gy, d.gy);
+    if (use_planes<T>(d)) {
+      max_planes = std::max(max_planes, d.K3);
+      max_plane = std::max(max_plane, d.K1 * d.K2);
+      shp = std::max(shp, plane_lds<T>(d));
+    } else {
+      max_gx = std::max(max_gx, d.gx);
+      max_gy = std::max(max_gy, d.gy);
+    }
     max_gz = std::max(max_gz, d.conv_nblk);
     max_gg = std::max(max_gg, d.gather_nblk);
     shx = std::max(shx, (2 * (size_t)d.tpx + 1) * d.K1 * sizeof(cx<T>));
     shy = std::max(shy, (2 * (size_t)d.tpy + 1) * d.K2 * sizeof(cx<T>));
-    shz = std::max(shz, (2 * (size_t)d.tpz + 1) * d.K3 * sizeof(cx<T>));
+    shz = std::max(shz, (2 * (size_t)d.tpz * (d.K3 + 1) + d.K3) * sizeof(cx<T>));
     // one spline order in the whole launch: the kernels written out for it
     order = s == 0 || order == d.order ? d.order : 0;
     max_order = std::max(max_order, d.order);
@@ -841,11 +1027,18 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
     hipLaunchKernelGGL(k_spread<T>, dim3((unsigned)((max_work + 255) / 256), nsys), blk, 0, st, d_desc);
   }
   if (ev) ORAC_HIP(hipEventRecord(ev[1], st));
-  hipLaunchKernelGGL(k_fft_x_r2c<T>, dim3(max_gx, nsys), blk, shx, st, d_desc);
-  hipLaunchKernelGGL((k_fft_pencil<T, -1>), dim3(max_gy, nsys), blk, shy, st, d_desc, 2);
+  const dim3 pl(max_planes, nsys), bp(max_plane <= 64 * 64 ? 512 : 1024);
+  if (max_planes) hipLaunchKernelGGL(k_fft_plane_r2c<T>, pl, bp, shp, st, d_desc);
+  if (max_gx) {
+    hipLaunchKernelGGL(k_fft_x_r2c<T>, dim3(max_gx, nsys), blk, shx, st, d_desc);
+    hipLaunchKernelGGL((k_fft_pencil<T, -1>), dim3(max_gy, nsys), blk, shy, st, d_desc, 2);
+  }
   hipLaunchKernelGGL(k_fft_z_conv<T>, dim3(max_gz, nsys), blk, shz, st, d_desc);
-  hipLaunchKernelGGL((k_fft_pencil<T, +1>), dim3(max_gy, nsys), blk, shy, st, d_desc, 2);
-  hipLaunchKernelGGL(k_fft_x_c2r<T>, dim3(max_gx, nsys), blk, shx, st, d_desc);
+  if (max_planes) hipLaunchKernelGGL(k_fft_plane_c2r<T>, pl, bp, shp, st, d_desc);
+  if (max_gx) {
+    hipLaunchKernelGGL((k_fft_pencil<T, +1>), dim3(max_gy, nsys), blk, shy, st, d_desc, 2);
+    hipLaunchKernelGGL(k_fft_x_c2r<T>, dim3(max_gx, nsys), blk, shx, st, d_desc);
+  }
   if (ev) ORAC_HIP(hipEventRecord(ev[2], st));
   switch (order) {
     case 4: hipLaunchKernelGGL((k_gather<T, 4>), dim3(max_gg, nsys), blk, 0, st, d_desc); break;
