@@ -777,12 +777,20 @@ static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events
   // streams cost more than it overlapped (a fork before the centres with a
   // wait at the gather, and a third stream for the corrections: 279 against
   // 231 us for the 24,460-atom system; everything on one stream 269).
+  // The corrections go with the shorter of the two: beside the pair kernel alone
+  // (dynamics, whose list is built now and then) the reciprocal sum takes its
+  // 70 us of latencies however small the system, the pair kernel 3 us per 1,000
+  // atoms.  10 steps of 16k atoms 1,450 us with the corrections behind the
+  // reciprocal sum, 1,361 behind the pairs; of 76k atoms 2,950 and 3,065.
   const bool side = !events && ctx->side;
+  long atoms = 0;
+  for (const System *S : b.sys) atoms += S->natoms;
+  const bool corr_pairs = md_lists && atoms <= 30000;
   if (side) {
     ORAC_HIP(hipEventRecord(b.fork, st));
     ORAC_HIP(hipStreamWaitEvent(ctx->side, b.fork, 0));
     pme(ctx->side);
-    if (b.any_corr) launch_corr(b.dc, b.hc.data(), n, ctx->side, false);
+    if (b.any_corr && !corr_pairs) launch_corr(b.dc, b.hc.data(), n, ctx->side, false);
     ORAC_HIP(hipEventRecord(b.join, ctx->side));
   }
   if (lists) {
@@ -797,6 +805,7 @@ static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events
     launch_pairs<float>(b.dq, b.hq.data(), n, st, b.tu, pack, false, kb, ke);
   mark(ST_PAIRS);
   if (side) {
+    if (b.any_corr && corr_pairs) launch_corr(b.dc, b.hc.data(), n, st, false);
     ORAC_HIP(hipStreamWaitEvent(st, b.join, 0));
     mark(ST_PME);
   } else {
