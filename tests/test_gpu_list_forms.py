@@ -25,6 +25,8 @@ CASES = {
     "faces": dict(n=600, ncell=8, box=0.3, shift=-0.3),  # members across all three faces
     "skewed": dict(n=800, ncell=9, skew=0.3),
     "few": dict(n=3, ncell=8),
+    "scan_rows": dict(n=300, ncell=16),     # one cell past the scan's rows of 4,096
+    "scan_rounds": dict(n=300, ncell=27),   # more cells than one round of the scan
 }
 
 
