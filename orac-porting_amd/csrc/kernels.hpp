@@ -398,8 +398,8 @@ struct MdDesc {
 // Connected atoms per workgroup.  Larger sets, and sets with rigid units, go by
 // launches, a kick or substep each.  A step with four substeps of a chain of
 // 2,048 atoms takes 109 us in one workgroup and 137 by launches; each further
-// 1,024 atoms add 20 to the one and 4 to the other, and the positions of 3,072
-// exceed 64 KB of LDS.
+// 1,024 atoms add 20 to the one and 4 to the other, and the state of a third atom
+// a thread no longer fits the 128 registers of a 1,024-thread workgroup.
 constexpr int MD_WG = 1024, MD_WG_SLOTS = 2 * MD_WG, MD_FREE = 256;
 // stages, applied in this order when combined: half kick by the fast forces
 // over h + RATTLE; the half kicks that end a step, by the inner-shell forces

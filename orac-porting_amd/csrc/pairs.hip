@@ -1,6 +1,8 @@
 // pairs.hip -- centres, linked-cell lists and the correction pair lists on gfx950.
 //
-//   k_group_centres / k_mol_com   appbou.f group centres, molecule centres of mass
+//   k_prepare                     appbou.f group centres, molecule centres of mass, the
+//                                 pair kernel's records, the spread's bins
+//   k_tail                        forces combined, every partial sum reduced
 //   k_cell_*                      linked-cell binning of group centres (lc_list.f:93-109)
 //   k_list_count / k_list_offsets / k_list_write
 //                                 stencil walk and pair test (lc_list.f:133-201), two
