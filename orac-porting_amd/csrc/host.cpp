@@ -251,6 +251,23 @@ size_t mapnl_length(const int32_t *mapnl, int nato) {
   return na;
 }
 
+// A stencil {dx, dy, dz} as runs of cells along z {dx, dy, first dz, last dz},
+// where every (dx, dy) has one that run_cells can wrap; empty otherwise.
+std::vector<int4> stencil_runs(const std::vector<int> &sten, int ncx, int ncy, int ncz) {
+  std::map<std::pair<int, int>, std::vector<int>> runs;
+  for (size_t m = 0; m + 2 < sten.size(); m += 3) runs[{sten[m], sten[m + 1]}].push_back(sten[m + 2]);
+  std::vector<int4> col;
+  for (auto &r : runs) {
+    std::vector<int> &z = r.second;
+    std::sort(z.begin(), z.end());
+    if (z.back() - z.front() + 1 != (int)z.size() || (int)z.size() > ncz || std::abs(r.first.first) >= ncx ||
+        std::abs(r.first.second) >= ncy || z.front() <= -ncz || z.back() >= ncz)
+      return {};
+    col.push_back(make_int4(r.first.first, r.first.second, z.front(), z.back()));
+  }
+  return col;
+}
+
 CellGrid make_cellgrid(BufSet &B, const std::string &pfx, int ncx, int ncy, int ncz, const int32_t *nind,
                               const int32_t *indxi, const int32_t *indxj, const int32_t *indxk, double rcut,
                               const double *co, int half, hipStream_t st) {
@@ -266,23 +283,10 @@ CellGrid make_cellgrid(BufSet &B, const std::string &pfx, int ncx, int ncy, int 
     sten[3 * m + 2] = indxk[1 + 2 * m];
   }
   cg.sten = B.put_vec(pfx + "sten", sten, st, true);
-  // the stencil's runs along z, where every (x, y) offset has one
   cg.ncol = 0;
   cg.col = nullptr;
   if (!half) {
-    std::map<std::pair<int, int>, std::vector<int>> runs;
-    for (int m = 0; m < cg.nsten; ++m) runs[{sten[3 * m], sten[3 * m + 1]}].push_back(sten[3 * m + 2]);
-    std::vector<int4> col;
-    for (auto &r : runs) {
-      std::vector<int> &z = r.second;
-      std::sort(z.begin(), z.end());
-      if (z.back() - z.front() + 1 != (int)z.size() || (int)z.size() > ncz || std::abs(r.first.first) >= ncx ||
-          std::abs(r.first.second) >= ncy || z.front() <= -ncz || z.back() >= ncz) {
-        col.clear();
-        break;
-      }
-      col.push_back(make_int4(r.first.first, r.first.second, z.front(), z.back()));
-    }
+    const std::vector<int4> col = stencil_runs(sten, ncx, ncy, ncz);
     cg.ncol = (int)col.size();
     if (cg.ncol > 0) cg.col = B.put_vec(pfx + "col", col, st, true);
   }

@@ -115,6 +115,7 @@ PmeDesc pme_desc_base(BufSet &B, const std::string &pfx, const PmePlan &P, int n
                       double volume, double alpha, double rkcut, bool fp64, const Tuning &tu, hipStream_t st);
 // apply the tuning's FFT tiling and spread path to a descriptor built by pme_desc_base
 void pme_apply_tuning(PmeDesc &d, const Tuning &tu);
+std::vector<int4> stencil_runs(const std::vector<int> &sten, int ncx, int ncy, int ncz);
 CellGrid make_cellgrid(BufSet &B, const std::string &pfx, int ncx, int ncy, int ncz, const int32_t *nind,
                        const int32_t *indxi, const int32_t *indxj, const int32_t *indxk, double rcut,
                        const double *co, int half, hipStream_t st);

@@ -215,6 +215,26 @@ struct CellGrid {
   const int4 *col;
 };
 
+// The cells k + z0 .. k + z1 of a periodic column of n cells (z0 <= z1, at most
+// n of them, |z0| and |z1| below n), as [a0, b0) and, where the run wraps at a
+// face, [a1, b1).  In a skewed cell a run may lie wholly past a face: it is then
+// one segment on the other side.
+struct RunCells {
+  int a0, b0, a1, b1;
+};
+__host__ __device__ inline RunCells run_cells(int k, int z0, int z1, int n) {
+  int a = k + z0, b = k + z1 + 1;
+  const int shift = b <= 0 ? n : (a >= n ? -n : 0);
+  a += shift;
+  b += shift;
+  RunCells r;
+  r.a0 = a < 0 ? 0 : a;
+  r.b0 = b > n ? n : b;
+  r.a1 = a < 0 ? a + n : 0;
+  r.b1 = a < 0 ? n : (b > n ? b - n : 0);
+  return r;
+}
+
 // One system's list build: cells of the group centres, then the stencil walk.
 struct ListDesc {
   int ngrp;

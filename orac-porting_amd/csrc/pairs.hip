@@ -376,15 +376,12 @@ __device__ __forceinline__ int list_walk_runs(int n, const ListDesc &d, int *out
       ny += ny < 0 ? ncy : 0;
       ny -= ny >= ncy ? ncy : 0;
       const auto start = gmem(d.cell_start + ncz * (ny + ncy * nx));
-      const int za = k + col.z, zb = k + col.w;
-      s[0] = start[max(za, 0)];
-      cnt[0] = start[min(zb, ncz - 1) + 1] - s[0];
-      if (za < 0) {
-        s[1] = start[za + ncz];
-        cnt[1] = start[ncz] - s[1];
-      } else if (zb >= ncz) {
-        s[1] = start[0];
-        cnt[1] = start[zb - ncz + 1] - s[1];
+      const RunCells z = run_cells(k, col.z, col.w, ncz);
+      s[0] = start[z.a0];
+      cnt[0] = start[z.b0] - s[0];
+      if (z.a1 < z.b1) {
+        s[1] = start[z.a1];
+        cnt[1] = start[z.b1] - s[1];
       }
     }
     for (int w = 0; w < 2; ++w) {
