@@ -148,12 +148,17 @@ __host__ __device__ inline T recip_km1(int k) {
   }
 }
 
-// (one rounding per written operation, no contraction: every caller, unrolled
-// or not, gets the same weights bit for bit, and the host the reference's)
+// (no contraction by the compiler: every caller, unrolled or not, gets the same
+// weights bit for bit, with the sum fused on the device and each operation
+// rounded on the host, as the reference's is)
 template <typename T>
 __host__ __device__ inline T bspline_term(T div, T w, int k, int j, T lo, T hi) {
 #pragma clang fp contract(off)
+#ifdef __HIP_DEVICE_COMPILE__
+  return div * fma(w + T(j), lo, (T(k - j) - w) * hi);
+#else
   return div * ((w + T(j)) * lo + (T(k - j) - w) * hi);
+#endif
 }
 
 template <typename T>

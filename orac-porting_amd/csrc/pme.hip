@@ -102,24 +102,41 @@ __device__ inline void dft(cx<T> *v) {
     v[4] = csub(a1, b1);
     v[2] = cadd(a2, b2);
     v[3] = csub(a2, b2);
-  } else {  // 6 and 8: even and odd inputs, then one radix-2 step
-    constexpr int Q = R / 2;
-    constexpr double c1 = R == 6 ? 0.5 : 0.7071067811865475244, s1 = R == 6 ? 0.8660254037844386468 : c1;
-    constexpr double C[4][2] = {{1.0, 0.0}, {c1, s1}, {-0.5, s1}, {-c1, s1}};  // ([2] of 8 is i)
-    cx<T> e[Q], o[Q];
+  } else if constexpr (R == 6) {
+    // prime factors: input 3 n1 + 2 n2, output 3 k1 + 4 k2 (mod 6), and no twiddles between the
+    // radix-2 and the radix-3 step, which in FP32 would round once more
+    cx<T> s[3], d[3];
 #pragma unroll
-    for (int k = 0; k < Q; ++k) {
+    for (int n = 0; n < 3; ++n) {
+      const cx<T> p = v[2 * n], q = v[(2 * n + 3) % 6];
+      s[n] = cadd(p, q);
+      d[n] = csub(p, q);
+    }
+    dft<T, 3, S>(s);
+    dft<T, 3, S>(d);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      v[4 * k % 6] = s[k];
+      v[(4 * k + 3) % 6] = d[k];
+    }
+  } else {  // 8: even and odd inputs, then one radix-2 step
+    static_assert(R == 8);
+    const T h = T(0.7071067811865475244);
+    cx<T> e[4], o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
       e[k] = v[2 * k];
       o[k] = v[2 * k + 1];
     }
-    dft<T, Q, S>(e);
-    dft<T, Q, S>(o);
+    dft<T, 4, S>(e);
+    dft<T, 4, S>(o);
+    o[1] = cmul(o[1], cx<T>{h, T(S) * h});
+    o[2] = cmuli<T, S>(o[2]);
+    o[3] = cmul(o[3], cx<T>{-h, T(S) * h});
 #pragma unroll
-    for (int k = 0; k < Q; ++k) {
-      if (R == 8 && k == 2) o[k] = cmuli<T, S>(o[k]);
-      else if (k > 0) o[k] = cmul(o[k], cx<T>{T(C[k][0]), T(S * C[k][1])});
+    for (int k = 0; k < 4; ++k) {
       v[k] = cadd(e[k], o[k]);
-      v[k + Q] = csub(e[k], o[k]);
+      v[k + 4] = csub(e[k], o[k]);
     }
   }
 }
