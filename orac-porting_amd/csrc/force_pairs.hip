@@ -259,7 +259,7 @@ __device__ __forceinline__ AlchTerms<T> alch_terms(const PairDesc &d, T xc, T yc
       conf0 = T(F[3]) * (eps * (gp20 - gp10));
     }
     if (!d.lskip_ewald) {
-      const T alphar = T(d.alpha) * (rsq * rinv);
+      const T r = rsq * rinv, alphar = T(d.alpha) * r;
       const T qt = pair_rcp<T>(T(1) + T(AS_QP) * alphar);
       const T expcst = pair_exp2<T>(T(d.ew_exp2) * rsq);
       const T erfcst = ((((T(AS_A5) * qt + T(AS_A4)) * qt + T(AS_A3)) * qt + T(AS_A2)) * qt + T(AS_A1)) * qt * expcst;
@@ -279,6 +279,43 @@ __device__ __forceinline__ AlchTerms<T> alch_terms(const PairDesc &d, T xc, T yc
   r.cou = cou;
   r.dw = (double)(conf - conf0) + (double)(cou - cou0);
   return r;
+}
+
+// One plain atom pair: the force over the separation (force = qf * (x, y, z))
+// and the two energies.  Every fused operation is written out, here and in the
+// sums, so that all forms of the kernel round alike: a system's results do not
+// depend on the systems beside it.
+template <typename T>
+struct PairTerms {
+  T qf, conf, cou;
+};
+
+template <typename T>
+__device__ __forceinline__ PairTerms<T> plain_terms(const PairDesc &d, T x, T y, T z, T qq, bool lskip, bool plainq,
+                                                    bool lj, T c12, T c6) {
+#pragma clang fp contract(off)
+  const T rsq = fma(z, z, fma(y, y, x * x));
+  const T rinv = pair_rsqrt<T>(rsq);
+  const T rsqi = rinv * rinv;
+  PairTerms<T> p;
+  p.conf = T(0);
+  if (!lskip) {
+    const T r = rsq * rinv, expcst = pair_exp2<T>(T(d.ew_exp2) * rsq);
+    const T erfcst = erfc_poly<T>(pair_rcp<T>(fma(T(d.ew_qp), r, T(1)))) * expcst;
+    const T qr = qq * rinv;
+    p.cou = qr * erfcst;
+    p.qf = fma(T(d.ew_twa) * r, expcst, erfcst) * (qr * rsqi);
+  } else {
+    p.cou = plainq ? qq * rinv : T(0);
+    p.qf = p.cou * rsqi;
+  }
+  if (lj) {
+    const T r6 = rsqi * rsqi * rsqi;
+    const T e6 = c6 * r6, e12 = c12 * r6 * r6;
+    p.conf = e12 - e6;
+    p.qf = fma(fma(T(12), e12, T(-6) * e6), rsqi, p.qf);
+  }
+  return p;
 }
 
 constexpr int PAIR_NACC = 16;      // energies and virial of a block: uconf[3], ucoul[3], st[9], dwrk
@@ -488,11 +525,11 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
               if (gg.drj >= d.r2out && gg.drj < d.r2out0) {
                 const double auxa = (d.arsout1 + 2.0 * rsp) * inv_o2, auxb = d.rout0 - rsp;
                 sw = auxa * (auxb * auxb);
-                dsw = (-(2.0 * auxa * auxb) + 2.0 * (auxb * auxb) * inv_o2) * rinv;
+                dsw = fma(2.0 * (auxb * auxb), inv_o2, -(2.0 * auxa * auxb)) * rinv;
               } else {
                 const double auxa = (d.arsinn1 + 2.0 * rsp) * inv_i2, auxb = d.rinn0 - rsp;
-                sw = 1.0 - auxa * (auxb * auxb);
-                dsw = (2.0 * auxa * auxb - 2.0 * (auxb * auxb) * inv_i2) * rinv;
+                sw = fma(-auxa, auxb * auxb, 1.0);
+                dsw = -fma(2.0 * (auxb * auxb), inv_i2, -(2.0 * auxa * auxb)) * rinv;
               }
             }
             if constexpr (F32) {
@@ -606,48 +643,31 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
                 qq = masked ? T(0) : qq;
                 x = masked ? T(1) : x;
               }
-              T qf, cou, conf = T(0);
+              T qf, cou, conf;
               double dw = 0.0;
               if (MODE == PAIR_ALCH && (soft_b || (alch && (fl & ATOM_ALCH)))) {
                 const double4 ap = gload_at(d.alch_pair, (fl >> ATOM_FLAG_BITS) * d.ntypes + tb);
                 const AlchTerms<T> r = alch_terms<T>(d, x, y, z, qq, ap, sh.alch[(int)ap.z]);
-                qf = r.qf;
-                conf = r.conf;
-                cou = r.cou;
-                dw = r.dw;
+                // (the soft core takes its own parameters)
+                qf = masked ? T(0) : r.qf;
+                conf = masked ? T(0) : r.conf;
+                cou = masked ? T(0) : r.cou;
+                dw = masked ? 0.0 : r.dw;
               } else {
-                const T rsq = x * x + y * y + z * z;
-                const T rinv = pair_rsqrt<T>(rsq);
-                const T rsqi = rinv * rinv;
-                if (!lskip) {
-                  const T expcst = pair_exp2<T>(T(d.ew_exp2) * rsq), r = rsq * rinv;
-                  const T erfcst = erfc_poly<T>(pair_rcp<T>(T(1) + T(d.ew_qp) * r)) * expcst;
-                  const T qr = qq * rinv;
-                  cou = qr * erfcst;
-                  qf = (erfcst + (T(d.ew_twa) * r) * expcst) * (qr * rsqi);
-                } else {
-                  cou = plainq ? qq * rinv : T(0);
-                  qf = cou * rsqi;
-                }
-                if (fl & ATOM_LJ) {  // some type has LJ with this owner atom's
-                  T c12 = c12a, c6 = c6a;
+                const bool lj = (fl & ATOM_LJ) != 0;  // some type has LJ with this owner atom's
+                T c12 = c12a, c6 = c6a;
+                if (lj) {
                   if (u > 0) pair_lj<T, MODE == PAIR_PLAIN>(d, fl >> ATOM_FLAG_BITS, tb, c12, c6);
                   c12 = masked ? T(0) : c12;
                   c6 = masked ? T(0) : c6;
-                  const T r6 = rsqi * rsqi * rsqi;
-                  const T e6 = c6 * r6, e12 = c12 * r6 * r6;
-                  conf = e12 - e6;
-                  if (MODE != PAIR_ALCH) vc += (double)conf;
-                  qf += (T(12) * e12 - T(6) * e6) * rsqi;
                 }
+                const PairTerms<T> r = plain_terms<T>(d, x, y, z, qq, lskip, plainq, lj, c12, c6);
+                qf = r.qf;
+                conf = r.conf;
+                cou = r.cou;
               }
-              if (MODE == PAIR_ALCH) {  // (the soft core takes its own parameters)
-                qf = masked ? T(0) : qf;
-                conf = masked ? T(0) : conf;
-                cou = masked ? T(0) : cou;
-                seg += masked ? 0.0 : dw;
-              }
-              if (MODE == PAIR_ALCH) vc += (double)conf;
+              if (MODE == PAIR_ALCH) seg += dw;
+              if (MODE == PAIR_ALCH || (fl & ATOM_LJ)) vc += (double)conf;
               vq += (double)cou;
               double w = (double)qf * sw;
               if (MODE == PAIR_REM) {
@@ -661,13 +681,13 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
                 if (sel) seg += en;
                 vr += f * en;
               }
-              fr[u][0] += w * (double)x;
-              fr[u][1] += w * (double)y;
-              fr[u][2] += w * (double)z;
+              fr[u][0] = fma(w, (double)x, fr[u][0]);
+              fr[u][1] = fma(w, (double)y, fr[u][1]);
+              fr[u][2] = fma(w, (double)z, fr[u][2]);
               if (ST) {
-                fsx += w * (double)x;
-                fsy += w * (double)y;
-                fsz += w * (double)z;
+                fsx = fma(w, (double)x, fsx);
+                fsy = fma(w, (double)y, fsy);
+                fsz = fma(w, (double)z, fsz);
               }
             }
           }
@@ -684,8 +704,8 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
           ec[1] += solute ? 0.0 : sw * vc;
           eq[1] += solute ? 0.0 : sw * vq;
         } else {
-          ec[1] += sw * vc;
-          eq[1] += sw * vq;
+          ec[1] = fma(sw, vc, ec[1]);
+          eq[1] = fma(sw, vq, eq[1]);
         }
         if (DW) dwl += sw * seg;
         double gx, gy, gz;
@@ -699,18 +719,18 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
           gz = W.gz[e];
         }
         const double v = -dsw * (MODE == PAIR_REM ? vr : vc + vq);
-        x3[0] += v * gx;
-        x3[1] += v * gy;
-        x3[2] += v * gz;
+        x3[0] = fma(v, gx, x3[0]);
+        x3[1] = fma(v, gy, x3[1]);
+        x3[2] = fma(v, gz, x3[2]);
         if (pass_st) {
-          fsx += v * gx;
-          fsy += v * gy;
-          fsz += v * gz;
+          fsx = fma(v, gx, fsx);
+          fsy = fma(v, gy, fsy);
+          fsz = fma(v, gz, fsz);
           const double sx = shifted ? (double)W.sx[e] : 0.0, sy = shifted ? (double)W.sy[e] : 0.0,
                        sz = shifted ? (double)W.sz[e] : 0.0;
-          st[0] -= fsx * sx; st[1] -= fsx * sy; st[2] -= fsx * sz;
-          st[3] -= fsy * sx; st[4] -= fsy * sy; st[5] -= fsy * sz;
-          st[6] -= fsz * sx; st[7] -= fsz * sy; st[8] -= fsz * sz;
+          const double fs[3] = {fsx, fsy, fsz}, sh3[3] = {sx, sy, sz};
+#pragma unroll
+          for (int k = 0; k < 9; ++k) st[k] = fma(-fs[k / 3], sh3[k % 3], st[k]);
         }
         shead = (shead + np) & (SLOT_RING - 1);
         ns -= np;
