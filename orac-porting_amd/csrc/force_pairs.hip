@@ -96,8 +96,7 @@ __device__ __forceinline__ double fma_const(double a, double b, double c) {
   return d;
 }
 // 2^y for the Ewald factor exp(-(alpha r)^2) = 2^(-alpha^2 log2(e) r^2), from
-// the squared distance, beside the reciprocal square root rather than after
-// it.  y = n + f, |f| <= 1/2 (exact), and 2^f = 1 + f q(f) with q of degree 8
+// the squared distance.  y = n + f, |f| <= 1/2 (exact), and 2^f = 1 + f q(f) with q of degree 8
 // interpolating (2^f - 1) / f at the Chebyshev nodes (3.7e-14 relative).
 template <typename T>
 __device__ inline T pair_exp2(T y);
@@ -117,6 +116,16 @@ __device__ inline double pair_exp2<double>(double y) {
 }
 template <>
 __device__ inline float pair_exp2<float>(float y) { return __builtin_amdgcn_exp2f(y); }
+
+// exp(-(alpha r)^2), r = rsq * rsqrt(rsq): FP64 from rsq, beside the reciprocal
+// square root rather than after it.  FP32 from r: the seed's error (1 ulp) then
+// enters with the opposite sign to that of the force's 1 / r^3, of which it takes
+// part back; from rsq the Coulomb forces are 1 to 2 % further from 64 bits.
+template <typename T>
+__device__ __forceinline__ T pair_ewald_exp(const PairDesc &d, T rsq, T r) {
+  if constexpr (sizeof(T) == 8) return pair_exp2<T>(T(d.ew_exp2) * rsq);
+  else return pair_exp2<T>(T(d.ew_exp2) * (r * r));
+}
 
 // The A&S 7.1.26 polynomial of erfc at qt = 1 / (1 + p x), without its exponential
 template <typename T>
@@ -234,7 +243,7 @@ __device__ __forceinline__ AlchTerms<T> alch_terms(const PairDesc &d, T xc, T yc
     if (!d.lskip_ewald) {
       const T alphar = T(d.alpha) * r;
       const T qt = pair_rcp<T>(T(1) + T(AS_QP) * alphar);
-      const T expcst = pair_exp2<T>(T(d.ew_exp2) * rsq);
+      const T expcst = pair_ewald_exp<T>(d, rsq, r);
       const T erfcst = ((((T(AS_A5) * qt + T(AS_A4)) * qt + T(AS_A3)) * qt + T(AS_A2)) * qt + T(AS_A1)) * qt * expcst;
       const T furpar = T(F[5]) * qq;
       cou = furpar * erfcst * irq;
@@ -261,7 +270,7 @@ __device__ __forceinline__ AlchTerms<T> alch_terms(const PairDesc &d, T xc, T yc
     if (!d.lskip_ewald) {
       const T r = rsq * rinv, alphar = T(d.alpha) * r;
       const T qt = pair_rcp<T>(T(1) + T(AS_QP) * alphar);
-      const T expcst = pair_exp2<T>(T(d.ew_exp2) * rsq);
+      const T expcst = pair_ewald_exp<T>(d, rsq, r);
       const T erfcst = ((((T(AS_A5) * qt + T(AS_A4)) * qt + T(AS_A3)) * qt + T(AS_A2)) * qt + T(AS_A1)) * qt * expcst;
       const T furpar = T(F[5]) * qq, furpar0 = T(F[7]) * qq;
       cou = furpar * erfcst * auxaa;
@@ -300,7 +309,7 @@ __device__ __forceinline__ PairTerms<T> plain_terms(const PairDesc &d, T x, T y,
   PairTerms<T> p;
   p.conf = T(0);
   if (!lskip) {
-    const T r = rsq * rinv, expcst = pair_exp2<T>(T(d.ew_exp2) * rsq);
+    const T r = rsq * rinv, expcst = pair_ewald_exp<T>(d, rsq, r);
     const T erfcst = erfc_poly<T>(pair_rcp<T>(fma(T(d.ew_qp), r, T(1)))) * expcst;
     const T qr = qq * rinv;
     p.cou = qr * erfcst;
@@ -310,7 +319,9 @@ __device__ __forceinline__ PairTerms<T> plain_terms(const PairDesc &d, T x, T y,
     p.qf = p.cou * rsqi;
   }
   if (lj) {
-    const T r6 = rsqi * rsqi * rsqi;
+    // FP32: from rsq, whose power rounds without the seed's bias (12 to 14 times it in rinv's
+    // powers, which showed in the energy and the stress)
+    const T r6 = sizeof(T) == 4 ? pair_rcp<T>(rsq * rsq * rsq) : rsqi * rsqi * rsqi;
     const T e6 = c6 * r6, e12 = c12 * r6 * r6;
     p.conf = e12 - e6;
     p.qf = fma(fma(T(12), e12, T(-6) * e6), rsqi, p.qf);
@@ -577,23 +588,21 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
         const AtomRec<T> rb = atom_rec<T>(d, js);
         const int2 ib = gload_at(d.sai, js);
         const double sw = have ? W.sw[e] : 0.0, dsw = have ? W.dsw[e] : 0.0;
-        // separation = (owner centre - neighbour centre - image) + owner offset - neighbour offset;
-        // FP32: the centre separation as hi + lo, so that the last addition alone rounds at its size
-        T bx, by, bz, hx = T(0), hy = T(0), hz = T(0), lx = T(0), ly = T(0), lz = T(0);
+        // separation = owner centre - neighbour centre - image (bx) + owner offset - neighbour offset.  FP32:
+        // the centre separation as hi + lo, and every rounding the same from either side, so that a
+        // pair's two forces cancel exactly and leave no net force to the virial
+        T bx, by, bz, lx, ly, lz;
         if constexpr (F32) {
           float2 g;
           __builtin_memcpy(&g, &W.gx[e], 8);
-          hx = g.x;
+          bx = g.x;
           lx = g.y;
           __builtin_memcpy(&g, &W.gy[e], 8);
-          hy = g.x;
+          by = g.x;
           ly = g.y;
           __builtin_memcpy(&g, &W.gz[e], 8);
-          hz = g.x;
+          bz = g.x;
           lz = g.y;
-          bx = lx - rb.x;
-          by = ly - rb.y;
-          bz = lz - rb.z;
         } else {
           bx = W.gx[e] - rb.x;
           by = W.gy[e] - rb.y;
@@ -620,9 +629,9 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
               __builtin_memcpy(&ra, &W.own[u], sizeof ra);
               T x, y, z;
               if constexpr (F32) {
-                x = hx + (bx + ra.x);
-                y = hy + (by + ra.y);
-                z = hz + (bz + ra.z);
+                x = bx + (lx + (ra.x - rb.x));
+                y = by + (ly + (ra.y - rb.y));
+                z = bz + (lz + (ra.z - rb.z));
               } else {
                 x = bx + ra.x;
                 y = by + ra.y;
@@ -710,9 +719,14 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
         if (DW) dwl += sw * seg;
         double gx, gy, gz;
         if constexpr (F32) {
-          gx = (double)hx + (double)lx;
-          gy = (double)hy + (double)ly;
-          gz = (double)hz + (double)lz;
+          auto wide = [](double w) {
+            float2 g;
+            __builtin_memcpy(&g, &w, 8);
+            return (double)g.x + (double)g.y;
+          };
+          gx = wide(W.gx[e]);
+          gy = wide(W.gy[e]);
+          gz = wide(W.gz[e]);
         } else {
           gx = W.gx[e];
           gy = W.gy[e];
@@ -1059,7 +1073,7 @@ __device__ __forceinline__ void own_item(const PairDesc &d, int blk, OwnShared &
               const T rsp = rsq * rinv;
               const T alphar = T(d.alpha) * rsp;
               const T qt = pair_rcp<T>(T(1) + T(AS_QP) * alphar);
-              const T expcst = pair_exp2<T>(T(d.ew_exp2) * rsq);
+              const T expcst = pair_ewald_exp<T>(d, rsq, rsp);
               const T erfcst =
                   ((((T(AS_A5) * qt + T(AS_A4)) * qt + T(AS_A3)) * qt + T(AS_A2)) * qt + T(AS_A1)) * qt * expcst;
               cou = qq * erfcst * rinv;

@@ -29,6 +29,43 @@ def _removed(s, n=40, lam=0.4):
     return synth.alchemy_for(s, np.arange(n)), synth.lambda_state(lam, lrm0=lam + 0.1)
 
 
+def _direct(ctx, s, precision, alchemy=None):
+    """The direct sum's forces: those beyond the same system's with a cutoff that no pair is within."""
+    far = dataclasses.replace(s, rcut=0.5, rtol=0.01, rnei=0.01)
+    return _eval(ctx, s, precision, alchemy)["f"] - _eval(ctx, far, precision, alchemy)["f"]
+
+
+@pytest.mark.parametrize("charges", [False, True])
+@pytest.mark.parametrize("name", ["waters", "mixed", "seven_one"])
+def test_pair_forces_cancel(gpu_ctx, name, charges):
+    """Both sides of a pair round alike in FP32, so the direct forces sum to
+    zero but for the FP64 sums (1,728 atoms of ~100 terms each: a few hundred
+    roundings of 1e-16 of the largest; a single FP32 rounding is 6e-8)."""
+    from test_gpu_pair_forms import CASES
+    s = grouped(**CASES[name])
+    if not charges:
+        s = dataclasses.replace(s, charge=0.0 * s.charge)
+    f = _direct(gpu_ctx, s, 1)
+    assert np.abs(f.sum(axis=1)).max() < 1e-12 * np.abs(f).max()
+
+
+def test_lj_energy_has_no_bias(gpu_ctx):
+    """LJ constants that FP32 holds exactly: what is left of the energy's and
+    the forces' error is the arithmetic's, whose roundings (6e-8 a pair) average
+    out over 100,000 pairs unless a seed's bias is raised to the twelfth power
+    (1.4e-7 of the energy where r^-6 came from the reciprocal square root)."""
+    s = grouped(sizes=[3])
+    s = dataclasses.replace(s, charge=0.0 * s.charge, ecc12=np.exp2(np.round(np.log2(s.ecc12.clip(1e-300)))) * (s.ecc12 > 0),
+                            ecc6=np.exp2(np.round(np.log2(s.ecc6.clip(1e-300)))) * (s.ecc6 > 0))
+    g, m = _eval(gpu_ctx, s, 0), _eval(gpu_ctx, s, 1)
+    e, em = (sum(r[k] for k in ("uconf_slt", "uconf_slv", "uconf_ss")) for r in (g, m))
+    tr, trm = (np.trace(r["stress"]) for r in (g, m))
+    print("LJ energy", (em - e) / abs(e), "stress", (trm - tr) / abs(tr), "f", relrms(m["f"], g["f"]))
+    # (energy: a sum of both signs; 1.1e-7 and 2.4e-8 here, 8.7e-7 and 2.1e-7 with the seed's powers)
+    assert abs(em - e) < 2e-7 * abs(e)
+    assert abs(trm - tr) < 6e-8 * abs(tr)
+
+
 @pytest.mark.parametrize("K,bound", [(72, 5.23e-7), (108, 7.55e-7)])
 def test_reciprocal_forces_fp32(gpu_ctx, K, bound):
     """FP32 splines and transforms, mean of eight systems (every sum of a run is
@@ -67,3 +104,27 @@ def test_plain_system_beside_an_alchemical_one(gpu_ctx, order):
         b.close()
         for rs in rss:
             rs.close()
+
+
+def test_window_against_fp64(gpu_ctx):
+    """Windows of a ligand being removed: forces, stress and the energy step to
+    the next window, whose terms nearly cancel."""
+    from orac_hip import api, synth
+    s, al, states = synth.alchemy_windows(n_windows=6, seed=41)
+    out = []
+    for precision in (0, 1):
+        f, st, dw = [], [], []
+        for lam in states:
+            rs = api.ResidentSystem(gpu_ctx, s, precision=precision)
+            rs.set_alchemy(al, lam)
+            rs.eval(rebuild_list=True)
+            r = rs.results()
+            f.append(r["f"])
+            st.append(r["stress"])
+            dw.append(rs.alchemy_results()["dwrk"])
+            rs.close()
+        out.append((np.array(f), np.array(st), np.array(dw)))
+    # (stress 3.4e-8; 1.9e-7 where a pair's two sides round apart and LJ takes the seed's powers)
+    assert relrms(out[1][1], out[0][1]) < 8e-8
+    print("windows f", relrms(out[1][0], out[0][0]), "stress", relrms(out[1][1], out[0][1]), "dwrk", out[0][2],
+          np.abs(out[1][2] - out[0][2]).max())
