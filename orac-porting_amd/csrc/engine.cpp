@@ -1558,6 +1558,7 @@ extern "C" int orac_hip_system_set_alchemy(orac_hip_ctx *ctx, int32_t sys, const
     S.pair.lj_dense = B.put_vec("aljd", A.lj, st, false);
     S.pair.lj_dense32 = nullptr;
     if (S.precision == 1) {
+      S.pair.sapc = B.get<double4>("sapc", n);  // (its pairs take FP64 separations)
       std::vector<float2> lj32(A.lj.size());
       for (size_t k = 0; k < lj32.size(); ++k) lj32[k] = make_float2((float)A.lj[k].x, (float)A.lj[k].y);
       S.pair.lj_dense32 = B.put_vec("aljd32", lj32, st, false);

@@ -369,13 +369,13 @@ constexpr int SLOT_RING = 256;  // lane slots: at most 63 waiting + one round's 
 constexpr int RED_STRIDE = 72;  // 8 rows of 64 values, rows 16 banks apart
 
 struct PairWave {
-  double gx[ENT_RING], gy[ENT_RING], gz[ENT_RING];  // centre separation, image applied (T = float: {hi, lo} floats)
+  double gx[ENT_RING], gy[ENT_RING], gz[ENT_RING];  // centre separation, image applied (R = float: {hi, lo} floats)
   double sw[ENT_RING], dsw[ENT_RING];               // S and S'(r) / r of the group distance (1 and 0 unswitched)
   int sx[ENT_RING], sy[ENT_RING], sz[ENT_RING];     // image shift (even integers, reduced units)
   int bs[ENT_RING];                                 // sorted first atom | solute neighbour << 26 | shifted << 27
   int tj[ENT_RING];                                 // neighbour group, sorted position
   unsigned short slot[SLOT_RING];                   // entry | atom within the group << 7
-  double4 own[OWN_U];                               // the owner atoms' records (T = float: four floats)
+  double4 own[OWN_U];                               // the owner atoms' records (R = float: four floats)
 };
 static_assert(sizeof(PairWave) >= 8 * RED_STRIDE * sizeof(double), "the lane sums reuse the ring");
 
@@ -437,11 +437,13 @@ enum { PAIR_PLAIN = 0, PAIR_ALCH = 1, PAIR_REM = 2, PAIR_ANY = 3 };
 template <typename T, int MODE>
 __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShared &sh) {
   if (blk >= d.nblk || d.half) return;
-  constexpr bool F32 = sizeof(T) == 4;
+  // Separations and charge products: alchemical systems form them in FP64 and round once, also where
+  // the pair arithmetic is FP32 (a window's dU/dlambda is a small difference of large terms).
+  using R = std::conditional_t<MODE == PAIR_ALCH, double, T>;
+  constexpr bool F32 = sizeof(R) == 4;
   constexpr bool DW = MODE == PAIR_ALCH || MODE == PAIR_REM;  // a 16th sum: dwrk or the segment energy
-  const bool alch = MODE == PAIR_ALCH && d.alch_pair != nullptr;
   if (MODE == PAIR_ALCH) {
-    if (alch && threadIdx.x < 72) sh.alch[threadIdx.x >> 3][threadIdx.x & 7] = gmem(d.alch_fac)[threadIdx.x];
+    if (threadIdx.x < 72) sh.alch[threadIdx.x >> 3][threadIdx.x & 7] = gmem(d.alch_fac)[threadIdx.x];
     __syncthreads();
   }
   // (wave-uniform for the compiler too: the loop control then stays in scalar registers)
@@ -493,7 +495,7 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
 #pragma unroll
       for (int u = 0; u < OWN_U; ++u) {
         const int a = as0 + u0 + min(u, nu - 1);
-        const AtomRec<T> r = atom_rec<T>(d, a);
+        const AtomRec<R> r = atom_rec<R>(d, a);
         if (lane == 0) __builtin_memcpy(&W.own[u], &r, sizeof r);
         ot[u] = uniform(gload_at(d.sai, a).x);
         fr[u][0] = fr[u][1] = fr[u][2] = 0.0;
@@ -585,13 +587,13 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
         const int e = sl & 127, k = sl >> 7;
         const int eb = W.bs[e];
         const int js = (eb & 0x3ffffff) + k;
-        const AtomRec<T> rb = atom_rec<T>(d, js);
+        const AtomRec<R> rb = atom_rec<R>(d, js);
         const int2 ib = gload_at(d.sai, js);
         const double sw = have ? W.sw[e] : 0.0, dsw = have ? W.dsw[e] : 0.0;
-        // separation = owner centre - neighbour centre - image (bx) + owner offset - neighbour offset.  FP32:
-        // the centre separation as hi + lo, and every rounding the same from either side, so that a
-        // pair's two forces cancel exactly and leave no net force to the virial
-        T bx, by, bz, lx, ly, lz;
+        // separation = owner centre - neighbour centre - image (bx) + owner offset - neighbour offset.  FP32
+        // pairs: the centre separation as hi + lo (or FP64), and every rounding the same from either
+        // side, so that a pair's two forces cancel exactly and leave no net force to the virial
+        R bx, by, bz, lx, ly, lz;
         if constexpr (F32) {
           float2 g;
           __builtin_memcpy(&g, &W.gx[e], 8);
@@ -604,17 +606,20 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
           bz = g.x;
           lz = g.y;
         } else {
-          bx = W.gx[e] - rb.x;
-          by = W.gy[e] - rb.y;
-          bz = W.gz[e] - rb.z;
+          bx = W.gx[e];
+          by = W.gy[e];
+          bz = W.gz[e];
+          if constexpr (sizeof(T) == 8) {
+            bx -= rb.x;
+            by -= rb.y;
+            bz -= rb.z;
+          }
         }
         const bool shifted = have && ((eb >> 27) & 1) != 0, solute = ((eb >> 26) & 1) != 0;
         const bool pass_st = __ballot(shifted) != 0ull, pass_solute = __ballot(have && solute) != 0ull;
         const bool pass_ex = __ballot((ib.x & ATOM_EX) != 0) != 0ull;
         any_st = any_st || pass_st;
         const int tb = ib.x >> ATOM_FLAG_BITS;
-        // a pass without alchemical atoms takes the plain form of an alchemical system's pairs
-        const bool soft_b = alch && __ballot(have && (ib.x & ATOM_ALCH)) != 0ull;
         // the first owner atom's LJ entry (a water's only one), requested before the arithmetic that hides it
         T c12a = T(0), c6a = T(0);
         if (ot[0] & ATOM_LJ) pair_lj<T, MODE == PAIR_PLAIN>(d, ot[0] >> ATOM_FLAG_BITS, tb, c12a, c6a);
@@ -625,19 +630,23 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
           for (int u = 0; u < OWN_U; ++u) {
             if (u < nu) {
               const int fl = here(ot[u]);
-              AtomRec<T> ra;
+              AtomRec<R> ra;
               __builtin_memcpy(&ra, &W.own[u], sizeof ra);
               T x, y, z;
-              if constexpr (F32) {
+              if constexpr (sizeof(T) == 8) {
+                x = bx + ra.x;
+                y = by + ra.y;
+                z = bz + ra.z;
+              } else if constexpr (F32) {
                 x = bx + (lx + (ra.x - rb.x));
                 y = by + (ly + (ra.y - rb.y));
                 z = bz + (lz + (ra.z - rb.z));
               } else {
-                x = bx + ra.x;
-                y = by + ra.y;
-                z = bz + ra.z;
+                x = T(bx + (ra.x - rb.x));
+                y = T(by + (ra.y - rb.y));
+                z = T(bz + (ra.z - rb.z));
               }
-              T qq = ra.q * rb.q;
+              T qq = T(ra.q * rb.q);
               bool masked = false;
               const bool heavy = MODE != PAIR_PLAIN && d.any_heavy != 0;
               if (((fl & ATOM_EX) && pass_ex) || heavy) {  // wave-uniform
@@ -654,7 +663,8 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
               }
               T qf, cou, conf;
               double dw = 0.0;
-              if (MODE == PAIR_ALCH && (soft_b || (alch && (fl & ATOM_ALCH)))) {
+              // (per lane: a pair takes the same form from either side)
+              if (MODE == PAIR_ALCH && ((fl | ib.x) & ATOM_ALCH)) {
                 const double4 ap = gload_at(d.alch_pair, (fl >> ATOM_FLAG_BITS) * d.ntypes + tb);
                 const AlchTerms<T> r = alch_terms<T>(d, x, y, z, qq, ap, sh.alch[(int)ap.z]);
                 // (the soft core takes its own parameters)
@@ -834,13 +844,23 @@ __device__ __forceinline__ void pairs_item_index(int h, int nitems, int nblkmax,
   blk = l - sys * nblkmax;
 }
 
+// the item in its system's form: a plain system in a launch with alchemical ones
+// gets what it gets alone
+template <typename T, int MODE>
+__device__ __forceinline__ void pairs_form(const PairDesc &d, int blk, PairShared &sh) {
+  if constexpr (MODE == PAIR_ALCH) {
+    if (!d.alch_pair) return pairs_item<T, PAIR_ANY>(d, blk, sh);
+  }
+  pairs_item<T, MODE>(d, blk, sh);
+}
+
 // W = minimum waves per SIMD the register allocation must allow (occupancy target)
 template <typename T, int W, int MODE>
 __global__ void __launch_bounds__(256, W) k_pairs(const PairDesc *__restrict__ D, int remap) {
   __shared__ PairShared sh;
   int sys, blk;
   pairs_item_index(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y, gridDim.x, remap, sys, blk);
-  pairs_item<T, MODE>(D[sys], blk, sh);
+  pairs_form<T, MODE>(D[sys], blk, sh);
 }
 
 // Persistent form: a fixed grid (a multiple of 8 workgroups, so each keeps to
@@ -852,7 +872,7 @@ __global__ void __launch_bounds__(256, W) k_pairs_persistent(const PairDesc *__r
   for (int h = blockIdx.x; h < nitems; h += gridDim.x) {
     int sys, blk;
     pairs_item_index(h, nitems, nblkmax, remap, sys, blk);
-    pairs_item<T, MODE>(D[sys], blk, sh);
+    pairs_form<T, MODE>(D[sys], blk, sh);
     __syncthreads();
   }
 }
@@ -1357,7 +1377,8 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
     // every system's groups are packed and its blocks launched, whichever form serves it
     max_grp = std::max(max_grp, h[s].ngrp);
     max_blk = std::max(max_blk, h[s].nblk);
-    if (sizeof(T) == 4 ? !h[s].sapf : !h[s].sapc) throw Error(E_STATE, "no atom records in this precision");
+    if ((sizeof(T) == 4 && !h[s].sapf) || ((sizeof(T) == 8 || h[s].alch_pair) && !h[s].sapc))
+      throw Error(E_STATE, "no atom records in this precision");
     if (h[s].half) {
       if (h[s].alch_pair || h[s].rematom || h[s].split != 1 || h[s].max_group > OWN_REG)
         throw Error(E_STATE, "half-list pair form on a system it does not serve");

@@ -90,7 +90,7 @@ struct PairDesc {
   double4 *sgp;                     // [ngrp] {xpg, ypg, zpg, two ints: sorted first atom, natoms | gss << 8}
   int4 *sgi;                        // half form: [ngrp] {sorted first atom, first atom, natoms | gss << 8, group}
   float4 *sapf;                     // [natoms] {Cartesian offset from the group centre, q}: mixed-precision pairs
-  double4 *sapc;                    // [natoms] the same in FP64 (FP64 pairs)
+  double4 *sapc;                    // [natoms] the same in FP64: FP64 pairs, and the pairs of alchemical systems
   // Half-list form (half = 1, split list layout): the list holds each group
   // pair once (forward entries, upper group l > owner); the forces on the
   // neighbour's atoms go to per-pair slots, mirror[t * nb_slab + e] the first

@@ -35,9 +35,10 @@ def _direct(ctx, s, precision, alchemy=None):
     return _eval(ctx, s, precision, alchemy)["f"] - _eval(ctx, far, precision, alchemy)["f"]
 
 
+@pytest.mark.parametrize("alchemical", [False, True])
 @pytest.mark.parametrize("charges", [False, True])
 @pytest.mark.parametrize("name", ["waters", "mixed", "seven_one"])
-def test_pair_forces_cancel(gpu_ctx, name, charges):
+def test_pair_forces_cancel(gpu_ctx, name, charges, alchemical):
     """Both sides of a pair round alike in FP32, so the direct forces sum to
     zero but for the FP64 sums (1,728 atoms of ~100 terms each: a few hundred
     roundings of 1e-16 of the largest; a single FP32 rounding is 6e-8)."""
@@ -45,7 +46,7 @@ def test_pair_forces_cancel(gpu_ctx, name, charges):
     s = grouped(**CASES[name])
     if not charges:
         s = dataclasses.replace(s, charge=0.0 * s.charge)
-    f = _direct(gpu_ctx, s, 1)
+    f = _direct(gpu_ctx, s, 1, _removed(s) if alchemical else None)
     assert np.abs(f.sum(axis=1)).max() < 1e-12 * np.abs(f).max()
 
 
