@@ -742,7 +742,8 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
           gy = W.gy[e];
           gz = W.gz[e];
         }
-        const double v = -dsw * (MODE == PAIR_REM ? vr : vc + vq);
+        // (unswitched pairs have no such term, also where two atoms coincide and their energy is not finite)
+        const double v = dsw != 0.0 ? -dsw * (MODE == PAIR_REM ? vr : vc + vq) : 0.0;
         x3[0] = fma(v, gx, x3[0]);
         x3[1] = fma(v, gy, x3[1]);
         x3[2] = fma(v, gz, x3[2]);

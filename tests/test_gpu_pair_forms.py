@@ -130,3 +130,26 @@ def test_half_list_transpose(gpu_ctx, water216, ngrp):
     o = O.force(s, nnlpp, fa=fa, **kw)
     assert np.abs(g["f"] - o["f"]).max() <= F_TOL * max(np.abs(o["f"]).max(), 1e-300)
     assert _stress_close(g["stress"], o["stress"])
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_coincident_atoms_spoil_their_own_forces_only(gpu_ctx, precision):
+    """Two atoms of different groups at one point have no finite force; the other
+    atoms of their groups do (within the switching range alone a group pair's
+    energy enters the forces of all its atoms), so that a relaxation can move them."""
+    from orac_hip.api import ResidentSystem
+    s = grouped(sizes=[3])
+    # the third atoms of the first group and of its neighbour along y
+    x = [np.array(v) for v in (s.xp0, s.yp0, s.zp0)]
+    for v in x:
+        v[14] = v[2]
+    t = s.nbtype.copy()
+    t[[2, 14]] = 1  # (a type with LJ: r^-12 overflows FP32)
+    s = dataclasses.replace(s, xp0=x[0], yp0=x[1], zp0=x[2], nbtype=t)
+    rs = ResidentSystem(gpu_ctx, s, precision=precision)
+    rs.eval()
+    f = rs.results()["f"]
+    rs.close()
+    bad = np.flatnonzero(~np.isfinite(f).all(axis=0)).tolist()
+    # (FP64 leaves a distance of its rounding between them, and a force of 1e200)
+    assert bad == [2, 14] if precision == 1 else set(bad) <= {2, 14}
