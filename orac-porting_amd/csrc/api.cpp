@@ -347,6 +347,7 @@ extern "C" int orac_hip_fft_pme_noalloc(orac_hip_ctx *ctx, int32_t ntap, const d
     }
     double *dout = B.get<double>("p_out", 40);
     d.out = dout;
+    pme_bins(B, "p_", d, ctx->tuning, st);  // (last: they take what room is left)
     PmeDesc *dd = B.put("p_desc", &d, 1, st, false);
     launch_pme<double>(dd, &d, 1, st, ctx->tuning);
     ORAC_HIP(hipGetLastError());

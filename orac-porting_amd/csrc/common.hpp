@@ -82,6 +82,7 @@ struct PmeDesc {
   double4 *bin_fr;              // [nb1*nb2*nb3][bin_cap] {fr1, fr2, fr3, q} of each bin's atoms
   double4 *over_fr;             // [natoms] the same of the atoms beyond their bin's capacity
   int bin_cap;
+  double bin_slots;             // slots allocated at bin_fr (0: not yet)
   int tiled;                    // 1: LDS-tiled spread, 0: global-atomic spread
   double *out;                  // [20]: eer, vir (3x3 col-major), stc1..stc9
   int energy_only;              // 1: spread, forward FFT and energy only (a lambda0 charge grid)

@@ -299,9 +299,9 @@ CellGrid make_cellgrid(BufSet &B, const std::string &pfx, int ncx, int ncy, int 
 // Spread tiles of the largest or smallest edges the grid admits, and the room
 // of their bins: 1.5 x the mean, or 0.2 atoms per cubic A of the tile (above
 // any liquid's or solid's density, so that vacuum elsewhere does not fill a
-// bin), at most about twice the atoms in all.  Atoms beyond it go through the
-// overflow list, which every tile reads.
-static void pme_tiling(PmeDesc &d, bool smallest) {
+// bin), at most 2 x the mean + 48 a bin, and at most what is allocated.  Atoms
+// beyond it go through the overflow list, which every tile reads.
+void pme_tiling(PmeDesc &d, bool smallest) {
   d.st1 = spread_tile_edge(d.K1, d.order, smallest);
   d.st2 = spread_tile_edge(d.K2, d.order, smallest);
   d.st3 = spread_tile_edge(d.K3, d.order, smallest);
@@ -311,10 +311,42 @@ static void pme_tiling(PmeDesc &d, bool smallest) {
   const double nbin = (double)d.nb1 * d.nb2 * d.nb3, mean = d.natoms / nbin;
   const double want = std::max(1.5 * mean, 0.2 * d.volume / nbin) + 16.0;
   d.bin_cap = (int)std::min({want, 2.0 * mean + 48.0, (double)std::max(1, d.natoms)});
+  if (d.bin_slots > 0) d.bin_cap = (int)std::min<double>(d.bin_cap, std::floor(d.bin_slots / nbin));
+}
+
+// The spread's bins, when every axis has a tile edge in [order - 1, 8] dividing
+// K: sized for the largest and the smallest tiles, which a tuning may ask for.
+// In an arena, of which they take the last pieces, sized for the tiling in use
+// and for what is left beside the descriptor.
+void pme_bins(BufSet &B, const std::string &pfx, PmeDesc &d, const Tuning &tu, hipStream_t st) {
+  if (!(spread_tile_edge(d.K1, d.order, true) && spread_tile_edge(d.K2, d.order, true) &&
+        spread_tile_edge(d.K3, d.order, true)))
+    return;
+  size_t nbin = 0, slots = 1;
+  for (const bool smallest : {false, true}) {
+    if (B.arena && smallest != (tu.spread_tiled == 2)) continue;
+    pme_tiling(d, smallest);
+    const size_t n = (size_t)d.nb1 * d.nb2 * d.nb3;
+    nbin = std::max(nbin, n);
+    slots = std::max(slots, n * d.bin_cap);
+  }
+  const size_t ncnt = (nbin + 2) / 2 * 2, nover = (size_t)std::max(1, d.natoms);
+  if (B.arena) {
+    const size_t other = ncnt * sizeof(int) + nover * sizeof(double4) + 2 * sizeof(PmeDesc) + 4 * 256;
+    if (B.room() < other + sizeof(double4)) return;  // (the atomic spread)
+    slots = std::min(slots, (B.room() - other) / sizeof(double4));
+  }
+  d.bin_cnt = B.get<int>(pfx + "bin_cnt", ncnt);
+  launch_zero_u64(reinterpret_cast<unsigned long long *>(d.bin_cnt), ncnt / 2, st);
+  d.over_fr = B.get<double4>(pfx + "over_fr", nover);
+  d.bin_fr = B.get<double4>(pfx + "bin_fr", slots);
+  d.bin_slots = (double)slots;
+  pme_apply_tuning(d, tu);
 }
 
 // Device PME descriptor of one system: grids, B-spline moduli, partial-sum
-// buffers sized for any tuning, spread bins when the grid admits tiles.
+// buffers sized for any tuning, spread bins when the grid admits tiles (in an
+// arena the caller adds them when all else is in place).
 PmeDesc pme_desc_base(BufSet &B, const std::string &pfx, const PmePlan &P, int natoms, const double *oc,
                       double volume, double alpha, double rkcut, bool fp64, const Tuning &tu, hipStream_t st) {
   PmeDesc d;
@@ -344,23 +376,8 @@ PmeDesc pme_desc_base(BufSet &B, const std::string &pfx, const PmePlan &P, int n
   // one K3 pencil per workgroup is the most blocks any tiling uses
   d.conv_part = B.get<double>(pfx + "conv_part", (size_t)H * P.K2 * 8);
   d.gather_part = B.get<double>(pfx + "gather_part", (size_t)std::max(1, (natoms + 31) / 32) * 9);
-  // LDS-tiled spread when every axis has a tile edge in [order-1, 8] dividing K;
-  // the bins are sized for the smallest tiles (the most bins any tuning uses)
-  const int e1 = spread_tile_edge(P.K1, P.order, true), e2 = spread_tile_edge(P.K2, P.order, true),
-            e3 = spread_tile_edge(P.K3, P.order, true);
-  if (e1 && e2 && e3) {
-    const size_t nbin = (size_t)(P.K1 / e1) * (P.K2 / e2) * (P.K3 / e3);
-    size_t slots = 0;
-    for (const bool smallest : {false, true}) {
-      pme_tiling(d, smallest);
-      slots = std::max(slots, (size_t)d.nb1 * d.nb2 * d.nb3 * d.bin_cap);
-    }
-    d.bin_cnt = B.get<int>(pfx + "bin_cnt", (nbin + 2) / 2 * 2);
-    launch_zero_u64(reinterpret_cast<unsigned long long *>(d.bin_cnt), (nbin + 2) / 2, st);
-    d.bin_fr = B.get<double4>(pfx + "bin_fr", std::max<size_t>(1, slots));
-    d.over_fr = B.get<double4>(pfx + "over_fr", std::max(1, natoms));
-  }
   pme_apply_tuning(d, tu);
+  if (!B.arena) pme_bins(B, pfx, d, tu, st);
   return d;
 }
 
@@ -372,7 +389,8 @@ void pme_apply_tuning(PmeDesc &d, const Tuning &tu) {
   d.tiled = 0;
   if (!d.bin_cnt || !tu.spread_tiled || std::getenv("ORAC_HIP_SPREAD_ATOMIC")) return;
   pme_tiling(d, tu.spread_tiled == 2);
-  d.tiled = 1;
+  // (where the bins' room is short of the atoms, most would go through the overflow list)
+  d.tiled = (double)d.bin_cap * d.nb1 * d.nb2 * d.nb3 >= d.natoms ? 1 : 0;
 }
 
 double erfc_as(double x) {

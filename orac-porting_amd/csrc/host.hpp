@@ -60,6 +60,10 @@ struct BufSet {
     return s;
   }
   void reset() { arena_used = 0; }
+  size_t room() const {  // of an arena, past the alignment of the next piece
+    const size_t off = (arena_used + 255) & ~(size_t)255;
+    return off < arena_cap ? arena_cap - off : 0;
+  }
   template <class T>
   T *get(const std::string &name, size_t n) {
     if (arena) {
@@ -113,6 +117,9 @@ void build_pme_plan(BufSet &B, const std::string &pfx, PmePlan &P, int k1, int k
 // descriptor of one system's reciprocal sum with its grids and partial-sum buffers
 PmeDesc pme_desc_base(BufSet &B, const std::string &pfx, const PmePlan &P, int natoms, const double *oc,
                       double volume, double alpha, double rkcut, bool fp64, const Tuning &tu, hipStream_t st);
+// the spread's bins of a descriptor (pme_desc_base adds them unless B is an arena)
+void pme_bins(BufSet &B, const std::string &pfx, PmeDesc &d, const Tuning &tu, hipStream_t st);
+void pme_tiling(PmeDesc &d, bool smallest);
 // apply the tuning's FFT tiling and spread path to a descriptor built by pme_desc_base
 void pme_apply_tuning(PmeDesc &d, const Tuning &tu);
 std::vector<int4> stencil_runs(const std::vector<int> &sten, int ncx, int ncy, int ncz);

@@ -41,6 +41,28 @@ def test_noalloc_matches_fft_pme_two_calls(gpu_ctx):
         assert rel(e_na, e_ref) == 0.0
 
 
+@pytest.mark.parametrize("natoms,nfft,order,L", [
+    (65536, (64, 64, 64), 3, 87.0),     # the largest call, at liquid density
+    (65536, (64, 64, 64), 3, 200.0),    # and thin
+    (65536, (64, 64, 64), 5, 87.0),
+    (65536, (64, 64, 64), 8, 87.0),
+    (65536, (81, 81, 36), 3, 87.0),     # the most tiles of the largest edge the grid admits (3 along K1, K2)
+    (65536, (243, 243, 4), 3, 87.0),
+    (2000, (81, 81, 36), 4, 300.0),     # more tiles than atoms
+])
+def test_noalloc_takes_what_the_region_promises(gpu_ctx, natoms, nfft, order, L):
+    """65,536 atoms and 64^3 points fit the region at every order and tiling, bit for bit as with allocation."""
+    from test_gpu_spread_forms import _random
+    s = _random(n=natoms, nfft=nfft, order=order, L=L)
+    gpu_ctx.fft_pme_init(s.natoms, *s.nfft, s.order)
+    zero, st0 = np.zeros((3, s.natoms)), np.zeros((3, 3))
+    e_ref, f_ref, st_ref = _call(gpu_ctx, s, False, zero, st0)
+    e_na, f_na, st_na = _call(gpu_ctx, s, True, zero, st0)
+    assert e_na == e_ref
+    assert np.array_equal(f_na, f_ref)
+    assert np.array_equal(st_na, st_ref)
+
+
 def test_noalloc_rejects_sizes_beyond_the_region(gpu_ctx):
     from orac_hip import synth
     from orac_hip.api import OracHipError
