@@ -748,8 +748,25 @@ static int batch_create(orac_hip_ctx *ctx, const int32_t *ids, int n) {
   return id;
 }
 
+// Everything an evaluation would refuse, before its first launch: the preparing
+// launch fills the spread's bins, which only the transforms empty, and a step of
+// dynamics has moved the atoms by then.
+static void batch_check(const Batch &b, bool rebuild, bool md_lists) {
+  const int n = (int)b.sys.size();
+  if (md_lists || rebuild) {
+    const std::vector<ListDesc> &hl = md_lists ? b.hl_md : b.hl;
+    check_list_build(hl.data(), n, LIST_COUNT | LIST_WRITE);
+    if (b.shells) check_list_inner(hl.data(), n);
+  }
+  for (const std::vector<PairDesc> *q : {&b.hq, &b.hqm}) {
+    if (b.precision == 0) check_pairs<double>(q->data(), (int)q->size());
+    else check_pairs<float>(q->data(), (int)q->size());
+  }
+}
+
 // the stages of one force evaluation of every system in the batch
 static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events, bool md_lists = false) {
+  batch_check(b, rebuild, md_lists);
   hipStream_t st = ctx->stream;
   const int n = (int)b.sys.size();
   const int npme = (int)b.hp.size();
@@ -1291,6 +1308,7 @@ static void md_run(orac_hip_ctx *ctx, Batch &b, int nsteps, double dt, int nmid,
     b.md_nmid = nmid;
   }
   hipStream_t st = ctx->stream;
+  batch_check(b, true, true);
   if (nsteps > 0) md_start(ctx, b, dt, nmid, ninner, nsteps);
   for (int s = 0; s < nsteps; ++s) {
     if (use_graph) {

@@ -1369,8 +1369,29 @@ bool use_owner_kernel() {
 }
 
 template <typename T>
+void check_pairs(const PairDesc *h, int nsys) {
+  bool any_alch = false, any_rem = false;
+  for (int s = 0; s < nsys; ++s) {
+    if ((sizeof(T) == 4 && !h[s].sapf) || ((sizeof(T) == 8 || h[s].alch_pair) && !h[s].sapc))
+      throw Error(E_STATE, "no atom records in this precision");
+    if (h[s].half) {
+      if (h[s].alch_pair || h[s].rematom || h[s].split != 1 || h[s].max_group > OWN_REG)
+        throw Error(E_STATE, "half-list pair form on a system it does not serve");
+      continue;
+    }
+    any_alch = any_alch || h[s].alch_pair != nullptr;
+    any_rem = any_rem || h[s].rematom != nullptr;
+    if (h[s].max_group > 64)
+      throw Error(E_UNSUPPORTED, "groups larger than 64 atoms are not supported by the pair kernel");
+  }
+  if (any_alch && any_rem) throw Error(E_STATE, "alchemical and REM systems in one launch");
+  if (any_rem && sizeof(T) == 4) throw Error(E_STATE, "REM pairs are evaluated in double precision");
+}
+
+template <typename T>
 void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream_t st, const Tuning &tu,
                   bool packed, bool finalize, hipEvent_t kbeg, hipEvent_t kend) {
+  check_pairs<T>(h, nsys);
   int max_grp = 1, max_blk = 1;
   // half-list systems take the half form, the others k_pairs
   bool any_alch = false, any_rem = false, any_other = false, any_half = false, any_full = false;
@@ -1378,11 +1399,7 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
     // every system's groups are packed and its blocks launched, whichever form serves it
     max_grp = std::max(max_grp, h[s].ngrp);
     max_blk = std::max(max_blk, h[s].nblk);
-    if ((sizeof(T) == 4 && !h[s].sapf) || ((sizeof(T) == 8 || h[s].alch_pair) && !h[s].sapc))
-      throw Error(E_STATE, "no atom records in this precision");
     if (h[s].half) {
-      if (h[s].alch_pair || h[s].rematom || h[s].split != 1 || h[s].max_group > OWN_REG)
-        throw Error(E_STATE, "half-list pair form on a system it does not serve");
       any_half = true;
       continue;
     }
@@ -1390,8 +1407,6 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
     any_alch = any_alch || h[s].alch_pair != nullptr;
     any_rem = any_rem || h[s].rematom != nullptr;
     any_other = any_other || h[s].lskip_ewald || h[s].any_heavy || !h[s].lj_dense;
-    if (h[s].max_group > 64)
-      throw Error(E_UNSUPPORTED, "groups larger than 64 atoms are not supported by the pair kernel");
   }
   if (!packed) hipLaunchKernelGGL(k_pack_sorted, dim3((max_grp + 255) / 256, nsys), dim3(256), 0, st, d_desc);
   dim3 grd(max_blk, nsys);
@@ -1424,13 +1439,10 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
     // (every system in the half-list form)
   } else if (any_alch) {
     // the soft-core form at the default occupancy target only
-    if (any_rem) throw Error(E_STATE, "alchemical and REM systems in one launch");
     launch_pair_kernel<T, 3, PAIR_ALCH>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
   } else if (any_rem) {
-    if constexpr (sizeof(T) == 8)
+    if constexpr (sizeof(T) == 8)  // (check_pairs)
       launch_pair_kernel<T, 3, PAIR_REM>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
-    else
-      throw Error(E_STATE, "REM pairs are evaluated in double precision");
   } else if (any_other) {
     launch_pair_kernel<T, 3, PAIR_ANY>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
   } else {
@@ -1444,6 +1456,8 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
   if (finalize) hipLaunchKernelGGL(k_pairs_finalize, dim3(PAIR_NACC, nsys), dim3(1024), 0, st, d_desc);
 }
 
+template void check_pairs<double>(const PairDesc *, int);
+template void check_pairs<float>(const PairDesc *, int);
 template void launch_pairs<double>(const PairDesc *, const PairDesc *, int, hipStream_t, const Tuning &, bool, bool,
                                    hipEvent_t, hipEvent_t);
 template void launch_pairs<float>(const PairDesc *, const PairDesc *, int, hipStream_t, const Tuning &, bool, bool,

@@ -174,6 +174,9 @@ __device__ inline void pack_atom(const PairDesc &d, int s, int a, double gx, dou
   if (d.sapf) gstore(d.sapf + s, make_float4((float)cx, (float)cy, (float)cz, (float)q));
 }
 
+// throws what launch_pairs would refuse, before anything is launched
+template <typename T>
+void check_pairs(const PairDesc *h, int nsys);
 // packed: the systems' records are in place (launch_centres with pack).
 // finalize: reduce the partial sums (else launch_tail does).
 // kbeg/kend (optional) are recorded right before and after the pair kernel itself
@@ -277,6 +280,9 @@ enum ListPhase { LIST_COUNT = 1, LIST_WRITE = 2, LIST_ZERO = 4 };
 // LIST_ZERO: the counters; LIST_COUNT: cells, per-group counts, offsets and the capacity check;
 // LIST_WRITE: the entries.  On overflow total[1] = 1 and nothing is written.
 void launch_list_build(const ListDesc *d_desc, const ListDesc *h, int nsys, int phases, hipStream_t st);
+// throw what the launches below would refuse, before anything is launched
+void check_list_build(const ListDesc *h, int nsys, int phases);
+void check_list_inner(const ListDesc *h, int nsys);
 // the inner lists of a batch's systems after a slab-layout build (systems with r2m > 0)
 void launch_list_inner(const ListDesc *d_desc, const ListDesc *h, int nsys, hipStream_t st);
 // dense {ecc12, ecc6} table (and its FP32 copy if dense32) and the types' flags from the packed

@@ -673,6 +673,7 @@ __device__ inline int2 list_walk_split(int n, const ListDesc &d, int *outf, int 
 // Split slab layout: the walk, then the reverse entries ranked in LDS by group
 // number (distinct) and stored in ascending order, as group numbers.
 // Dynamic LDS: one slab of ints per wavefront.
+static size_t split_lds(int slab) { return (size_t)4 * slab * sizeof(int); }
 __global__ void __launch_bounds__(256) k_list_write_split(const ListDesc *__restrict__ D) {
   extern __shared__ int lrev_all[];
   const ListDesc &d = D[blockIdx.y];
@@ -806,20 +807,29 @@ __global__ void __launch_bounds__(1024) k_list_total(const ListDesc *__restrict_
   list_total(D[blockIdx.x], split_written != 0);
 }
 
+// a batch uses one layout: all slab (resident systems) or none (plain lc_list);
+// slab systems may mix the split and the plain slab layouts
+void check_list_build(const ListDesc *h, int nsys, int phases) {
+  for (int s = 0; s < nsys; ++s) {
+    if ((h[s].slab > 0) != (h[0].slab > 0) || h[s].mode != h[0].mode)
+      throw Error(E_STATE, "list layouts differ within a batch");
+    if ((phases & LIST_WRITE) && h[s].mode == 0 && h[s].slab > 0 && h[s].split && split_lds(h[s].slab) > 65536)
+      throw Error(E_CAPACITY, "neighbour-list slab too large for the split layout's LDS sort");
+  }
+}
+
 void launch_list_build(const ListDesc *d_desc, const ListDesc *h, int nsys, int phases, hipStream_t st) {
+  check_list_build(h, nsys, phases);
   int max_cell = 1, max_grp = 1;
   for (int s = 0; s < nsys; ++s) {
     max_cell = std::max(max_cell, h[s].cg.ncx * h[s].cg.ncy * h[s].cg.ncz + 1);  // + the parking cell
     max_grp = std::max(max_grp, h[s].ngrp);
   }
   const dim3 b(256), gg((max_grp + 255) / 256, nsys), gw((max_grp + 3) / 4, nsys);
-  // a batch uses one layout: all slab (resident systems) or none (plain lc_list);
-  // slab systems may mix the split and the plain slab layouts
   const bool slab = h[0].slab > 0;
   bool any_split = false, any_plain = false;
   int max_slab = 0;
   for (int s = 0; s < nsys; ++s) {
-    if ((h[s].slab > 0) != slab || h[s].mode != h[0].mode) throw Error(E_STATE, "list layouts differ within a batch");
     if (h[s].split) {
       any_split = true;
       max_slab = std::max(max_slab, h[s].slab);
@@ -858,9 +868,7 @@ void launch_list_build(const ListDesc *d_desc, const ListDesc *h, int nsys, int 
     else if (layout == LW_SLAB) {
       if (any_plain) hipLaunchKernelGGL(k_list_write<LW_SLAB>, gw, b, 0, st, d_desc);
       if (any_split) {
-        const size_t shm = (size_t)4 * max_slab * sizeof(int);
-        if (shm > 65536) throw Error(E_CAPACITY, "neighbour-list slab too large for the split layout's LDS sort");
-        hipLaunchKernelGGL(k_list_write_split, gw, b, shm, st, d_desc);
+        hipLaunchKernelGGL(k_list_write_split, gw, b, split_lds(max_slab), st, d_desc);
       }
     } else {
       hipLaunchKernelGGL(k_list_write<LW_CSR>, gw, b, 0, st, d_desc);
@@ -904,12 +912,15 @@ __global__ void __launch_bounds__(256) k_list_inner(const ListDesc *__restrict__
   if (lane == 0) d.count_m[o] = w;
 }
 
-void launch_list_inner(const ListDesc *d_desc, const ListDesc *h, int nsys, hipStream_t st) {
-  int max_grp = 1;
-  for (int s = 0; s < nsys; ++s) {
+void check_list_inner(const ListDesc *h, int nsys) {
+  for (int s = 0; s < nsys; ++s)
     if (h[s].r2m > 0.0 && (h[s].slab <= 0 || h[s].split)) throw Error(E_STATE, "inner lists need the plain slab layout");
-    max_grp = std::max(max_grp, h[s].ngrp);
-  }
+}
+
+void launch_list_inner(const ListDesc *d_desc, const ListDesc *h, int nsys, hipStream_t st) {
+  check_list_inner(h, nsys);
+  int max_grp = 1;
+  for (int s = 0; s < nsys; ++s) max_grp = std::max(max_grp, h[s].ngrp);
   hipLaunchKernelGGL(k_list_inner, dim3((max_grp + 3) / 4, nsys), dim3(256), 0, st, d_desc);
 }
 

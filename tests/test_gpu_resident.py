@@ -215,3 +215,32 @@ def test_owner_form_mixed_batch_equals_alone(gpu_ctx, monkeypatch):
     b.close()
     for x in systems:
         x.close()
+
+
+def test_refused_evaluation_leaves_nothing_behind(gpu_ctx, water216, monkeypatch):
+    """A batch that is refused (one system's list is beyond the half-list form's
+    sort) launches nothing: the other system's reciprocal sum, whose atoms are
+    binned by an evaluation's first launch, is what it was."""
+    import dataclasses
+
+    from orac_hip.api import Batch, OracHipError, ResidentSystem
+    from test_gpu_spread_forms import _random
+    monkeypatch.setenv("ORAC_HIP_PAIR_KERNEL", "own")
+    big = _random(n=5200, nfft=(24, 24, 24), order=4, L=30.0)
+    big = dataclasses.replace(big, rcut=14.0, rtol=0.3, rnei=0.6)
+    a, b = ResidentSystem(gpu_ctx, water216), ResidentSystem(gpu_ctx, big)
+    a.eval(rebuild_list=True)
+    want = a.results()
+    batch = Batch(gpu_ctx, [a, b])
+    for stages_timed in (True, False):
+        batch.profile(stages_timed)
+        for graph in (False, True):
+            with pytest.raises(OracHipError) as e:
+                batch.eval(rebuild_list=True, graph=graph)
+            assert e.value.code == 2
+    batch.close()
+    a.eval(rebuild_list=True)
+    got = a.results()
+    assert got["eer"] == want["eer"] and np.array_equal(got["f"], want["f"])
+    a.close()
+    b.close()
