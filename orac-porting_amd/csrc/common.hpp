@@ -387,10 +387,17 @@ __device__ inline void bin_atom(const PmeDesc &d, int a) {
   base = __shfl(base, leader, 64);
   if (bin < 0) return;
   const int pos = base + __popcll(mine & ((1ull << lane) - 1ull));
-  if (pos < d.bin_cap)
+  if (pos < d.bin_cap) {
     gstore(d.bin_fr + (size_t)bin * d.bin_cap + pos, f);
-  else
-    gstore(d.over_fr + atomicAdd(&d.bin_cnt[d.nb1 * d.nb2 * d.nb3], 1), f);
+    return;
+  }
+  // the wavefront's atoms beyond their bins' room: one atomic on the list's count
+  const unsigned long long over = __ballot(1);
+  const int first = __ffsll((long long)over) - 1;
+  int at = 0;
+  if (lane == first) at = atomicAdd(&d.bin_cnt[d.nb1 * d.nb2 * d.nb3], __popcll(over));
+  at = __builtin_amdgcn_readlane(at, first) + lanes_below(over);
+  gstore(d.over_fr + at, f);
 }
 
 // lane J of each group of four lanes, to all four

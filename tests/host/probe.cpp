@@ -20,3 +20,18 @@ extern "C" void probe_run_cells(int k, int z0, int z1, int n, int *out) {
   const int v[4] = {r.a0, r.b0, r.a1, r.b1};
   std::copy(v, v + 4, out);
 }
+
+// room of one spread bin, and the tiles, for the largest or smallest tiles
+extern "C" int probe_bin_cap(const int *K, int order, int natoms, double volume, int smallest, int *nbin) {
+  PmeDesc d;
+  std::memset(&d, 0, sizeof d);
+  d.K1 = K[0];
+  d.K2 = K[1];
+  d.K3 = K[2];
+  d.order = order;
+  d.natoms = natoms;
+  d.volume = volume;
+  pme_tiling(d, smallest != 0);
+  *nbin = d.nb1 * d.nb2 * d.nb3;
+  return d.bin_cap;
+}

@@ -74,3 +74,21 @@ def test_stencil_runs_are_the_stencil(probe, name):
             cells += [(dx, dy, z) for z in (*range(a0, b0), *range(a1, b1))]
         want = [(dx, dy, (k + dz) % nc[2]) for dx, dy, dz in sten.tolist()]
         assert sorted(cells) == sorted(want)
+
+
+@pytest.mark.parametrize("smallest", [0, 1])
+@pytest.mark.parametrize("order", [3, 4, 5, 6, 8])
+@pytest.mark.parametrize("n,L,K", [(24000, 62.0, 64), (24000, 124.0, 96), (24000, 186.0, 144), (24000, 250.0, 160),
+                                   (24000, 250.0, 200), (648, 18.6, 20), (648, 80.0, 64), (3, 40.0, 32)])
+def test_spread_bins_hold_a_droplet(probe, n, L, K, order, smallest):
+    """Every bin has room for a condensed phase (0.13 atoms per cubic A) wherever
+    it lies in the box, and all bins together take no more than the grids or a
+    fixed amount per atom and tile."""
+    from math import ceil
+    if not any(K % e == 0 for e in range(max(2, order - 1), 9)):
+        pytest.skip("no tile edge")
+    nbin = C.c_int()
+    probe.probe_bin_cap.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_double, C.c_int, C.c_void_p]
+    cap = probe.probe_bin_cap(_ptr(np.array([K] * 3, np.int32)), order, n, L ** 3, smallest, C.byref(nbin))
+    assert cap >= min(n, ceil(0.13 * L ** 3 / nbin.value))
+    assert cap * nbin.value <= max(2 * n + 48 * nbin.value, K ** 3)
