@@ -696,6 +696,7 @@ static int force_impl(orac_hip_ctx *ctx, const int32_t *ss_index, const double *
     p.sapc = B.get<double4>("f_sapc", std::max(1, nato));
     p.sai = B.get<int2>("f_sai", std::max(1, nato));
     p.max_group = max_group;
+    p.many = pair_many_for(nato, ngrp);
     if (rem) {
       std::vector<int> rf(nato);
       for (int a = 0; a < nato; ++a) rf[a] = rem->rematom[a] != 0;

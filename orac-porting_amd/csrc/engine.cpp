@@ -506,6 +506,7 @@ static void system_build(orac_hip_ctx *ctx, System &S, const orac_hip_system_des
   p.sai = B.get<int2>("sai", n);
   p.out = S.out + 20;
   p.max_group = S.max_group;
+  p.many = pair_many_for(n, ng);
 
   // ---- linked cells and the full list
   ListDesc &L = S.list;

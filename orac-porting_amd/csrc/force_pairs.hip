@@ -363,11 +363,12 @@ constexpr int PAIR_NACC = 16;      // energies and virial of a block: uconf[3], 
 // atom, neighbour group) that recomputed the group geometry per lane; 26 M
 // vector instructions against 43 M.  16 systems in one launch: 56 us each (FP32).
 
-constexpr int OWN_U = 3;        // owner atoms whose sums stay in registers during a list walk
 constexpr int ENT_RING = 128;   // entries kept: at most 63 with atoms waiting + 64 new ones
 constexpr int SLOT_RING = 256;  // lane slots: at most 63 waiting + one round's atoms
 constexpr int RED_STRIDE = 72;  // 8 rows of 64 values, rows 16 banks apart
 
+// U: owner atoms whose sums stay in registers during a list walk
+template <int U>
 struct PairWave {
   double gx[ENT_RING], gy[ENT_RING], gz[ENT_RING];  // centre separation, image applied (R = float: {hi, lo} floats)
   double sw[ENT_RING], dsw[ENT_RING];               // S and S'(r) / r of the group distance (1 and 0 unswitched)
@@ -375,12 +376,13 @@ struct PairWave {
   int bs[ENT_RING];                                 // sorted first atom | solute neighbour << 26 | shifted << 27
   int tj[ENT_RING];                                 // neighbour group, sorted position
   unsigned short slot[SLOT_RING];                   // entry | atom within the group << 7
-  double4 own[OWN_U];                               // the owner atoms' records (R = float: four floats)
+  double4 own[U];                                   // the owner atoms' records (R = float: four floats)
 };
-static_assert(sizeof(PairWave) >= 8 * RED_STRIDE * sizeof(double), "the lane sums reuse the ring");
+static_assert(sizeof(PairWave<1>) >= 8 * RED_STRIDE * sizeof(double), "the lane sums reuse the ring");
 
+template <int U>
 struct PairShared {
-  PairWave w[PAIR_WAVES];
+  PairWave<U> w[PAIR_WAVES];
   double fsum[PAIR_WAVES][64][3];          // owner-atom forces of a wave's part of the list
   double red[PAIR_WAVES][3 + PAIR_NACC];   // S'V vector, then energies and virial
   double alch[9][8];                       // the system's soft-core factors (alchemical kernels)
@@ -433,10 +435,20 @@ __device__ __forceinline__ AtomRec<T> atom_rec(const PairDesc &d, int s) {
 // (an outer shell that skips the Ewald term, more than LJ_DENSE_MAX types).
 enum { PAIR_PLAIN = 0, PAIR_ALCH = 1, PAIR_REM = 2, PAIR_ANY = 3 };
 
+// Owner atoms a list walk takes (their sums stay in registers).  Three suit
+// waters and charge groups of a few atoms; groups of dozens of atoms walk their
+// list again for every three and have so few owners that eight at half the
+// occupancy are better.  13,824 to 21,952 atoms, us with 3 and with 8 (FP64;
+// FP32), and before the lanes took the neighbours: groups of 6 atoms 64 71 (88);
+// 54 62 (58), of 8 80 80 (80); 68 68 (64), of 12 115 92 (107); 103 80 (90), of 16
+// 178 121 (148); 161 102 (123), of 64 1,530 900 (1,046); 1,458 836 (919).
+constexpr int OWN_FEW = 3, OWN_MANY = 8;
+int pair_many_for(int natoms, int ngrp) { return (long long)natoms > 8ll * ngrp ? 1 : 0; }
+
 // One work item: block blk of system d (PAIR_WAVES waves, split of them per owner group).
-template <typename T, int MODE>
-__device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShared &sh) {
-  if (blk >= d.nblk || d.half) return;
+template <typename T, int MODE, int U>
+__device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShared<U> &sh) {
+  if (blk >= d.nblk || d.half || (d.many != 0) != (U == OWN_MANY)) return;
   // Separations and charge products: alchemical systems form them in FP64 and round once, also where
   // the pair arithmetic is FP32 (a window's dU/dlambda is a small difference of large terms).
   using R = std::conditional_t<MODE == PAIR_ALCH, double, T>;
@@ -451,7 +463,7 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
   // S waves share one owner group, each taking a contiguous part of its list
   const int S = d.split, part = wid % S;
   const int t = uniform(blk * (PAIR_WAVES / S) + wid / S);  // owner group, sorted position
-  PairWave &W = sh.w[wid];
+  PairWave<U> &W = sh.w[wid];
   double *buf = reinterpret_cast<double *>(&W);
   double x3[3] = {0.0, 0.0, 0.0};                 // S'(r) V vectors of the switched group pairs
   double ec[2] = {0.0, 0.0}, eq[2] = {0.0, 0.0};  // LJ and Coulomb energy by the neighbour's class
@@ -487,13 +499,13 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
     const int per_round = min(64, (SLOT_RING - 63) / mg);
     const bool lskip = (MODE == PAIR_ALCH || MODE == PAIR_ANY) && d.lskip_ewald != 0, plainq = !d.ewald;
     const double inv_o2 = d.inv_arsout2, inv_i2 = d.inv_arsinn2;
-    for (int u0 = 0; u0 < nI; u0 += OWN_U) {
-      const int nu = min(OWN_U, nI - u0);
-      int ot[OWN_U];  // type << ATOM_FLAG_BITS | flags
-      int xn[OWN_U], xv[OWN_U];
-      double fr[OWN_U][3];
+    for (int u0 = 0; u0 < nI; u0 += U) {
+      const int nu = min(U, nI - u0);
+      int ot[U];  // type << ATOM_FLAG_BITS | flags
+      int xn[U], xv[U];
+      double fr[U][3];
 #pragma unroll
-      for (int u = 0; u < OWN_U; ++u) {
+      for (int u = 0; u < U; ++u) {
         const int a = as0 + u0 + min(u, nu - 1);
         const AtomRec<R> r = atom_rec<R>(d, a);
         if (lane == 0) __builtin_memcpy(&W.own[u], &r, sizeof r);
@@ -627,7 +639,7 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
         auto owner_atoms = [&](auto st_tag) {
           constexpr bool ST = decltype(st_tag)::value;
 #pragma unroll
-          for (int u = 0; u < OWN_U; ++u) {
+          for (int u = 0; u < U; ++u) {
             if (u < nu) {
               const int fl = here(ot[u]);
               AtomRec<R> ra;
@@ -763,12 +775,12 @@ __device__ __forceinline__ void pairs_item(const PairDesc &d, int blk, PairShare
       // ---- this batch's owner-atom forces: value 3 u + c on lanes 8 (3 u + c) ..
       double v[8];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (h == 0 || nu >= 3) {
+      for (int h = 0; h < (3 * U + 7) / 8; ++h) {
+        if (8 * h < 3 * nu) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           const int w = 8 * h + q;
-          v[q] = w < 3 * OWN_U ? fr[w / 3 < OWN_U ? w / 3 : 0][w % 3] : 0.0;
+          v[q] = w < 3 * U ? fr[w < 3 * U ? w / 3 : 0][w % 3] : 0.0;
         }
         const double s = wave_sum8(v, buf, lane);
         const int w = 8 * h + (lane >> 3);
@@ -847,45 +859,45 @@ __device__ __forceinline__ void pairs_item_index(int h, int nitems, int nblkmax,
 
 // the item in its system's form: a plain system in a launch with alchemical ones
 // gets what it gets alone
-template <typename T, int MODE>
-__device__ __forceinline__ void pairs_form(const PairDesc &d, int blk, PairShared &sh) {
+template <typename T, int MODE, int U>
+__device__ __forceinline__ void pairs_form(const PairDesc &d, int blk, PairShared<U> &sh) {
   if constexpr (MODE == PAIR_ALCH) {
-    if (!d.alch_pair) return pairs_item<T, PAIR_ANY>(d, blk, sh);
+    if (!d.alch_pair) return pairs_item<T, PAIR_ANY, U>(d, blk, sh);
   }
-  pairs_item<T, MODE>(d, blk, sh);
+  pairs_item<T, MODE, U>(d, blk, sh);
 }
 
 // W = minimum waves per SIMD the register allocation must allow (occupancy target)
-template <typename T, int W, int MODE>
+template <typename T, int W, int MODE, int U>
 __global__ void __launch_bounds__(256, W) k_pairs(const PairDesc *__restrict__ D, int remap) {
-  __shared__ PairShared sh;
+  __shared__ PairShared<U> sh;
   int sys, blk;
   pairs_item_index(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y, gridDim.x, remap, sys, blk);
-  pairs_form<T, MODE>(D[sys], blk, sh);
+  pairs_form<T, MODE, U>(D[sys], blk, sh);
 }
 
 // Persistent form: a fixed grid (a multiple of 8 workgroups, so each keeps to
 // one XCD) walks all items of the batch with a grid stride.
-template <typename T, int W, int MODE>
+template <typename T, int W, int MODE, int U>
 __global__ void __launch_bounds__(256, W) k_pairs_persistent(const PairDesc *__restrict__ D, int remap, int nitems,
                                                              int nblkmax) {
-  __shared__ PairShared sh;
+  __shared__ PairShared<U> sh;
   for (int h = blockIdx.x; h < nitems; h += gridDim.x) {
     int sys, blk;
     pairs_item_index(h, nitems, nblkmax, remap, sys, blk);
-    pairs_form<T, MODE>(D[sys], blk, sh);
+    pairs_form<T, MODE, U>(D[sys], blk, sh);
     __syncthreads();
   }
 }
 
-template <typename T, int W, int MODE>
+template <typename T, int W, int MODE, int U>
 static void launch_pair_kernel(bool persistent, dim3 grd, int g, hipStream_t st, const PairDesc *d_desc, int remap,
                                int nitems, int max_blk) {
   const dim3 blk(64 * PAIR_WAVES);
   if (persistent)
-    hipLaunchKernelGGL((k_pairs_persistent<T, W, MODE>), dim3(g), blk, 0, st, d_desc, remap, nitems, max_blk);
+    hipLaunchKernelGGL((k_pairs_persistent<T, W, MODE, U>), dim3(g), blk, 0, st, d_desc, remap, nitems, max_blk);
   else
-    hipLaunchKernelGGL((k_pairs<T, W, MODE>), grd, blk, 0, st, d_desc, remap);
+    hipLaunchKernelGGL((k_pairs<T, W, MODE, U>), grd, blk, 0, st, d_desc, remap);
 }
 
 __global__ void __launch_bounds__(1024) k_pairs_finalize(const PairDesc *__restrict__ D) {
@@ -1394,7 +1406,8 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
   check_pairs<T>(h, nsys);
   int max_grp = 1, max_blk = 1;
   // half-list systems take the half form, the others k_pairs
-  bool any_alch = false, any_rem = false, any_other = false, any_half = false, any_full = false;
+  bool any_alch = false, any_rem = false, any_other = false, any_half = false;
+  bool any_many = false, any_few = false;
   for (int s = 0; s < nsys; ++s) {
     // every system's groups are packed and its blocks launched, whichever form serves it
     max_grp = std::max(max_grp, h[s].ngrp);
@@ -1403,7 +1416,8 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
       any_half = true;
       continue;
     }
-    any_full = true;
+    any_many = any_many || h[s].many;
+    any_few = any_few || !h[s].many;
     any_alch = any_alch || h[s].alch_pair != nullptr;
     any_rem = any_rem || h[s].rematom != nullptr;
     any_other = any_other || h[s].lskip_ewald || h[s].any_heavy || !h[s].lj_dense;
@@ -1435,23 +1449,25 @@ void launch_pairs(const PairDesc *d_desc, const PairDesc *h, int nsys, hipStream
     }
     hipLaunchKernelGGL(k_pairs_jsum, grd, dim3(64 * PAIR_WAVES), 0, st, d_desc);
   }
-  if (!any_full) {
-    // (every system in the half-list form)
-  } else if (any_alch) {
-    // the soft-core form at the default occupancy target only
-    launch_pair_kernel<T, 3, PAIR_ALCH>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
-  } else if (any_rem) {
-    if constexpr (sizeof(T) == 8)  // (check_pairs)
-      launch_pair_kernel<T, 3, PAIR_REM>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
-  } else if (any_other) {
-    launch_pair_kernel<T, 3, PAIR_ANY>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
-  } else {
-    switch (waves) {
-      case 3: launch_pair_kernel<T, 3, PAIR_PLAIN>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
-      case 4: launch_pair_kernel<T, 4, PAIR_PLAIN>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
-      default: launch_pair_kernel<T, 2, PAIR_PLAIN>(pers, grd, g, st, d_desc, remap, nitems, max_blk); break;
+  // (the soft-core, REM and general forms at one occupancy target)
+  auto full = [&](auto u) {
+    constexpr int U = decltype(u)::value, W = U == OWN_MANY ? 2 : 3;
+    if (any_alch) {
+      launch_pair_kernel<T, W, PAIR_ALCH, U>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
+    } else if (any_rem) {
+      if constexpr (sizeof(T) == 8)  // (check_pairs)
+        launch_pair_kernel<T, W, PAIR_REM, U>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
+    } else if (any_other) {
+      launch_pair_kernel<T, W, PAIR_ANY, U>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
+    } else if (U == OWN_MANY || waves < 3) {
+      launch_pair_kernel<T, 2, PAIR_PLAIN, U>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
+    } else if constexpr (U == OWN_FEW) {
+      if (waves == 3) launch_pair_kernel<T, 3, PAIR_PLAIN, U>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
+      else launch_pair_kernel<T, 4, PAIR_PLAIN, U>(pers, grd, g, st, d_desc, remap, nitems, max_blk);
     }
-  }
+  };
+  if (any_few) full(std::integral_constant<int, OWN_FEW>{});
+  if (any_many) full(std::integral_constant<int, OWN_MANY>{});
   if (kend) ORAC_HIP(hipEventRecord(kend, st));
   if (finalize) hipLaunchKernelGGL(k_pairs_finalize, dim3(PAIR_NACC, nsys), dim3(1024), 0, st, d_desc);
 }

@@ -41,6 +41,8 @@ int spread_tile_edge(int K, int order, bool smallest);
 // property of the system, never of a batch or a tuning: it fixes the
 // summation order.
 int pair_split_for(int ngrp);
+// whether a system's groups are so large that its owners take eight atoms a list walk
+int pair_many_for(int natoms, int ngrp);
 
 // ---------------------------------------------------------------- direct space
 
@@ -113,6 +115,7 @@ struct PairDesc {
   int2 *sai;                        // [natoms] {type << ATOM_FLAG_BITS | ATOM_* flags, atom}
   double *out;                      // [16]: uconf[3], ucoul[3] by typeij, st[9] row-major, dwrk
   int max_group;                    // largest group (atoms)
+  int many;                         // pair_many_for(natoms, ngrp): owner atoms a list walk takes in k_pairs
   // Alchemy (force_alchemy.f): with alch_pair set, `type` is each atom's
   // alchemical class (distinct rmin, epsm, ss_alchemy) and the pairs take the
   // soft-core form.

@@ -37,7 +37,7 @@ def _direct(ctx, s, precision, alchemy=None):
 
 @pytest.mark.parametrize("alchemical", [False, True])
 @pytest.mark.parametrize("charges", [False, True])
-@pytest.mark.parametrize("name", ["waters", "mixed", "seven_one"])
+@pytest.mark.parametrize("name", ["waters", "mixed", "seven_one", "tails"])
 def test_pair_forces_cancel(gpu_ctx, name, charges, alchemical):
     """Both sides of a pair round alike in FP32, so the direct forces sum to
     zero but for the FP64 sums (1,728 atoms of ~100 terms each: a few hundred

@@ -65,6 +65,12 @@ CASES = {
     "largest": dict(sizes=[64, 1, 3, 17]),
     "exclusions": dict(sizes=[1, 3], many_excluded=True),
     "few": dict(sizes=[3, 1], side=5, spacing=4.0),
+    # around a mean of eight atoms a group, where owners take eight atoms a list walk
+    "eight": dict(sizes=[8]),
+    "nine": dict(sizes=[9]),
+    "full": dict(sizes=[64]),
+    "tails": dict(sizes=[17, 8, 64, 3, 10, 1]),
+    "large_excluded": dict(sizes=[16, 7], many_excluded=True),
 }
 
 
@@ -87,7 +93,7 @@ def test_force_forms(gpu_ctx, name, shell):
     assert _stress_close(g["stress"], o["stress"])
 
 
-@pytest.mark.parametrize("name", ["mixed", "largest", "exclusions"])
+@pytest.mark.parametrize("name", ["mixed", "largest", "exclusions", "nine", "tails", "large_excluded"])
 def test_mixed_precision_forms(gpu_ctx, name):
     """The FP32 pair form on the same groups: forces within the mixed-precision bar of FP64."""
     from orac_hip.api import ResidentSystem
@@ -100,6 +106,62 @@ def test_mixed_precision_forms(gpu_ctx, name):
         rs.close()
     assert relrms(f[1]["f"], f[0]["f"]) < 5e-6
     assert rel(f[1]["uconf_ss"], f[0]["uconf_ss"]) < 1e-5
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_large_and_small_groups_in_one_batch(gpu_ctx, precision):
+    """Systems whose owners take three and eight atoms a list walk, and an
+    alchemical one of each, in one launch: each gets what it gets alone."""
+    from orac_hip import synth
+    from orac_hip.api import Batch, ResidentSystem
+    systems = [grouped(sizes=z, seed=k) for k, z in enumerate(([3], [9], [17, 8, 64, 3, 10, 1], [1, 2]))]
+    for alchemical in ((), (0, 2)):
+        rss = [ResidentSystem(gpu_ctx, s, precision=precision) for s in systems]
+        alone = []
+        for k, (s, rs) in enumerate(zip(systems, rss)):
+            if k in alchemical:
+                rs.set_alchemy(synth.alchemy_for(s, np.arange(40)), synth.lambda_state(0.4, lrm0=0.5))
+            rs.eval(rebuild_list=True)
+            alone.append(rs.results())
+        b = Batch(gpu_ctx, rss)
+        for persistent in (0, 1):
+            b.set_tuning(persistent=persistent)
+            b.eval(rebuild_list=True)
+            for r, a in zip(b.results(), alone):
+                assert np.array_equal(r["f"], a["f"]) and r["uconf_ss"] == a["uconf_ss"]
+                assert np.array_equal(r["stress"], a["stress"])
+        b.close()
+        for rs in rss:
+            rs.close()
+
+
+@pytest.mark.parametrize("name", ["waters", "nine", "tails"])
+def test_alchemical_forms_at_full_coupling(gpu_ctx, name):
+    """At lambda = 0 the soft core is the plain pair: the alchemical form of any
+    group size gives the plain form's forces."""
+    from orac_hip import synth
+    from orac_hip.api import ResidentSystem
+    s = grouped(**CASES[name])
+    rs = ResidentSystem(gpu_ctx, s)
+    rs.eval()
+    plain = rs.results()["f"]
+    # (mixed types by sigma and epsilon of each atom, as the system's own tables are)
+    rs.set_alchemy(synth.alchemy_for(s, np.arange(0, s.natoms, 3)), synth.lambda_state(0.0))
+    rs.eval()
+    f = rs.results()["f"]
+    rs.close()
+    assert relrms(f, plain) < F_TOL
+
+
+@pytest.mark.parametrize("name", ["mixed", "nine", "tails"])
+def test_rem_forms(gpu_ctx, name):
+    from test_gpu_rem import _check, _force_rem_gpu
+    s = grouped(**CASES[name])
+    nnlpp, fa, _ = _oracle_list(s)
+    rem = (np.random.default_rng(4).random(s.natoms) < 0.2).astype(np.int32)
+    kw = dict(rinn=3.5, rout=s.rcut, rtolinn=0.4, rtolout=s.rtol, rneigh=0.0)
+    g = _force_rem_gpu(gpu_ctx, s, nnlpp, fa, rem, 2, 0.55, **kw)
+    _check(g, O.force_rem(s, nnlpp, rem, rem_kind=2, rem_f3=0.55, fa=fa, **kw))
 
 
 def test_owner_atoms_order(gpu_ctx):
