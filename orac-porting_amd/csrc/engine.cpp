@@ -795,15 +795,19 @@ static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events
   // streams cost more than it overlapped (a fork before the centres with a
   // wait at the gather, and a third stream for the corrections: 279 against
   // 231 us for the 24,460-atom system; everything on one stream 269).
-  // The corrections go with the shorter of the two: beside the pair kernel alone
-  // (dynamics, whose list is built now and then) the reciprocal sum takes its
-  // 70 us of latencies however small the system, the pair kernel 3 us per 1,000
-  // atoms.  10 steps of 16k atoms 1,450 us with the corrections behind the
-  // reciprocal sum, 1,361 behind the pairs; of 76k atoms 2,950 and 3,065.
+  // In dynamics the corrections go behind the pair kernel, which ends before the
+  // reciprocal sum's chain of latencies in small systems and leaves the chip
+  // half empty in larger ones; behind the reciprocal sum in the largest.  A step,
+  // us, behind the pairs and behind the reciprocal sum (FP64; mixed), lists every
+  // 5 steps: 9,458 atoms 101 110; 91 99, 16,252 atoms 126 136; 115 121, 22,184
+  // atoms 154 166; 140 141, 32,842 atoms 202 214; 180 187, 53,214 atoms 300 310;
+  // 251 256, 78,722 atoms 447 453; 356 372.  With a list every step the gain is
+  // smaller (16,252 atoms 145 144; 135 128), and 78,722 atoms 479 467; 402 413
+  // set the line: below it neither schedule of the list turns the choice.
   const bool side = !events && ctx->side;
   long atoms = 0;
   for (const System *S : b.sys) atoms += S->natoms;
-  const bool corr_pairs = md_lists && atoms <= 30000;
+  const bool corr_pairs = md_lists && atoms <= 60000;
   if (side) {
     ORAC_HIP(hipEventRecord(b.fork, st));
     ORAC_HIP(hipStreamWaitEvent(ctx->side, b.fork, 0));

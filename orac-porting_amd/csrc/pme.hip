@@ -1044,6 +1044,11 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
     hipLaunchKernelGGL(k_spread<T>, dim3((unsigned)((max_work + 255) / 256), nsys), blk, 0, st, d_desc);
   }
   if (ev) ORAC_HIP(hipEventRecord(ev[1], st));
+  // Threads a plane: up to 64 x 64 two or more workgroups share a compute unit's LDS, and 512 threads
+  // let them overlap (12 systems, us with 512 and 1,024: 32^3 37 49, 48^3 68 88, 64^3 115 128 in FP64;
+  // one system 1 to 2 us the other way).  Larger planes have the unit to themselves in FP64 (80^3 235
+  // 225, 96^3 371 356); in FP32 72^3 to 96^3 still share it in a batch (12 systems of 80^3 156 181), one
+  // system not (48 45), and the single one decides.
   const dim3 pl(max_planes, nsys), bp(max_plane <= 64 * 64 ? 512 : 1024);
   if (max_planes) hipLaunchKernelGGL(k_fft_plane_r2c<T>, pl, bp, shp, st, d_desc);
   if (max_gx) {
