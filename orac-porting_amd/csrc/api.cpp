@@ -242,7 +242,7 @@ static int fft_pme_impl(orac_hip_ctx *ctx, int32_t ntap, const double *xp, const
       ndesc = 2;
     }
     PmeDesc *dd = B.put("p_desc", descs, ndesc, st, false);
-    launch_pme<double>(dd, descs, ndesc, st, ctx->tuning);
+    launch_pme<double>(dd, descs, ndesc, st);
     ORAC_HIP(hipGetLastError());
     std::vector<double> fx(ntap), fy(ntap), fz(ntap);
     double out[40];
@@ -349,7 +349,7 @@ extern "C" int orac_hip_fft_pme_noalloc(orac_hip_ctx *ctx, int32_t ntap, const d
     d.out = dout;
     pme_bins(B, "p_", d, ctx->tuning, st);  // (last: they take what room is left)
     PmeDesc *dd = B.put("p_desc", &d, 1, st, false);
-    launch_pme<double>(dd, &d, 1, st, ctx->tuning);
+    launch_pme<double>(dd, &d, 1, st);
     ORAC_HIP(hipGetLastError());
     double out[40];
     ORAC_HIP(hipMemcpyAsync(fpx, d.fx, ntap * sizeof(double), hipMemcpyDeviceToHost, st));

@@ -777,9 +777,9 @@ static void batch_enqueue(orac_hip_ctx *ctx, Batch &b, bool rebuild, bool events
   auto pme = [&](hipStream_t s) {
     const hipEvent_t *pev = events ? &b.ev[ST_P0] : nullptr;
     if (b.precision == 0)
-      launch_pme<double>(b.dp, b.hp.data(), npme, s, b.tu, pev, false, true);
+      launch_pme<double>(b.dp, b.hp.data(), npme, s, pev, false, true);
     else
-      launch_pme<float>(b.dp, b.hp.data(), npme, s, b.tu, pev, false, true);
+      launch_pme<float>(b.dp, b.hp.data(), npme, s, pev, false, true);
   };
   mark(ST_BEGIN);
   // in group order (no cell permutation) the pair kernel's records are written with the centres
@@ -983,7 +983,7 @@ static void md_partition(BufSet &B, MdDesc &d, const std::vector<int> &ufirst,
                          const std::vector<int> &bj, const std::vector<double> &bk, const std::vector<double> &br0,
                          hipStream_t st) {
   const int n = d.natoms, nu = (int)ufirst.size();
-  std::vector<int> root(n), size(n, 1), unit_of(n);
+  std::vector<int> root(n), size(n, 1);
   for (int a = 0; a < n; ++a) root[a] = a;
   auto find = [&](int a) {
     while (root[a] != a) a = root[a] = root[root[a]];
@@ -1000,10 +1000,8 @@ static void md_partition(BufSet &B, MdDesc &d, const std::vector<int> &ufirst,
   for (int t = 0; t < d.nbond; ++t) join(bi[t], bj[t]);
   std::vector<char> rigid_set(n, 0);  // (by root) terms reach a rigid unit
   for (int u = 0; u < nu; ++u)
-    for (int k = 0; k < (urigid[u] ? 3 : 1); ++k) {
-      unit_of[ufirst[u] + k] = u;
-      if (urigid[u] && goff[ufirst[u] + k + 1] > goff[ufirst[u] + k]) rigid_set[find(ufirst[u] + k)] = 1;
-    }
+    for (int k = 0; k < (urigid[u] ? 3 : 0); ++k)
+      if (goff[ufirst[u] + k + 1] > goff[ufirst[u] + k]) rigid_set[find(ufirst[u] + k)] = 1;
   std::vector<int> free_atom, rest;
   std::vector<double> free_d2;
   std::vector<std::vector<int>> sets;

@@ -32,8 +32,8 @@ template <typename T>
 // before the gather and after it (the stage timings of a profiled evaluation).
 // finalize: reduce the partial sums (else launch_tail does).
 // binned: the atoms are in their tiles' bins (launch_centres).
-void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st, const Tuning &tu,
-                const hipEvent_t *ev = nullptr, bool finalize = true, bool binned = false);
+void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st, const hipEvent_t *ev = nullptr,
+                bool finalize = true, bool binned = false);
 // tile edge of the LDS-tiled spread along an axis of K points (0: use the atomic spread)
 int spread_tile_edge(int K, int order, bool smallest);
 // Waves per owner group of the pair kernel for a system of ngrp groups (1

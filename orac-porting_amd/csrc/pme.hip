@@ -458,9 +458,6 @@ int spread_tile_edge(int K, int order, bool smallest) {
   return 0;
 }
 
-// ---------------------------------------------------------------- FFT passes
-
-// Rows along K1: fixed-point grid -> half spectrum.  TP rows per block.
 // ---------------------------------------------------------------- transforms
 
 // The transforms along K1 and K2 of one K3 plane in one workgroup, where two
@@ -571,6 +568,7 @@ __global__ void __launch_bounds__(1024) k_fft_plane_c2r(const PmeDesc *__restric
 
 constexpr int CONV_PTS = 8;  // grid points per thread of k_fft_z_conv at most
 
+// Rows along K1: fixed-point grid -> half spectrum.  TP rows per block.
 template <typename T>
 __global__ void __launch_bounds__(256) k_fft_x_r2c(const PmeDesc *__restrict__ D) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -605,19 +603,17 @@ __global__ void __launch_bounds__(256) k_fft_x_r2c(const PmeDesc *__restrict__ D
   }
 }
 
-// Complex pencils along a strided axis of the half grid: pencil p has base
-// (p % H) + (p / H) * S1 and element stride Se.
+// Complex pencils along K2 of the half grid: pencil p has base (p % H) +
+// (p / H) * H * K2 and element stride H.
 template <typename T, int S>
-__global__ void __launch_bounds__(256) k_fft_pencil(const PmeDesc *__restrict__ D, int axis) {
+__global__ void __launch_bounds__(256) k_fft_pencil(const PmeDesc *__restrict__ D) {
   extern __shared__ __align__(16) unsigned char smem[];
   const PmeDesc &d = D[blockIdx.y];
   const int H = d.K1 / 2 + 1, TP = d.tpy;
   if ((int)blockIdx.x >= d.gy || (S > 0 && d.energy_only) || use_planes<T>(d)) return;
-  const FftAxis &ax = axis == 2 ? d.ax2 : d.ax3;
-  const int N = ax.n;
-  const int npen = axis == 2 ? H * d.K3 : H * d.K2;
-  const size_t S1 = axis == 2 ? (size_t)H * d.K2 : (size_t)H;
-  const size_t Se = axis == 2 ? (size_t)H : (size_t)H * d.K2;
+  const FftAxis &ax = d.ax2;
+  const int N = ax.n, npen = H * d.K3;
+  const size_t S1 = (size_t)H * d.K2, Se = (size_t)H;
   const int p0 = blockIdx.x * TP;
   if (p0 >= npen) return;
   cx<T> *a = reinterpret_cast<cx<T> *>(smem);
@@ -989,9 +985,8 @@ void pme_set_tiles(PmeDesc &d, int lds_elems) {
 }
 
 template <typename T>
-void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st, const Tuning &tu,
-                const hipEvent_t *ev, bool finalize, bool binned) {
-  (void)tu;
+void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t st, const hipEvent_t *ev, bool finalize,
+                bool binned) {
   if (nsys <= 0) return;
   int max_atoms = 1, max_bins = 1, any_tiled = 0, any_atomic = 0, max_gx = 0, max_gy = 0, max_gz = 1, max_gg = 1;
   int max_planes = 0, max_plane = 0;
@@ -1053,12 +1048,12 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
   if (max_planes) hipLaunchKernelGGL(k_fft_plane_r2c<T>, pl, bp, shp, st, d_desc);
   if (max_gx) {
     hipLaunchKernelGGL(k_fft_x_r2c<T>, dim3(max_gx, nsys), blk, shx, st, d_desc);
-    hipLaunchKernelGGL((k_fft_pencil<T, -1>), dim3(max_gy, nsys), blk, shy, st, d_desc, 2);
+    hipLaunchKernelGGL((k_fft_pencil<T, -1>), dim3(max_gy, nsys), blk, shy, st, d_desc);
   }
   hipLaunchKernelGGL(k_fft_z_conv<T>, dim3(max_gz, nsys), blk, shz, st, d_desc);
   if (max_planes) hipLaunchKernelGGL(k_fft_plane_c2r<T>, pl, bp, shp, st, d_desc);
   if (max_gx) {
-    hipLaunchKernelGGL((k_fft_pencil<T, +1>), dim3(max_gy, nsys), blk, shy, st, d_desc, 2);
+    hipLaunchKernelGGL((k_fft_pencil<T, +1>), dim3(max_gy, nsys), blk, shy, st, d_desc);
     hipLaunchKernelGGL(k_fft_x_c2r<T>, dim3(max_gx, nsys), blk, shx, st, d_desc);
   }
   if (ev) ORAC_HIP(hipEventRecord(ev[2], st));
@@ -1072,9 +1067,7 @@ void launch_pme(const PmeDesc *d_desc, const PmeDesc *h, int nsys, hipStream_t s
   if (finalize) hipLaunchKernelGGL(k_pme_finalize, dim3(16, nsys), dim3(1024), 0, st, d_desc);
 }
 
-template void launch_pme<double>(const PmeDesc *, const PmeDesc *, int, hipStream_t, const Tuning &,
-                                 const hipEvent_t *, bool, bool);
-template void launch_pme<float>(const PmeDesc *, const PmeDesc *, int, hipStream_t, const Tuning &,
-                                const hipEvent_t *, bool, bool);
+template void launch_pme<double>(const PmeDesc *, const PmeDesc *, int, hipStream_t, const hipEvent_t *, bool, bool);
+template void launch_pme<float>(const PmeDesc *, const PmeDesc *, int, hipStream_t, const hipEvent_t *, bool, bool);
 
 }  // namespace orac

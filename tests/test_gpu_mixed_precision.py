@@ -84,24 +84,29 @@ def test_reciprocal_forces_fp32(gpu_ctx, K, bound):
     assert np.mean(err) < bound
 
 
+@pytest.mark.parametrize("beside", ["alchemical", "two_shells"])
 @pytest.mark.parametrize("order", [0, 1])
-def test_plain_system_beside_an_alchemical_one(gpu_ctx, order):
-    """A plain system gets, in a launch with alchemical ones, what it gets alone."""
+def test_plain_system_beside_another(gpu_ctx, order, beside):
+    """A plain system gets, in a launch with alchemical ones or with outer shells
+    that skip the Ewald term, what it gets alone; so does the other."""
     from orac_hip.api import Batch, ResidentSystem
     for precision in (0, 1):
         s, a = grouped(sizes=[1, 3, 2]), grouped(sizes=[3], seed=5)
         rss = [ResidentSystem(gpu_ctx, x, precision=precision) for x in ([s, a] if order == 0 else [a, s])]
-        k = rss[order]
+        k, other = rss[order], rss[1 - order]
         k.eval(rebuild_list=True)
         alone = k.results()
-        rss[1 - order].set_alchemy(*_removed(a))
-        rss[1 - order].eval(rebuild_list=True)
-        window = rss[1 - order].results()
+        if beside == "alchemical":
+            other.set_alchemy(*_removed(a))
+        else:
+            other.set_shells(4.5, 0.5)
+        other.eval(rebuild_list=True)
+        want = other.results()
         b = Batch(gpu_ctx, rss)
         b.eval(rebuild_list=True)
         r = b.results()
         assert np.array_equal(r[order]["f"], alone["f"]) and r[order]["uconf_ss"] == alone["uconf_ss"]
-        assert np.array_equal(r[1 - order]["f"], window["f"])
+        assert np.array_equal(r[1 - order]["f"], want["f"])
         b.close()
         for rs in rss:
             rs.close()
