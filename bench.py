@@ -40,10 +40,10 @@ FP64_PEAK_TFLOPS = 78.6
 FP32_PEAK_TFLOPS = 157.3
 HBM_PEAK_GBS = 8000.0
 FLOP_PER_PAIR = 89
-# HBM bytes per launch of k_pairs<double, 4, 0> on the 24,460-atom system, from the
+# HBM bytes per launch of k_pairs<double, 4, 0, 3> on the 24,460-atom system, from the
 # committed FETCH_SIZE / WRITE_SIZE profile (rocprof_summary traffic)
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "bytes_k_pairs_fp64_solvated24k.txt")
-PAIR_KERNEL = "k_pairs<double, 4, 0>"
+PAIR_KERNEL = "k_pairs<double, 4, 0, 3>"
 
 
 def pme_stage_roofline(s, stages, fp64):

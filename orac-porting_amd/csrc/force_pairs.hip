@@ -335,7 +335,7 @@ constexpr int PAIR_NACC = 16;      // energies and virial of a block: uconf[3], 
 //
 // The lanes of a wavefront take the atoms of the owner's in-shell neighbour
 // groups, one atom each, and loop over the owner group's atoms, whose records
-// are the same across the wavefront and sit in SGPRs: a pair costs three
+// are the same across the wavefront and sit in LDS: a pair costs a few
 // additions before its distance and reads no memory but its LJ entry, and a
 // neighbour atom's record is read once for all owner atoms.  The list entries
 // are classified 64 at a time; a kept entry's Cartesian group separation,
@@ -359,9 +359,13 @@ constexpr int PAIR_NACC = 16;      // energies and virial of a block: uconf[3], 
 //  * the 64-lane sums go through LDS eight values at a time (8 writes, 8 reads
 //    per lane and three exchanges for eight sums).
 // Measured on the 24,460-atom system (11.9 M pair evaluations from both sides):
-// 86 us in FP64 and 79 us in FP32, against 182 and 151 us with lanes on (owner
-// atom, neighbour group) that recomputed the group geometry per lane; 26 M
-// vector instructions against 43 M.  16 systems in one launch: 56 us each (FP32).
+// 85 us in FP64 and 78 us in FP32, against 182 and 155 us with lanes on (owner
+// atom, neighbour group) that recomputed the group geometry per lane; 27 M
+// vector instructions (26 M in FP32) against 43 M.  16 systems in one launch:
+// 58 us each (FP32).  FP32 separations from a rounded centre separation that
+// differed between a pair's two sides took 2.5% less at 103,000 atoms (236 us,
+// now 242), but the two forces of a pair did not cancel, and what they left
+// made the virial's error 1.6e-7 for 0.5e-7 (24,460 atoms; 2.4 for 1.2 at 103,000).
 
 constexpr int ENT_RING = 128;   // entries kept: at most 63 with atoms waiting + 64 new ones
 constexpr int SLOT_RING = 256;  // lane slots: at most 63 waiting + one round's atoms
@@ -1351,11 +1355,11 @@ int pair_split_for(int ngrp) {
   const int v = e ? atoi(e) : 0;
   if (v == 1 || v == 2 || v == 4) return v;
   (void)ngrp;
-  return 1;  // measured: extra waves per owner cost more than the tail they trim
+  return 1;  // extra waves per owner cost more than the tail they trim (24,460 atoms, 2: 92 us for 82)
 }
 
 // Occupancy target of k_pairs (plain form): on the 24.5k-atom system 4 waves
-// per SIMD take 86 us in FP64 (3 registers spilled) and 3 take 96; FP32 fits
+// per SIMD take 85 us in FP64 (4 registers spilled) and 3 take 96; FP32 fits
 // 4.  The tuning value, then ORAC_HIP_PAIR_WAVES=2|3|4, override it.
 template <typename T>
 static int pair_occupancy(int tuned) {
@@ -1374,7 +1378,7 @@ static int pair_occupancy(int tuned) {
 // Measured on MI355X on the 24,460-atom system (one evaluation with a list
 // rebuild): the half-list form's per-pair slots and its list build (split,
 // reverse ranking, mirror search) cost more than the halved arithmetic saves
-// (0.454 vs 0.346 ms in FP64).
+// (0.473 vs 0.192 ms in FP64, 0.390 vs 0.181 in FP32).
 bool use_owner_kernel() {
   const char *e = getenv("ORAC_HIP_PAIR_KERNEL");
   return e && std::string(e) == "own";
