@@ -371,9 +371,18 @@ PmeDesc pme_desc_base(BufSet &B, const std::string &pfx, const PmePlan &P, int n
   d.Qfix = B.get<unsigned long long>(pfx + "Qfix", G);
   d.FQ = fp64 ? (void *)B.get<double2>(pfx + "FQ", Gc) : (void *)B.get<float2>(pfx + "FQ32", Gc);
   d.Qr = fp64 ? (void *)B.get<double>(pfx + "Qr", G) : (void *)B.get<float>(pfx + "Qr32", G);
-  d.bsp1 = B.put_vec(pfx + "bsp1", P.bsp[0], st, true);
-  d.bsp2 = B.put_vec(pfx + "bsp2", P.bsp[1], st, true);
-  d.bsp3 = B.put_vec(pfx + "bsp3", P.bsp[2], st, true);
+  // FP32 weights carry the rounding of their recurrence's factors 1/3, 1/5, ..., alike in every weight of an
+  // axis (order 5: 3e-8 more charge).  The moduli are those of the rounded weights, so the sum does not: its
+  // energy was 1.8e-7 too large at order 5 and 7.5e-7 at 8, its forces half of that
+  double gain = 1.0;
+  if (!fp64)
+    for (int k = 3; k <= P.order; ++k) gain *= (double)recip_km1<float>(k) * (k - 1);
+  const double **const bsp[3] = {&d.bsp1, &d.bsp2, &d.bsp3};
+  for (int a = 0; a < 3; ++a) {
+    std::vector<double> m = P.bsp[a];
+    for (double &v : m) v *= gain * gain;
+    *bsp[a] = B.put_vec(pfx + "bsp" + std::to_string(a + 1), m, st, true);
+  }
   d.ax1 = P.ax[0];
   d.ax2 = P.ax[1];
   d.ax3 = P.ax[2];

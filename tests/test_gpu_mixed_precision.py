@@ -84,6 +84,28 @@ def test_reciprocal_forces_fp32(gpu_ctx, K, bound):
     assert np.mean(err) < bound
 
 
+def _reciprocal_energy(ctx, K, order):
+    """Relative error of the FP32 reciprocal energy, mean of eight systems."""
+    err = []
+    for seed in range(8):
+        s = grouped(sizes=[1], side=12, spacing=K / 12.0, seed=seed)
+        s = dataclasses.replace(s, nfft=(K, K, K), order=order, rcut=0.3, rtol=0.01, rnei=0.01, ecc12=0 * s.ecc12,
+                                ecc6=0 * s.ecc6)
+        g, m = _eval(ctx, s, 0), _eval(ctx, s, 1)
+        err.append((m["eer"] - g["eer"]) / abs(g["eer"]))
+    print("reciprocal energy", K, order, np.mean(err), err)
+    return np.mean(err)
+
+
+@pytest.mark.parametrize("order", [4, 5, 6, 7, 8])
+def test_reciprocal_energy_has_the_splines_charge(gpu_ctx, order):
+    """The factors 1/3, 1/5, ... of the splines' recurrence, rounded, scale every
+    weight of an axis alike, and the energy by their sixth power (order 5: 1.8e-7;
+    6: 2.7e-7): the moduli take it out.  What is left is below two roundings, 1.2e-7
+    (3.5e-8 to 4.3e-8 measured; 2.1e-7 to 7.6e-7 with the exact splines' moduli)."""
+    assert abs(_reciprocal_energy(gpu_ctx, 40, order)) < 2.0 ** -23
+
+
 @pytest.mark.parametrize("beside", ["alchemical", "two_shells"])
 @pytest.mark.parametrize("order", [0, 1])
 def test_plain_system_beside_another(gpu_ctx, order, beside):
