@@ -318,6 +318,37 @@ void pme_tiling(PmeDesc &d, bool smallest) {
   if (d.bin_slots > 0) d.bin_cap = (int)std::min<double>(d.bin_cap, std::floor(d.bin_slots / nbin));
 }
 
+// How much larger each mode of an axis is than it should be, by the rounding
+// to FP32 of the transform's constants (sqrt(3/4) in radix 3, ...) and twiddle
+// factors: the mean over a mode's inputs, pass by pass, to first order.  Mode k
+// of radix R after passes of product Ns takes input r with the twiddle r (k mod
+// Ns) / (Ns R) and row q = k / Ns mod R of the radix's own matrix.
+static std::vector<double> fft_gain_f32(const FftAxis &ax) {
+  const double pi = 3.14159265358979323846;
+  // (a rounded unit vector along the exact one, less 1)
+  auto unit = [&](int m, int n) {
+    const double c = cos(2.0 * pi * m / n), s = sin(2.0 * pi * m / n);
+    return ((double)(float)c - c) * c + ((double)(float)s - s) * s;
+  };
+  std::vector<double> g(ax.n, 1.0);
+  int Ns = 1;
+  for (int p = 0; p < ax.nr; ++p) {
+    const int R = ax.radix[p];
+    double own = 0.0;  // mean over the inputs of a row that has the constants
+    for (int t = 1; t < R; ++t) own += R == 3 || R == 5 ? unit(t, R) / R : 0.0;
+    if (R == 6) own = 2.0 / 3.0 * unit(1, 3);  // (a radix-3 step without twiddles)
+    if (R == 8) own = 0.5 * unit(1, 8);        // (odd inputs of odd rows)
+    for (int k = 0; k < ax.n; ++k) {
+      const int q = k / Ns % R;
+      double e = q % (R == 6 ? 3 : R == 8 ? 2 : R) ? own : 0.0;
+      for (int t = 1; t < R; ++t) e += unit(t * (k % Ns) % (Ns * R), Ns * R) / R;
+      g[k] *= 1.0 + e;
+    }
+    Ns *= R;
+  }
+  return g;
+}
+
 // The spread's bins, when every axis has a tile edge in [order - 1, 8] dividing
 // K: sized for the largest and the smallest tiles, which a tuning may ask for.
 // In an arena, of which they take the last pieces, sized for the tiling in use
@@ -373,14 +404,18 @@ PmeDesc pme_desc_base(BufSet &B, const std::string &pfx, const PmePlan &P, int n
   d.Qr = fp64 ? (void *)B.get<double>(pfx + "Qr", G) : (void *)B.get<float>(pfx + "Qr32", G);
   // FP32 weights carry the rounding of their recurrence's factors 1/3, 1/5, ..., alike in every weight of an
   // axis (order 5: 3e-8 more charge).  The moduli are those of the rounded weights, so the sum does not: its
-  // energy was 1.8e-7 too large at order 5 and 7.5e-7 at 8, its forces half of that
+  // energy was 1.8e-7 too large at order 5 and 7.5e-7 at 8.  The transforms' own gain, up to 1.0e-7 of the
+  // energy, goes the same way; what is left of the bias is 0.1e-7 (mean of 12 grids of 20 to 96 points)
   double gain = 1.0;
   if (!fp64)
     for (int k = 3; k <= P.order; ++k) gain *= (double)recip_km1<float>(k) * (k - 1);
   const double **const bsp[3] = {&d.bsp1, &d.bsp2, &d.bsp3};
   for (int a = 0; a < 3; ++a) {
     std::vector<double> m = P.bsp[a];
-    for (double &v : m) v *= gain * gain;
+    if (!fp64) {
+      const std::vector<double> g = fft_gain_f32(P.ax[a]);
+      for (size_t k = 0; k < m.size(); ++k) m[k] *= gain * gain * g[k] * g[k];
+    }
     *bsp[a] = B.put_vec(pfx + "bsp" + std::to_string(a + 1), m, st, true);
   }
   d.ax1 = P.ax[0];

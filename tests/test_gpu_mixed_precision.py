@@ -71,7 +71,8 @@ def test_lj_energy_has_no_bias(gpu_ctx):
 def test_reciprocal_forces_fp32(gpu_ctx, K, bound):
     """FP32 splines and transforms, mean of eight systems (every sum of a run is
     in fixed order).  The bounds lie between the error with the splines' sums
-    fused and no twiddles inside radix 6 (5.07e-7, 7.34e-7) and with each product
+    fused and no twiddles inside radix 6 (5.07e-7, 7.34e-7; 4.95e-7, 7.28e-7 with
+    the moduli of the rounded splines and transforms) and with each product
     rounded and radix 6 as 2 x 3 (5.39e-7, 7.75e-7)."""
     err = []
     for seed in range(8):
@@ -102,8 +103,19 @@ def test_reciprocal_energy_has_the_splines_charge(gpu_ctx, order):
     """The factors 1/3, 1/5, ... of the splines' recurrence, rounded, scale every
     weight of an axis alike, and the energy by their sixth power (order 5: 1.8e-7;
     6: 2.7e-7): the moduli take it out.  What is left is below two roundings, 1.2e-7
-    (3.5e-8 to 4.3e-8 measured; 2.1e-7 to 7.6e-7 with the exact splines' moduli)."""
+    (3.5e-8 to 4.3e-8 measured; 2.1e-7 to 7.6e-7 with the exact splines' moduli; 0.4e-8
+    to 1.2e-8 where the transforms' gain is taken out too)."""
     assert abs(_reciprocal_energy(gpu_ctx, 40, order)) < 2.0 ** -23
+
+
+@pytest.mark.parametrize("K", [24, 32, 36, 48, 54, 72, 80, 96])
+def test_reciprocal_energy_fp32(gpu_ctx, K):
+    """Grids of every radix: the rounding of the transforms' constants (sqrt(3/4),
+    cos(2 pi / 5), ...) and twiddle factors scales a mode, and the moduli carry
+    that.  The mean error is at most 3.6e-8 (a system's deviation of 1 to 3e-8 is
+    the rounding of the arithmetic), and 7.6e-8 to 1.0e-7 without; the bound is one
+    rounding, 2^-24."""
+    assert abs(_reciprocal_energy(gpu_ctx, K, 5)) < 2.0 ** -24
 
 
 @pytest.mark.parametrize("beside", ["alchemical", "two_shells"])
